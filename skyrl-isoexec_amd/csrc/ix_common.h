@@ -126,10 +126,42 @@ __device__ __forceinline__ float ix_xor_lane(float v) {
     return __shfl_xor(v, S, IX_WAVE);
   }
 }
+// The value of the partner group (lane ^ S) inside a tree or a maximum, where every lane of a group of S already holds
+// the same value, so that ANY lane of the partner group will do: distance 4 is then the mirror inside a half row (one
+// lane control on the add itself instead of two rotates and a select), and 16 and 32 are the row and half-wave swaps of
+// the vector ALU instead of a trip through the LDS crossbar.
+template <int S>
+__device__ __forceinline__ float ix_partner(float v) {
+  if constexpr (S == 4) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x141, 0xF, 0xF, true));  // row_half_mirror
+  } else {
+    return ix_xor_lane<S>(v);
+  }
+}
+// (own, partner) of distance 16 or 32, in the order the swap leaves them: for operations that commute.
+template <int S>
+__device__ __forceinline__ void ix_swap_pair(float v, float& a, float& b) {
+  const uint32_t u = __float_as_uint(v);
+  if constexpr (S == 16) {
+    const auto r = __builtin_amdgcn_permlane16_swap(u, u, false, false);
+    a = __uint_as_float(r[0]);
+    b = __uint_as_float(r[1]);
+  } else {
+    const auto r = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+    a = __uint_as_float(r[0]);
+    b = __uint_as_float(r[1]);
+  }
+}
 template <int L, int S = 1>
 __device__ __forceinline__ float ix_lane_tree(float v) {
   if constexpr (S < L) {
-    v = v + ix_xor_lane<S>(v);
+    if constexpr (S >= 16) {
+      float a, b;
+      ix_swap_pair<S>(v, a, b);
+      v = a + b;
+    } else {
+      v = v + ix_partner<S>(v);
+    }
     return ix_lane_tree<L, S * 2>(v);
   } else {
     return v;
@@ -138,7 +170,13 @@ __device__ __forceinline__ float ix_lane_tree(float v) {
 template <int L, int S = 1>
 __device__ __forceinline__ float ix_lane_max(float v) {
   if constexpr (S < L) {
-    v = fmaxf(v, ix_xor_lane<S>(v));
+    if constexpr (S >= 16) {
+      float a, b;
+      ix_swap_pair<S>(v, a, b);
+      v = fmaxf(a, b);
+    } else {
+      v = fmaxf(v, ix_partner<S>(v));
+    }
     return ix_lane_max<L, S * 2>(v);
   } else {
     return v;

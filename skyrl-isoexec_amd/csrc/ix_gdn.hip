@@ -213,7 +213,26 @@ __global__ __launch_bounds__(256) void k_gdn_scan(const TIO* __restrict__ q, con
 // for bit, and which one runs is a staging choice like the time tile. What changes is the cost: 15 of the 16 tree
 // adds per dot product no longer cross lanes, and a wave instruction serves 32 rows with 64 elements each instead
 // of 4 rows x RPL with 8: about 9.4 instead of 11.3 vector instructions per row and token.
-// Compact state form only (one pool row per sequence, stored after the last token).
+// Compact state form only (one pool row per sequence, stored after the last token; without a pool the sequences start
+// from zero and nothing is stored).
+#define IX_GDN_SORT_MAX 256  // sequences a workgroup ranks by length
+// The sequence of rank `n` when sequences are taken longest first (ties in packed order), so that the long ones do not
+// start last: every workgroup of a launch over 2..IX_GDN_SORT_MAX sequences ranks them itself, one per thread. `lens`:
+// IX_GDN_SORT_MAX + 1 ints of LDS, free again on return.
+__device__ __forceinline__ int ix_gdn_nth_longest(const int* __restrict__ cu, int N, int n, int* lens) {
+  if (N < 2 || N > IX_GDN_SORT_MAX) return n;
+  const int tid = threadIdx.x;
+  const int mine = tid < N ? cu[tid + 1] - cu[tid] : 0;
+  if (tid < N) lens[tid] = mine;
+  __syncthreads();
+  int rank = 0;
+  for (int j = 0; j < N; ++j) rank += (lens[j] > mine || (lens[j] == mine && j < tid)) ? 1 : 0;
+  if (tid < N && rank == n) lens[IX_GDN_SORT_MAX] = tid;
+  __syncthreads();
+  const int r = lens[IX_GDN_SORT_MAX];
+  __syncthreads();
+  return r;
+}
 __device__ __forceinline__ float ix_add_halves(float v) {
   const uint32_t u = __float_as_uint(v);
   const auto r = __builtin_amdgcn_permlane32_swap(u, u, false, false);
@@ -225,7 +244,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3)))
 void k_gdn_scan_pairs(const TIO* __restrict__ q, const TIO* __restrict__ k, const TIO* __restrict__ v,
                       const float* __restrict__ g, const TIO* __restrict__ beta, TIO* __restrict__ o,
                       float* __restrict__ state, const int* __restrict__ cu, const int* __restrict__ sidx,
-                      long q_pitch, long k_pitch, long v_pitch, int H, int HV, int V, float scale, int TT,
+                      long q_pitch, long k_pitch, long v_pitch, int N, int H, int HV, int V, float scale, int TT,
                       const bf16_t* __restrict__ gate, long gate_stride_t, const bf16_t* __restrict__ norm_w,
                       float norm_eps, int zero_centered) {
   constexpr int K = 128;
@@ -243,7 +262,7 @@ void k_gdn_scan_pairs(const TIO* __restrict__ q, const TIO* __restrict__ k, cons
   const int vb = (int)(bid % VB);
   bid /= VB;
   const int hv = (int)(bid % HV);
-  const int n = (int)(bid / HV);
+  const int n = ix_gdn_nth_longest(cu, N, (int)(bid / HV), reinterpret_cast<int*>(ix_lds));
   const int h = hv / (HV / H);
   const int tid = threadIdx.x;
   const int lane = tid & 63, wave = tid >> 6;
@@ -254,7 +273,7 @@ void k_gdn_scan_pairs(const TIO* __restrict__ q, const TIO* __restrict__ k, cons
   const int t_begin = cu[n], t_end = cu[n + 1];
   const int len = t_end - t_begin;
   if (len <= 0) return;
-  const int row0 = sidx[n];
+  const int row0 = sidx ? sidx[n] : 1;
   // What leaves for the nt tokens of the tile at t0 whose outputs stand in `of`: the outputs themselves, or, with a gate,
   // the layer's gated output norm of them (ix_gated_out_norm: RMSNorm over the head's V = 128 values, bf16(1 + w),
   // silu(gate)) instead of a launch that reads them back. A token's head is sixteen consecutive threads of eight
@@ -318,7 +337,7 @@ void k_gdn_scan_pairs(const TIO* __restrict__ q, const TIO* __restrict__ k, cons
   float* srow = state + (((long)row0 * HV + hv) * V + vrow) * K + 64 * hf;
 #pragma unroll
   for (int c = 0; c < 16; ++c) {
-    const float4 a = *reinterpret_cast<const float4*>(srow + 4 * c);
+    const float4 a = state ? *reinterpret_cast<const float4*>(srow + 4 * c) : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
     S[4 * c] = a.x; S[4 * c + 1] = a.y; S[4 * c + 2] = a.z; S[4 * c + 3] = a.w;
   }
 
@@ -402,7 +421,7 @@ void k_gdn_scan_pairs(const TIO* __restrict__ q, const TIO* __restrict__ k, cons
       const float ov = ix_add_halves(ix_tree8(part));
       if (hf == 0) of[tt * R + r] = ov;
     }
-    if (t0 + nt == len) {
+    if (state && t0 + nt == len) {
 #pragma unroll
       for (int c = 0; c < 16; ++c)
         *reinterpret_cast<float4*>(srow + 4 * c) = make_float4(S[4 * c], S[4 * c + 1], S[4 * c + 2], S[4 * c + 3]);
@@ -410,6 +429,345 @@ void k_gdn_scan_pairs(const TIO* __restrict__ q, const TIO* __restrict__ k, cons
     __syncthreads();
     if (o) emit(t0, nt);
   }
+}
+
+// ---- prefill of few sequences: the walk ---------------------------------------------------------------------
+// One sequence has HV * V row recurrences and a token's step is a chain through each of them (decay, multiply-adds, tree,
+// update): with few sequences the time is tokens x the latency of that chain, and with some more the vector issue of the
+// waves that share a SIMD. So the layout is the sixteen-lane one (one sequence of HV = 32, V = 128 heads is then
+// exactly one wave per SIMD), and everything that is not the chain is kept out of its way:
+//   * tiles of 16 tokens, staged twice in LDS: the next tile's global loads are issued before this tile's tokens and
+//     written to LDS after them; one barrier per tile;
+//   * no LDS store between a tile's tokens (an LDS load may not pass one): a token's output is the same in all lanes of
+//     its row, so lane tt keeps token tt's and the tile is written out at its end;
+//   * sixteen tokens of straight-line code, so the output's tree runs in the shadow of the next token's decay and dot.
+// The statements per token are ix_gdn_step's: same bits as k_gdn_scan and k_gdn_scan_pairs.
+// Sequences are taken longest first when there are 2..256 of them (ranked by every workgroup from cu), and a sequence's
+// workgroups are spread over all XCDs with the row blocks of a key head on one of them.
+// CPR: the boundary form (gdn_cpr.py:296-319). Two states walk together: the fp32 chain, and the running state, which
+// restarts from the chain rounded to the io type at every multiple of `chunk` tokens and makes the outputs. The pass that
+// first computes every boundary state, its pool, and the second pass over all tokens are then not there at all.
+// Measured (HV = 32, V = K = 128, bf16), k_gdn_scan / walk: one sequence of 8192 tokens 1990 / 1129 us (138 ns a token;
+// vector issue alone would be 75), five of 33..1203 tokens 883 / 247, 8 x 1000 1330 / 667; boundary form of nine sequences
+// of 120..1500 tokens, boundary pass + segmented scan / walk: 3900 / 975. With first and second halves of the 8-element
+// slices apart in LDS a 16-byte read of sixteen lanes is one contiguous row (8 x 1000: 714 -> 667).
+template <typename TIO>
+struct IxRaw8 {
+  uint4 u;
+  __device__ __forceinline__ void load(const TIO* p) { u = *reinterpret_cast<const uint4*>(p); }
+  __device__ __forceinline__ void get(float (&o)[8]) const { ix_unpack8(u, o); }
+};
+template <>
+struct IxRaw8<float> {
+  float4 a, b;
+  __device__ __forceinline__ void load(const float* p) {
+    a = *reinterpret_cast<const float4*>(p);
+    b = *reinterpret_cast<const float4*>(p + 4);
+  }
+  __device__ __forceinline__ void get(float (&o)[8]) const {
+    o[0] = a.x; o[1] = a.y; o[2] = a.z; o[3] = a.w; o[4] = b.x; o[5] = b.y; o[6] = b.z; o[7] = b.w;
+  }
+};
+__device__ __forceinline__ float ix_wire(float x, const bf16_t*) { return ix_rbf(x); }
+__device__ __forceinline__ float ix_wire(float x, const float*) { return x; }
+
+
+template <int KS, int RPL, typename TIO, bool CPR>
+__global__ __launch_bounds__(256) void k_gdn_walk(const TIO* __restrict__ q, const TIO* __restrict__ k,
+                                                  const TIO* __restrict__ v, const float* __restrict__ g,
+                                                  const TIO* __restrict__ beta, TIO* __restrict__ o,
+                                                  float* __restrict__ state, const int* __restrict__ cu,
+                                                  const int* __restrict__ sidx, long q_pitch, long k_pitch,
+                                                  long v_pitch, int N, int H, int HV, int V, float scale, int chunk) {
+  constexpr int T = KS == 32 ? 8 : 16;  // tokens per tile (K = 256: half as many, for the LDS)
+  constexpr int K = KS * 8;
+  constexpr int RW = 256 / KS;
+  constexpr int R = RW * RPL;
+  constexpr int QK = 2 * T * KS;                 // 8-element groups of k and q in a tile
+  constexpr int QC = (QK + 255) / 256;           // groups per thread
+  constexpr int VC = (T * R + 255) / 256;        // v elements per thread
+  constexpr int NK = (T + KS - 1) / KS;          // tokens a lane keeps the output of
+  __shared__ __align__(16) float kq[2][2][T][K];  // [buffer][k, q * scale][token]
+  __shared__ float vf[2][T][R];
+  __shared__ float of[2][T][R];
+  __shared__ float2 eb[2][T];                    // exp(g), beta
+
+  const int VB = V / R;
+  const int per_seq = HV * VB;
+  const int tid = threadIdx.x;
+  int n, w;
+  {
+    const unsigned bid = blockIdx.x;
+    if ((per_seq & 7) == 0) {  // hardware deals consecutive ids to the XCDs round-robin
+      const unsigned per8 = (unsigned)per_seq >> 3;
+      n = (int)((bid >> 3) / per8);
+      w = (int)((bid & 7u) * per8 + (bid >> 3) % per8);
+    } else {
+      n = (int)(bid / (unsigned)per_seq);
+      w = (int)(bid % (unsigned)per_seq);
+    }
+  }
+  static_assert(sizeof(kq) >= (IX_GDN_SORT_MAX + 1) * sizeof(int), "the ranking uses the staging buffer");
+  n = ix_gdn_nth_longest(cu, N, n, reinterpret_cast<int*>(&kq[0][0][0][0]));
+  const int vb = w % VB;
+  const int hv = w / VB;
+  const int h = hv / (HV / H);
+  const int sub = tid % KS, r = tid / KS;
+  const int t_begin = cu[n];
+  const int len = cu[n + 1] - t_begin;
+  if (len <= 0) return;
+  const int row0 = sidx ? sidx[n] : 1;
+  TIO* ob = o + (long)hv * V + vb * R;
+  if (row0 <= 0) {  // null lane: no state, outputs defined as zero
+    for (int i = tid; i < len * R; i += 256) ix_st(ob + (long)(t_begin + i / R) * HV * V + i % R, 0.0f);
+    return;
+  }
+
+  float S[RPL][8], C[CPR ? RPL : 1][8];
+#pragma unroll
+  for (int j = 0; j < RPL; ++j) {
+    if (state) {
+      const float* sp = state + (((long)row0 * HV + hv) * V + vb * R + r + j * RW) * K + sub * 8;
+      const float4 a = *reinterpret_cast<const float4*>(sp);
+      const float4 b = *reinterpret_cast<const float4*>(sp + 4);
+      S[j][0] = a.x; S[j][1] = a.y; S[j][2] = a.z; S[j][3] = a.w;
+      S[j][4] = b.x; S[j][5] = b.y; S[j][6] = b.z; S[j][7] = b.w;
+    } else {
+#pragma unroll
+      for (int i = 0; i < 8; ++i) S[j][i] = 0.0f;
+    }
+    if constexpr (CPR) {
+#pragma unroll
+      for (int i = 0; i < 8; ++i) C[j][i] = S[j][i];
+    }
+  }
+
+  IxRaw8<TIO> rq[QC];
+  // raw, as loaded: a conversion here would wait for the loads that the tile's tokens are meant to cover
+  TIO rv[VC], rb = 0;
+  float rg = 0.0f;
+  auto fetch = [&](int t0) __attribute__((always_inline)) {  // tokens past the end read the last one's values, unused
+#pragma unroll
+    for (int c = 0; c < QC; ++c) {
+      const int i = tid + 256 * c;
+      if (QK % 256 == 0 || i < QK) {
+        const int e = i % (T * KS), isq = i / (T * KS);
+        const long tok = t_begin + min(t0 + e / KS, len - 1);
+        rq[c].load((isq ? q + tok * q_pitch : k + tok * k_pitch) + h * K + (e % KS) * 8);
+      }
+    }
+#pragma unroll
+    for (int c = 0; c < VC; ++c) {
+      const int i = tid + 256 * c;
+      if ((T * R) % 256 == 0 || i < T * R) {
+        const long tok = t_begin + min(t0 + i / R, len - 1);
+        rv[c] = v[tok * v_pitch + (long)hv * V + vb * R + i % R];
+      }
+    }
+    if (tid < T) {
+      const long tok = t_begin + min(t0 + tid, len - 1);
+      rg = g[tok * HV + hv];
+      rb = beta[tok * HV + hv];
+    }
+  };
+  auto commit = [&](int b) __attribute__((always_inline)) {
+#pragma unroll
+    for (int c = 0; c < QC; ++c) {
+      const int i = tid + 256 * c;
+      if (QK % 256 == 0 || i < QK) {
+        const int e = i % (T * KS), isq = i / (T * KS);
+        float x[8];
+        rq[c].get(x);
+        const float m = isq ? scale : 1.0f;  // k * 1 is k
+        float* d = &kq[b][isq][e / KS][(e % KS) * 4];  // first halves of all slices, then second halves
+        *reinterpret_cast<float4*>(d) = make_float4(x[0] * m, x[1] * m, x[2] * m, x[3] * m);
+        *reinterpret_cast<float4*>(d + K / 2) = make_float4(x[4] * m, x[5] * m, x[6] * m, x[7] * m);
+      }
+    }
+#pragma unroll
+    for (int c = 0; c < VC; ++c) {
+      const int i = tid + 256 * c;
+      if ((T * R) % 256 == 0 || i < T * R) vf[b][i / R][i % R] = ix_ld(&rv[c]);
+    }
+    if (tid < T) eb[b][tid] = make_float2(ix_exp(rg), ix_ld(&rb));
+  };
+  auto emit = [&](int t0, int nt, int b) __attribute__((always_inline)) {
+#pragma unroll
+    for (int c = 0; c < VC; ++c) {
+      const int i = tid + 256 * c;
+      if (i < nt * R) ix_st(ob + (long)(t_begin + t0 + i / R) * HV * V + i % R, of[b][i / R][i % R]);
+    }
+  };
+  auto token = [&](int b, int tt, float (&ov)[RPL]) __attribute__((always_inline)) {
+    float kk[8], qs[8];
+    {
+      const float4 a = *reinterpret_cast<const float4*>(&kq[b][0][tt][sub * 4]);
+      const float4 c = *reinterpret_cast<const float4*>(&kq[b][0][tt][K / 2 + sub * 4]);
+      kk[0] = a.x; kk[1] = a.y; kk[2] = a.z; kk[3] = a.w; kk[4] = c.x; kk[5] = c.y; kk[6] = c.z; kk[7] = c.w;
+      const float4 d = *reinterpret_cast<const float4*>(&kq[b][1][tt][sub * 4]);
+      const float4 e = *reinterpret_cast<const float4*>(&kq[b][1][tt][K / 2 + sub * 4]);
+      qs[0] = d.x; qs[1] = d.y; qs[2] = d.z; qs[3] = d.w; qs[4] = e.x; qs[5] = e.y; qs[6] = e.z; qs[7] = e.w;
+    }
+    const float2 gb = eb[b][tt];
+#pragma unroll
+    for (int j = 0; j < RPL; ++j) {
+      const float vv = vf[b][tt][j * RW + r];
+      if constexpr (CPR) {  // ix_gdn_step without its output, on the chain
+#pragma unroll
+        for (int i = 0; i < 8; ++i) C[j][i] = C[j][i] * gb.x;
+        const float kv = ix_lane_tree<KS>(ix_dot8(C[j], kk));
+        const float d = (vv - kv) * gb.y;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) C[j][i] = __builtin_fmaf(d, kk[i], C[j][i]);
+      }
+      ov[j] = ix_gdn_step<KS>(S[j], kk, qs, vv, gb.x, gb.y);
+    }
+  };
+
+  fetch(0);
+  commit(0);
+  __syncthreads();
+  int b = 0;
+  for (int t0 = 0; t0 < len; t0 += T, b ^= 1) {
+    const int nt = min(T, len - t0);
+    const bool more = t0 + T < len;
+    if (more) fetch(t0 + T);
+    if (t0 > 0) emit(t0 - T, T, b ^ 1);
+    if constexpr (CPR) {
+      if (t0 % chunk == 0) {
+#pragma unroll
+        for (int j = 0; j < RPL; ++j)
+#pragma unroll
+          for (int i = 0; i < 8; ++i) S[j][i] = ix_wire(C[j][i], (const TIO*)nullptr);
+      }
+    }
+    if (nt == T) {
+      // Skewed by half a token: an iteration joins the two trees that are pending (k dot of this token, q dot of the one
+      // before, so that neither waits alone for its lane exchanges), updates the state, and issues the dots of its own q
+      // and the next token's k. k is loaded two tokens ahead, q one; the scheduling barrier keeps those loads at the top
+      // of the iteration, a whole one in front of their use (left alone, the compiler sinks them to it).
+      float keep[RPL][NK];
+      float kb[3][8], qb[2][8], vb3[3][RPL], kp[RPL], qp[RPL], cp[RPL];
+      float2 gb[3];
+      auto load_k = [&](int tt) __attribute__((always_inline)) {
+        const float4 a = *reinterpret_cast<const float4*>(&kq[b][0][tt][sub * 4]);
+        const float4 c = *reinterpret_cast<const float4*>(&kq[b][0][tt][K / 2 + sub * 4]);
+        float(&x)[8] = kb[tt % 3];
+        x[0] = a.x; x[1] = a.y; x[2] = a.z; x[3] = a.w; x[4] = c.x; x[5] = c.y; x[6] = c.z; x[7] = c.w;
+        gb[tt % 3] = eb[b][tt];
+#pragma unroll
+        for (int j = 0; j < RPL; ++j) vb3[tt % 3][j] = vf[b][tt][j * RW + r];
+      };
+      auto load_q = [&](int tt) __attribute__((always_inline)) {
+        const float4 a = *reinterpret_cast<const float4*>(&kq[b][1][tt][sub * 4]);
+        const float4 c = *reinterpret_cast<const float4*>(&kq[b][1][tt][K / 2 + sub * 4]);
+        float(&x)[8] = qb[tt % 2];
+        x[0] = a.x; x[1] = a.y; x[2] = a.z; x[3] = a.w; x[4] = c.x; x[5] = c.y; x[6] = c.z; x[7] = c.w;
+      };
+      auto decay_dot = [&](int tt) __attribute__((always_inline)) {
+#pragma unroll
+        for (int j = 0; j < RPL; ++j) {
+#pragma unroll
+          for (int i = 0; i < 8; ++i) S[j][i] = S[j][i] * gb[tt % 3].x;
+          kp[j] = ix_dot8(S[j], kb[tt % 3]);
+          if constexpr (CPR) {
+#pragma unroll
+            for (int i = 0; i < 8; ++i) C[j][i] = C[j][i] * gb[tt % 3].x;
+            cp[j] = ix_dot8(C[j], kb[tt % 3]);
+          }
+        }
+      };
+      auto keep_out = [&](int tt, int j, float ov) __attribute__((always_inline)) {
+        if ((tt % KS) == 0) keep[j][tt / KS] = ov;
+        else keep[j][tt / KS] = sub == tt % KS ? ov : keep[j][tt / KS];
+      };
+      load_k(0);
+      load_k(1);
+      load_q(0);
+      decay_dot(0);
+#pragma unroll
+      for (int tt = 0; tt < T; ++tt) {
+        if (tt + 2 < T) load_k(tt + 2);
+        if (tt + 1 < T) load_q(tt + 1);
+        __builtin_amdgcn_sched_barrier(0);
+        float ov[RPL], kv[RPL], cv[RPL];
+#pragma unroll
+        for (int j = 0; j < RPL; ++j) {
+          kv[j] = ix_lane_tree<KS>(kp[j]);
+          if constexpr (CPR) cv[j] = ix_lane_tree<KS>(cp[j]);
+          if (tt > 0) ov[j] = ix_lane_tree<KS>(qp[j]);
+        }
+#pragma unroll
+        for (int j = 0; j < RPL; ++j) {
+          if (tt > 0) keep_out(tt - 1, j, ov[j]);
+          const float d = (vb3[tt % 3][j] - kv[j]) * gb[tt % 3].y;
+#pragma unroll
+          for (int i = 0; i < 8; ++i) S[j][i] = __builtin_fmaf(d, kb[tt % 3][i], S[j][i]);
+          qp[j] = ix_dot8(S[j], qb[tt % 2]);
+          if constexpr (CPR) {
+            const float dc = (vb3[tt % 3][j] - cv[j]) * gb[tt % 3].y;
+#pragma unroll
+            for (int i = 0; i < 8; ++i) C[j][i] = __builtin_fmaf(dc, kb[tt % 3][i], C[j][i]);
+          }
+        }
+        if (tt + 1 < T) decay_dot(tt + 1);
+      }
+#pragma unroll
+      for (int j = 0; j < RPL; ++j) keep_out(T - 1, j, ix_lane_tree<KS>(qp[j]));
+      if (KS <= T || sub < T) {
+#pragma unroll
+        for (int j = 0; j < RPL; ++j)
+#pragma unroll
+          for (int i = 0; i < NK; ++i) of[b][sub + KS * i][j * RW + r] = keep[j][i];
+      }
+    } else {
+      for (int tt = 0; tt < nt; ++tt) {
+        float ov[RPL];
+        token(b, tt, ov);
+        if (sub == 0) {
+#pragma unroll
+          for (int j = 0; j < RPL; ++j) of[b][tt][j * RW + r] = ov[j];
+        }
+      }
+    }
+    if (more) commit(b ^ 1);
+    __syncthreads();
+  }
+  const int last = (len - 1) / T;
+  emit(last * T, len - last * T, last & 1);
+  if (state && !CPR) {
+#pragma unroll
+    for (int j = 0; j < RPL; ++j) {
+      float* sp = state + (((long)row0 * HV + hv) * V + vb * R + r + j * RW) * K + sub * 8;
+      *reinterpret_cast<float4*>(sp) = make_float4(S[j][0], S[j][1], S[j][2], S[j][3]);
+      *reinterpret_cast<float4*>(sp + 4) = make_float4(S[j][4], S[j][5], S[j][6], S[j][7]);
+    }
+  }
+}
+
+// q and k rows that can be fetched 8 elements at a time: every row start on a 16-byte (bf16) or 32-byte (fp32) boundary
+template <typename TIO>
+static bool ix_gdn_vec_qk(const void* q, const void* k, long q_pitch, long k_pitch) {
+  return q_pitch % 8 == 0 && k_pitch % 8 == 0 && ix_aligned(q, 8 * sizeof(TIO)) && ix_aligned(k, 8 * sizeof(TIO));
+}
+
+template <int KS, typename TIO, bool CPR>
+static int ix_gdn_walk_launch(const void* q, const void* k, const void* v, const float* g, const void* beta, void* o,
+                              float* state, const int* cu, const int* sidx, long q_pitch, long k_pitch, long v_pitch,
+                              long N, int H, int HV, int V, float scale, int chunk, int rpl, hipStream_t st) {
+  constexpr int RW = 256 / KS;
+  if (V % RW != 0 || !ix_gdn_vec_qk<TIO>(q, k, q_pitch, k_pitch)) return IX_DECLINED;
+  if (rpl == 2 && V % (2 * RW) != 0) rpl = 1;
+  const long grid = N * HV * (V / (RW * rpl));
+  if (grid > 0x7fffffffL) return IX_DECLINED;
+#define IX_WALK(RPL_)                                                                                                \
+  hipLaunchKernelGGL((k_gdn_walk<KS, RPL_, TIO, CPR>), dim3((unsigned)grid), dim3(256), 0, st, (const TIO*)q,        \
+                     (const TIO*)k, (const TIO*)v, g, (const TIO*)beta, (TIO*)o, state, cu, sidx, q_pitch, k_pitch,  \
+                     v_pitch, (int)N, H, HV, V, scale, chunk)
+  if (rpl == 2) IX_WALK(2);
+  else IX_WALK(1);
+#undef IX_WALK
+  return ix_launch_status();
 }
 
 static size_t ix_gdn_lds_bytes(int K, int R, int TT) {
@@ -467,6 +825,61 @@ static int ix_gdn_scan_launch(const void* q, const void* k, const void* v, const
 #undef IX_RPL_CASE
 }
 
+// chunk > 0: the boundary form. rpl: state rows per lane group, 0 = by the rule.
+static int ix_gdn_walk(const void* q, const void* k, const void* v, const float* g, const void* beta, void* o,
+                       int io_dtype, float* state, const int* cu, const int* sidx, long q_pitch, long k_pitch, long v_pitch,
+                       long N, int H, int HV, long K, int V, float scale, int chunk, int rpl, hipStream_t st) {
+  // Two rows per lane group share the LDS reads of k and q and give a wave two chains to interleave, one leaves twice the
+  // waves. Measured at HV = 32, V = K = 128, us one / two rows: one sequence of 8192 tokens 1129 / 1823, five of 33..1203
+  // 247 / 307, nine of 120..1500 608 / 591, 16 x 1000 1266 / 1180; K = V = 64, HV = 16
+  // and 32: 8 x 500 72 / 110, 32 x 500 329 / 323. The line: eight waves per SIMD at one row.
+  if (rpl <= 0) rpl = N * HV * V * (K / 8) >= 8L * 1024 * 64 ? 2 : 1;
+#define IX_WALK_CASE(KSV)                                                                                             \
+  if (K == KSV * 8) {                                                                                                 \
+    if (io_dtype == IX_DT_BF16)                                                                                       \
+      return chunk > 0 ? ix_gdn_walk_launch<KSV, bf16_t, true>(q, k, v, g, beta, o, state, cu, sidx, q_pitch, k_pitch, \
+                                                               v_pitch, N, H, HV, V, scale, chunk, rpl, st)           \
+                       : ix_gdn_walk_launch<KSV, bf16_t, false>(q, k, v, g, beta, o, state, cu, sidx, q_pitch,        \
+                                                                k_pitch, v_pitch, N, H, HV, V, scale, 0, rpl, st);    \
+    return chunk > 0 ? ix_gdn_walk_launch<KSV, float, true>(q, k, v, g, beta, o, state, cu, sidx, q_pitch, k_pitch,   \
+                                                            v_pitch, N, H, HV, V, scale, chunk, rpl, st)              \
+                     : ix_gdn_walk_launch<KSV, float, false>(q, k, v, g, beta, o, state, cu, sidx, q_pitch, k_pitch,  \
+                                                             v_pitch, N, H, HV, V, scale, 0, rpl, st);                \
+  }
+  IX_WALK_CASE(4)
+  IX_WALK_CASE(8)
+  IX_WALK_CASE(16)
+  IX_WALK_CASE(32)
+#undef IX_WALK_CASE
+  return IX_DECLINED;
+}
+
+// Workgroups (128 rows each) from which a batch of whole sequences takes the lane-pair layout. It issues 36 vector
+// instructions per four rows and token where the walk issues 42, but a token takes one of its waves five times as long:
+// it wins once every SIMD has several waves through to the end. Measured at HV = 32, V = 128 (one such workgroup per
+// sequence and head), us pairs / walk: 64 x 1000 tokens 3953 / 4364, 32 x 1000 2314 / 2227, 16 x 1000 1201 / 1180, 20
+// sequences of 60..1485 tokens 1788 / 1134.
+#define IX_GDN_PAIR_MIN 2048
+
+static int ix_gdn_pairs(const void* q, const void* k, const void* v, const float* g, const void* beta, void* o, int io_dtype,
+                        long q_pitch, long k_pitch, long v_pitch, float* state, const int* cu, const int* sidx, long N,
+                        int H, int HV, int V, float scale, int TT, const bf16_t* gate, long gate_stride_t,
+                        const bf16_t* norm_w, float norm_eps, int zero_centered, hipStream_t st) {
+  const long grid = N * HV * (V / 128);
+  if (grid > 0x7fffffffL) return IX_DECLINED;
+  size_t lds = ix_gdn_lds_bytes(128, 128, TT);
+  if (lds < (IX_GDN_SORT_MAX + 1) * sizeof(int)) lds = (IX_GDN_SORT_MAX + 1) * sizeof(int);
+  if (io_dtype == IX_DT_BF16)
+    hipLaunchKernelGGL((k_gdn_scan_pairs<bf16_t>), dim3((unsigned)grid), dim3(256), lds, st, (const bf16_t*)q,
+                       (const bf16_t*)k, (const bf16_t*)v, g, (const bf16_t*)beta, (bf16_t*)o, state, cu, sidx, q_pitch,
+                       k_pitch, v_pitch, (int)N, H, HV, V, scale, TT, gate, gate_stride_t, norm_w, norm_eps, zero_centered);
+  else
+    hipLaunchKernelGGL((k_gdn_scan_pairs<float>), dim3((unsigned)grid), dim3(256), lds, st, (const float*)q,
+                       (const float*)k, (const float*)v, g, (const float*)beta, (float*)o, state, cu, sidx, q_pitch, k_pitch,
+                       v_pitch, (int)N, H, HV, V, scale, TT, (const bf16_t*)nullptr, 0L, (const bf16_t*)nullptr, 0.0f, 0);
+  return ix_launch_status();
+}
+
 static int ix_gdn_scan_impl(const void* q, const void* k, const void* v, const float* g, const void* beta, void* o,
                             int io_dtype, long q_pitch, long k_pitch, long v_pitch, float* state_pool,
                             const int* cu_seqlens, const int* state_indices, long state_indices_stride, long N,
@@ -485,30 +898,25 @@ static int ix_gdn_scan_impl(const void* q, const void* k, const void* v, const f
   if (TT <= 0) TT = (N * HV * (V / 16) >= 4096) ? 16 : 64;
   if (TT > 64) TT = 64;
   hipStream_t st = (hipStream_t)stream;
-  // The lane-pair layout: compact state form, K = 128, whole groups of 128 rows, and enough workgroups to fill the
-  // chip (or forced by rows-per-lane-group code 16 in bits 8.. of time_tile). Same bits as the kernels below. A
-  // time tile of 1 says one token per sequence (a decode step): that is a pure stream of the state, which the
-  // 16-lane layout does with more waves in flight.
+  // The lane-pair layout: compact state form, K = 128, whole groups of 128 rows, and IX_GDN_PAIR_MIN workgroups (or forced
+  // by code 16 in bits 8.. of time_tile). A time tile of 1 says one token per sequence (a decode step): that is a pure
+  // stream of the state, which the 16-lane layout does with more waves in flight.
   if (state_indices_stride == 0 && K == 128 && V % 128 == 0 &&
-      (rpl == 16 || (rpl == 0 && (time_tile & 0xff) != 1 && N * HV * (V / 128) >= 512))) {
-    const long grid = N * HV * (V / 128);
-    if (grid > 0x7fffffffL) return IX_DECLINED;
-    const int tt = time_tile > 0 && (time_tile & 0xff) > 0 ? TT : 16;
-    const size_t lds = ix_gdn_lds_bytes(128, 128, tt);
-    if (io_dtype == IX_DT_BF16)
-      hipLaunchKernelGGL((k_gdn_scan_pairs<bf16_t>), dim3((unsigned)grid), dim3(256), lds, st, (const bf16_t*)q,
-                         (const bf16_t*)k, (const bf16_t*)v, g, (const bf16_t*)beta, (bf16_t*)o, state_pool,
-                         cu_seqlens, state_indices, q_pitch, k_pitch, v_pitch, (int)H, (int)HV, (int)V, scale, tt, gate,
-                         gate_stride_t, norm_w, norm_eps, zero_centered);
-    else
-      hipLaunchKernelGGL((k_gdn_scan_pairs<float>), dim3((unsigned)grid), dim3(256), lds, st, (const float*)q,
-                         (const float*)k, (const float*)v, g, (const float*)beta, (float*)o, state_pool, cu_seqlens,
-                         state_indices, q_pitch, k_pitch, v_pitch, (int)H, (int)HV, (int)V, scale, tt,
-                         (const bf16_t*)nullptr, 0L, (const bf16_t*)nullptr, 0.0f, 0);
-    return ix_launch_status();
-  }
+      (rpl == 16 || (rpl == 0 && (time_tile & 0xff) != 1 && N * HV * (V / 128) >= IX_GDN_PAIR_MIN)))
+    return ix_gdn_pairs(q, k, v, g, beta, o, io_dtype, q_pitch, k_pitch, v_pitch, state_pool, cu_seqlens, state_indices, N,
+                        (int)H, (int)HV, (int)V, scale, time_tile > 0 && (time_tile & 0xff) > 0 ? TT : 16, gate,
+                        gate_stride_t, norm_w, norm_eps, zero_centered, st);
   if (gate) return IX_DECLINED;       // the norm rides on the lane-pair layout only
   if (rpl == 16) return IX_DECLINED;  // the lane-pair layout was asked for and does not apply
+  // Sequences of more than one token in the compact form: the walk (codes 17 and 18 force it with one and two rows per
+  // lane group). k_gdn_scan below keeps the decode step, the per-token index map, the state-only pass and the operands
+  // whose rows are not aligned.
+  if (state_indices_stride == 0 && o && (time_tile <= 0 || rpl == 17 || rpl == 18)) {
+    const int rc = ix_gdn_walk(q, k, v, g, beta, o, io_dtype, state_pool, cu_seqlens, state_indices, q_pitch, k_pitch,
+                               v_pitch, N, (int)H, (int)HV, K, (int)V, scale, 0, rpl >= 17 ? rpl - 16 : 0, st);
+    if (rc != IX_DECLINED) return rc;
+  }
+  if (rpl >= 17) return IX_DECLINED;
 #define IX_SCAN_CASE(KSV)                                                                                         \
   if (K == KSV * 8) {                                                                                             \
     if (io_dtype == IX_DT_BF16)                                                                                   \
@@ -537,7 +945,7 @@ extern "C" int ix_gdn_scan(const void* q, const void* k, const void* v, const fl
 
 // ix_gdn_scan whose output leaves through the layer's gated output norm (ix_gated_out_norm with N = V) in the same
 // launch: o receives bf16(norm(o_scan) * silu(gate)) instead of o_scan -- the bits of the two calls. Served where the
-// lane-pair layout runs (one state row per sequence, K = V = 128, bf16, at least 512 (sequence, head) pairs) with
+// lane-pair layout runs (one state row per sequence, K = V = 128, bf16, at least IX_GDN_PAIR_MIN (sequence, head) pairs) with
 // 16-byte aligned gate rows and weight; IX_DECLINED otherwise, before anything is launched or the state is touched.
 extern "C" int ix_gdn_scan_gated_norm(const void* q, const void* k, const void* v, const float* g, const void* beta,
                                       void* o, long q_pitch, long k_pitch, long v_pitch, float* state_pool,
@@ -546,11 +954,37 @@ extern "C" int ix_gdn_scan_gated_norm(const void* q, const void* k, const void* 
                                       const void* norm_weight, float norm_eps, int zero_centered, void* stream) {
   if (!o || !gate || !norm_weight || gate_stride_t < HV * V) return IX_ERR_ARG;
   if (K != 128 || V != 128 || (gate_stride_t % 8) || !ix_aligned(gate, 16) || !ix_aligned(norm_weight, 16) ||
-      !ix_aligned(o, 16) || (time_tile & 0xff) == 1 || (time_tile >> 8) != 0 || N * HV < 512)
+      !ix_aligned(o, 16) || (time_tile & 0xff) == 1 || (time_tile >> 8) != 0 || N * HV < IX_GDN_PAIR_MIN)
     return IX_DECLINED;
   return ix_gdn_scan_impl(q, k, v, g, beta, o, IX_DT_BF16, q_pitch, k_pitch, v_pitch, state_pool, cu_seqlens,
                           state_indices, 0, N, H, HV, K, V, scale, time_tile, (const bf16_t*)gate, gate_stride_t,
                           (const bf16_t*)norm_weight, norm_eps, zero_centered, stream);
+}
+
+// The stateless forward: every sequence starts from a zero state, which is not kept. chunk 0: the recurrence; chunk > 0:
+// the boundary form, whose running state restarts every `chunk` tokens from the fp32 chain rounded to io_dtype.
+extern "C" int ix_gdn_forward(const void* q, const void* k, const void* v, const float* g, const void* beta, void* o,
+                              int io_dtype, long q_pitch, long k_pitch, long v_pitch, const int* cu_seqlens, long N, long H,
+                              long HV, long K, long V, float scale, long chunk, const void* gate, long gate_stride_t,
+                              const void* norm_weight, float norm_eps, int zero_centered, void* stream) {
+  if (!q || !k || !v || !g || !beta || !o || !cu_seqlens) return IX_ERR_ARG;
+  if (N < 0 || H <= 0 || HV <= 0 || K <= 0 || V <= 0 || HV % H != 0 || chunk < 0) return IX_ERR_ARG;
+  if (q_pitch < H * K || k_pitch < H * K || v_pitch < HV * V) return IX_ERR_ARG;
+  if (gate && (!norm_weight || gate_stride_t < HV * V)) return IX_ERR_ARG;
+  if (io_dtype != IX_DT_F32 && io_dtype != IX_DT_BF16) return IX_DECLINED;
+  if (chunk % 16 || chunk > 0x7fffffffL) return IX_DECLINED;  // the restart falls on a tile's first token
+  hipStream_t st = (hipStream_t)stream;
+  const bool pairs = chunk == 0 && K == 128 && V % 128 == 0 && N * HV * (V / 128) >= IX_GDN_PAIR_MIN;
+  if (gate && (!pairs || V != 128 || io_dtype != IX_DT_BF16 || (gate_stride_t % 8) || !ix_aligned(gate, 16) ||
+               !ix_aligned(norm_weight, 16) || !ix_aligned(o, 16)))
+    return IX_DECLINED;  // the norm rides on the lane-pair layout only
+  if (N == 0) return IX_OK;
+  if (pairs)
+    return ix_gdn_pairs(q, k, v, g, beta, o, io_dtype, q_pitch, k_pitch, v_pitch, nullptr, cu_seqlens, nullptr, N, (int)H,
+                        (int)HV, (int)V, scale, 16, (const bf16_t*)gate, gate_stride_t, (const bf16_t*)norm_weight,
+                        norm_eps, zero_centered, st);
+  return ix_gdn_walk(q, k, v, g, beta, o, io_dtype, nullptr, cu_seqlens, nullptr, q_pitch, k_pitch, v_pitch, N, (int)H,
+                     (int)HV, K, (int)V, scale, (int)chunk, 0, st);
 }
 
 // ---------------------------------------------------------------------------------------------

@@ -92,6 +92,11 @@ SIGNATURES = {
         [P, P, P, P, P, P, c_long, c_long, c_long, P, P, P, c_long, c_long, c_long, c_long, c_long, c_float, c_int, P,
          c_long, P, c_float, c_int, P],
     ),
+    "ix_gdn_forward": (
+        c_int,
+        [P, P, P, P, P, P, c_int, c_long, c_long, c_long, P, c_long, c_long, c_long, c_long, c_long, c_float, c_long, P,
+         c_long, P, c_float, c_int, P],
+    ),
     "ix_gdn_conv": (c_int, [P, c_long, P, P, P, P, P, P, P, c_long, c_long, c_long, c_long, c_int, P]),
     "ix_gdn_conv_l2norm": (c_int, [P, c_long, P, P, P, P, P, P, P, c_long, c_long, c_long, c_long, c_int, c_long, c_long,
                                    c_float, P]),

@@ -152,6 +152,56 @@ def gdn_recurrent_kernel(
     return o.view(B, T, HV, V) if cu_seqlens is None else o.unsqueeze(0)
 
 
+def stateless_forward(q, k, v, g, beta, *, cu_seqlens=None, chunk_size: int = 0, gated_norm: tuple | None = None):
+    """The delta-rule forward from a zero state that is not kept (``ix_gdn_forward``): ``q, k`` L2-normalised, layouts as
+    ``gdn_recurrent_kernel``'s. ``chunk_size`` > 0 is the boundary form (``gdn_cpr_fwd``), in the same single pass over the
+    tokens. With ``gated_norm`` the output comes back through the layer's gated output norm. Returns ``o`` shaped like
+    ``v``, or ``None`` when the library does not serve the operands (nothing launched: the caller scans with a pool)."""
+    _lib.require_device(q, k, v, g, beta, cu_seqlens)
+    if q.ndim != 4 or v.ndim != 4:
+        raise RuntimeError(f"[isoexec-amd] the delta-rule forward expects [B,T,H,K]/[B,T,HV,V], got {tuple(q.shape)}")
+    B, T, H, K = q.shape
+    HV, V = v.shape[-2], v.shape[-1]
+    io, dev = v.dtype, q.device
+    if q.dtype is not io or k.dtype is not io:
+        raise RuntimeError("[isoexec-amd] q/k/v must share a dtype")
+    if cu_seqlens is None:
+        cu, n_seq = _uniform_cu(B, T, dev), B
+    else:
+        if B != 1:
+            raise RuntimeError("[isoexec-amd] a packed batch (cu_seqlens) needs B == 1")
+        cu = cu_seqlens.to(torch.int32).contiguous()
+        n_seq = cu.numel() - 1
+    qf, kf, vf = _flatten_tokens(q, 2), _flatten_tokens(k, 2), _flatten_tokens(v, 2)
+    gf = _flatten_tokens(g, 1).to(torch.float32).contiguous()
+    bf = _flatten_tokens(beta, 1).to(io).contiguous()
+    o = torch.empty(qf.shape[0], HV, V, dtype=io, device=dev)
+
+    def launch(gate, weight, eps, zero_centered):
+        return _lib.check(
+            _lib.lib().ix_gdn_forward(
+                qf.data_ptr(), kf.data_ptr(), vf.data_ptr(), gf.data_ptr(), bf.data_ptr(), o.data_ptr(),
+                _lib.dtype_code(io), _token_pitch(qf), _token_pitch(kf), _token_pitch(vf), cu.data_ptr(), n_seq, H, HV, K,
+                V, float(K) ** -0.5, int(chunk_size), _lib.ptr(gate), 0 if gate is None else gate.stride(0),
+                _lib.ptr(weight), float(eps), int(zero_centered), _lib.current_stream(dev)), "ix_gdn_forward")
+
+    if gated_norm is None:
+        return o.view(B, T, HV, V) if launch(None, None, 0.0, 0) == _lib.IX_OK else None
+    gate, weight, eps, zero_centered = gated_norm
+    _lib.require_device(gate, weight)
+    if tuple(gate.shape) != (qf.shape[0], HV, V):
+        raise RuntimeError("[isoexec-amd] gated_norm needs a gate [tokens, HV, V]")
+    fusable = (io is torch.bfloat16 and gate.dtype is io and weight.dtype is io and gate.stride(2) == 1
+               and gate.stride(1) == V and weight.is_contiguous() and weight.numel() == V)
+    if fusable and launch(gate, weight, eps, zero_centered) == _lib.IX_OK:
+        return o.view(B, T, HV, V)
+    if launch(None, None, 0.0, 0) != _lib.IX_OK:
+        return None
+    from ..norms.fused_outnorm import fused_gated_out_norm
+
+    return fused_gated_out_norm(o, gate, weight, eps, zero_centered=zero_centered).view(B, T, HV, V)
+
+
 def gdn_l2norm(x: torch.Tensor) -> torch.Tensor:
     """Row-local L2 normalisation ``x * rsqrt(sum x^2 + 1e-6)`` over the last dim; ``[..., H, K]``."""
     _lib.require_device(x)
@@ -326,15 +376,22 @@ def gdn_causal_conv_batched(x, weight, bias=None, *, initial_state=None, activat
 
 
 def _recurrent_scratch_state(q, v, cu_seqlens):
-    """A throwaway zero pool + row indices for a stateless forward (gdn_ops.py:444-464): row 0 unused,
-    sequence n at row n+1. One row per sequence (the compact form): the final state lands in the throwaway
-    pool instead of nowhere, which costs one 2 MB store per sequence and lets the scan run its branch-free
-    token loop; the outputs do not depend on where, or whether, the state is stored."""
+    """A throwaway zero pool + row indices for a stateless forward that ``ix_gdn_forward`` does not serve
+    (gdn_ops.py:444-464): row 0 unused, sequence n at row n+1, one row per sequence."""
     N = cu_seqlens.numel() - 1 if cu_seqlens is not None else q.shape[0]
     HV, V, K = v.shape[-2], v.shape[-1], q.shape[-1]
     ssm_state = torch.zeros(N + 1, HV, V, K, dtype=torch.float32, device=q.device)
     idx = torch.arange(1, N + 1, dtype=torch.int32, device=q.device)
     return ssm_state, idx
+
+
+def _stateless(q, k, v, g, beta, cu_seqlens, gated_norm=None):
+    o = stateless_forward(q, k, v, g, beta, cu_seqlens=cu_seqlens, gated_norm=gated_norm)
+    if o is not None:
+        return o
+    ssm_state, idx = _recurrent_scratch_state(q, v, cu_seqlens)
+    return gdn_recurrent_kernel(q, k, v, g, beta, ssm_state=ssm_state, state_indices=idx, cu_seqlens=cu_seqlens,
+                                gated_norm=gated_norm)
 
 
 def gdn_recurrent(q, k, v, g, beta, *, initial_state=None, output_final_state=False, cu_seqlens=None):
@@ -344,9 +401,7 @@ def gdn_recurrent(q, k, v, g, beta, *, initial_state=None, output_final_state=Fa
             "isoexec GDN: gdn_recurrent is the stateless (training/prefill-from-zero) entry point. "
             "The engine carries state through gdn_recurrent_kernel + a real state pool.")
     with torch.no_grad():
-        ssm_state, idx = _recurrent_scratch_state(q, v, cu_seqlens)
-        o = gdn_recurrent_kernel(q, k, v, g, beta, ssm_state=ssm_state, state_indices=idx, cu_seqlens=cu_seqlens)
-    return o, None
+        return _stateless(q, k, v, g, beta, cu_seqlens), None
 
 
 def gdn_kernel_mode() -> str:
@@ -422,17 +477,12 @@ def gdn_native_core_normed(qn, kn, v, a, b, A_log, dt_bias, *, cu_seqlens=None, 
     the scan of the same composition, without its two l2norm launches. Same bits as ``gdn_native_core`` on the raw heads.
     ``gated_norm`` as in ``gdn_recurrent_kernel``: the output then comes back through the layer's gated output norm."""
     with torch.no_grad():
-        ssm_state, idx = _recurrent_scratch_state(qn, v, cu_seqlens)
         HV = v.shape[-2]
         g, beta = gate_and_beta_fp32(a.reshape(-1, HV), b.reshape(-1, HV), A_log, dt_bias)
         lead = v.shape[:2]
-        return gdn_recurrent_kernel(qn, kn, v, g.view(*lead, HV), beta.view(*lead, HV), ssm_state=ssm_state,
-                                    state_indices=idx, cu_seqlens=cu_seqlens, gated_norm=gated_norm)
+        return _stateless(qn, kn, v, g.view(*lead, HV), beta.view(*lead, HV), cu_seqlens, gated_norm)
 
 
 def gdn_native_core(q, k, v, a, b, A_log, dt_bias, *, cu_seqlens=None):
     """Stateless entry for the native composition (gdn_ops.py:702-716)."""
-    with torch.no_grad():
-        ssm_state, idx = _recurrent_scratch_state(q, v, cu_seqlens)
-        return gdn_native_core_kernel(q, k, v, a, b, A_log, dt_bias, ssm_state=ssm_state, state_indices=idx,
-                                      cu_seqlens=cu_seqlens)
+    return gdn_native_core_normed(gdn_l2norm(q), gdn_l2norm(k), v, a, b, A_log, dt_bias, cu_seqlens=cu_seqlens)

@@ -25,7 +25,7 @@ import torch
 from ..debug.trace import get_tracer
 from ..ops.attention.varlen_attn import KVCache, varlen_attention
 from ..ops.gdn.gdn_ops import conv_packed, gdn_native_core, gdn_native_core_normed
-from ..ops.gdn.gdn_cpr import gdn_native_cpr_fwd
+from ..ops.gdn.gdn_cpr import gdn_native_cpr_fwd, gdn_native_cpr_normed
 from ..ops.gdn.gdn_cpr_state import CprGDN
 from ..ops.gdn.gdn_recurrent_state import RecurrentGDN
 from ..ops.logprobs.rowinv import leaves, sampled_forward
@@ -364,17 +364,18 @@ class TrainerModel:
                 return b.attn_out(i, varlen_attention(q, k, v, cu, max_len))
             qkv, z, bb, a = b.gdn_in(i, x)
             kd = c.gdn_k_heads * c.gdn_head_dim
-            # the recurrent form takes q and k normalised by the convolution's own launch and hands its output to the
+            # q and k come normalised from the convolution's own launch, and the recurrent form hands its output to the
             # gated norm inside the scan's (where the library serves those forms; the same bits as the ops apart)
-            fused = b.fuse_ops and c.gdn_kernel != "cpr"
+            fused = b.fuse_ops
             y = conv_packed(qkv, lw["conv_weight"], lw["conv_bias"], cu_seqlens=cu, l2norm_qk=2 * kd if fused else 0,
                             head_k_dim=c.gdn_head_dim)
             q = y[:, :kd].unflatten(1, (c.gdn_k_heads, c.gdn_head_dim))
             k = y[:, kd : 2 * kd].unflatten(1, (c.gdn_k_heads, c.gdn_head_dim))
             v = y[:, 2 * kd :].unflatten(1, (c.gdn_v_heads, c.gdn_head_dim))
             if c.gdn_kernel == "cpr":
-                o = gdn_native_cpr_fwd(q.unsqueeze(0), k.unsqueeze(0), v.unsqueeze(0), a, bb, lw["A_log"], lw["dt_bias"],
-                                       cu_seqlens=cu, chunk_size=c.gdn_chunk)
+                core = gdn_native_cpr_normed if fused else gdn_native_cpr_fwd
+                o = core(q.unsqueeze(0), k.unsqueeze(0), v.unsqueeze(0), a, bb, lw["A_log"], lw["dt_bias"], cu_seqlens=cu,
+                         chunk_size=c.gdn_chunk)
             elif fused:
                 o = gdn_native_core_normed(q.unsqueeze(0), k.unsqueeze(0), v.unsqueeze(0), a, bb, lw["A_log"],
                                            lw["dt_bias"], cu_seqlens=cu, gated_norm=b.gdn_gated_norm(i, z))

@@ -100,6 +100,12 @@ int ix_logprob_rowinv_full(const void* logits, int dtype, long rows, long V, lon
                            float* out_full, long out_stride, float* out_lse, void* workspace,
                            size_t workspace_bytes, int force_shape, const float* row_max_in, void* stream);
 
+/* Backward of the sampled logprob (rowinv.py:573-612): grad[row, j] = -u exp(x[row, j] - lse[row]) + (j == target[row]) u with
+ * u = upstream[row], or 0 for a target outside [0, V); rounded to dtype. target int64, upstream and lse fp32 [rows]; grad
+ * [rows, V] of the logits' dtype with row pitch grad_stride. */
+int ix_logprob_rowinv_backward(const void* logits, int dtype, long rows, long V, long row_stride, const int64_t* target,
+                               const float* upstream, const float* lse, void* grad, long grad_stride, void* stream);
+
 /* rowmax[r] = max_p parts[r*parts_ld + p], p < P (torch.amax of rowinv.py:479 over partials). */
 int ix_rowmax_reduce(const float* parts, long parts_ld, long P, long rows, float* rowmax, void* stream);
 

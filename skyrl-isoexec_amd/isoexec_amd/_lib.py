@@ -50,6 +50,7 @@ SIGNATURES = {
         c_int,
         [P, c_int, c_long, c_long, c_long, c_int, P, c_long, P, P, c_size_t, c_int, P, P],
     ),
+    "ix_logprob_rowinv_backward": (c_int, [P, c_int, c_long, c_long, c_long, P, P, P, P, c_long, P]),
     "ix_rowmax_reduce": (c_int, [P, c_long, c_long, c_long, P, P]),
     "ix_rmsnorm_gamma": (c_int, [P, P, P, c_long, c_long, c_float, c_int, P]),
     "ix_gated_out_norm": (c_int, [P, P, c_long, P, P, c_long, c_long, c_long, c_float, c_int, P]),

@@ -106,6 +106,22 @@ def sampled_forward(x: torch.Tensor, t: torch.Tensor, g: int, *, force_shape: in
     return out, lse
 
 
+def sampled_backward(x: torch.Tensor, t: torch.Tensor, upstream: torch.Tensor, lse: torch.Tensor):
+    """Gradient of ``sampled_forward``'s logprobs with respect to ``x [rows, V]`` (in its dtype) from ``upstream [rows]``
+    and the forward's ``lse [rows]``; ``None`` if declined."""
+    _lib.require_device(x, t, upstream, lse)
+    if x.stride(1) != 1:
+        return None
+    rows, vocab = x.shape
+    grad = torch.empty(rows, vocab, dtype=x.dtype, device=x.device)
+    rc = _lib.check(
+        _lib.lib().ix_logprob_rowinv_backward(x.data_ptr(), _lib.dtype_code(x.dtype), rows, vocab, x.stride(0),
+                                              t.contiguous().data_ptr(), upstream.contiguous().data_ptr(),
+                                              lse.contiguous().data_ptr(), grad.data_ptr(), grad.stride(0),
+                                              _lib.current_stream(x.device)), "ix_logprob_rowinv_backward")
+    return grad if rc == _lib.IX_OK else None
+
+
 def full_forward(x: torch.Tensor, g: int, *, force_shape: int = 0):
     _lib.require_device(x)
     rows, vocab = x.shape
@@ -120,7 +136,7 @@ def full_forward(x: torch.Tensor, g: int, *, force_shape: int = 0):
 
 
 class _RowInvSampledLogprob(torch.autograd.Function):
-    """Kernel forward; rank-local backward from per-row scalars (rowinv.py:573-612)."""
+    """Kernel forward; rank-local backward from per-row scalars (rowinv.py:573-612), one kernel as well."""
 
     @staticmethod
     def forward(ctx, logits, target, g):
@@ -138,6 +154,11 @@ class _RowInvSampledLogprob(torch.autograd.Function):
         x = logits.reshape(-1, vocab)
         t = target.reshape(-1).to(torch.int64)
         upstream = grad_out.reshape(-1).to(torch.float32)
+        if not torch.is_grad_enabled():
+            grad = sampled_backward(x, t, upstream, lse)
+            if grad is not None:
+                return grad.reshape(logits.shape), None, None
+        # the same expression in differentiable pieces (a caller that builds a graph of the gradient)
         valid = (t >= 0) & (t < vocab)
         upstream = torch.where(valid, upstream, torch.zeros_like(upstream))
         grad = torch.exp(x - lse.unsqueeze(1)).mul_(-upstream.unsqueeze(1))

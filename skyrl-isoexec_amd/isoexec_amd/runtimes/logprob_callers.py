@@ -105,8 +105,13 @@ def _ix_try_rowinv_logprobs(
     served = []
     with torch.set_grad_enabled(grad_on):
         # torch.split gives the same views as slicing (so the same forward bits) with one backward
-        # node for the walk instead of one zero-filled gradient per chunk.
-        for chunk, target_chunk in zip(torch.split(vocab_parallel_logits, step, dim=1), torch.split(target, step, dim=1)):
+        # node for the walk instead of one zero-filled gradient per chunk. An unchunked call hands the tensors over as they
+        # are: even a single view's backward would copy the whole gradient once more.
+        if step >= seq_len:
+            pieces = [(vocab_parallel_logits, target)]
+        else:
+            pieces = zip(torch.split(vocab_parallel_logits, step, dim=1), torch.split(target, step, dim=1))
+        for chunk, target_chunk in pieces:
             if not chunk.is_contiguous():
                 chunk = chunk.contiguous()
 

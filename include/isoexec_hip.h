@@ -351,6 +351,7 @@ int ix_moe_router_topk(const float* logits, long ld, long T, long E, long k, int
 long ix_moe_max_tiles(long T, long k, long E, long BM);   /* ceil(T*k/BM) + E */
 size_t ix_moe_permute_scratch_ints(long T, long E);
 int ix_moe_pick_bm(long T, long k, long E);               /* 32, 128 or 256 */
+int ix_moe_pick_bm_packed(long T, long k, long E);        /* 32, 64, 128 or 256: for callers that hold packed matrices */
 
 /* fused_permute_index / ref_permute_index (moe_router_o2_kernel.py:313-351,389-397) plus the
  * block map (moe_fused_experts.py:156-205) and the inverse permutation of
@@ -430,8 +431,12 @@ int ix_moe_experts_tile(const void* x, long ldx, const int* sorted_token, const 
  *   W1f [E][F / 128][wave 4][Hd / 64][b 2][s 4][lane 64]   row = b F + 128 nt + 32 wave + r   (b: gate, up)
  *   W2f [E][Hd / 256][wave 4][F / 64][b 2][s 4][lane 64]   row = 256 nt + 64 wave + 32 b + r
  * Serves Hd % 256 == 0, F % 128 == 0 with Hd / 64 and F / 64 in {8, 12, 16, 24, 32, 48, 64}; else declined. Pack once per
- * weight version (one pass over each matrix), not per step. ix_moe_experts_decode takes a block map of BM = 32. */
+ * weight version (one pass over each matrix), not per step. ix_moe_experts_packed takes a block map of BM = 32 or 64,
+ * ix_moe_experts_decode one of BM = 32. */
 int ix_moe_pack_decode(const void* W1, const void* W2, void* W1f, void* W2f, long E, long Hd, long F, void* stream);
+int ix_moe_experts_packed(const void* x, long ldx, const int* sorted_token, const float* permuted_prob, const void* W1f,
+                          const void* W2f, const int* tile_meta, long max_tiles, long BM, void* inter, void* expert_out,
+                          long T, long rows, long Hd, long F, void* stream);
 int ix_moe_experts_decode(const void* x, long ldx, const int* sorted_token, const float* permuted_prob, const void* W1f,
                           const void* W2f, const int* tile_meta, long max_tiles, void* inter, void* expert_out, long T,
                           long rows, long Hd, long F, void* stream);

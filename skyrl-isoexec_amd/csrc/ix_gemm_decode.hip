@@ -8,7 +8,8 @@
 //     wave's four matrix instructions take as their A operands, in (step, lane) order, so a load instruction is 1 KiB
 //     of contiguous memory and a wave walks one contiguous stream;
 //   * a lane holds the fragments of the next D = 8 k-tiles in registers (32 loads of 16 bytes in flight per lane; with
-//     eight waves on a CU 256 KiB of weight bytes in flight per CU);
+//     eight waves on a CU 256 KiB of weight bytes in flight per CU), loaded past the caches (ix_load16_once: LM head
+//     151936 x 4096 at M = 16 216 -> 189 us = 6.6 TB/s, 151936 x 2048 115 -> 101 us);
 //   * the activations -- the same at most 64 rows for every unit -- are staged once per workgroup: each k-tile of A is
 //     fetched straight into LDS in B-operand fragment order (memory -> LDS, 1 KiB pieces shared out over the waves), as
 //     far ahead as the weights, and every wave reads its B fragments from there. One barrier per k-tile, which couples
@@ -90,7 +91,7 @@ __global__ __launch_bounds__(NW * 64) void k_gemm_dec(const bf16_t* __restrict__
   auto load_w = [&](auto ktc) {
     constexpr int kt = decltype(ktc)::value;
 #pragma unroll
-    for (int c = 0; c < 4; ++c) wreg[kt % D][c] = wp[kt * 256 + c * 64];
+    for (int c = 0; c < 4; ++c) wreg[kt % D][c] = ix_load16_once(wp + kt * 256 + c * 64);
   };
 
   ix_f32x16 acc[TB];

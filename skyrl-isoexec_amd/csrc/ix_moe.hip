@@ -689,9 +689,22 @@ extern "C" size_t ix_moe_permute_scratch_ints(long T, long E) {
   return (size_t)(2 * ntiles * E);
 }
 
+// Rows per tile of the ring kernels, from the mean rows per expert. Measured (E = 128, Hd = 2048, F = 768, top-8; us fc1 + fc2
+// with tiles of 32 x 256 / 128 x 128 / 256 x 256): 128 tokens 221 / 221 / 237, 256 223 / 224 / 238, 400 246 / 233 / 242, 512
+// 260 / 233 / 245, 700 289 / 240 / 250, 1000 328 / 253 / 253, 1500 - / 272 / 272, 2000 - / 326 / 276. 128-row tiles go with
+// 128-column tiles (128 x 256: 256 at 700 tokens).
 extern "C" int ix_moe_pick_bm(long T, long k, long E) {
-  const long avg = (T * k) / (E > 0 ? E : 1);
-  return avg >= 96 ? 256 : (avg >= 48 ? 128 : 32);
+  const long rows = T * k, e = E > 0 ? E : 1;
+  return rows >= 88 * e ? 256 : (rows >= 20 * e ? 128 : 32);
+}
+
+// The same when fragment-packed copies of the matrices are at hand: the streaming kernels as long as every touched expert's
+// weights are the traffic. Measured (us fc1 + fc2 with streamed tiles of 32 / 64 rows, ring 128 x 128 / 256 x 256): 64 tokens
+// 176 / 177 / 219 / 242, 256 186 / 186 / 227 / 239, 512 282 / 222 / 235 / 248, 700 367 / 246 / 241 / 253, 1000 - / 366 / 254 /
+// 267.
+extern "C" int ix_moe_pick_bm_packed(long T, long k, long E) {
+  const long rows = T * k, e = E > 0 ? E : 1;
+  return rows >= 40 * e ? ix_moe_pick_bm(T, k, E) : (rows >= 16 * e ? 64 : 32);
 }
 
 extern "C" int ix_moe_permute(const int* topk_idx, const float* topk_prob, long T, long E, long k, long BM,
@@ -1435,19 +1448,23 @@ extern "C" int ix_moe_experts(const void* x, long ldx, const int* sorted_token, 
 //   * weights are stored FRAGMENT-PACKED (ix_moe_pack_decode): per (expert, column tile, wave, k-tile) the 8 KiB a wave's
 //     eight matrix instructions of that k-tile take as their A operands, in (block, step, lane) order, so that a load
 //     instruction is 1 KiB of contiguous memory and a wave walks one contiguous stream;
-//   * a lane keeps the fragments of the next D k-tiles in registers (D x 8 loads of 16 bytes in flight per lane, two
-//     workgroups per CU: up to 256 KiB of weight bytes in flight per CU);
-//   * activations (at most 32 token rows per tile, typically four live ones) come straight from memory as B operands,
+//   * a lane keeps the fragments of the next D k-tiles in registers (D x 8 loads of 16 bytes in flight per lane, eight
+//     waves per CU: up to 256 KiB of weight bytes in flight per CU), loaded past the caches (ix_load16_once);
+//   * activations (at most 32 token rows per block, typically four live ones) come straight from memory as B operands,
 //     a lane loading the 16 bytes of its own token, as far ahead as the weights; a dead token's lanes load a live row
-//     and multiply zeros instead. No barrier, no shared state: the four waves of a workgroup only share the tile.
+//     and multiply zeros instead;
+//   * a workgroup is ONE wave (a column tile's four waves share nothing), so that a step that touches few experts spreads
+//     over the chip: one token's eight experts are 192 workgroups instead of 48 (fc1 23.3 -> 10.4 us);
+//   * a block map of 64-row tiles (BM = 64) multiplies up to two blocks of 32 tokens with the same weight registers.
+// Measured (E = 128, Hd = 2048, F = 768, top-8; us fc1 / fc2, four waves and default loads -> this): T = 1 23.3 / 8.3 ->
+// 10.4 / 5.7; T = 64 132 / 68 -> 116 / 57 (7.0 TB/s); T = 512 (32-row tiles, experts with more rows read twice) 175 / 89 ->
+// 136 / 80 (64-row tiles).
 // Arithmetic is that of every other tile shape: v_mfma_f32_32x32x16_bf16, weights the A operand, K in tiles of 64, step
 // s consuming k = 8 s .. 8 s + 7 (lane group 0) and 32 + 8 s .. (lane group 1), one fp32 accumulator per element, the
 // epilogues of k_moe_fc1_glu / k_moe_fc2 statement for statement.
 // Packed layouts (16-byte chunk index; r = lane % 32, g = lane / 32; chunk = W[row][64 kt + 32 g + 8 s .. + 7]):
 //   W1f [E][F / 128][wave 4][Hd / 64][b 2][s 4][lane 64]   row = b F + 128 nt + 32 wave + r      (b: gate, up)
 //   W2f [E][Hd / 256][wave 4][F / 64][b 2][s 4][lane 64]   row = 256 nt + 64 wave + 32 b + r
-#define IX_DEC_D 4  // k-tiles of weight fragments a lane holds ahead of the matrix instructions
-
 __global__ __launch_bounds__(256) void k_moe_pack_frag(const bf16_t* __restrict__ W, bf16_t* __restrict__ Wf,
                                                        int rows_per_expert, int K, int nb, int is_fc1, long chunks) {
   const long i = (long)blockIdx.x * 256 + threadIdx.x;
@@ -1467,125 +1484,162 @@ __global__ __launch_bounds__(256) void k_moe_pack_frag(const bf16_t* __restrict_
   *reinterpret_cast<uint4*>(Wf + i * 8) = v;
 }
 
-template <int D>
+// D: k-tiles of fragments a lane holds ahead of the matrix instructions. TB: blocks of 32 token rows.
+template <int D, int TB>
 struct IxDecStream {
-  const uint4* wp;   // this lane's first chunk of the wave's stream: k-tile kt, chunk c at wp[kt * 512 + c * 64]
-  const bf16_t* xp;  // this lane's token row + 32 g (a dead token's lanes point at a live row and discard what they load)
-  bool live;
+  const uint4* wp;       // this lane's first chunk of the wave's stream: k-tile kt, chunk c at wp[kt * 512 + c * 64]
+  const bf16_t* xp[TB];  // this lane's token row + 32 g (a dead token's lanes point at a live row and discard what they load)
+  bool live[TB];
   uint4 wreg[D][8];
-  uint4 xreg[D][4];
-  __device__ __forceinline__ void load_w(uint4 (&dst)[8], int kt) {
+  uint4 xreg[D][TB][4];
+  __device__ __forceinline__ void load(int d, int kt) {
 #pragma unroll
-    for (int c = 0; c < 8; ++c) dst[c] = wp[(long)kt * 512 + c * 64];
-  }
-  __device__ __forceinline__ void load_x(uint4 (&dst)[4], int kt) {
+    for (int t = 0; t < TB; ++t)
 #pragma unroll
-    for (int st = 0; st < 4; ++st) dst[st] = *reinterpret_cast<const uint4*>(xp + 64 * kt + 8 * st);
-  }
-  template <int d>
-  __device__ __forceinline__ void multiply(const uint4 (&xc)[4], ix_f32x16& a0, ix_f32x16& a1) {
+      for (int st = 0; st < 4; ++st) xreg[d][t][st] = *reinterpret_cast<const uint4*>(xp[t] + 64 * kt + 8 * st);
 #pragma unroll
-    for (int st = 0; st < 4; ++st) {
-      uint4 xv = xc[st];
-      if (!live) xv = make_uint4(0u, 0u, 0u, 0u);  // a select, not a branch
-      const ix_bf16x8 xf = *reinterpret_cast<const ix_bf16x8*>(&xv);
-      a0 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(*reinterpret_cast<const ix_bf16x8*>(&wreg[d][st]), xf, a0, 0, 0, 0);
-      a1 = __builtin_amdgcn_mfma_f32_32x32x16_bf16(*reinterpret_cast<const ix_bf16x8*>(&wreg[d][4 + st]), xf, a1, 0, 0, 0);
-    }
+    for (int c = 0; c < 8; ++c) wreg[d][c] = ix_load16_once(wp + (long)kt * 512 + c * 64);
   }
-  // The whole product of a wave: two 32 x 32 blocks (weight chunks 0..3 -> a0, 4..7 -> a1) over KT_ k-tiles. KT_ is a
-  // compile-time constant and the walk is straight-line code: with a loop (or any branch) the compiler's wait
+  __device__ __forceinline__ void multiply(int d, ix_f32x16 (&a0)[TB], ix_f32x16 (&a1)[TB]) {
+#pragma unroll
+    for (int st = 0; st < 4; ++st)
+#pragma unroll
+      for (int t = 0; t < TB; ++t) {
+        uint4 xv = xreg[d][t][st];
+        if (!live[t]) xv = make_uint4(0u, 0u, 0u, 0u);  // a select, not a branch
+        const ix_bf16x8 xf = *reinterpret_cast<const ix_bf16x8*>(&xv);
+        a0[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(*reinterpret_cast<const ix_bf16x8*>(&wreg[d][st]), xf, a0[t], 0, 0, 0);
+        a1[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(*reinterpret_cast<const ix_bf16x8*>(&wreg[d][4 + st]), xf, a1[t], 0, 0, 0);
+      }
+  }
+  // The whole product of a wave: two 32 x 32 blocks per token block (weight chunks 0..3 -> a0, 4..7 -> a1) over KT_ k-tiles.
+  // KT_ is a compile-time constant and the walk is straight-line code: with a loop (or any branch) the compiler's wait
   // bookkeeping falls back to "wait for every load" at the join, which would drain the D k-tiles in flight at every
   // step; in straight-line code it waits for exactly the loads a matrix instruction reads.
   template <int KT_>
-  __device__ __forceinline__ void run(ix_f32x16& a0, ix_f32x16& a1) {
+  __device__ __forceinline__ void run(ix_f32x16 (&a0)[TB], ix_f32x16 (&a1)[TB]) {
     static_assert(KT_ >= D, "the ring is filled before the first multiply");
+#pragma unroll
+    for (int t = 0; t < TB; ++t)
+#pragma unroll
+      for (int i = 0; i < 16; ++i) a0[t][i] = a1[t][i] = 0.0f;
     // sched_barrier(0): the compiler's scheduler may not move a load across it -- left alone it sinks every load down
     // to its first use (fewest live registers), which is a ring of depth zero. Loads retire in order, so the
     // activation fragments of a k-tile are requested together with its weight fragments, D k-tiles ahead: a wait for
-    // k-tile kt then leaves the (D - 1) x 12 younger loads in flight.
-    ix_static_for<0, D>([&](auto dc) {
-      load_x(xreg[decltype(dc)::value], decltype(dc)::value);
-      load_w(wreg[decltype(dc)::value], decltype(dc)::value);
-    });
+    // k-tile kt then leaves the younger k-tiles' loads in flight.
+    ix_static_for<0, D>([&](auto dc) { load(decltype(dc)::value, decltype(dc)::value); });
     __builtin_amdgcn_sched_barrier(0);
     ix_static_for<0, KT_>([&](auto kc) {
       constexpr int kt = decltype(kc)::value, d = kt % D;
-      multiply<d>(xreg[d], a0, a1);
+      multiply(d, a0, a1);
       __builtin_amdgcn_sched_barrier(0);
-      if constexpr (kt + D < KT_) {
-        load_x(xreg[d], kt + D);
-        load_w(wreg[d], kt + D);
-      }
+      if constexpr (kt + D < KT_) load(d, kt + D);
       __builtin_amdgcn_sched_barrier(0);
     });
   }
 };
 
-template <int D, int KT>
-__global__ __launch_bounds__(256, 2) void k_moe_fc1_dec(const bf16_t* __restrict__ x, long ldx,
-                                                        const int* __restrict__ sorted_token,
-                                                        const float* __restrict__ permuted_prob,
-                                                        const bf16_t* __restrict__ W1f, const int* __restrict__ meta,
-                                                        int max_tiles, bf16_t* __restrict__ inter, int Hd, int F,
-                                                        int nb_n) {
-  int mt, nt;
-  if (!ix_moe_tile_of_block(blockIdx.x, meta[0], nb_n, &mt, &nt)) return;
-  const long e = meta[1 + mt];
-  const long row0 = meta[1 + max_tiles + mt];
-  const int nrows = meta[1 + 2 * max_tiles + mt];
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  const int r = lane & 31, g = lane >> 5;
-  const bool live = r < nrows;
-  IxDecStream<D> st;
-  st.wp = reinterpret_cast<const uint4*>(W1f) + (((e * nb_n + nt) * 4 + w) * (long)KT) * 512 + lane;
-  st.live = live;
-  st.xp = x + (long)sorted_token[row0 + (live ? r : 0)] * ldx + 32 * g;  // a tile has at least one row
-  ix_f32x16 ag, au;
+// unit -> (row tile, column tile, wave of the packed layout)
+struct IxDecUnit {
+  long e, row0, stream;  // stream: index of the unit's packed stream
+  int nrows, nt, w;
+  __device__ __forceinline__ bool init(const int* __restrict__ meta, int max_tiles, int nb_n) {
+    int mt, u;
+    if (!ix_moe_tile_of_block(blockIdx.x, meta[0], nb_n * 4, &mt, &u)) return false;
+    e = meta[1 + mt];
+    row0 = meta[1 + max_tiles + mt];
+    nrows = meta[1 + 2 * max_tiles + mt];
+    nt = u >> 2;
+    w = u & 3;
+    stream = (e * nb_n + nt) * 4 + w;
+    return true;
+  }
+};
+
+template <int D, int TB, int KT>
+__device__ __forceinline__ void ix_moe_fc1_dec_unit(const IxDecUnit& un, const bf16_t* __restrict__ x, long ldx,
+                                                    const int* __restrict__ sorted_token,
+                                                    const float* __restrict__ permuted_prob, const bf16_t* __restrict__ W1f,
+                                                    bf16_t* __restrict__ inter, int F) {
+  const int lane = threadIdx.x, r = lane & 31, g = lane >> 5;
+  IxDecStream<D, TB> st;
+  st.wp = reinterpret_cast<const uint4*>(W1f) + un.stream * (long)KT * 512 + lane;
 #pragma unroll
-  for (int i = 0; i < 16; ++i) ag[i] = au[i] = 0.0f;
+  for (int t = 0; t < TB; ++t) {
+    st.live[t] = 32 * t + r < un.nrows;
+    st.xp[t] = x + (long)sorted_token[un.row0 + (st.live[t] ? 32 * t + r : 0)] * ldx + 32 * g;  // a tile has at least one row
+  }
+  ix_f32x16 ag[TB], au[TB];
   st.template run<KT>(ag, au);
-  if (!live) return;
-  const long m = row0 + r;
-  const float prob = permuted_prob[m];
-  const int c0 = nt * 128 + w * 32;
+  const int c0 = un.nt * 128 + un.w * 32;
 #pragma unroll
-  for (int q = 0; q < 4; ++q) {
-    const int col = c0 + ix_acc_row(q * 4, lane);
-    const uint32_t lo = IxMoeFc1StreamJob::chain2(ag[q * 4], ag[q * 4 + 1], au[q * 4], au[q * 4 + 1], prob);
-    const uint32_t hi = IxMoeFc1StreamJob::chain2(ag[q * 4 + 2], ag[q * 4 + 3], au[q * 4 + 2], au[q * 4 + 3], prob);
-    *reinterpret_cast<uint2*>(inter + m * F + col) = make_uint2(lo, hi);  // col % 4 == 0, F % 8 == 0, inter 16-byte aligned
+  for (int t = 0; t < TB; ++t) {
+    if (!st.live[t]) continue;
+    const long m = un.row0 + 32 * t + r;
+    const float prob = permuted_prob[m];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const int col = c0 + ix_acc_row(q * 4, lane);
+      const uint32_t lo = IxMoeFc1StreamJob::chain2(ag[t][q * 4], ag[t][q * 4 + 1], au[t][q * 4], au[t][q * 4 + 1], prob);
+      const uint32_t hi =
+          IxMoeFc1StreamJob::chain2(ag[t][q * 4 + 2], ag[t][q * 4 + 3], au[t][q * 4 + 2], au[t][q * 4 + 3], prob);
+      *reinterpret_cast<uint2*>(inter + m * F + col) = make_uint2(lo, hi);  // col % 4 == 0, F % 8 == 0, inter 16-byte aligned
+    }
   }
 }
 
-template <int D, int KT>
-__global__ __launch_bounds__(256, 2) void k_moe_fc2_dec(const bf16_t* __restrict__ inter, const bf16_t* __restrict__ W2f,
-                                                        const int* __restrict__ meta, int max_tiles,
-                                                        bf16_t* __restrict__ out, int Hd, int F, int nb_n) {
-  int mt, nt;
-  if (!ix_moe_tile_of_block(blockIdx.x, meta[0], nb_n, &mt, &nt)) return;
-  const long e = meta[1 + mt];
-  const long row0 = meta[1 + max_tiles + mt];
-  const int nrows = meta[1 + 2 * max_tiles + mt];
-  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-  const int r = lane & 31, g = lane >> 5;
-  const bool live = r < nrows;
-  IxDecStream<D> st;
-  st.wp = reinterpret_cast<const uint4*>(W2f) + (((e * nb_n + nt) * 4 + w) * (long)KT) * 512 + lane;
-  st.live = live;
-  st.xp = inter + (row0 + (live ? r : 0)) * (long)F + 32 * g;  // a tile has at least one row
-  ix_f32x16 a0, a1;
+template <int D, int TB, int KT>
+__device__ __forceinline__ void ix_moe_fc2_dec_unit(const IxDecUnit& un, const bf16_t* __restrict__ inter,
+                                                    const bf16_t* __restrict__ W2f, bf16_t* __restrict__ out, int Hd, int F) {
+  const int lane = threadIdx.x, r = lane & 31, g = lane >> 5;
+  IxDecStream<D, TB> st;
+  st.wp = reinterpret_cast<const uint4*>(W2f) + un.stream * (long)KT * 512 + lane;
 #pragma unroll
-  for (int i = 0; i < 16; ++i) a0[i] = a1[i] = 0.0f;
-  st.template run<KT>(a0, a1);
-  if (!live) return;
-  const long m = row0 + r;
-#pragma unroll
-  for (int q = 0; q < 4; ++q) {
-    const long n = (long)nt * 256 + w * 64 + ix_acc_row(q * 4, lane);
-    ix_store4_bf16(out + m * Hd + n, 4, true, a0[q * 4], a0[q * 4 + 1], a0[q * 4 + 2], a0[q * 4 + 3]);
-    ix_store4_bf16(out + m * Hd + n + 32, 4, true, a1[q * 4], a1[q * 4 + 1], a1[q * 4 + 2], a1[q * 4 + 3]);
+  for (int t = 0; t < TB; ++t) {
+    st.live[t] = 32 * t + r < un.nrows;
+    st.xp[t] = inter + (un.row0 + (st.live[t] ? 32 * t + r : 0)) * (long)F + 32 * g;
   }
+  ix_f32x16 a0[TB], a1[TB];
+  st.template run<KT>(a0, a1);
+#pragma unroll
+  for (int t = 0; t < TB; ++t) {
+    if (!st.live[t]) continue;
+    const long m = un.row0 + 32 * t + r;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const long n = (long)un.nt * 256 + un.w * 64 + ix_acc_row(q * 4, lane);
+      ix_store4_bf16(out + m * Hd + n, 4, true, a0[t][q * 4], a0[t][q * 4 + 1], a0[t][q * 4 + 2], a0[t][q * 4 + 3]);
+      ix_store4_bf16(out + m * Hd + n + 32, 4, true, a1[t][q * 4], a1[t][q * 4 + 1], a1[t][q * 4 + 2], a1[t][q * 4 + 3]);
+    }
+  }
+}
+
+// BM = 32 or 64: the block map's rows per tile. Four k-tiles ahead for one block of tokens (three where a long K's addresses
+// would push registers out to memory), two for two: both leave two waves per SIMD; deeper rings with one wave measured slower.
+template <int KT, int BM>
+__global__ __launch_bounds__(64, 2) void k_moe_fc1_dec(const bf16_t* __restrict__ x, long ldx,
+                                                       const int* __restrict__ sorted_token,
+                                                       const float* __restrict__ permuted_prob,
+                                                       const bf16_t* __restrict__ W1f, const int* __restrict__ meta,
+                                                       int max_tiles, bf16_t* __restrict__ inter, int F, int nb_n) {
+  IxDecUnit un;
+  if (!un.init(meta, max_tiles, nb_n)) return;
+  if (BM == 32 || un.nrows <= 32)
+    ix_moe_fc1_dec_unit<(KT <= 32 ? 4 : 3), 1, KT>(un, x, ldx, sorted_token, permuted_prob, W1f, inter, F);
+  else
+    ix_moe_fc1_dec_unit<2, 2, KT>(un, x, ldx, sorted_token, permuted_prob, W1f, inter, F);
+}
+
+template <int KT, int BM>
+__global__ __launch_bounds__(64, 2) void k_moe_fc2_dec(const bf16_t* __restrict__ inter, const bf16_t* __restrict__ W2f,
+                                                       const int* __restrict__ meta, int max_tiles,
+                                                       bf16_t* __restrict__ out, int Hd, int F, int nb_n) {
+  IxDecUnit un;
+  if (!un.init(meta, max_tiles, nb_n)) return;
+  if (BM == 32 || un.nrows <= 32)
+    ix_moe_fc2_dec_unit<(KT <= 12 ? 4 : 3), 1, KT>(un, inter, W2f, out, Hd, F);
+  else
+    ix_moe_fc2_dec_unit<2, 2, KT>(un, inter, W2f, out, Hd, F);
 }
 
 // The k-tile counts the straight-line kernels are instantiated for (K = 64 KT).
@@ -1617,34 +1671,52 @@ extern "C" int ix_moe_pack_decode(const void* W1, const void* W2, void* W1f, voi
   return ix_launch_status();
 }
 
-// ix_moe_experts for a block map of 32-row tiles (BM = 32), reading the fragment-packed matrices.
-extern "C" int ix_moe_experts_decode(const void* x, long ldx, const int* sorted_token, const float* permuted_prob,
-                                     const void* W1f, const void* W2f, const int* tile_meta, long max_tiles, void* inter,
-                                     void* expert_out, long T, long rows, long Hd, long F, void* stream) {
+// ix_moe_experts for a block map of 32- or 64-row tiles, reading the fragment-packed matrices.
+extern "C" int ix_moe_experts_packed(const void* x, long ldx, const int* sorted_token, const float* permuted_prob,
+                                     const void* W1f, const void* W2f, const int* tile_meta, long max_tiles, long BM,
+                                     void* inter, void* expert_out, long T, long rows, long Hd, long F, void* stream) {
   if (!x || !sorted_token || !permuted_prob || !W1f || !W2f || !tile_meta || !inter || !expert_out) return IX_ERR_ARG;
-  if (T < 0 || rows < 0 || Hd <= 0 || F <= 0 || max_tiles < 0 || ldx < Hd) return IX_ERR_ARG;
+  if (T < 0 || rows < 0 || Hd <= 0 || F <= 0 || max_tiles < 0 || ldx < Hd || (BM != 32 && BM != 64)) return IX_ERR_ARG;
   if (!ix_moe_decode_serves(Hd, F) || (ldx % 8) || !ix_aligned(x, 16) || !ix_aligned(W1f, 16) || !ix_aligned(W2f, 16) ||
       !ix_aligned(inter, 16) || !ix_aligned(expert_out, 16))
     return IX_DECLINED;
   if (rows == 0 || max_tiles == 0) return IX_OK;
   const long nb1 = F / 128, nb2 = Hd / 256;
-  if (max_tiles * nb1 > 0x7fffffffL || max_tiles * nb2 > 0x7fffffffL) return IX_DECLINED;
+  const long tiles = max_tiles < rows ? max_tiles : rows;  // every tile has a row
+  const long u1 = tiles * nb1 * 4, u2 = tiles * nb2 * 4;
+  if (u1 > 0x7ffffff0L || u2 > 0x7ffffff0L) return IX_DECLINED;
+  const dim3 g1((unsigned)(8 * ((u1 + 7) / 8))), g2((unsigned)(8 * ((u2 + 7) / 8)));
   hipStream_t st = (hipStream_t)stream;
-#define IX_DEC_FC1(KT_)                                                                                               \
-  if (Hd / 64 == KT_)                                                                                                 \
-    hipLaunchKernelGGL((k_moe_fc1_dec<IX_DEC_D, KT_>), dim3((unsigned)(8 * ((max_tiles * nb1 + 7) / 8))), dim3(256), 0, st, \
-                       (const bf16_t*)x, ldx, sorted_token, permuted_prob, (const bf16_t*)W1f, tile_meta, (int)max_tiles, \
-                       (bf16_t*)inter, (int)Hd, (int)F, (int)nb1);
-#define IX_DEC_FC2(KT_)                                                                                               \
-  if (F / 64 == KT_)                                                                                                  \
-    hipLaunchKernelGGL((k_moe_fc2_dec<IX_DEC_D, KT_>), dim3((unsigned)(8 * ((max_tiles * nb2 + 7) / 8))), dim3(256), 0, st, \
-                       (const bf16_t*)inter, (const bf16_t*)W2f, tile_meta, (int)max_tiles, (bf16_t*)expert_out, (int)Hd, \
-                       (int)F, (int)nb2);
+#define IX_DEC_FC1_BM(KT_, BM_)                                                                                     \
+  hipLaunchKernelGGL((k_moe_fc1_dec<KT_, BM_>), g1, dim3(64), 0, st, (const bf16_t*)x, ldx, sorted_token, permuted_prob, \
+                     (const bf16_t*)W1f, tile_meta, (int)max_tiles, (bf16_t*)inter, (int)F, (int)nb1)
+#define IX_DEC_FC2_BM(KT_, BM_)                                                                                      \
+  hipLaunchKernelGGL((k_moe_fc2_dec<KT_, BM_>), g2, dim3(64), 0, st, (const bf16_t*)inter, (const bf16_t*)W2f, tile_meta, \
+                     (int)max_tiles, (bf16_t*)expert_out, (int)Hd, (int)F, (int)nb2)
+#define IX_DEC_FC1(KT_)                          \
+  if (Hd / 64 == KT_) {                          \
+    if (BM == 32) IX_DEC_FC1_BM(KT_, 32);        \
+    else IX_DEC_FC1_BM(KT_, 64);                 \
+  }
+#define IX_DEC_FC2(KT_)                          \
+  if (F / 64 == KT_) {                           \
+    if (BM == 32) IX_DEC_FC2_BM(KT_, 32);        \
+    else IX_DEC_FC2_BM(KT_, 64);                 \
+  }
   IX_DEC_KTS(IX_DEC_FC1)
   IX_DEC_KTS(IX_DEC_FC2)
 #undef IX_DEC_FC1
 #undef IX_DEC_FC2
+#undef IX_DEC_FC1_BM
+#undef IX_DEC_FC2_BM
   return ix_launch_status();
+}
+
+extern "C" int ix_moe_experts_decode(const void* x, long ldx, const int* sorted_token, const float* permuted_prob,
+                                     const void* W1f, const void* W2f, const int* tile_meta, long max_tiles, void* inter,
+                                     void* expert_out, long T, long rows, long Hd, long F, void* stream) {
+  return ix_moe_experts_packed(x, ldx, sorted_token, permuted_prob, W1f, W2f, tile_meta, max_tiles, 32, inter, expert_out, T,
+                               rows, Hd, F, stream);
 }
 
 // ---------------------------------------------------------------------------------------------

@@ -129,6 +129,11 @@ SIGNATURES = {
         [P, c_long, P, P, P, P, P, c_long, c_long, c_long, P, P, c_long, c_long, c_long, c_long, P],
     ),
     "ix_moe_pack_decode": (c_int, [P, P, P, P, c_long, c_long, c_long, P]),
+    "ix_moe_pick_bm_packed": (c_int, [c_long, c_long, c_long]),
+    "ix_moe_experts_packed": (
+        c_int,
+        [P, c_long, P, P, P, P, P, c_long, c_long, P, P, c_long, c_long, c_long, c_long, P],
+    ),
     "ix_moe_experts_decode": (
         c_int,
         [P, c_long, P, P, P, P, P, c_long, P, P, c_long, c_long, c_long, c_long, P],

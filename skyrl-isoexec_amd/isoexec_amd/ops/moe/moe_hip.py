@@ -64,7 +64,7 @@ def permute(topk_idx: torch.Tensor, topk_prob: torch.Tensor, E: int, *, BM: int 
     p = Permutation()
     p.T, p.E, p.k = T, E, k
     p.BM = int(BM or L.ix_moe_pick_bm(T, k, E))
-    p.BN = int(BN or 256)          # weight-tile width of the grouped GEMMs: 256, or 128 with BM = 128
+    p.BN = int(BN or (128 if p.BM == 128 else 256))  # weight-tile width of the grouped GEMMs: 256, or 128 with BM = 128
     p.max_tiles = int(L.ix_moe_max_tiles(T, k, E, p.BM))
     i32 = dict(dtype=torch.int32, device=dev)
     p.counts = torch.empty(E, **i32)
@@ -111,7 +111,7 @@ def route_and_permute(logits: torch.Tensor, k: int, *, pre_softmax: bool = False
     p = Permutation()
     p.T, p.E, p.k = T, E, k
     p.BM = int(BM or L.ix_moe_pick_bm(T, k, E))
-    p.BN = 256
+    p.BN = 128 if p.BM == 128 else 256
     p.max_tiles = int(L.ix_moe_max_tiles(T, k, E, p.BM))
     i32 = dict(dtype=torch.int32, device=dev)
     idx = torch.empty(T, k, **i32)
@@ -166,7 +166,8 @@ def experts_forward(x: torch.Tensor, w1: torch.Tensor, w2: torch.Tensor, p: Perm
     """Grouped fc1 + SwiGLU + prob epilogue + fc2 over the permuted rows. ``x [T, H]`` bf16,
     ``w1 [E, 2F, H]``, ``w2 [E, H, F]``. Returns ``expert_out [T*k, H]`` in permuted order; with ``return_inter`` also
     the activation that enters fc2, ``inter [T*k, F]`` = bf16(bf16(bf16(silu(gate)) * up) * prob). ``packed``
-    (``pack_decode(w1, w2)``): read by the decode-size tile (BM = 32) instead of ``w1`` / ``w2``; same bits."""
+    (``pack_decode(w1, w2)``): read by the decode-size tiles (BM = 32 or 64) instead of ``w1`` / ``w2``; same bits. A plan with
+    BM = 64 needs them."""
     _lib.require_device(x, w1, w2)
     if x.dtype is not torch.bfloat16 or w1.dtype is not torch.bfloat16 or w2.dtype is not torch.bfloat16:
         raise RuntimeError("[isoexec-amd] experts serve bf16 only")
@@ -178,15 +179,15 @@ def experts_forward(x: torch.Tensor, w1: torch.Tensor, w2: torch.Tensor, p: Perm
     inter = torch.empty(rows, F, dtype=torch.bfloat16, device=dev)
     out = torch.empty(rows, H, dtype=torch.bfloat16, device=dev)
     xc = x if x.stride(1) == 1 else x.contiguous()
-    if packed is not None and p.BM == 32 and p.BN == 256:
+    if packed is not None and p.BM in (32, 64) and p.BN == 256:
         w1f, w2f = packed
         if w1f.shape != w1.shape or w2f.shape != w2.shape or w1f.dtype is not torch.bfloat16 or w2f.dtype is not torch.bfloat16:
             raise RuntimeError("[isoexec-amd] packed must come from pack_decode(w1, w2)")
         rc = _lib.check(
-            _lib.lib().ix_moe_experts_decode(xc.data_ptr(), xc.stride(0), p.sorted_token.data_ptr(),
+            _lib.lib().ix_moe_experts_packed(xc.data_ptr(), xc.stride(0), p.sorted_token.data_ptr(),
                                              p.permuted_prob.data_ptr(), w1f.data_ptr(), w2f.data_ptr(),
-                                             p.tile_meta.data_ptr(), p.max_tiles, inter.data_ptr(), out.data_ptr(), T, rows,
-                                             H, F, _lib.current_stream(dev)), "ix_moe_experts_decode")
+                                             p.tile_meta.data_ptr(), p.max_tiles, p.BM, inter.data_ptr(), out.data_ptr(), T,
+                                             rows, H, F, _lib.current_stream(dev)), "ix_moe_experts_packed")
         if rc == _lib.IX_OK:
             return (out, inter) if return_inter else out
     rc = _lib.check(
@@ -246,6 +247,8 @@ def moe_ffn_forward(x: torch.Tensor, router_weight: torch.Tensor, w1: torch.Tens
         raise RuntimeError("[isoexec-amd] router GEMM declined")
     if logit_bias is not None:
         logits = logits + logit_bias  # elementwise, per token
+    if BM is None and packed is not None:
+        BM = int(_lib.lib().ix_moe_pick_bm_packed(logits.shape[0], k, logits.shape[1]))
     idx, prob, p = route_and_permute(logits, k, pre_softmax=pre_softmax, scaling_factor=scaling_factor, BM=BM)
     if routing_out is not None:
         routing_out.append(idx)

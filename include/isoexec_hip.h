@@ -456,6 +456,45 @@ int ix_moe_combine(const void* expert_out, const int* combine_rows, void* out, l
 int ix_moe_combine_weighted(const void* expert_out, int in_dtype, const float* row_weight, int arith_dtype,
                             const int* combine_rows, void* out, int out_dtype, long T, long Hd, long k, void* stream);
 
+/* ---- one decode step of the hybrid model in one call ------------------------------------------
+ * The engine's step (the role of gptmodel_vllm.py's forward at one token per sequence): embedding + norm, then per layer the
+ * mixer (GatedDeltaNet out of its state pools, or attention out of its key/value cache), the residual add + norm and the
+ * mixture of experts, by the entry points above in this order; the bits of calling them one by one. */
+typedef struct IxDecodeDims {
+  int64_t n, layers, hidden, vocab;
+  int64_t max_positions;                          /* rows of the rotary tables */
+  int64_t gdn_k_heads, gdn_v_heads, gdn_head_dim; /* K = V = gdn_head_dim = 128, conv width 4, silu */
+  int64_t q_heads, kv_heads, head_dim;            /* rotary over the whole head */
+  int64_t experts, topk, expert_inter;            /* softmax, top-k, renormalise */
+  int64_t packed_experts;                         /* 1: every layer has w1_packed / w2_packed */
+  int64_t combine_fp32;                           /* sum of a token's expert rows in fp32 (else bf16) */
+} IxDecodeDims;
+
+/* Device pointers of one layer; every tensor contiguous and 16-byte aligned, bf16 unless noted. Fields of the other kind of
+ * layer are ignored. *_packed: ix_gemm_pack_decode / ix_moe_pack_decode copies, or NULL. */
+typedef struct IxDecodeLayer {
+  int64_t kind; /* 0: GatedDeltaNet, 1: attention */
+  const void *post_norm, *next_norm, *router, *w1, *w2, *w1_packed, *w2_packed; /* next_norm: the norm after the layer */
+  const void *w_in, *w_in_packed, *w_out, *w_out_packed; /* [q k v z beta a | q k v, hidden], [hidden, heads * dim] */
+  const void *conv_weight, *conv_bias;
+  const float *A_log, *dt_bias;
+  const void* out_norm;
+  float* ssm_state;
+  void* conv_state;
+  const int64_t* slot2row; /* [map_n]: slot id -> pool row */
+  int64_t map_n;
+  int64_t *last_used, *clock;
+  void *k_cache, *v_cache; /* [rows * max_len, kv_heads, head_dim] */
+} IxDecodeLayer;
+
+size_t ix_decode_step_workspace_bytes(const IxDecodeDims* dims); /* 0: not served */
+
+/* dims and layers in HOST memory, read during the call. tokens, slots int64 [n]; ctx int32 [n]: each sequence's position of
+ * this token, advanced by one on the device; kv_start int64 [n]. out bf16 [n, hidden]: the normed hidden states. */
+int ix_decode_step(const IxDecodeDims* dims, const IxDecodeLayer* layers, const void* embed, const void* pre_norm,
+                   const void* cos_table, const void* sin_table, const int64_t* tokens, const int64_t* slots, int* ctx,
+                   const int64_t* kv_start, float eps, void* workspace, size_t workspace_bytes, void* out, void* stream);
+
 /* ---- order-invariant digests: debug/thash ------------------------------------------------- */
 
 #define IX_DIGEST_MAX_MASKS 8

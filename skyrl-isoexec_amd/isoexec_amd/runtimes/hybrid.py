@@ -17,11 +17,13 @@ Layer layout (pre-norm residual stream, hidden H):
 
 from __future__ import annotations
 
+from array import array
 from dataclasses import dataclass, field
 
 import numpy as np
 import torch
 
+from .. import _lib
 from ..debug.trace import get_tracer
 from ..ops.attention.varlen_attn import KVCache, varlen_attention
 from ..ops.gdn.gdn_ops import conv_packed, gdn_native_core, gdn_native_core_normed
@@ -491,24 +493,107 @@ class RolloutEngine:
 
     def _decode_state(self, slots: list):
         """Device-resident description of a decode batch: slot ids, each sequence's context length
-        (advanced on the device after every step) and where its keys start."""
-        dev = self.blocks.w.embed.device
+        (advanced on the device after every step) and where its keys start. One asynchronous upload."""
         n = len(slots)
-        ctx = np.array([self.context[s] for s in slots], dtype=np.int32)
-        rows = np.array([self.kv_rows[s] for s in slots], dtype=np.int64)
+        host = torch.empty(2 * n + (n + 1) // 2, dtype=torch.int64, pin_memory=True)
+        a = host.numpy()
+        a[:n] = slots
+        a[n : 2 * n] = [self.kv_rows[s] * self.max_len for s in slots]
+        a[2 * n :].view(np.int32)[:n] = [self.context[s] for s in slots]
+        t = host.to(self.blocks.w.embed.device, non_blocking=True)
         return {
             "slots": list(slots),
-            "slots_t": torch.tensor(slots, dtype=torch.int64, device=dev),
-            "ctx": torch.from_numpy(ctx).to(dev),
-            "kv_start": torch.from_numpy(rows * self.max_len).to(dev),
-            "cu": torch.arange(n + 1, dtype=torch.int32, device=dev),
+            "slots_t": t[:n],
+            "ctx": t[2 * n :].view(torch.int32)[:n],
+            "kv_start": t[n : 2 * n],
         }
+
+    def _native_step_tables(self, n: int):
+        """``(dims, layers)`` for ``ix_decode_step``: the layers' device pointers as they are now (tables are built anew for
+        every step, so a replaced weight or a moved pool is seen), or ``None`` when the step has to be taken op by op: a
+        log or a trace wants the ops' outputs, or something is not the plain contiguous tensor the call expects."""
+        b, c = self.blocks, self.cfg
+        if b.region_log is not None or b.routing_log is not None or c.gdn_kernel != "recurrent" or c.conv_width != 4:
+            return None
+        bf16, f32, i64 = torch.bfloat16, torch.float32, torch.int64
+        ok = True
+
+        def ptr(t, dtype, *shape):
+            nonlocal ok
+            p = t.data_ptr()
+            if t.dtype is not dtype or not t.is_contiguous() or p % 16 or (shape and tuple(t.shape) != shape) or not t.is_cuda:
+                ok = False
+            return p
+
+        H, F, E, D = c.hidden, c.expert_inter, c.experts, c.gdn_qkv
+        packed_all = len(b.packed_experts) == c.layers
+        table = []
+        for i, lw in enumerate(b.w.layers):
+            attention = c.is_attention(i)
+            nxt = b.w.layers[i + 1]["pre_norm"] if i + 1 < c.layers else b.w.final_norm
+            row = [int(attention), ptr(lw["post_norm"], bf16, H), ptr(nxt, bf16, H), ptr(lw["router"], bf16, E, H),
+                   ptr(lw["w1"], bf16, E, 2 * F, H), ptr(lw["w2"], bf16, E, H, F)]
+            row += [t.data_ptr() for t in b.packed_experts[i]] if packed_all else [0, 0]
+            names = ("qkv_proj", "o_proj") if attention else ("in_proj", "out_proj")
+            for name in names:
+                pk = b.packed_dense.get((i, name))
+                row += [ptr(lw[name], bf16), 0 if pk is None else pk.packed.data_ptr()]
+            if attention:
+                kv = self.kv[i]
+                row += [0] * 11 + [ptr(kv.k, bf16), ptr(kv.v, bf16)]
+                ok = ok and lw["qkv_proj"].shape == ((c.q_heads + 2 * c.kv_heads) * c.head_dim, H)
+            else:
+                g = self.gdn[i]
+                if type(g) is not RecurrentGDN or g.table is None or g.activation not in ("silu", "swish") or not g.fused_decode_prep:
+                    return None
+                row += [ptr(g.conv_weight, bf16, D, 4), 0 if g.conv_bias is None else ptr(g.conv_bias, bf16, D),
+                        ptr(g.A_log, f32), ptr(g.dt_bias, f32), ptr(lw["out_norm"], bf16, c.gdn_head_dim),
+                        ptr(g.ssm_state, f32), ptr(g.conv_state, bf16), ptr(g.slot2row, i64), g.slot2row.numel(),
+                        ptr(g.last_used, i64), ptr(g._clock, i64), 0, 0]
+                ok = ok and lw["in_proj"].shape == (D + c.gdn_z + 2 * c.gdn_v_heads, H)
+            table += row
+        if not ok:
+            return None
+        dims = array("q", [n, c.layers, H, c.vocab, b.cos.shape[0], c.gdn_k_heads, c.gdn_v_heads, c.gdn_head_dim, c.q_heads,
+                           c.kv_heads, c.head_dim, E, c.topk, F, int(packed_all), int(c.moe_combine_dtype == "fp32")])
+        return dims, array("q", table)
+
+    def _decode_native(self, st: dict, tokens: torch.Tensor):
+        """The step by ``ix_decode_step``: every launch of every layer from one call. Same bits as the ops one by one.
+        ``None`` when it has to be taken op by op (nothing launched)."""
+        b = self.blocks
+        n = tokens.shape[0]
+        if tokens.dtype is not torch.int64 or tokens.ndim != 1 or not tokens.is_contiguous() or n == 0 or n != len(st["slots"]):
+            return None
+        tables = self._native_step_tables(n)
+        if tables is None:
+            return None
+        dims, layers = tables
+        L = _lib.lib()
+        need = int(L.ix_decode_step_workspace_bytes(dims.buffer_info()[0]))
+        w = b.w
+        if need == 0 or not w.embed.is_contiguous() or w.embed.dtype is not torch.bfloat16:
+            return None
+        dev = w.embed.device
+        _lib.require_device(tokens, w.embed)
+        work = torch.empty(need, dtype=torch.uint8, device=dev)
+        out = torch.empty(n, self.cfg.hidden, dtype=torch.bfloat16, device=dev)
+        rc = _lib.check(
+            L.ix_decode_step(dims.buffer_info()[0], layers.buffer_info()[0], w.embed.data_ptr(),
+                             w.layers[0]["pre_norm"].data_ptr(), b.cos.data_ptr(), b.sin.data_ptr(), tokens.data_ptr(),
+                             st["slots_t"].data_ptr(), st["ctx"].data_ptr(), st["kv_start"].data_ptr(), float(self.cfg.eps),
+                             work.data_ptr(), need, out.data_ptr(), _lib.current_stream(dev)), "ix_decode_step")
+        return out if rc == _lib.IX_OK else None
 
     def _decode_device(self, st: dict, tokens: torch.Tensor) -> torch.Tensor:
         """One decode step from device tensors only (no host read, fixed shapes): what a captured graph
         replays. Advances ``st["ctx"]`` in place."""
+        x = self._decode_native(st, tokens)
+        if x is not None:
+            return x
         b, c = self.blocks, self.cfg
-        positions, kv_start, cu, slots_t = st["ctx"], st["kv_start"], st["cu"], st["slots_t"]
+        positions, kv_start, slots_t = st["ctx"], st["kv_start"], st["slots_t"]
+        cu = torch.arange(len(st["slots"]) + 1, dtype=torch.int32, device=positions.device)
         kv_index = kv_start + positions
 
         def mixer(i, x):
@@ -576,8 +661,7 @@ class RolloutEngine:
 class DecodeGraph:
     """One decode step of a fixed batch, captured once and replayed.
 
-    A decode step is ~45 small launches per layer; at batch 64 their launch cost is about half the step.
-    The step reads nothing on the host and every shape is fixed, so the whole step is recorded into one
+    A decode step is ~11 small launches per layer. The step reads nothing on the host and every shape is fixed, so the whole step is recorded into one
     HIP graph: the token ids live in a static input tensor, each sequence's position in a device counter
     the graph itself advances, and the output in a static tensor the caller must consume before the next
     replay. Replays run the same kernels on the same data as the eager step, so the bits are identical.

@@ -1,0 +1,86 @@
+"""The decode step as one native call against the same step op by op: hidden states, every pool and the context counters."""
+
+import pytest
+import torch
+
+from _util import cpu_gen, same_bits
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+def config(**kw):
+    from isoexec_amd.runtimes.hybrid import HybridConfig
+
+    base = dict(hidden=512, vocab=1024, layers=4, attention_every=2, gdn_k_heads=2, gdn_v_heads=4, q_heads=4, kv_heads=2,
+                experts=16, topk=4, expert_inter=256, max_positions=256)
+    return HybridConfig(**{**base, **kw})
+
+
+def pools(engine):
+    for i, g in engine.gdn.items():
+        for name in ("ssm_state", "conv_state", "last_used", "_clock"):
+            yield f"gdn {i} {name}", getattr(g, name)
+    for i, kv in engine.kv.items():
+        yield f"keys {i}", kv.k
+        yield f"values {i}", kv.v
+
+
+@pytest.mark.parametrize("n,kw", [
+    (1, {}), (5, {}), (70, {}), (300, {}),                           # one-launch routing up to 256 tokens, packed dense up to 64
+    (3, dict(hidden=2048, topk=8, experts=128, expert_inter=512)),
+    (4, dict(experts=200, topk=2, hidden=2048)),                     # more experts than the one-launch routing holds
+    (6, dict(moe_combine_dtype="bf16", attention_every=4)),
+])
+@pytest.mark.parametrize("packed", [True, False])
+def test_native_step_equals_the_step_op_by_op(n, kw, packed):
+    from isoexec_amd.runtimes.hybrid import HybridWeights, RolloutEngine
+
+    cfg = config(**kw)
+    w = HybridWeights.make(cfg, seed=3, device=DEV)
+    g = cpu_gen(n)
+    lens = [1 + (7 * i) % 11 for i in range(n)]
+    tokens = torch.randint(0, cfg.vocab, (sum(lens),), generator=g).to(DEV)
+    engines = [RolloutEngine(cfg, w, max_num_seqs=n, max_len=32, pack_expert_weights=packed) for _ in range(2)]
+    slots = [(5 * i + 2) % 1021 for i in range(n)]
+    for e in engines:
+        e.prefill(slots, tokens, lens)
+    one, ops = engines
+    for step in range(3):
+        tok = torch.randint(0, cfg.vocab, (n,), generator=g).to(DEV)
+        ops.blocks.routing_log = []          # the log wants every layer's routing: op by op
+        want = ops.decode(slots, tok)
+        assert len(ops.blocks.routing_log) == cfg.layers
+        got = one.decode(slots, tok)
+        assert same_bits(got, want), step
+        for (name, a), (_, b) in zip(pools(one), pools(ops)):
+            assert torch.equal(a.reshape(-1).view(torch.uint8), b.reshape(-1).view(torch.uint8)), (step, name)
+    # a captured step replays the native call: counters advance on the device, a replaced weight is seen by the next eager step
+    graph = one.capture_decode(slots)
+    ops.blocks.routing_log = None
+    for step in range(3):
+        tok = torch.randint(0, cfg.vocab, (n,), generator=g).to(DEV)
+        ops.blocks.routing_log = []
+        want = ops.decode(slots, tok)
+        assert same_bits(graph.step(tok), want), step
+        assert graph.state["ctx"].tolist() == [one.context[s] for s in slots]
+
+
+def test_native_step_is_taken_and_sees_replaced_weights():
+    from isoexec_amd.runtimes.hybrid import HybridWeights, RolloutEngine
+
+    cfg = config()
+    w = HybridWeights.make(cfg, seed=4, device=DEV)
+    e = RolloutEngine(cfg, w, max_num_seqs=2, max_len=32)
+    e.prefill([0, 1], torch.tensor([1, 2, 3], device=DEV), [2, 1])
+    tok = torch.tensor([5, 6], device=DEV)
+    st = e._decode_state([0, 1])
+    first = e._decode_native(st, tok)
+    assert first is not None and st["ctx"].tolist() == [3, 2]
+    # tables are built per call: another norm weight, then a tensor the call cannot take (strided), which goes op by op
+    w.final_norm = w.final_norm + 1.0
+    moved = e._decode_native(e._decode_state([0, 1]), tok)
+    assert moved is not None and not same_bits(moved, first)
+    w.layers[0]["out_proj"] = torch.cat([w.layers[0]["out_proj"]] * 2, dim=1)[:, : cfg.gdn_z]
+    assert e._decode_native(e._decode_state([0, 1]), tok) is None
+    assert torch.isfinite(e.decode([0, 1], tok).float()).all()

@@ -69,7 +69,7 @@ __device__ __forceinline__ bool ix_tile_of_block(unsigned bid, int nb_m, int nb_
 // TC = bf16_t: C is the bf16 round of the fp32 accumulator; TC = float: the accumulator itself.
 // row_max_parts (optional): [M, parts_ld] fp32, entry (m, tn) = max over the tile's columns of the
 // values stored to C (exact, order-free), so a consumer can skip its own max pass over C.
-template <int BM, int BN, int WM, int WN, typename TC, int PW = 0>
+template <int BM, int BN, int WM, int WN, typename TC, int PW = 0, bool W_ONCE = false>
 __global__ __launch_bounds__((WM * WN + PW) * 64) void k_gemm_bf16_nt(const bf16_t* __restrict__ A, long lda,
                                                               const bf16_t* __restrict__ W, long ldw,
                                                               const bf16_t* __restrict__ bias,
@@ -77,7 +77,7 @@ __global__ __launch_bounds__((WM * WN + PW) * 64) void k_gemm_bf16_nt(const bf16
                                                               int nb_m, int nb_n, int vec_store,
                                                               float* __restrict__ row_max_parts, long parts_ld,
                                                               long batch_a, long batch_w, long batch_c) {
-  using Cfg = IxGemmCfg<BM, BN, WM, WN, PW>;
+  using Cfg = IxGemmCfg<BM, BN, WM, WN, PW, W_ONCE>;
   extern __shared__ __align__(16) char ix_lds[];
   // a batch of independent products (bmm): workgroup row blockIdx.y works on matrices batch strides further on
   A += (long)blockIdx.y * batch_a;
@@ -236,13 +236,13 @@ struct IxDenseStreamSeq {
   }
 };
 
-template <bool PARTS>
+template <bool PARTS, bool W_ONCE>
 __global__ __launch_bounds__(256) void k_gemm_bf16_nt_stream(const bf16_t* __restrict__ A, long lda,
                                                              const bf16_t* __restrict__ W, long ldw,
                                                              bf16_t* __restrict__ C, long ldc, int M, int N, int K,
                                                              int nb_m, int nb_n, int gm, int gn,
                                                              float* __restrict__ row_max_parts, long parts_ld) {
-  using Cfg = IxGemmCfg<256, 256, 2, 2>;
+  using Cfg = IxGemmCfg<256, 256, 2, 2, 0, W_ONCE>;
   extern __shared__ __align__(16) char ix_lds[];
   IxPlainStreamJob<Cfg, IxDenseStreamSeq, PARTS> job;
   job.seq.gm = gm;
@@ -270,35 +270,45 @@ static bool ix_gemm_stream_fits(const void* C, long ldc, long M, long N, long K,
          ix_aligned(C, 16) && ldc * 512 < 0x40000000L && tiles >= min_tiles;
 }
 
+// Weights with one reader in the launch (ix_dma16): a single row tile, and more of them than the caches would keep for the
+// next launch anyway.
+static bool ix_gemm_once(long nb_m, long N, long K) { return nb_m == 1 && N * K * 2 >= (64L << 20); }
+
+template <auto KERN, typename... Args>
+static int ix_gemm_stream_start(int lds, hipStream_t st, Args... args) {
+  static bool attr_set = false;  // per kernel
+  if (!attr_set) {
+    if (hipFuncSetAttribute((const void*)KERN, hipFuncAttributeMaxDynamicSharedMemorySize, lds) != hipSuccess)
+      return IX_ERR_LAUNCH;
+    attr_set = true;
+  }
+  hipLaunchKernelGGL(KERN, dim3(IX_STREAM_WORKGROUPS), dim3(256), lds, st, args...);
+  return ix_launch_status();
+}
+
 static int ix_gemm_bf16_stream_launch(const bf16_t* A, long lda, const bf16_t* W, long ldw, bf16_t* C, long ldc, long M,
                                       long N, long K, float* parts, long parts_ld, hipStream_t st) {
   using Cfg = IxGemmCfg<256, 256, 2, 2>;
   const long nb_m = (M + 255) / 256, nb_n = (N + 255) / 256;
   if (nb_m * nb_n > 0x7fffffffL) return IX_DECLINED;
   if (parts && parts_ld < nb_n * 2) return IX_ERR_ARG;
-  static bool attr_set = false;
-  if (!attr_set) {
-    if (hipFuncSetAttribute((const void*)k_gemm_bf16_nt_stream<true>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                            Cfg::LDS_BYTES) != hipSuccess ||
-        hipFuncSetAttribute((const void*)k_gemm_bf16_nt_stream<false>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                            Cfg::LDS_BYTES) != hipSuccess)
-      return IX_ERR_LAUNCH;
-    attr_set = true;
-  }
   // Group shape of the tile order: with many row tiles the activations are the operand that streams, and a group
   // that is wider in weight tiles re-uses each activation tile more often (163840 x 2048 x 12352: 6.40 -> 6.20 ms,
   // 32768 x 2048 x 151936: 15.7 -> 15.5); with few row tiles the default serves the weights better.
   const int gm = nb_m >= 64 ? 4 : IX_GEMM_GM, gn = nb_m >= 64 ? 16 : IX_GEMM_GN;
-  if (parts)
-    hipLaunchKernelGGL(k_gemm_bf16_nt_stream<true>, dim3(IX_STREAM_WORKGROUPS), dim3(256), Cfg::LDS_BYTES, st, A, lda, W,
-                       ldw, C, ldc, (int)M, (int)N, (int)K, (int)nb_m, (int)nb_n, gm, gn, parts, parts_ld);
-  else
-    hipLaunchKernelGGL(k_gemm_bf16_nt_stream<false>, dim3(IX_STREAM_WORKGROUPS), dim3(256), Cfg::LDS_BYTES, st, A, lda, W,
-                       ldw, C, ldc, (int)M, (int)N, (int)K, (int)nb_m, (int)nb_n, gm, gn, parts, parts_ld);
-  return ix_launch_status();
+#define IX_STREAM_GO(PARTS_, ONCE_)                                                                                       \
+  return ix_gemm_stream_start<k_gemm_bf16_nt_stream<PARTS_, ONCE_>>(Cfg::LDS_BYTES, st, A, lda, W, ldw, C, ldc, (int)M, (int)N, \
+                                                                    (int)K, (int)nb_m, (int)nb_n, gm, gn, parts, parts_ld)
+  if (ix_gemm_once(nb_m, N, K)) {
+    if (parts) IX_STREAM_GO(true, true);
+    IX_STREAM_GO(false, true);
+  }
+  if (parts) IX_STREAM_GO(true, false);
+  IX_STREAM_GO(false, false);
+#undef IX_STREAM_GO
 }
 
-template <int BM, int BN, int WM, int WN, typename TC, int PW = 0>
+template <int BM, int BN, int WM, int WN, typename TC, int PW = 0, bool W_ONCE = false>
 static int ix_gemm_bf16_launch(const bf16_t* A, long lda, const bf16_t* W, long ldw, const bf16_t* bias, TC* C,
                                long ldc, long M, long N, long K, float* parts, long parts_ld, hipStream_t st,
                                long batch = 1, long batch_a = 0, long batch_w = 0, long batch_c = 0) {
@@ -307,7 +317,7 @@ static int ix_gemm_bf16_launch(const bf16_t* A, long lda, const bf16_t* W, long 
   const long grid = 8 * ((nb_m * nb_n + 7) / 8);  // 8 XCD runs of the tile order, the longest one sets the count
   if (grid > 0x7fffffffL) return IX_DECLINED;
   if (parts && parts_ld < nb_n * ix_gemm_parts_per_tile<BM, BN, WM, WN, PW>()) return IX_ERR_ARG;
-  auto kern = k_gemm_bf16_nt<BM, BN, WM, WN, TC, PW>;
+  auto kern = k_gemm_bf16_nt<BM, BN, WM, WN, TC, PW, W_ONCE>;
   static bool attr_set = false;  // per instantiation
   if (!attr_set) {
     if (hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, Cfg::LDS_BYTES) !=
@@ -378,7 +388,10 @@ static int ix_gemm_bf16_dispatch(const bf16_t* a, long lda, const bf16_t* w, lon
 #define IX_BATCH_ARGS , batch, sa, sw, sc
   switch (ix_gemm_tile_for(M * (batch > 1 ? batch : 1), N, K, tile)) {
     case 1: return ix_gemm_bf16_launch<32, 256, 1, 4, TC, 4>(a, lda, w, ldw, b, c, ldc, M, N, K, parts, parts_ld, st IX_BATCH_ARGS);
-    case 2: return ix_gemm_bf16_launch<128, 128, 2, 2, TC>(a, lda, w, ldw, b, c, ldc, M, N, K, parts, parts_ld, st IX_BATCH_ARGS);
+    case 2:
+      if (batch == 1 && ix_gemm_once((M + 127) / 128, N, K))
+        return ix_gemm_bf16_launch<128, 128, 2, 2, TC, 0, true>(a, lda, w, ldw, b, c, ldc, M, N, K, parts, parts_ld, st);
+      return ix_gemm_bf16_launch<128, 128, 2, 2, TC>(a, lda, w, ldw, b, c, ldc, M, N, K, parts, parts_ld, st IX_BATCH_ARGS);
     case 3: return ix_gemm_bf16_launch<256, 256, 2, 4, TC>(a, lda, w, ldw, b, c, ldc, M, N, K, parts, parts_ld, st IX_BATCH_ARGS);
     case 4:
       if constexpr (sizeof(TC) == 2) {

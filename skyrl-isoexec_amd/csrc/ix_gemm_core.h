@@ -45,8 +45,10 @@ __device__ __forceinline__ int ix_lds_off(int row, int chunk) { return row * 128
 __device__ __forceinline__ int ix_acc_row(int i, int lane) { return ((i >> 2) << 3) + ((lane >> 5) << 2) + (i & 3); }
 
 // PW_ > 0: PW_ extra waves that only fetch (pipeline D below); NT counts the computing threads, NTT all of them.
-template <int BM_, int BN_, int WM_, int WN_, int PW_ = 0>
+// W_ONCE_: every weight tile has one reader in the launch (ix_dma16); the pipelines C and F take it.
+template <int BM_, int BN_, int WM_, int WN_, int PW_ = 0, bool W_ONCE_ = false>
 struct IxGemmCfg {
+  static constexpr bool W_ONCE = W_ONCE_;
   static constexpr int BM = BM_, BN = BN_, WM = WM_, WN = WN_, PW = PW_;
   static constexpr int NT = WM * WN * 64;
   static constexpr int NTT = NT + PW * 64;
@@ -116,19 +118,24 @@ __device__ __forceinline__ ix_rsrc_t ix_make_rsrc(const void* base, uint32_t byt
 // vector-memory instruction reads it as descriptor word or scalar offset -- the load would otherwise go to the address
 // the old value gives, and the scalar offset is not even range-checked. IDLE = 0 gives the one state for M0 and is right
 // where every scalar operand comes from scalar arithmetic; a kernel short of scalar registers takes IDLE = 3.
-template <int IDLE = 0>
+// ONCE: the non-temporal hint, for weights that one workgroup of the launch reads. Lines that nobody asks for again then
+// leave the caches to the operand that is shared. Measured on ring tiles with the 1.2 GB LM head 151936 x 4096: 7 rows
+// 228 -> 202 us (6.2 TB/s), 64 rows 238 -> 232, 200 rows (256-row tile) 315 -> 307. With several row tiles it costs what the
+// second reader would have found (200 rows in 128-row tiles: 366 -> 489), and weights of a few MB lose too (5120 x 2048,
+// 128 rows: 19.6 -> 22.5).
+template <int IDLE = 0, bool ONCE = false>
 __device__ __forceinline__ void ix_dma16(ix_rsrc_t rsrc, uint32_t lds_addr, uint32_t voff, int soff) {
   static_assert(IDLE == 0 || IDLE == 3, "one wait state for M0, or five for scalar operands a vector instruction wrote");
-  if constexpr (IDLE == 0)
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
-                 :
-                 : "s"(lds_addr), "v"(voff), "s"(rsrc), "s"(soff)
-                 : "memory", "m0");
-  else
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 3\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
-                 :
-                 : "s"(lds_addr), "v"(voff), "s"(rsrc), "s"(soff)
-                 : "memory", "m0");
+#define IX_DMA16(NOP, HINT)                                                                    \
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop " NOP "\n\tbuffer_load_dwordx4 %1, %2, %3 offen" HINT " lds" \
+               :                                                                               \
+               : "s"(lds_addr), "v"(voff), "s"(rsrc), "s"(soff)                                \
+               : "memory", "m0")
+  if constexpr (IDLE == 0 && !ONCE) IX_DMA16("0", "");
+  else if constexpr (IDLE == 0) IX_DMA16("0", " nt");
+  else if constexpr (!ONCE) IX_DMA16("3", "");
+  else IX_DMA16("3", " nt");
+#undef IX_DMA16
 }
 // Stores through a descriptor: an offset outside its range (IX_OOB, or a row past the tile) is dropped by the hardware,
 // so a predicated store needs no branch.
@@ -397,13 +404,13 @@ __device__ __forceinline__ void ix_gemm_mainloop_units(ix_rsrc_t x_rsrc, const X
     w_voff[j] = w_row(r) + kb[j];
   }
   // unit u -> slot u % NU, tracked incrementally
-  auto issue = [&](ix_rsrc_t rsrc, const uint32_t (&voff)[CH], int kt, int slot) {
+  auto issue = [&](auto is_w, ix_rsrc_t rsrc, const uint32_t (&voff)[CH], int kt, int slot) {
     const int soff = kt * IX_BK * 2;
     const uint32_t sbase = lds_base + slot * UNIT;
 #pragma unroll
     for (int j = 0; j < CH; ++j) {
       const uint32_t dead = (uint32_t)((K2 - 1 - (soff + kb[j])) >> 31) & IX_OOB;
-      ix_dma16(rsrc, sbase + j * NT * 16, voff[j] | dead, soff);
+      ix_dma16<0, Cfg::W_ONCE && decltype(is_w)::value>(rsrc, sbase + j * NT * 16, voff[j] | dead, soff);
     }
   };
   const int frow = lane & 31, fg = lane >> 5;
@@ -432,7 +439,8 @@ __device__ __forceinline__ void ix_gemm_mainloop_units(ix_rsrc_t x_rsrc, const X
   int is = 0;  // slot of the next unit to issue
 #pragma unroll
   for (int u = 0; u < NU - 2; ++u) {
-    if (u & 1) issue(x_rsrc, x_voff, u >> 1, is); else issue(w_rsrc, w_voff, u >> 1, is);
+    if (u & 1) issue(std::false_type{}, x_rsrc, x_voff, u >> 1, is);
+    else issue(std::true_type{}, w_rsrc, w_voff, u >> 1, is);
     is = is + 1 == NU ? 0 : is + 1;
   }
   int cs = 0;            // slot of the W unit being consumed
@@ -442,7 +450,8 @@ __device__ __forceinline__ void ix_gemm_mainloop_units(ix_rsrc_t x_rsrc, const X
     __syncthreads();
 #pragma unroll
     for (int r = 0; r < 2; ++r) {
-      if (nu & 1) issue(x_rsrc, x_voff, nu >> 1, is); else issue(w_rsrc, w_voff, nu >> 1, is);
+      if (nu & 1) issue(std::false_type{}, x_rsrc, x_voff, nu >> 1, is);
+      else issue(std::true_type{}, w_rsrc, w_voff, nu >> 1, is);
       is = is + 1 == NU ? 0 : is + 1;
       ++nu;
     }

@@ -115,8 +115,11 @@ __device__ __forceinline__ void ix_gemm_stream4(Job& job, int KT, char* lds) {
   job.advance();
 
   // chunk j of k-tile t of the tile that `rsrc` describes into ring slot `slot` (K is a multiple of 64 here: no tail)
-  auto fetch = [&](const ix_rsrc_t& rsrc, uint32_t voff, int t, int slot, int j) {
+  auto fetch_x = [&](const ix_rsrc_t& rsrc, uint32_t voff, int t, int slot, int j) {
     ix_dma16<Job::DMA_IDLE>(rsrc, lds_base + slot * UNIT + j * NT * 16, voff, t * (IX_BK * 2));
+  };
+  auto fetch_w = [&](const ix_rsrc_t& rsrc, uint32_t voff, int t, int slot, int j) {
+    ix_dma16<Job::DMA_IDLE, Cfg::W_ONCE>(rsrc, lds_base + slot * UNIT + j * NT * 16, voff, t * (IX_BK * 2));
   };
   const int frow = lane & 31, fg = lane >> 5;
   int x_foff[4], w_foff[4];
@@ -143,9 +146,9 @@ __device__ __forceinline__ void ix_gemm_stream4(Job& job, int KT, char* lds) {
         __builtin_amdgcn_mfma_f32_32x32x16_bf16(F[(J) & 3], fx[(J) >> 2], acc[(J) >> 2][(J) & 3], 0, 0, 0)
   // One phase (pipeline E's): 16 matrix instructions on weight buffer FM and the activation fragments; after
   // instructions 0, 1, 2, 4 a weight fragment of step S of the k-tile at (XS, WS) into buffer FR, after 3, 7, 11, 15 its
-  // activation fragments 0..3, after 8, 10, 12, 14 one fetch (chunks J0..J0+3 of k-tile T of the tile behind RSRC / VOFF
-  // into ring slot SLOT); after every instruction micro-step SLICE * 64 + PH * 16 + j.
-#define IXS_PHASE(FM, FR, XS, WS, S, RSRC, VOFF, T, SLOT, J0, PH, Z, SLICE)                             \
+  // activation fragments 0..3, after 8, 10, 12, 14 one fetch (chunks J0..J0+3 of k-tile T of the tile behind RSRC, OP = x
+  // or w, into ring slot SLOT); after every instruction micro-step SLICE * 64 + PH * 16 + j.
+#define IXS_PHASE(FM, FR, XS, WS, S, RSRC, OP, T, SLOT, J0, PH, Z, SLICE)                               \
   ix_static_for<0, 16>([&](auto jc) {                                                                   \
     constexpr int j = decltype(jc)::value;                                                              \
     IXS_MFMA(FM, j, Z);                                                                                 \
@@ -155,7 +158,7 @@ __device__ __forceinline__ void ix_gemm_stream4(Job& job, int KT, char* lds) {
     } else if constexpr (j < 3 || j == 4) {                                                             \
       IXS_READ_W(FR, WS, S, j < 3 ? j : 3);                                                             \
     } else if constexpr (j >= 8 && (j & 1) == 0) {                                                      \
-      fetch(RSRC, job.template VOFF<(J0) + ((j - 8) >> 1)>(), T, SLOT, (J0) + ((j - 8) >> 1));          \
+      fetch_##OP(RSRC, job.template OP##_voff<(J0) + ((j - 8) >> 1)>(), T, SLOT, (J0) + ((j - 8) >> 1)); \
     }                                                                                                   \
     if constexpr ((SLICE) >= 0) job.template micro<((SLICE) < 0 ? 0 : (SLICE)) * 64 + (PH) * 16 + j>(); \
     __builtin_amdgcn_sched_barrier(0);                                                                  \
@@ -164,19 +167,19 @@ __device__ __forceinline__ void ix_gemm_stream4(Job& job, int KT, char* lds) {
   // ---- the first tile's first units: W(0), X(0), W(1) and half of X(1), as in pipeline E
   ix_static_for<0, CH>([&](auto jc) {
     constexpr int j = decltype(jc)::value;
-    fetch(wr_c, job.template w_voff<j>(), 0, 0, j);
+    fetch_w(wr_c, job.template w_voff<j>(), 0, 0, j);
   });
   ix_static_for<0, CH>([&](auto jc) {
     constexpr int j = decltype(jc)::value;
-    fetch(xr_c, job.template x_voff<j>(), 0, 1, j);
+    fetch_x(xr_c, job.template x_voff<j>(), 0, 1, j);
   });
   ix_static_for<0, CH>([&](auto jc) {
     constexpr int j = decltype(jc)::value;
-    fetch(wr_c, job.template w_voff<j>(), 1, 2, j);
+    fetch_w(wr_c, job.template w_voff<j>(), 1, 2, j);
   });
   ix_static_for<0, 4>([&](auto jc) {
     constexpr int j = decltype(jc)::value;
-    fetch(xr_c, job.template x_voff<j>(), 1, 3, j);
+    fetch_x(xr_c, job.template x_voff<j>(), 1, 3, j);
   });
   int slot = 3;  // ring slot of X(kt + 1)
   int cs = 0;    // slot of the W unit of the k-tile being read
@@ -207,10 +210,10 @@ __device__ __forceinline__ void ix_gemm_stream4(Job& job, int KT, char* lds) {
     }
     const int t1 = TAIL == 1 ? 0 : kt + 1;                       // k-tile of the X half fetched in the first phase
     const int t2 = TAIL == 2 ? 0 : (TAIL == 1 ? 1 : kt + 2);     // k-tile of the W unit and the X half after it
-    IXS_PHASE(fa, fb, xs, ws, 1, (TAIL == 1 ? xr_n : xr_c), x_voff, t1, slot_x, 4, 0, ZERO, SLICE);
+    IXS_PHASE(fa, fb, xs, ws, 1, (TAIL == 1 ? xr_n : xr_c), x, t1, slot_x, 4, 0, ZERO, SLICE);
     if constexpr (TAIL == 2) job.turn_offsets();  // the current tile has made its last fetch through them
-    IXS_PHASE(fb, fa, xs, ws, 2, ((TAIL == 1 || TAIL == 2) ? wr_n : wr_c), w_voff, t2, slot_w, 0, 1, false, SLICE);
-    IXS_PHASE(fa, fb, xs, ws, 3, ((TAIL == 1 || TAIL == 2) ? wr_n : wr_c), w_voff, t2, slot_w, 4, 2, false, SLICE);
+    IXS_PHASE(fb, fa, xs, ws, 2, ((TAIL == 1 || TAIL == 2) ? wr_n : wr_c), w, t2, slot_w, 0, 1, false, SLICE);
+    IXS_PHASE(fa, fb, xs, ws, 3, ((TAIL == 1 || TAIL == 2) ? wr_n : wr_c), w, t2, slot_w, 4, 2, false, SLICE);
     // Every fragment of this k-tile is in registers, and everything older than the W unit just requested (and the
     // stores of this k-tile's micro-steps) has landed: k-tile kt + 1 is complete.
     constexpr int NST = SLICE >= 0 ? Job::stores_after_p1(SLICE < 0 ? 0 : SLICE) : 0;
@@ -218,7 +221,7 @@ __device__ __forceinline__ void ix_gemm_stream4(Job& job, int KT, char* lds) {
     __syncthreads();
     const char* ws1 = lds + cs * UNIT;
     const char* xs1 = lds + (cs + 1 == NU ? 0 : cs + 1) * UNIT;
-    IXS_PHASE(fb, fa, xs1, ws1, 0, ((TAIL == 1 || TAIL == 2) ? xr_n : xr_c), x_voff, t2, slot, 0, 3, false, SLICE);
+    IXS_PHASE(fb, fa, xs1, ws1, 0, ((TAIL == 1 || TAIL == 2) ? xr_n : xr_c), x, t2, slot, 0, 3, false, SLICE);
   };
 
   // The first tile runs the same code as every other: its "pending tile" is the empty one the job starts with (no rows,

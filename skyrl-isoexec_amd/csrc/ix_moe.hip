@@ -1044,10 +1044,11 @@ struct IxMoeFc2Seq {
   }
 };
 
+template <bool W_ONCE>
 __global__ __launch_bounds__(256) void k_moe_fc2_stream(const bf16_t* __restrict__ inter, const bf16_t* __restrict__ W2,
                                                         const int* __restrict__ meta, int max_tiles,
                                                         bf16_t* __restrict__ out, int Hd, int F, int nb_n) {
-  using Cfg = IxGemmCfg<256, 256, 2, 2>;
+  using Cfg = IxGemmCfg<256, 256, 2, 2, 0, W_ONCE>;
   extern __shared__ __align__(16) char ix_lds[];
   IxPlainStreamJob<Cfg, IxMoeFc2Seq, false> job;
   job.seq.inter = inter;
@@ -1310,13 +1311,14 @@ struct IxMoeFc1StreamJob {
   }
 };
 
+template <bool W_ONCE>
 __global__ __launch_bounds__(256) void k_moe_fc1_glu_stream(const bf16_t* __restrict__ x, long ldx, int T, int rows,
                                                             const int* __restrict__ sorted_token,
                                                             const float* __restrict__ permuted_prob,
                                                             const bf16_t* __restrict__ W1, const int* __restrict__ meta,
                                                             int max_tiles, bf16_t* __restrict__ inter, int Hd, int F,
                                                             int nb_n) {
-  using Cfg = IxGemmCfg<256, 256, 2, 2>;
+  using Cfg = IxGemmCfg<256, 256, 2, 2, 0, W_ONCE>;
   extern __shared__ __align__(16) char ix_lds[];
   IxMoeFc1StreamJob job;
   job.x = x;
@@ -1355,6 +1357,11 @@ static int ix_moe_experts_launch(const bf16_t* x, long ldx, int T, long rows, co
   const long nb1 = (F + BN / 2 - 1) / (BN / 2);
   const long nb2 = (Hd + BN - 1) / BN;
   if (max_tiles * nb1 > 0x7fffffffL || max_tiles * nb2 > 0x7fffffffL) return IX_DECLINED;
+  // Weights read past the caches (ix_dma16) while nearly every expert has one 256-row tile, i.e. each of its weight tiles
+  // one reader: mean rows per expert up to 224 (max_tiles counts one tile per expert beside the full ones). us fc1 + fc2,
+  // 128 experts of 2048 x 768: 512 tokens 278 -> 259, 1500 300 -> 287, 3500 335 -> 310; 4096 tokens, where half the experts
+  // have a second tile, 410 -> 419.
+  const bool once = rows <= 224 * (max_tiles - rows / 256);
   // 8 XCD runs of the tile order; the longest run sets the count
   bool fc1_streamed = false;
   if constexpr (BM == 256 && BN == 256 && WM == 2 && WN == 2) {
@@ -1364,12 +1371,14 @@ static int ix_moe_experts_launch(const bf16_t* x, long ldx, int T, long rows, co
         ((long)F + 128) * Hd * 2 < 0x40000000L && max_tiles * nb1 >= 2 * IX_STREAM_WORKGROUPS) {
       static bool attr1_set = false;
       if (!attr1_set) {
-        if (hipFuncSetAttribute((const void*)k_moe_fc1_glu_stream, hipFuncAttributeMaxDynamicSharedMemorySize,
+        if (hipFuncSetAttribute((const void*)k_moe_fc1_glu_stream<false>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                Cfg::LDS_BYTES) != hipSuccess ||
+            hipFuncSetAttribute((const void*)k_moe_fc1_glu_stream<true>, hipFuncAttributeMaxDynamicSharedMemorySize,
                                 Cfg::LDS_BYTES) != hipSuccess)
           return IX_ERR_LAUNCH;
         attr1_set = true;
       }
-      hipLaunchKernelGGL(k_moe_fc1_glu_stream, dim3(IX_STREAM_WORKGROUPS), dim3(256), Cfg::LDS_BYTES, st, x, ldx, T,
+      hipLaunchKernelGGL(once ? k_moe_fc1_glu_stream<true> : k_moe_fc1_glu_stream<false>, dim3(IX_STREAM_WORKGROUPS), dim3(256), Cfg::LDS_BYTES, st, x, ldx, T,
                          (int)rows, sorted_token, permuted_prob, W1, meta, (int)max_tiles, inter, Hd, F, (int)nb1);
       fc1_streamed = true;
     }
@@ -1383,12 +1392,14 @@ static int ix_moe_experts_launch(const bf16_t* x, long ldx, int T, long rows, co
         max_tiles * nb2 >= 2 * IX_STREAM_WORKGROUPS) {
       static bool attr2_set = false;
       if (!attr2_set) {
-        if (hipFuncSetAttribute((const void*)k_moe_fc2_stream, hipFuncAttributeMaxDynamicSharedMemorySize,
+        if (hipFuncSetAttribute((const void*)k_moe_fc2_stream<false>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                Cfg::LDS_BYTES) != hipSuccess ||
+            hipFuncSetAttribute((const void*)k_moe_fc2_stream<true>, hipFuncAttributeMaxDynamicSharedMemorySize,
                                 Cfg::LDS_BYTES) != hipSuccess)
           return IX_ERR_LAUNCH;
         attr2_set = true;
       }
-      hipLaunchKernelGGL(k_moe_fc2_stream, dim3(IX_STREAM_WORKGROUPS), dim3(256), Cfg::LDS_BYTES, st, inter, W2, meta,
+      hipLaunchKernelGGL(once ? k_moe_fc2_stream<true> : k_moe_fc2_stream<false>, dim3(IX_STREAM_WORKGROUPS), dim3(256), Cfg::LDS_BYTES, st, inter, W2, meta,
                          (int)max_tiles, out, Hd, F, (int)nb2);
       return ix_launch_status();
     }

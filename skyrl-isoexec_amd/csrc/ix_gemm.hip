@@ -5,6 +5,8 @@
 #include "ix_gemm_core.h"
 #include "ix_gemm_stream.h"
 #include "../../include/isoexec_hip.h"
+#include <algorithm>
+#include <cmath>
 
 // Workgroup -> tile map. Hardware hands consecutive workgroup ids to the 8 XCDs round-robin, and each XCD has
 // its own L2. The tiles are put in one order -- groups of GM M-tiles x GN weight tiles, about what an XCD's 32
@@ -263,11 +265,9 @@ __global__ __launch_bounds__(256) void k_gemm_bf16_nt_stream(const bf16_t* __res
   ix_gemm_stream4<Cfg>(job, K / IX_BK, ix_lds);
 }
 
-static bool ix_gemm_stream_fits(const void* C, long ldc, long M, long N, long K, const void* bias, long batch,
-                                long min_tiles) {
-  const long tiles = ((M + 255) / 256) * ((N + 255) / 256);
+static bool ix_gemm_stream_fits(const void* C, long ldc, long M, long N, long K, const void* bias, long batch) {
   return !bias && batch == 1 && (K % IX_BK == 0) && K / IX_BK >= IX_STREAM_MIN_KT && (N % 8 == 0) && (ldc % 8 == 0) &&
-         ix_aligned(C, 16) && ldc * 512 < 0x40000000L && tiles >= min_tiles;
+         ix_aligned(C, 16) && ldc * 512 < 0x40000000L;
 }
 
 // Weights with one reader in the launch (ix_dma16): a single row tile, and more of them than the caches would keep for the
@@ -333,42 +333,44 @@ static int ix_gemm_bf16_launch(const bf16_t* A, long lda, const bf16_t* W, long 
   return ix_launch_status();
 }
 
-// Which tile shape runs (0 = choose). Never changes a bit. The choice minimises a small cost model fitted to
-// measurements on MI355X: a launch runs in ceil(tiles / slots) waves of workgroups (one or two per CU), a workgroup costs
-// about 6 us plus K/64 k-tiles at a per-shape rate, and no shape streams the operands faster than ~5 TB/s. Big
-// square tiles win when there are enough of them to fill the chip several times over; a product with few rows or
-// few columns takes smaller tiles so that every CU has one.
+// Which tile shape runs (0 = choose). Never changes a bit. The choice minimises a cost model: a CU works through
+// ceil(tiles / 256) tiles -- the two small shapes two at a time -- at `fixed` us plus K/64 k-tiles each, and no shape streams
+// the operands faster than `stream` bytes per us. The figures are a fit to 139 measured shapes (weights 2048 x 4096, 5120 x
+// 2048, 12352 x 2048, 8192 x 8192, 151936 x 2048 and x 4096, 1 to 4000 rows): the shape it picks is within 0.2 % of the
+// fastest of the five in the geometric mean, 6 % at worst. The model before it counted waves of whole workgroups and was
+// 4.9 % off, 80 % at worst. us, before -> after: 8192 x 8192 at 384 rows 135 -> 75, 151936 x 4096 at 384 612 -> 488, 12352 x
+// 2048 at 700 54 -> 42, 5120 x 2048 at 4000 100 -> 81, 2048 x 4096 at 1000 40 -> 31.
 static int ix_gemm_tile_for(long M, long N, long K, int tile) {
   if (tile != 0) return tile;
   // One 128-wide column of tiles (the router's gating product): 128-row tiles once there are enough of them to fill
   // the chip, the small tile below that (2048 x 2048 x 128: 20.7 -> 8.5 us; equal at 16384 rows).
   if (M > 128 && N <= 128) return M >= 16384 ? 2 : 6;
-  // slots: workgroups resident on the chip at once; us_per_ktile: with the CU to itself / shared with a second one;
-  // us_fixed: launch, first fetches and the store phase of one workgroup
-  struct Shape { int id, bm, bn; double slots, us_per_ktile, us_per_ktile_shared, us_fixed; };
-  // preference order on ties: larger tiles first. The 256 x 256 tile runs on four waves (id 4: a third fewer LDS reads,
-  // 1.4 us per k-tile) unless the product is short in K, where the eight-wave form's shorter store phase wins.
-  static const Shape shapes[] = {{4, 256, 256, 256.0, 1.4, 1.4, 8.0},   {5, 128, 256, 256.0, 0.75, 0.75, 6.0},
-                                 {2, 128, 128, 512.0, 0.6, 1.0, 6.0},   {1, 32, 256, 256.0, 0.55, 0.55, 6.0},
-                                 {6, 64, 32, 512.0, 0.16, 0.16, 6.0}};
+  // us_ktile: a tile with its CU to itself; us_ktile_more: one of several (for id 2 and 6: of a pair that shares the CU)
+  struct Shape { int id, bm, bn; double us_ktile, us_ktile_more, fixed, stream; };
+  static const Shape shapes[] = {{4, 256, 256, 0.98, 1.4, 4.4, 4.4e6}, {5, 128, 256, 0.95, 1.1, 7.0, 4.1e6},
+                                 {2, 128, 128, 0.51, 0.95, 5.3, 4.7e6}, {1, 32, 256, 0.38, 0.42, 3.7, 4.4e6},
+                                 {6, 64, 32, 0.20, 0.29, 1.3, 3.7e6}};  // preference on ties: larger tiles first
   const double kt = (double)((K + 63) / 64);
-  const double stream_us = (double)(N + M) * (double)K * 2.0 / 5.0e6;  // both operands once at 5 TB/s
   int best = 4;
-  double best_cost = 1e300, big_cost = 0.0;
+  double best_cost = 1e300;
   for (const Shape& sh : shapes) {
     const double tiles = (double)((M + sh.bm - 1) / sh.bm) * (double)((N + sh.bn - 1) / sh.bn);
-    const double waves = (double)(long)((tiles + sh.slots - 1.0) / sh.slots);
-    double cost = waves * (sh.us_fixed + kt * (tiles > 256.0 ? sh.us_per_ktile_shared : sh.us_per_ktile));
-    if (cost < stream_us) cost = sh.id == 2 ? 0.9 * stream_us : stream_us;  // two workgroups per CU stream best
-    if (sh.id == 4) big_cost = cost;
+    const double turns = std::ceil(tiles / 256.0);
+    double cost;
+    if (sh.id == 4) {  // one workgroup per CU streams its tiles: 3 us between two of them
+      cost = sh.fixed + turns * (kt * (turns == 1.0 ? sh.us_ktile : sh.us_ktile_more) + 3.0);
+    } else if (sh.id == 2 || sh.id == 6) {
+      const double pairs = std::floor(turns / 2.0);
+      cost = pairs * (sh.fixed + kt * sh.us_ktile_more) + (turns - 2.0 * pairs) * (sh.fixed + kt * sh.us_ktile);
+    } else {
+      cost = turns * (sh.fixed + kt * (turns == 1.0 ? sh.us_ktile : sh.us_ktile_more));
+    }
+    cost = std::max(cost, (double)(N + M) * (double)K * 2.0 / sh.stream);
     if (cost < best_cost * 0.97) {  // a later (smaller) shape must win by a margin
       best_cost = cost;
       best = sh.id;
     }
   }
-  // With more than half a big tile of rows, the big tile keeps its place unless another shape is clearly ahead:
-  // at scale the smaller shapes pull more bytes through L2 than the per-k-tile rates above say.
-  if (M > 128 && big_cost <= 1.25 * best_cost) best = 4;
   return best;
 }
 
@@ -395,8 +397,8 @@ static int ix_gemm_bf16_dispatch(const bf16_t* a, long lda, const bf16_t* w, lon
     case 3: return ix_gemm_bf16_launch<256, 256, 2, 4, TC>(a, lda, w, ldw, b, c, ldc, M, N, K, parts, parts_ld, st IX_BATCH_ARGS);
     case 4:
       if constexpr (sizeof(TC) == 2) {
-        // worth it from two tiles per workgroup up
-        if (ix_gemm_stream_fits(c, ldc, M, N, K, b, batch, 2 * IX_STREAM_WORKGROUPS))
+        // with one tile per workgroup too (12352 x 2048 at 700 rows 53 -> 42 us, 8192 x 8192 at 1100 157 -> 145)
+        if (ix_gemm_stream_fits(c, ldc, M, N, K, b, batch))
           return ix_gemm_bf16_stream_launch(a, lda, w, ldw, (bf16_t*)c, ldc, M, N, K, parts, parts_ld, st);
       }
       [[fallthrough]];
@@ -406,7 +408,7 @@ static int ix_gemm_bf16_dispatch(const bf16_t* a, long lda, const bf16_t* w, lon
     case 6: return ix_gemm_bf16_launch<64, 32, 2, 1, TC, 2>(a, lda, w, ldw, b, c, ldc, M, N, K, parts, parts_ld, st IX_BATCH_ARGS);
     case 8:  // the streaming form whatever the number of tiles (declines what it does not serve)
       if constexpr (sizeof(TC) == 2) {
-        if (ix_gemm_stream_fits(c, ldc, M, N, K, b, batch, 1))
+        if (ix_gemm_stream_fits(c, ldc, M, N, K, b, batch))
           return ix_gemm_bf16_stream_launch(a, lda, w, ldw, (bf16_t*)c, ldc, M, N, K, parts, parts_ld, st);
       }
       return IX_DECLINED;

@@ -40,6 +40,25 @@ __device__ __forceinline__ void ix_best_step(float& bv, int& bi, int sentinel) {
   if (ix_beats(ov, oi, bv, bi, sentinel)) { bv = ov; bi = oi; }
 }
 
+// Minimum over the 16 lanes of a row.
+__device__ __forceinline__ int ix_row_min(int v) {
+  v = min(v, __float_as_int(ix_partner<1>(__int_as_float(v))));
+  v = min(v, __float_as_int(ix_partner<2>(__int_as_float(v))));
+  v = min(v, __float_as_int(ix_partner<4>(__int_as_float(v))));
+  return min(v, __float_as_int(ix_partner<8>(__int_as_float(v))));
+}
+
+// Inclusive sum over the lanes of a wave: within rows by shifts, then each row's total into the rows above it.
+__device__ __forceinline__ int ix_wave_scan(int v) {
+  v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, true);   // row_shr:1
+  v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, true);   // row_shr:2
+  v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, true);   // row_shr:4
+  v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, true);   // row_shr:8
+  v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);  // row_bcast:15 into rows 1 and 3
+  v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);  // row_bcast:31 into rows 2 and 3
+  return v;
+}
+
 __device__ __forceinline__ float ix_tree_k(float (&t)[IX_MOE_KMAX], int k) {
 #pragma unroll
   for (int s = 1; s < IX_MOE_KMAX; s <<= 1) {
@@ -206,68 +225,60 @@ __device__ __forceinline__ void ix_moe_route_row16(const float* __restrict__ log
 #pragma unroll
     for (int c = 0; c < 8; ++c) s[c] = s[c] / z;
   }
-  float vals[IX_MOE_KMAX];
-  int idxs[IX_MOE_KMAX];
+  // k rounds of "the largest value left, the lowest expert among equals" (ix_beats). A round is a maximum over the row and a
+  // minimum over the experts that reach it, both of which ride the vector ALU's lane controls as one instruction a step
+  // (value and index exchanged as a pair and compared cost twice the instructions; at 64 tokens four waves share a SIMD and
+  // issue is what a round costs). A taken or missing expert is a NaN: the maximum passes it over and nothing equals it.
+  // Scores that are NaN (an infinite logit under mode 1: then the whole row is) rank with -inf.
+  const float none = __uint_as_float(0x7fc00000u);
+  float sel[8];
+#pragma unroll
+  for (int c = 0; c < 8; ++c) sel[c] = live[c] ? (s[c] != s[c] ? IX_NEG_INF : s[c]) : none;
+  float top = 0.0f, mine = 0.0f;  // round 0's value; lane j of the row keeps round j's
+  int mine_e = 0;
 #pragma unroll
   for (int j = 0; j < IX_MOE_KMAX; ++j) {
-    vals[j] = 0.0f;
-    idxs[j] = 0;
     if (j < k) {
-      float bv = 0.0f;
-      int bi = E;
+      const float m = ix_lane_max<16>(fmaxf(fmaxf(fmaxf(sel[0], sel[1]), fmaxf(sel[2], sel[3])),
+                                            fmaxf(fmaxf(sel[4], sel[5]), fmaxf(sel[6], sel[7]))));
+      int bi = IX_MOE_EMAX;  // no expert of this lane
 #pragma unroll
-      for (int c = 0; c < 8; ++c)
-        if (live[c] && ix_beats(s[c], eid[c], bv, bi, E)) { bv = s[c]; bi = eid[c]; }
-      ix_best_step<1>(bv, bi, E);
-      ix_best_step<2>(bv, bi, E);
-      ix_best_step<4>(bv, bi, E);
-      ix_best_step<8>(bv, bi, E);
-      bi = min(bi, E - 1);
-      vals[j] = bv;
-      idxs[j] = bi;
+      for (int c = 7; c >= 0; --c) bi = sel[c] == m ? eid[c] : bi;  // eid[] ascends
+      bi = ix_row_min(bi);
+      if (j == 0) top = m;
+      if (li == j) { mine = m; mine_e = bi; }
 #pragma unroll
-      for (int c = 0; c < 8; ++c)
-        if (eid[c] == bi) live[c] = false;
+      for (int c = 0; c < 8; ++c) sel[c] = eid[c] == bi ? none : sel[c];
     }
   }
-  float p[IX_MOE_KMAX], tmp[IX_MOE_KMAX];
-  if (mode == 0) {
-    const float m = vals[0];
-#pragma unroll
-    for (int j = 0; j < IX_MOE_KMAX; ++j) { p[j] = (j < k) ? ix_exp(vals[j] - m) : 0.0f; tmp[j] = p[j]; }
-  } else {
-#pragma unroll
-    for (int j = 0; j < IX_MOE_KMAX; ++j) { p[j] = (j < k) ? vals[j] : 0.0f; tmp[j] = p[j]; }
-  }
-  const float den = ix_tree_k(tmp, k);
-#pragma unroll
-  for (int j = 0; j < IX_MOE_KMAX; ++j) {
-    p[j] = p[j] / den;
-    if (scaling != 0.0f) p[j] = p[j] * scaling;
-  }
-#pragma unroll
-  for (int j = 0; j < IX_MOE_KMAX; ++j) {
-    if (j < k && li == j) {
-      topk_idx[t * k + j] = idxs[j];
-      topk_prob[t * k + j] = p[j];
-      if (lds_idx) {  // a kernel that goes on to permute keeps the winners in LDS as well
-        lds_idx[t * k + j] = idxs[j];
-        lds_prob[t * k + j] = p[j];
-      }
+  // lane j < k holds winner j; the tree over k lanes goes on over zeros, which change no bit of a sum of non-negatives
+  float p = li < k ? (mode == 0 ? ix_exp(mine - top) : mine) : 0.0f;
+  p = p / ix_lane_tree<16>(p);
+  if (scaling != 0.0f) p = p * scaling;
+  if (li < k) {
+    topk_idx[t * k + li] = mine_e;
+    topk_prob[t * k + li] = p;
+    if (lds_idx) {  // a kernel that goes on to permute keeps the winners in LDS as well
+      lds_idx[t * k + li] = mine_e;
+      lds_prob[t * k + li] = p;
     }
   }
   if (dense_probs || dense_map) {
+    float dp[8] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
+    uint8_t dm[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+    for (int j = 0; j < k; ++j) {
+      const int ej = __shfl(mine_e, j, 16);
+      const float pj = __shfl(p, j, 16);
+#pragma unroll
+      for (int c = 0; c < 8; ++c)
+        if (ej == eid[c]) { dp[c] = pj; dm[c] = 1; }
+    }
 #pragma unroll
     for (int c = 0; c < 8; ++c) {
       const int e = eid[c];
       if (e < E) {
-        float dp = 0.0f;
-        uint8_t dm = 0;
-#pragma unroll
-        for (int j = 0; j < IX_MOE_KMAX; ++j)
-          if (j < k && idxs[j] == e) { dp = p[j]; dm = 1; }
-        if (dense_probs) dense_probs[t * E + e] = dp;
-        if (dense_map) dense_map[t * E + e] = dm;
+        if (dense_probs) dense_probs[t * E + e] = dp[c];
+        if (dense_map) dense_map[t * E + e] = dm[c];
       }
     }
   }
@@ -314,15 +325,13 @@ extern "C" int ix_moe_router_topk(const float* logits, long ld, long T, long E, 
 // which makes every expert's rows token-ascending without any ordered loop or counter.
 __device__ __forceinline__ void ix_moe_build_masks(const int* __restrict__ topk_idx, int t0, int nt, int E, int k,
                                                    uint32_t* s_mask /* [E][8] */, int* s_idx /* [256][k] */) {
-  for (int i = threadIdx.x; i < E * 8; i += 256) s_mask[i] = 0u;
-  for (int i = threadIdx.x; i < nt * k; i += 256) s_idx[i] = topk_idx[(long)t0 * k + i];
+  const int nthreads = blockDim.x;
+  for (int i = threadIdx.x; i < E * 8; i += nthreads) s_mask[i] = 0u;
+  for (int i = threadIdx.x; i < nt * k; i += nthreads) s_idx[i] = topk_idx[(long)t0 * k + i];
   __syncthreads();
-  const int t = threadIdx.x;
-  if (t < nt) {
-    for (int j = 0; j < k; ++j) {
-      const int e = s_idx[t * k + j];
-      atomicOr(&s_mask[e * 8 + (t >> 5)], 1u << (t & 31));
-    }
+  for (int i = threadIdx.x; i < nt * k; i += nthreads) {
+    const int t = i / k;
+    atomicOr(&s_mask[s_idx[i] * 8 + (t >> 5)], 1u << (t & 31));
   }
   __syncthreads();
 }
@@ -432,7 +441,9 @@ __global__ __launch_bounds__(256) void k_moe_offsets(int E, int BM, int max_tile
   }
 }
 
-__global__ __launch_bounds__(256) void k_moe_scatter(const int* __restrict__ topk_idx,
+// 1024 threads, a (token, choice) pair at a time: bound by the latency of a pair's lookups (10 us with a token per thread
+// that walks its choices one after the other).
+__global__ __launch_bounds__(1024) void k_moe_scatter(const int* __restrict__ topk_idx,
                                                      const float* __restrict__ topk_prob, int T, int E, int k,
                                                      const int* __restrict__ tile_base,
                                                      const int* __restrict__ offsets, int* __restrict__ sorted_token,
@@ -444,53 +455,50 @@ __global__ __launch_bounds__(256) void k_moe_scatter(const int* __restrict__ top
   const int t0 = tile * IX_MOE_TILE_T;
   const int nt = min(IX_MOE_TILE_T, T - t0);
   ix_moe_build_masks(topk_idx, t0, nt, E, k, s_mask, s_idx);
-  const int t = threadIdx.x;
-  if (t >= nt) return;
-  const long tg = t0 + t;
-  for (int j = 0; j < k; ++j) {
-    const int e = s_idx[t * k + j];
+  for (int i = threadIdx.x; i < nt * k; i += 1024) {
+    const int t = i / k, e = s_idx[i];
+    const long first = (long)t0 * k;
     int local = __popc(s_mask[e * 8 + (t >> 5)] & ((1u << (t & 31)) - 1u));
     for (int w = 0; w < (t >> 5); ++w) local += __popc(s_mask[e * 8 + w]);
     int rank = 0;
     for (int j2 = 0; j2 < k; ++j2) rank += (s_idx[t * k + j2] < e);
     const int pos = offsets[e] + tile_base[(long)tile * E + e] + local;
-    sorted_token[pos] = (int)tg;
-    permuted_prob[pos] = topk_prob[tg * k + j];
-    combine_rows[tg * k + rank] = pos;
+    sorted_token[pos] = t0 + t;
+    permuted_prob[pos] = topk_prob[first + i];
+    combine_rows[first + t * k + rank] = pos;
   }
 }
 
 // The three steps above in one launch for a batch of at most one token tile (a decode step): the membership masks
 // stay in LDS, the expert offsets come from a workgroup-wide scan (two experts per lane), and every output is the
 // integer the general path writes.
-// Body of the one-tile permutation for the first 256 threads of a workgroup (`tid`; threads past 255 of a larger
-// workgroup pass through and only meet the barriers). s_idx [T * k] holds the winners already when `idx_in_lds`; the
-// routing weights come from `prob_src` (global or LDS). Every thread of the workgroup must call it.
+// Body of the one-tile permutation, by every thread of a workgroup of at least 256: a (token, choice) pair per thread
+// where the work is per pair, and one scan whose lanes each own two experts (rows and tiles ride in one integer: at most
+// 4096 of either), a wave at a time with one barrier between. Bound by latency: a serial loop over a token's choices and
+// a workgroup-wide scan of sixteen barriers made this 9 of 14 us of a decode step's routing. s_idx [T * k] holds the
+// winners already when `idx_in_lds`; the routing weights come from `prob_src` (global or LDS).
 __device__ __forceinline__ void ix_moe_permute_tile_body(const int* __restrict__ topk_idx, const float* prob_src, int T,
                                                          int E, int k, int BM, int max_tiles, int* __restrict__ counts,
                                                          int* __restrict__ offsets, int* __restrict__ sorted_token,
                                                          float* __restrict__ permuted_prob,
                                                          int* __restrict__ combine_rows, int* __restrict__ meta,
-                                                         int* s_idx, uint32_t* s_mask, int* s_off, int* s_rows,
-                                                         int* s_tiles, bool idx_in_lds) {
-  const int tid = threadIdx.x;
-  const bool worker = tid < 256;
-  if (worker) {
-    for (int i = tid; i < E * 8; i += 256) s_mask[i] = 0u;
-    if (!idx_in_lds)
-      for (int i = tid; i < T * k; i += 256) s_idx[i] = topk_idx[i];
-  }
+                                                         int* s_idx, uint32_t* s_mask, int* s_off, int* s_sums,
+                                                         bool idx_in_lds) {
+  static_assert(IX_MOE_TILE_T * IX_MOE_KMAX <= 0xffff && IX_MOE_EMAX <= 512, "rows and tiles in 16 bits each");
+  const int tid = threadIdx.x, nthreads = blockDim.x;
+  const bool scans = tid < 256;
+  for (int i = tid; i < E * 8; i += nthreads) s_mask[i] = 0u;
+  if (!idx_in_lds)
+    for (int i = tid; i < T * k; i += nthreads) s_idx[i] = topk_idx[i];
   __syncthreads();
-  if (worker && tid < T) {
-    for (int j = 0; j < k; ++j) {
-      const int e = s_idx[tid * k + j];
-      atomicOr(&s_mask[e * 8 + (tid >> 5)], 1u << (tid & 31));
-    }
+  for (int i = tid; i < T * k; i += nthreads) {
+    const int t = i / k;
+    atomicOr(&s_mask[s_idx[i] * 8 + (t >> 5)], 1u << (t & 31));
   }
   __syncthreads();
   // lane owns experts 2 tid and 2 tid + 1
-  int c[2] = {0, 0}, tl[2] = {0, 0};
-  if (worker) {
+  int c[2] = {0, 0}, tl[2] = {0, 0}, own = 0, upto = 0;
+  if (scans) {
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
       const int e = 2 * tid + h;
@@ -500,23 +508,15 @@ __device__ __forceinline__ void ix_moe_permute_tile_body(const int* __restrict__
       }
       tl[h] = (c[h] + BM - 1) / BM;
     }
-    s_rows[tid] = c[0] + c[1];
-    s_tiles[tid] = tl[0] + tl[1];
+    own = (c[0] + c[1]) | ((tl[0] + tl[1]) << 16);
+    upto = ix_wave_scan(own);
+    if ((tid & 63) == 63) s_sums[tid >> 6] = upto;
   }
   __syncthreads();
-  for (int d = 1; d < 256; d <<= 1) {  // inclusive scan over the 256 lane sums
-    const int a = (worker && tid >= d) ? s_rows[tid - d] : 0;
-    const int b = (worker && tid >= d) ? s_tiles[tid - d] : 0;
-    __syncthreads();
-    if (worker) {
-      s_rows[tid] += a;
-      s_tiles[tid] += b;
-    }
-    __syncthreads();
-  }
-  if (worker) {
-    int row0 = s_rows[tid] - (c[0] + c[1]);   // rows before expert 2 tid
-    int tile0 = s_tiles[tid] - (tl[0] + tl[1]);
+  if (scans) {
+    for (int w = 0; w < (tid >> 6); ++w) upto += s_sums[w];
+    int row0 = (upto - own) & 0xffff;  // rows before expert 2 tid
+    int tile0 = (upto - own) >> 16;
     int* tile_expert = meta + 1;
     int* tile_row0 = tile_expert + max_tiles;
     int* tile_nrows = tile_row0 + max_tiles;
@@ -538,22 +538,21 @@ __device__ __forceinline__ void ix_moe_permute_tile_body(const int* __restrict__
       tile0 += tl[h];
     }
     if (tid == 255) {
-      offsets[E] = s_rows[255];
-      meta[0] = min(s_tiles[255], max_tiles);
+      offsets[E] = upto & 0xffff;
+      meta[0] = min(upto >> 16, max_tiles);
     }
   }
   __syncthreads();
-  if (!worker || tid >= T) return;
-  for (int j = 0; j < k; ++j) {
-    const int e = s_idx[tid * k + j];
-    int local = __popc(s_mask[e * 8 + (tid >> 5)] & ((1u << (tid & 31)) - 1u));
-    for (int w = 0; w < (tid >> 5); ++w) local += __popc(s_mask[e * 8 + w]);
+  for (int i = tid; i < T * k; i += nthreads) {
+    const int t = i / k, e = s_idx[i];
+    int local = __popc(s_mask[e * 8 + (t >> 5)] & ((1u << (t & 31)) - 1u));
+    for (int w = 0; w < (t >> 5); ++w) local += __popc(s_mask[e * 8 + w]);
     int rank = 0;
-    for (int j2 = 0; j2 < k; ++j2) rank += (s_idx[tid * k + j2] < e);
+    for (int j2 = 0; j2 < k; ++j2) rank += (s_idx[t * k + j2] < e);
     const int pos = s_off[e] + local;
-    sorted_token[pos] = tid;
-    permuted_prob[pos] = prob_src[(long)tid * k + j];
-    combine_rows[(long)tid * k + rank] = pos;
+    sorted_token[pos] = t;
+    permuted_prob[pos] = prob_src[i];
+    combine_rows[t * k + rank] = pos;
   }
 }
 
@@ -567,9 +566,9 @@ __global__ __launch_bounds__(256) void k_moe_permute_one_tile(const int* __restr
   __shared__ int s_idx[IX_MOE_TILE_T * IX_MOE_KMAX];
   __shared__ uint32_t s_mask[IX_MOE_EMAX * 8];
   __shared__ int s_off[IX_MOE_EMAX + 1];
-  __shared__ int s_rows[256], s_tiles[256];
+  __shared__ int s_sums[4];
   ix_moe_permute_tile_body(topk_idx, topk_prob, T, E, k, BM, max_tiles, counts, offsets, sorted_token, permuted_prob,
-                           combine_rows, meta, s_idx, s_mask, s_off, s_rows, s_tiles, false);
+                           combine_rows, meta, s_idx, s_mask, s_off, s_sums, false);
 }
 
 // Router and permutation of a batch of at most one token tile (a decode step) in ONE launch: a workgroup of 1024
@@ -587,7 +586,7 @@ __global__ __launch_bounds__(1024) void k_moe_route_one_tile(const float* __rest
   __shared__ float s_prob[IX_MOE_TILE_T * IX_MOE_KMAX];
   __shared__ uint32_t s_mask[128 * 8];
   __shared__ int s_off[128 + 1];
-  __shared__ int s_rows[256], s_tiles[256];
+  __shared__ int s_sums[4];
   for (int t0 = 0; t0 < T; t0 += 64) {
     const int t = t0 + (int)(threadIdx.x >> 4);
     if (t < T)
@@ -596,7 +595,7 @@ __global__ __launch_bounds__(1024) void k_moe_route_one_tile(const float* __rest
   }
   // (the body's first barrier publishes s_idx and s_prob)
   ix_moe_permute_tile_body(topk_idx, s_prob, T, E, k, BM, max_tiles, counts, offsets, sorted_token, permuted_prob,
-                           combine_rows, meta, s_idx, s_mask, s_off, s_rows, s_tiles, true);
+                           combine_rows, meta, s_idx, s_mask, s_off, s_sums, true);
 }
 
 // Block map for rows that are ALREADY grouped by expert (the caller holds tokens_per_expert, e.g. a dispatcher's
@@ -734,7 +733,7 @@ extern "C" int ix_moe_permute(const int* topk_idx, const float* topk_prob, long 
   hipLaunchKernelGGL(k_moe_offsets, dim3(1), dim3(256), 0, st, (int)E, (int)BM, (int)max_tiles, counts, offsets,
                      tile_meta);
   if (ntiles > 0)
-    hipLaunchKernelGGL(k_moe_scatter, dim3((unsigned)ntiles), dim3(256), 0, st, topk_idx, topk_prob, (int)T, (int)E,
+    hipLaunchKernelGGL(k_moe_scatter, dim3((unsigned)ntiles), dim3(1024), 0, st, topk_idx, topk_prob, (int)T, (int)E,
                        (int)k, tile_base, offsets, sorted_token, permuted_prob, combine_rows);
   return ix_launch_status();
 }

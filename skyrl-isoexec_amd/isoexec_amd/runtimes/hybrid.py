@@ -534,24 +534,28 @@ class RolloutEngine:
             row = [int(attention), ptr(lw["post_norm"], bf16, H), ptr(nxt, bf16, H), ptr(lw["router"], bf16, E, H),
                    ptr(lw["w1"], bf16, E, 2 * F, H), ptr(lw["w2"], bf16, E, H, F)]
             row += [t.data_ptr() for t in b.packed_experts[i]] if packed_all else [0, 0]
-            names = ("qkv_proj", "o_proj") if attention else ("in_proj", "out_proj")
-            for name in names:
+            if attention:
+                q_width = c.q_heads * c.head_dim
+                shapes = {"qkv_proj": (q_width + 2 * c.kv_heads * c.head_dim, H), "o_proj": (H, q_width)}
+            else:
+                shapes = {"in_proj": (D + c.gdn_z + 2 * c.gdn_v_heads, H), "out_proj": (H, c.gdn_z)}
+            for name, shape in shapes.items():
                 pk = b.packed_dense.get((i, name))
-                row += [ptr(lw[name], bf16), 0 if pk is None else pk.packed.data_ptr()]
+                row += [ptr(lw[name], bf16, *shape), 0 if pk is None else pk.packed.data_ptr()]
             if attention:
                 kv = self.kv[i]
                 row += [0] * 11 + [ptr(kv.k, bf16), ptr(kv.v, bf16)]
-                ok = ok and lw["qkv_proj"].shape == ((c.q_heads + 2 * c.kv_heads) * c.head_dim, H)
             else:
                 g = self.gdn[i]
                 if type(g) is not RecurrentGDN or g.table is None or g.activation not in ("silu", "swish") or not g.fused_decode_prep:
                     return None
                 row += [ptr(g.conv_weight, bf16, D, 4), 0 if g.conv_bias is None else ptr(g.conv_bias, bf16, D),
-                        ptr(g.A_log, f32), ptr(g.dt_bias, f32), ptr(lw["out_norm"], bf16, c.gdn_head_dim),
+                        ptr(g.A_log, f32, c.gdn_v_heads), ptr(g.dt_bias, f32, c.gdn_v_heads), ptr(lw["out_norm"], bf16, c.gdn_head_dim),
                         ptr(g.ssm_state, f32), ptr(g.conv_state, bf16), ptr(g.slot2row, i64), g.slot2row.numel(),
                         ptr(g.last_used, i64), ptr(g._clock, i64), 0, 0]
-                ok = ok and lw["in_proj"].shape == (D + c.gdn_z + 2 * c.gdn_v_heads, H)
             table += row
+        ptr(b.w.embed, bf16, c.vocab, H)
+        ptr(b.w.layers[0]["pre_norm"], bf16, H)
         if not ok:
             return None
         dims = array("q", [n, c.layers, H, c.vocab, b.cos.shape[0], c.gdn_k_heads, c.gdn_v_heads, c.gdn_head_dim, c.q_heads,
@@ -572,7 +576,7 @@ class RolloutEngine:
         L = _lib.lib()
         need = int(L.ix_decode_step_workspace_bytes(dims.buffer_info()[0]))
         w = b.w
-        if need == 0 or not w.embed.is_contiguous() or w.embed.dtype is not torch.bfloat16:
+        if need == 0:
             return None
         dev = w.embed.device
         _lib.require_device(tokens, w.embed)

@@ -84,3 +84,19 @@ def test_native_step_is_taken_and_sees_replaced_weights():
     w.layers[0]["out_proj"] = torch.cat([w.layers[0]["out_proj"]] * 2, dim=1)[:, : cfg.gdn_z]
     assert e._decode_native(e._decode_state([0, 1]), tok) is None
     assert torch.isfinite(e.decode([0, 1], tok).float()).all()
+
+
+@pytest.mark.parametrize("layer,name,cut", [(0, "out_proj", lambda w: w[:, :-8]), (0, "in_proj", lambda w: w[:-8]),
+                                            (1, "o_proj", lambda w: w[:, :-8]), (1, "qkv_proj", lambda w: w[:-8]),
+                                            (None, "embed", lambda w: w[:-8])])
+def test_a_weight_of_another_shape_is_not_handed_to_the_native_step(layer, name, cut):
+    from isoexec_amd.runtimes.hybrid import HybridWeights, RolloutEngine
+
+    w = HybridWeights.make(config(), seed=4, device=DEV)
+    e = RolloutEngine(config(), w, max_num_seqs=2, max_len=32)
+    assert e._native_step_tables(2) is not None
+    if layer is None:
+        setattr(w, name, cut(getattr(w, name)).contiguous())
+    else:
+        w.layers[layer][name] = cut(w.layers[layer][name]).contiguous()
+    assert e._native_step_tables(2) is None

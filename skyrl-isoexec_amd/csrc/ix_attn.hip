@@ -40,7 +40,8 @@ typedef __attribute__((address_space(3))) ix_s16x4 ix_lds_s16x4;
 //   V: chunk c of key r sits at slot c ^ ((r & 3) << 2)   a transpose read takes 4 chunks of 4 consecutive keys
 // so that either read spreads over all LDS banks. A lane's LDS destination is fixed by its position in the
 // wave (destination = base + 16 * lane), so the permutation is applied to the memory address it fetches.
-template <int NT>
+// ONCE: the workgroup is its blocks' only reader (ix_dma16).
+template <int NT, bool ONCE>
 struct IxAttnFetch {
   static constexpr int CPT = 512 / NT;  // chunks per thread per tile
   uint32_t voff_k[CPT], voff_v[CPT];    // byte offsets inside a block: key row * pitch + chunk * 16
@@ -68,8 +69,8 @@ struct IxAttnFetch {
     const uint32_t dst = __builtin_amdgcn_readfirstlane(lds0 + stage * IX_ATTN_STAGE);
 #pragma unroll
     for (int j = 0; j < CPT; ++j) {
-      ix_dma16(rk, dst + j * NT * 16, voff_k[j], 0);
-      ix_dma16(rv, dst + IX_ATTN_TILE + j * NT * 16, voff_v[j], 0);
+      ix_dma16<0, ONCE>(rk, dst + j * NT * 16, voff_k[j], 0);
+      ix_dma16<0, ONCE>(rv, dst + IX_ATTN_TILE + j * NT * 16, voff_v[j], 0);
     }
   }
 };
@@ -193,7 +194,7 @@ __device__ __forceinline__ void ix_attn_step(const char* stage, const char* stag
 // workgroup never reaches the arithmetic. Two workgroups per CU (register limit below).
 // Inside a wave the loop is skewed by one block: while block kb goes through its softmax, the scores of block
 // kb + 1 are already in the matrix pipeline.
-template <int GROUP, int NW, int S>
+template <int GROUP, int NW, int S, bool ONCE>
 __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2, 2))) void k_attn_varlen(const bf16_t* __restrict__ q, long q_pitch,
                                                      const bf16_t* __restrict__ k, const bf16_t* __restrict__ v,
                                                      long kv_pitch, bf16_t* __restrict__ o,
@@ -267,7 +268,7 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2, 2)))
   float m = IX_NEG_INF, l = 0.0f;
   const float c = scale * IX_LOG2E;
 
-  IxAttnFetch<NT> fetch;
+  IxAttnFetch<NT, ONCE> fetch;
   fetch.init(ix_attn_lds, (uint32_t)(kv_pitch * 2));
   IxAttnLane ln;
   ln.init();
@@ -324,12 +325,12 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2, 2)))
   }
 }
 
-template <int GROUP, int NW, int S>
+template <int GROUP, int NW, int S, bool ONCE>
 static int ix_attn_launch(const void* q, long q_pitch, const void* k, const void* v, long kv_pitch, void* o,
                           const int* cu_q, const long* kv_start, const int* q_pos0, long N, long max_q_len, long HQ,
                           long HKV, float scale, hipStream_t st) {
   constexpr int LDS = S * IX_ATTN_STAGE;
-  auto kern = k_attn_varlen<GROUP, NW, S>;
+  auto kern = k_attn_varlen<GROUP, NW, S, ONCE>;
   static bool attr_set = false;  // per instantiation
   if (!attr_set) {
     if (hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, LDS) != hipSuccess)
@@ -366,10 +367,17 @@ extern "C" int ix_attn_varlen(const void* q, long q_pitch, const void* k, const 
   // barrier, so one's matrix work meets the other's softmax arithmetic (measured: an eight-wave workgroup, whose
   // two waves per SIMD stand behind the same barrier, is 4 % slower on long prefills although it stages half as
   // many key/value bytes per query; and a decode step runs 20-40 % faster with two workgroups per CU).
+  // One query tile per sequence (a decode step, short continuations): a (sequence, head) pair's keys and values have one
+  // reader, so their loads go past the caches. What they would displace there is the activations and, in the memory-side
+  // cache, lines other kernels left dirty, which have to be written back first: behind a 2 GiB copy, 64 sequences of 2060
+  // keys took 82 us with the default policy and 52 without, and 53 -> 47 with nothing in front (256 x 2000 183 -> 160, 128 x
+  // 300 19.4 -> 17.4, one sequence of 700 unchanged: there it is the chain of 0.65 us per block of 32 keys, for which a ring
+  // of 5, 6 or 9 stages does nothing either). With more tiles the pair's other tiles find the blocks in the L2.
+#define IX_ATTN_GO(G, S, ONCE) \
+  ix_attn_launch<G, 4, S, ONCE>(q, q_pitch, k, v, kv_pitch, o, cu_q, kv_start, q_pos0, N, max_q_len, HQ, HKV, scale, st)
 #define IX_ATTN_LAUNCH(G)                                                                                          \
   case G:                                                                                                          \
-    return ix_attn_launch<G, 4, IX_ATTN_STAGES>(q, q_pitch, k, v, kv_pitch, o, cu_q, kv_start, q_pos0, N, max_q_len, \
-                                                HQ, HKV, scale, st);
+    return max_q_len > 4 * (32 / G) ? IX_ATTN_GO(G, IX_ATTN_STAGES, false) : IX_ATTN_GO(G, IX_ATTN_STAGES, true);
   switch (group) {
     IX_ATTN_LAUNCH(1)
     IX_ATTN_LAUNCH(2)
@@ -381,6 +389,7 @@ extern "C" int ix_attn_varlen(const void* q, long q_pitch, const void* k, const 
       return IX_DECLINED;
   }
 #undef IX_ATTN_LAUNCH
+#undef IX_ATTN_GO
 }
 
 // ---- rotary position embedding -------------------------------------------------------------------

@@ -310,3 +310,27 @@ def test_rope_positions_outside_the_tables_read_nothing_and_give_nan():
     want = o_attn.rope(x[:2].float().numpy(), co, so, pos[:2].numpy())
     assert np.array_equal(got[:2], want)
     assert np.isnan(got[2:]).all()
+
+
+@pytest.mark.parametrize("HQ,HKV", [(1, 1), (8, 1), (32, 4), (64, 2)])
+@pytest.mark.parametrize("extra", [0, 1])
+def test_single_reader_form_equals_the_tiled_form(HQ, HKV, extra):
+    """Up to 4 x 32 / (HQ / HKV) queries per sequence take the loads past the caches; the same queries in a call that also
+    holds a longer sequence take the other form. Same bits; the sequences end on and beside block edges."""
+    from isoexec_amd.ops.attention.varlen_attn import varlen_attention
+
+    tile = 4 * 32 // (HQ // HKV)
+    lens = [1, tile, max(1, tile - 1)]
+    context = [0, 63, 1027]                      # keys in front of the first query
+    starts = [5, 200, 700]
+    q, k, v = (t.to(DEV) for t in rand_qkv(sum(lens) + tile + extra, HQ, HKV, HQ + extra)[:1] + rand_qkv(2048, HQ, HKV, 9)[1:])
+    i32 = dict(dtype=torch.int32, device=DEV)
+
+    def call(lengths, ctx, first):
+        cu = torch.tensor(np.cumsum([0] + lengths), **i32)
+        return varlen_attention(q[: sum(lengths)], k, v, cu, max(lengths), q_pos0=torch.tensor(ctx, **i32),
+                                kv_start=torch.tensor(first, dtype=torch.int64, device=DEV))
+
+    n = sum(lens)
+    both = call(lens + [tile + extra], context + [30], starts + [0])   # extra = 1: more than one tile
+    assert same_bits(call(lens, context, starts), both[:n])

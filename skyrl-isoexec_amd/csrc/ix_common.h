@@ -219,6 +219,11 @@ __device__ __forceinline__ uint4 ix_load16_once(const uint4* p) {
   return make_uint4(v.x, v.y, v.z, v.w);
 }
 
+__device__ __forceinline__ void ix_store16_once(uint4* p, uint4 u) {
+  typedef __attribute__((ext_vector_type(4))) uint32_t v4;
+  __builtin_nontemporal_store(v4{u.x, u.y, u.z, u.w}, reinterpret_cast<v4*>(p));
+}
+
 // Eight bf16 held in a 16-byte register group, widened.
 __device__ __forceinline__ void ix_unpack8(const uint4 u, float (&o)[8]) {
   const uint32_t q[4] = {u.x, u.y, u.z, u.w};

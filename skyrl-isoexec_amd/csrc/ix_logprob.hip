@@ -327,41 +327,45 @@ __global__ __launch_bounds__(256) void k_lp_fullwrite(const T* __restrict__ x, l
 // ---------------------------------------------------------------------------------------------
 // Gradient of the sampled logprob (rowinv.py:573-612): grad[j] = -u * exp(x[j] - lse), plus u at the target, u = upstream[row]
 // (0 for a target outside the vocabulary), rounded to the logits' type at the store. One pass: every logit is read once and
-// every gradient written once. Bound by HBM: [1000, 151936] fp32 225 us = 5.4 TB/s, bf16
-// 120 us; the same expression in elementwise passes took 600 us.
-// A workgroup owns a segment of IX_LP_SEG columns of a row, in memory order; a thread requests its four groups of eight
-// before it uses the first.
-template <typename T>
-__device__ __forceinline__ void ix_lp_store8(T* __restrict__ p, const float (&v)[8]);
-template <>
-__device__ __forceinline__ void ix_lp_store8<bf16_t>(bf16_t* __restrict__ p, const float (&v)[8]) {
-  ix_store8_bf16(p, 8, true, v);
+// every gradient written once. Bound by HBM: behind its forward, [1000, 151936] fp32 207 us with the default cache policy
+// and 32 bytes per lane, 188 us = 6.5 TB/s past the caches with 16 (a non-temporal store has to fill whole lines by itself:
+// 220 us with 32 bytes per lane); bf16 107 -> 106 and the forward behind it 109 -> 93. The same expression in elementwise
+// passes took 600 us.
+// A workgroup owns a segment of IX_LP_SEG columns of a row, in memory order; a thread requests all its columns before it
+// uses the first.
+__device__ __forceinline__ void ix_lp_widen16(const uint4 u, float (&v)[8]) { ix_unpack8(u, v); }
+__device__ __forceinline__ void ix_lp_widen16(const uint4 u, float (&v)[4]) {
+  v[0] = __uint_as_float(u.x); v[1] = __uint_as_float(u.y); v[2] = __uint_as_float(u.z); v[3] = __uint_as_float(u.w);
 }
-template <>
-__device__ __forceinline__ void ix_lp_store8<float>(float* __restrict__ p, const float (&v)[8]) {
-  *reinterpret_cast<float4*>(p) = make_float4(v[0], v[1], v[2], v[3]);
-  *reinterpret_cast<float4*>(p + 4) = make_float4(v[4], v[5], v[6], v[7]);
+__device__ __forceinline__ uint4 ix_lp_pack16(const float (&v)[8]) {
+  return make_uint4(ix_pack_bf2(v[0], v[1]), ix_pack_bf2(v[2], v[3]), ix_pack_bf2(v[4], v[5]), ix_pack_bf2(v[6], v[7]));
+}
+__device__ __forceinline__ uint4 ix_lp_pack16(const float (&v)[4]) {
+  return make_uint4(__float_as_uint(v[0]), __float_as_uint(v[1]), __float_as_uint(v[2]), __float_as_uint(v[3]));
 }
 __device__ __forceinline__ void ix_lp_store1(bf16_t* p, float v) { *p = ix_f2bf(v); }
 __device__ __forceinline__ void ix_lp_store1(float* p, float v) { *p = v; }
 
-template <typename T>
+// ONCE: the caches are too small for the logits and the gradient; both go past them.
+template <typename T, bool ONCE>
 __global__ __launch_bounds__(256) void k_lp_backward(const T* __restrict__ x, long row_stride, int V, int P,
                                                      const int64_t* __restrict__ target,
                                                      const float* __restrict__ upstream, const float* __restrict__ lse,
                                                      T* __restrict__ grad, long grad_stride, int vec) {
-  constexpr int GROUPS = IX_LP_SEG / (256 * 8);
+  constexpr int W = 16 / sizeof(T);  // columns of one 16-byte access; a wave's access is 1 KiB of the row
+  constexpr int GROUPS = IX_LP_SEG / (256 * W);
   const long row = blockIdx.x / P;  // segments fastest
   const int lo = (int)(blockIdx.x % P) * IX_LP_SEG;
   const int hi = min(V, lo + IX_LP_SEG);
   const T* xr = x + row * row_stride;
   T* gr = grad + row * grad_stride;
   if (vec) {  // V is a multiple of 8: a group is whole or absent (an absent one reads the segment's first columns)
-    IxRaw8<T> raw[GROUPS];
+    uint4 raw[GROUPS];
 #pragma unroll
     for (int c = 0; c < GROUPS; ++c) {
-      const int off = lo + (c * 256 + (int)threadIdx.x) * 8;
-      raw[c].load(xr + (off < hi ? off : lo));
+      const int off = lo + (c * 256 + (int)threadIdx.x) * W;
+      const uint4* p = reinterpret_cast<const uint4*>(xr + (off < hi ? off : lo));
+      raw[c] = ONCE ? ix_load16_once(p) : *p;
     }
     __builtin_amdgcn_sched_barrier(0);
     const int64_t t64 = target[row];
@@ -370,15 +374,18 @@ __global__ __launch_bounds__(256) void k_lp_backward(const T* __restrict__ x, lo
     const float u = valid ? upstream[row] : 0.0f, ls = lse[row];
 #pragma unroll
     for (int c = 0; c < GROUPS; ++c) {
-      const int off = lo + (c * 256 + (int)threadIdx.x) * 8;
-      float v[8];
-      raw[c].widen(v);
+      const int off = lo + (c * 256 + (int)threadIdx.x) * W;
+      float v[W];
+      ix_lp_widen16(raw[c], v);
 #pragma unroll
-      for (int i = 0; i < 8; ++i) {
+      for (int i = 0; i < W; ++i) {
         v[i] = ix_exp(v[i] - ls) * -u;
         if (off + i == t) v[i] = v[i] + u;
       }
-      if (off < hi) ix_lp_store8<T>(gr + off, v);
+      if (off >= hi) continue;
+      uint4* d = reinterpret_cast<uint4*>(gr + off);
+      if (ONCE) ix_store16_once(d, ix_lp_pack16(v));
+      else *d = ix_lp_pack16(v);
     }
     return;
   }
@@ -515,14 +522,23 @@ extern "C" int ix_logprob_rowinv_backward(const void* logits, int dtype, long ro
   if (rows == 0) return IX_OK;
   const long P = (V + IX_LP_SEG - 1) / IX_LP_SEG;
   if (V > 0x7fff0000L || rows * P > 0x7fffffffL) return IX_DECLINED;
-  const size_t al = 8 * (dtype == IX_DT_BF16 ? sizeof(bf16_t) : sizeof(float));
-  const int vec = (V % 8 == 0) && (row_stride % 8 == 0) && (grad_stride % 8 == 0) && ix_aligned(logits, al) && ix_aligned(grad, al);
+  const int vec = (V % 8 == 0) && (row_stride % 8 == 0) && (grad_stride % 8 == 0) && ix_aligned(logits, 16) && ix_aligned(grad, 16);
+  // Logits of 256 MiB and more (the memory-side cache): a default store leaves dirty lines that the next kernel's reads
+  // have to wait for, and a default load only displaces lines. Forward + backward, us, default / past the caches: fp32
+  // 1000 rows of 151936 413 / 367, 2900 1165 / 1086, bf16 1000 217 / 200, 2900 602 / 572; below the line the logits are
+  // still there for the next pass (fp32 300 rows 122 / 124, 100 rows 48 / 51).
+  const bool once = rows * V * (long)(dtype == IX_DT_BF16 ? sizeof(bf16_t) : sizeof(float)) >= (256L << 20);
   hipStream_t st = (hipStream_t)stream;
-  if (dtype == IX_DT_BF16)
-    hipLaunchKernelGGL(k_lp_backward<bf16_t>, dim3((unsigned)(rows * P)), dim3(256), 0, st, (const bf16_t*)logits,
-                       row_stride, (int)V, (int)P, target, upstream, lse, (bf16_t*)grad, grad_stride, vec);
-  else
-    hipLaunchKernelGGL(k_lp_backward<float>, dim3((unsigned)(rows * P)), dim3(256), 0, st, (const float*)logits,
-                       row_stride, (int)V, (int)P, target, upstream, lse, (float*)grad, grad_stride, vec);
+#define IX_LP_BACK(T, ONCE)                                                                                         \
+  hipLaunchKernelGGL((k_lp_backward<T, ONCE>), dim3((unsigned)(rows * P)), dim3(256), 0, st, (const T*)logits, row_stride, \
+                     (int)V, (int)P, target, upstream, lse, (T*)grad, grad_stride, vec)
+  if (dtype == IX_DT_BF16) {
+    if (once) IX_LP_BACK(bf16_t, true);
+    else IX_LP_BACK(bf16_t, false);
+  } else {
+    if (once) IX_LP_BACK(float, true);
+    else IX_LP_BACK(float, false);
+  }
+#undef IX_LP_BACK
   return ix_launch_status();
 }

@@ -46,3 +46,20 @@ def test_gradient_through_the_function_equals_the_differentiable_form():
     (a,) = torch.autograd.grad(_RowInvSampledLogprob.apply(x, t, 8), x, u)
     (b,) = torch.autograd.grad(_RowInvSampledLogprob.apply(x, t, 8), x, u, create_graph=True)
     assert b.requires_grad and float((a - b.detach()).abs().max()) <= 2.0 ** -22 * float(a.abs().max())
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_a_gradient_larger_than_the_caches_equals_its_rows_taken_by_themselves(dtype):
+    """From 256 MiB of logits both streams go past the caches: the bits of calls below that line."""
+    from isoexec_amd.ops.logprobs.rowinv import sampled_backward
+
+    vocab = 16384 + 8
+    rows = (256 << 20) // (vocab * dtype.itemsize) + 2
+    x = torch.randn(rows, vocab, generator=torch.Generator(device=DEV).manual_seed(1), device=DEV).to(dtype)
+    t = torch.randint(-1, vocab + 1, (rows,), generator=cpu_gen(3)).to(DEV)
+    u = torch.randn(rows, generator=cpu_gen(4)).to(DEV)
+    lse = torch.logsumexp(x.float(), 1)
+    whole = sampled_backward(x, t, u, lse)
+    half = rows // 2
+    parts = [sampled_backward(x[a:b], t[a:b], u[a:b], lse[a:b]) for a, b in ((0, half), (half, rows))]
+    assert torch.equal(whole, torch.cat(parts))

@@ -113,11 +113,12 @@ def sampled_backward(x: torch.Tensor, t: torch.Tensor, upstream: torch.Tensor, l
     if x.stride(1) != 1:
         return None
     rows, vocab = x.shape
+    # named: a copy made here has to outlive the call (the allocator hands a freed one out again for the next)
+    tc, uc, lc = t.contiguous(), upstream.contiguous(), lse.contiguous()
     grad = torch.empty(rows, vocab, dtype=x.dtype, device=x.device)
     rc = _lib.check(
         _lib.lib().ix_logprob_rowinv_backward(x.data_ptr(), _lib.dtype_code(x.dtype), rows, vocab, x.stride(0),
-                                              t.contiguous().data_ptr(), upstream.contiguous().data_ptr(),
-                                              lse.contiguous().data_ptr(), grad.data_ptr(), grad.stride(0),
+                                              tc.data_ptr(), uc.data_ptr(), lc.data_ptr(), grad.data_ptr(), grad.stride(0),
                                               _lib.current_stream(x.device)), "ix_logprob_rowinv_backward")
     return grad if rc == _lib.IX_OK else None
 

@@ -63,3 +63,19 @@ def test_a_gradient_larger_than_the_caches_equals_its_rows_taken_by_themselves(d
     half = rows // 2
     parts = [sampled_backward(x[a:b], t[a:b], u[a:b], lse[a:b]) for a, b in ((0, half), (half, rows))]
     assert torch.equal(whole, torch.cat(parts))
+
+
+def test_strided_targets_and_an_expanded_upstream(monkeypatch):
+    """Targets that are a view of a wider label tensor, and the upstream of a ``.sum()`` (one element, expanded): both are
+    copied for the kernel, and the gradient is the one of contiguous operands."""
+    from isoexec_amd.ops.logprobs.rowinv import rowinv_sampled_logprobs
+
+    monkeypatch.setenv("SKYRL_ISOEXEC", "1")
+    g = cpu_gen(5)
+    x = torch.randn(2, 300, 512, generator=g).to(DEV).requires_grad_(True)
+    labels = torch.randint(0, 512, (2, 300, 2), generator=g).to(DEV)
+    call = lambda t: rowinv_sampled_logprobs(x, t, vocab_start_index=0, vocab_end_index=512, group=None,
+                                             src_dtype=torch.float32, reference=None)
+    (want,) = torch.autograd.grad(call(labels[:, :, 0].contiguous()), x, torch.ones(2, 300, device=DEV))
+    (got,) = torch.autograd.grad(call(labels[:, :, 0]).sum(), x)
+    assert torch.equal(got, want)

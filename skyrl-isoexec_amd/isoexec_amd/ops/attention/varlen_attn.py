@@ -61,10 +61,11 @@ def varlen_attention(
     o = torch.empty(Tq, HQ, D, dtype=torch.bfloat16, device=q.device)
     if Tq == 0 or n_seq == 0:
         return o
+    starts, pos0 = kv_start.contiguous(), None if q_pos0 is None else q_pos0.contiguous()  # named: they outlive the call
     rc = _lib.check(
         _lib.lib().ix_attn_varlen(
             q.data_ptr(), q.stride(0), k.data_ptr(), v.data_ptr(), k.stride(0), o.data_ptr(), cu_seqlens_q.data_ptr(),
-            kv_start.contiguous().data_ptr(), _lib.ptr(None if q_pos0 is None else q_pos0.contiguous()), n_seq,
+            starts.data_ptr(), _lib.ptr(pos0), n_seq,
             int(max_q_len), HQ, HKV, D, float(D) ** -0.5 if scale is None else float(scale),
             _lib.current_stream(q.device)),
         "ix_attn_varlen")

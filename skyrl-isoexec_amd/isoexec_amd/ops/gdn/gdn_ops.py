@@ -282,11 +282,11 @@ def decode_prep(x, a, b, conv_weight, conv_bias, A_log, dt_bias, conv_state, row
     beta = torch.empty(N, HV, dtype=x.dtype, device=x.device)
     wc = conv_weight if conv_weight.is_contiguous() else conv_weight.contiguous()
     bc = None if conv_bias is None else (conv_bias if conv_bias.is_contiguous() else conv_bias.contiguous())
+    ac, dc = A_log.contiguous(), dt_bias.contiguous()  # named: the copies have to outlive the call
     rc = _lib.check(
         _lib.lib().ix_gdn_decode_prep(x.data_ptr(), x.stride(0), a.data_ptr(), a.stride(0), b.data_ptr(), b.stride(0),
-                                      wc.data_ptr(), _lib.ptr(bc), A_log.contiguous().data_ptr(),
-                                      dt_bias.contiguous().data_ptr(), conv_state.data_ptr(), rows.data_ptr(),
-                                      y.data_ptr(), g.data_ptr(), beta.data_ptr(), N, H, K, HV, V, 4,
+                                      wc.data_ptr(), _lib.ptr(bc), ac.data_ptr(), dc.data_ptr(), conv_state.data_ptr(),
+                                      rows.data_ptr(), y.data_ptr(), g.data_ptr(), beta.data_ptr(), N, H, K, HV, V, 4,
                                       int(activation is not None), L2NORM_EPS, _lib.current_stream(x.device)),
         "ix_gdn_decode_prep")
     return (y, g, beta) if rc == _lib.IX_OK else None

@@ -73,8 +73,10 @@ def permute(topk_idx: torch.Tensor, topk_prob: torch.Tensor, E: int, *, BM: int 
     p.permuted_prob = torch.empty(T * k, dtype=torch.float32, device=dev)
     p.combine_rows = torch.empty(T, k, **i32)
     p.tile_meta = torch.empty(1 + 3 * p.max_tiles, **i32)
+    # named: a copy made here has to outlive the call (the allocator hands a freed one out again for the next)
+    idx, prob = topk_idx.contiguous(), topk_prob.contiguous()
     if static_scratch:
-        rc = L.ix_moe_permute_static(topk_idx.contiguous().data_ptr(), topk_prob.contiguous().data_ptr(), T, E, k, p.BM,
+        rc = L.ix_moe_permute_static(idx.data_ptr(), prob.data_ptr(), T, E, k, p.BM,
                                      p.counts.data_ptr(), p.offsets.data_ptr(), p.sorted_token.data_ptr(),
                                      p.permuted_prob.data_ptr(), p.combine_rows.data_ptr(), p.tile_meta.data_ptr(),
                                      p.max_tiles, _lib.current_stream(dev))
@@ -86,7 +88,7 @@ def permute(topk_idx: torch.Tensor, topk_prob: torch.Tensor, E: int, *, BM: int 
         return p
     scratch = torch.empty(max(1, int(L.ix_moe_permute_scratch_ints(T, E))), **i32)
     _lib.check(
-        L.ix_moe_permute(topk_idx.contiguous().data_ptr(), topk_prob.contiguous().data_ptr(), T, E, k, p.BM,
+        L.ix_moe_permute(idx.data_ptr(), prob.data_ptr(), T, E, k, p.BM,
                          p.counts.data_ptr(), p.offsets.data_ptr(), p.sorted_token.data_ptr(),
                          p.permuted_prob.data_ptr(), p.combine_rows.data_ptr(), p.tile_meta.data_ptr(), p.max_tiles,
                          scratch.data_ptr(), _lib.current_stream(dev)), "ix_moe_permute")
@@ -190,10 +192,10 @@ def experts_forward(x: torch.Tensor, w1: torch.Tensor, w2: torch.Tensor, p: Perm
                                              rows, H, F, _lib.current_stream(dev)), "ix_moe_experts_packed")
         if rc == _lib.IX_OK:
             return (out, inter) if return_inter else out
+    w1c, w2c = w1.contiguous(), w2.contiguous()  # named: the copies have to outlive the call
     rc = _lib.check(
         _lib.lib().ix_moe_experts_tile(xc.data_ptr(), xc.stride(0), p.sorted_token.data_ptr(),
-                                       p.permuted_prob.data_ptr(), w1.contiguous().data_ptr(),
-                                       w2.contiguous().data_ptr(), p.tile_meta.data_ptr(), p.max_tiles, p.BM,
+                                       p.permuted_prob.data_ptr(), w1c.data_ptr(), w2c.data_ptr(), p.tile_meta.data_ptr(), p.max_tiles, p.BM,
                                        p.BN, inter.data_ptr(), out.data_ptr(), T, rows, H, F,
                                        _lib.current_stream(dev)),
         "ix_moe_experts")

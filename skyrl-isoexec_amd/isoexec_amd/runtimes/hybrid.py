@@ -28,6 +28,7 @@ from ..debug.trace import get_tracer
 from ..ops.attention.varlen_attn import KVCache, varlen_attention
 from ..ops.gdn.gdn_ops import conv_packed, gdn_native_core, gdn_native_core_normed
 from ..ops.gdn.gdn_cpr import gdn_native_cpr_fwd, gdn_native_cpr_normed
+from ..ops.gdn.gdn_cpr_rows import fused_rows_enabled
 from ..ops.gdn.gdn_cpr_state import CprGDN
 from ..ops.gdn.gdn_recurrent_state import RecurrentGDN
 from ..ops.logprobs.rowinv import leaves, sampled_forward
@@ -511,9 +512,12 @@ class RolloutEngine:
     def _native_step_tables(self, n: int):
         """``(dims, layers)`` for ``ix_decode_step``: the layers' device pointers as they are now (tables are built anew for
         every step, so a replaced weight or a moved pool is seen), or ``None`` when the step has to be taken op by op: a
-        log or a trace wants the ops' outputs, or something is not the plain contiguous tensor the call expects."""
+        log or a trace wants the ops' outputs, the fused row lookup is switched off, or something is not the plain
+        contiguous tensor the call expects."""
         b, c = self.blocks, self.cfg
         if b.region_log is not None or b.routing_log is not None or c.gdn_kernel != "recurrent" or c.conv_width != 4:
+            return None
+        if not fused_rows_enabled():
             return None
         bf16, f32, i64 = torch.bfloat16, torch.float32, torch.int64
         ok = True

@@ -100,3 +100,22 @@ def test_a_weight_of_another_shape_is_not_handed_to_the_native_step(layer, name,
     else:
         w.layers[layer][name] = cut(w.layers[layer][name]).contiguous()
     assert e._native_step_tables(2) is None
+
+
+def test_the_row_lookup_switch_sends_the_step_op_by_op(monkeypatch):
+    from isoexec_amd.ops.gdn import gdn_cpr_rows
+    from isoexec_amd.runtimes.hybrid import HybridWeights, RolloutEngine
+
+    w = HybridWeights.make(config(), seed=6, device=DEV)
+    engines = [RolloutEngine(config(), w, max_num_seqs=2, max_len=32) for _ in range(2)]
+    tok = torch.tensor([5, 6], device=DEV)
+    for e in engines:
+        e.prefill([0, 1], torch.tensor([1, 2, 3], device=DEV), [2, 1])
+    want = engines[0].decode([0, 1], tok)
+    monkeypatch.setenv("SKYRL_ISOEXEC_GDN_CPR_FUSED_ROWS", "0")
+    assert engines[1]._native_step_tables(2) is None
+    served = gdn_cpr_rows._served
+    got = engines[1].decode([0, 1], tok)
+    assert gdn_cpr_rows._served == served and same_bits(got, want)
+    for (name, a), (_, b) in zip(pools(engines[1]), pools(engines[0])):
+        assert torch.equal(a.reshape(-1).view(torch.uint8), b.reshape(-1).view(torch.uint8)), name

@@ -520,12 +520,13 @@ class RolloutEngine:
         if not fused_rows_enabled():
             return None
         bf16, f32, i64 = torch.bfloat16, torch.float32, torch.int64
-        ok = True
+        dev = b.w.embed.device
+        ok = dev.type == "cuda"
 
-        def ptr(t, dtype, *shape):
+        def ptr(t, dtype, *shape):  # the kernels have no extents to check an index against: every shape is pinned here
             nonlocal ok
             p = t.data_ptr()
-            if t.dtype is not dtype or not t.is_contiguous() or p % 16 or (shape and tuple(t.shape) != shape) or not t.is_cuda:
+            if t.dtype is not dtype or t.shape != shape or not t.is_contiguous() or p % 16 or t.device != dev:
                 ok = False
             return p
 
@@ -537,7 +538,11 @@ class RolloutEngine:
             nxt = b.w.layers[i + 1]["pre_norm"] if i + 1 < c.layers else b.w.final_norm
             row = [int(attention), ptr(lw["post_norm"], bf16, H), ptr(nxt, bf16, H), ptr(lw["router"], bf16, E, H),
                    ptr(lw["w1"], bf16, E, 2 * F, H), ptr(lw["w2"], bf16, E, H, F)]
-            row += [t.data_ptr() for t in b.packed_experts[i]] if packed_all else [0, 0]
+            if packed_all:
+                w1f, w2f = b.packed_experts[i]
+                row += [ptr(w1f, bf16, E, 2 * F, H), ptr(w2f, bf16, E, H, F)]
+            else:
+                row += [0, 0]
             if attention:
                 q_width = c.q_heads * c.head_dim
                 shapes = {"qkv_proj": (q_width + 2 * c.kv_heads * c.head_dim, H), "o_proj": (H, q_width)}
@@ -545,21 +550,29 @@ class RolloutEngine:
                 shapes = {"in_proj": (D + c.gdn_z + 2 * c.gdn_v_heads, H), "out_proj": (H, c.gdn_z)}
             for name, shape in shapes.items():
                 pk = b.packed_dense.get((i, name))
-                row += [ptr(lw[name], bf16, *shape), 0 if pk is None else pk.packed.data_ptr()]
+                if pk is None:
+                    row += [ptr(lw[name], bf16, *shape), 0]
+                else:  # as linear_nt: the weight the copy was made of beside the copy
+                    row += [ptr(pk.weight, bf16, *shape), ptr(pk.packed, bf16, shape[0] * shape[1])]
             if attention:
                 kv = self.kv[i]
-                row += [0] * 11 + [ptr(kv.k, bf16), ptr(kv.v, bf16)]
+                cache = (kv.k.shape[0], self.max_len, c.kv_heads, c.head_dim)
+                row += [0] * 11 + [ptr(kv.k, bf16, *cache), ptr(kv.v, bf16, *cache)]
             else:
                 g = self.gdn[i]
                 if type(g) is not RecurrentGDN or g.table is None or g.activation not in ("silu", "swish") or not g.fused_decode_prep:
                     return None
                 row += [ptr(g.conv_weight, bf16, D, 4), 0 if g.conv_bias is None else ptr(g.conv_bias, bf16, D),
                         ptr(g.A_log, f32, c.gdn_v_heads), ptr(g.dt_bias, f32, c.gdn_v_heads), ptr(lw["out_norm"], bf16, c.gdn_head_dim),
-                        ptr(g.ssm_state, f32), ptr(g.conv_state, bf16), ptr(g.slot2row, i64), g.slot2row.numel(),
-                        ptr(g.last_used, i64), ptr(g._clock, i64), 0, 0]
+                        ptr(g.ssm_state, f32, g.capacity + 1, c.gdn_v_heads, c.gdn_head_dim, c.gdn_head_dim),
+                        ptr(g.conv_state, bf16, g.capacity + 1, D, c.conv_width - 1),
+                        ptr(g.slot2row, i64, g.table.map_size), g.table.map_size, ptr(g.last_used, i64, g.capacity + 1),
+                        ptr(g._clock, i64), 0, 0]
             table += row
         ptr(b.w.embed, bf16, c.vocab, H)
         ptr(b.w.layers[0]["pre_norm"], bf16, H)
+        ptr(b.cos, bf16, b.cos.shape[0], c.head_dim)
+        ptr(b.sin, bf16, b.cos.shape[0], c.head_dim)
         if not ok:
             return None
         dims = array("q", [n, c.layers, H, c.vocab, b.cos.shape[0], c.gdn_k_heads, c.gdn_v_heads, c.gdn_head_dim, c.q_heads,

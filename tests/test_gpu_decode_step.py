@@ -119,3 +119,29 @@ def test_the_row_lookup_switch_sends_the_step_op_by_op(monkeypatch):
     assert gdn_cpr_rows._served == served and same_bits(got, want)
     for (name, a), (_, b) in zip(pools(engines[1]), pools(engines[0])):
         assert torch.equal(a.reshape(-1).view(torch.uint8), b.reshape(-1).view(torch.uint8)), name
+
+
+@pytest.mark.parametrize("what", ["keys", "values", "ssm_state", "conv_state", "last_used", "slot2row", "sin", "cos", "experts"])
+def test_a_pool_table_or_copy_of_another_shape_is_not_handed_to_the_native_step(what):
+    """The kernels index these with what the pools' own tables say: a tensor of another shape, or of another type, goes op by
+    op, where the ops' own checks refuse it."""
+    from isoexec_amd.runtimes.hybrid import HybridWeights, RolloutEngine
+
+    cfg = config(expert_inter=512)
+    e = RolloutEngine(cfg, HybridWeights.make(cfg, seed=4, device=DEV), max_num_seqs=2, max_len=32)
+    assert e._native_step_tables(2) is not None
+    if what in ("keys", "values"):
+        kv, name = e.kv[1], what[0]
+        setattr(kv, name, getattr(kv, name)[:, :16].contiguous())
+    elif what in ("sin", "cos"):
+        setattr(e.blocks, what, getattr(e.blocks, what).float())
+    elif what == "experts":
+        w1f, w2f = e.blocks.packed_experts[2]
+        e.blocks.packed_experts[2] = (w1f[:-1].contiguous(), w2f)
+    else:
+        g = e.gdn[0]
+        setattr(g, what, getattr(g, what)[:-1].contiguous())
+    assert e._native_step_tables(2) is None
+    if what == "experts":
+        with pytest.raises(RuntimeError, match="pack_decode"):
+            e.blocks.moe(2, torch.zeros(2, 512, dtype=torch.bfloat16, device=DEV))

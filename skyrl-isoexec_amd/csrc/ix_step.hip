@@ -7,9 +7,9 @@
 // entry points, so every value is computed by the code that computes it when the ops are called one at a time, plus three
 // kernels that exist only here because they fold what the runtime does with tensor ops between the calls:
 //   k_step_begin     slot -> row of every GatedDeltaNet layer with its use stamp (ix_gdn_resolve_rows, one launch per layer
-//                    otherwise), the step's positions copied out of the context counters and the counters advanced, the
-//                    packed offsets 0..n
-//   k_embed_rmsnorm  the embedding rows gathered into the residual stream and normalised
+//                    otherwise), the step's positions copied out of the context counters and checked, the packed offsets
+//                    0..n
+//   k_embed_rmsnorm  the embedding rows gathered into the residual stream and normalised, the context counters advanced
 //   k_rope_append    q and k rotated (k_rope8's statements), k and v written to the caches at the step's positions
 #include "ix_common.h"
 #include "../../include/isoexec_hip.h"
@@ -27,10 +27,25 @@ struct IxStepMaps {
   IxStepMap m[IX_STEP_GDN_MAX];
 };
 
-// Workgroup l < layers: layer l's rows; the last workgroup: positions, counters, offsets. ctx NULL: rows only.
+// What a sequence's next token is checked against: nothing behind this kernel knows an extent.
+struct IxStepLimits {
+  const int* ctx;           // [n] the position of this token
+  const int64_t* kv_start;  // [n] first cache token of the sequence
+  int64_t cache_len;        // positions that the sequence's part of the cache and the rotary tables both hold
+  int64_t cache_tokens;     // tokens of the whole cache
+  __device__ __forceinline__ bool fits(int i) const {
+    const int64_t p = ctx[i], start = kv_start[i];
+    return p >= 0 && p < cache_len && start >= 0 && start < cache_tokens && p < cache_tokens - start;
+  }
+};
+
+// Workgroup l < layers: layer l's rows; the last workgroup (pos not NULL): positions and offsets. A sequence whose position
+// does not fit takes the step as a null lane -- row 0 of every state pool, position -1: no key and no state is stored, none
+// is read, its output is NaN -- and is reported in error[0]. The counters are advanced by a later launch (k_embed_rmsnorm),
+// so every workgroup here checks the same values.
 __global__ __launch_bounds__(256) void k_step_begin(IxStepMaps maps, int layers, const int64_t* __restrict__ slots, int n,
-                                                    int* __restrict__ rows, int* __restrict__ ctx, int* __restrict__ pos,
-                                                    int* __restrict__ cu) {
+                                                    IxStepLimits lim, int* __restrict__ rows, int* __restrict__ pos,
+                                                    int* __restrict__ cu, int* __restrict__ error) {
   const int l = blockIdx.x;
   if (l < layers) {
     const IxStepMap m = maps.m[l];
@@ -38,7 +53,7 @@ __global__ __launch_bounds__(256) void k_step_begin(IxStepMaps maps, int layers,
     for (int i = threadIdx.x; i < n; i += 256) {
       int64_t s = slots[i];
       s = s < 0 ? 0 : (s > m.map_n - 1 ? m.map_n - 1 : s);
-      const int64_t r = m.slot2row[s];
+      const int64_t r = lim.fits(i) ? m.slot2row[s] : 0;
       rows[(long)l * n + i] = (int)r;
       m.last_used[r] = stamp;
     }
@@ -46,29 +61,32 @@ __global__ __launch_bounds__(256) void k_step_begin(IxStepMaps maps, int layers,
     if (threadIdx.x == 0) m.clock[0] = stamp;
     return;
   }
-  if (!ctx) return;
+  if (!pos) return;
   for (int i = threadIdx.x; i <= n; i += 256) {
     cu[i] = i;
     if (i < n) {
-      const int p = ctx[i];
-      pos[i] = p;
-      ctx[i] = p + 1;
+      const bool fits = lim.fits(i);
+      pos[i] = fits ? lim.ctx[i] : -1;
+      // host memory: seen by the host once the launch has ended, whatever the caller waits for
+      if (!fits && error) __hip_atomic_store(error, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     }
   }
 }
 
 // h[i] = table[tokens[i]], x[i] = norm(h[i]): k_rmsnorm_reg<64, 0, NG>'s statements (ix_norm.hip) on the gathered row. A
-// token outside the table reads nothing and gives a row of NaNs.
+// token outside the table reads nothing and gives a row of NaNs, a null lane (pos < 0) as well. Advances ctx.
 template <int NG>
 __global__ __launch_bounds__(64) void k_embed_rmsnorm(const bf16_t* __restrict__ table, long vocab,
-                                                      const int64_t* __restrict__ tokens, const bf16_t* __restrict__ w,
+                                                      const int64_t* __restrict__ tokens, const int* __restrict__ pos,
+                                                      int* __restrict__ ctx, const bf16_t* __restrict__ w,
                                                       bf16_t* __restrict__ h, bf16_t* __restrict__ x, float eps,
                                                       int zero_centered) {
   constexpr int LPR = 64, N = LPR * 8 * NG;
   const int sub = threadIdx.x;
   const long row = blockIdx.x;
   const int64_t t = tokens[row];
-  const bool held = t >= 0 && t < vocab;
+  const bool held = t >= 0 && t < vocab && pos[row] >= 0;
+  if (sub == 0) ctx[row] += 1;
   const bf16_t* src = table + (held ? t : 0) * N + sub * 8;
   uint4 xp[NG], wp[NG];
 #pragma unroll
@@ -107,12 +125,12 @@ __global__ __launch_bounds__(64) void k_embed_rmsnorm(const bf16_t* __restrict__
 
 static bool ix_embed_rmsnorm_serves(long N) { return N == 512 || N == 1024 || N == 2048 || N == 4096; }
 
-static int ix_embed_rmsnorm(const void* table, long vocab, const int64_t* tokens, const void* w, void* h, void* x, long n,
-                            long N, float eps, hipStream_t st) {
+static int ix_embed_rmsnorm(const void* table, long vocab, const int64_t* tokens, const int* pos, int* ctx, const void* w,
+                            void* h, void* x, long n, long N, float eps, hipStream_t st) {
 #define IX_EMB(NG_)                                                                                                     \
   if (N == 512 * NG_) {                                                                                                 \
     hipLaunchKernelGGL((k_embed_rmsnorm<NG_>), dim3((unsigned)n), dim3(64), 0, st, (const bf16_t*)table, vocab, tokens, \
-                       (const bf16_t*)w, (bf16_t*)h, (bf16_t*)x, eps, 1);                                               \
+                       pos, ctx, (const bf16_t*)w, (bf16_t*)h, (bf16_t*)x, eps, 1);                                     \
     return ix_launch_status();                                                                                          \
   }
   IX_EMB(1) IX_EMB(2) IX_EMB(4) IX_EMB(8)
@@ -121,13 +139,13 @@ static int ix_embed_rmsnorm(const void* table, long vocab, const int64_t* tokens
 }
 
 // The projection row of a token holds HQ + HKV heads to rotate and HKV value heads, D each. Rotated q heads go back to the
-// row, rotated k heads and the v heads to cache token kv_start[n] + pos[n] ([*, HKV, D]). Eight pairs (or, for v, sixteen
-// values) per thread; the rotation is k_rope8's (ix_attn.hip), statement for statement.
+// row, rotated k heads and the v heads to cache token kv_start[n] + pos[n] ([*, HKV, D]), which k_step_begin has checked
+// against the cache and the tables; a null lane (pos < 0) stores neither. Eight pairs (or, for v, sixteen values) per
+// thread; the rotation is k_rope8's (ix_attn.hip), statement for statement.
 __global__ __launch_bounds__(256) void k_rope_append(bf16_t* __restrict__ proj, long pitch, const bf16_t* __restrict__ cs,
-                                                     const bf16_t* __restrict__ sn, int table_rows,
-                                                     const int* __restrict__ pos, const int64_t* __restrict__ kv_start,
-                                                     bf16_t* __restrict__ kc, bf16_t* __restrict__ vc, int HQ, int HKV,
-                                                     int D) {
+                                                     const bf16_t* __restrict__ sn, const int* __restrict__ pos,
+                                                     const int64_t* __restrict__ kv_start, bf16_t* __restrict__ kc,
+                                                     bf16_t* __restrict__ vc, int HQ, int HKV, int D) {
   const int n = blockIdx.y;
   const int chunks = D >> 4;  // 8-pair chunks per head
   const int i = blockIdx.x * 256 + threadIdx.x;
@@ -135,6 +153,7 @@ __global__ __launch_bounds__(256) void k_rope_append(bf16_t* __restrict__ proj, 
   const int c = i % chunks, hd = i / chunks, half = D >> 1;
   bf16_t* row = proj + (long)n * pitch + (long)hd * D + c * 8;
   const int p = pos[n];
+  if (p < 0 && hd >= HQ) return;
   const uint4 a4 = *reinterpret_cast<const uint4*>(row), b4 = *reinterpret_cast<const uint4*>(row + half);
   const long slot = kv_start[n] + p;
   if (hd >= HQ + HKV) {
@@ -144,7 +163,7 @@ __global__ __launch_bounds__(256) void k_rope_append(bf16_t* __restrict__ proj, 
     return;
   }
   uint4 lo4, hi4;
-  if (p < 0 || p >= table_rows) {
+  if (p < 0) {
     lo4 = hi4 = make_uint4(0x7fc07fc0u, 0x7fc07fc0u, 0x7fc07fc0u, 0x7fc07fc0u);
   } else {
     const bf16_t* ct = cs + (long)p * D + c * 8;
@@ -247,6 +266,7 @@ Work carve(const IxDecodeDims& d, void* base) {
 
 bool served(const IxDecodeDims& d) {
   if (d.n <= 0 || d.n > 65535 || d.layers <= 0 || d.vocab <= 0 || d.max_positions <= 0 || d.max_positions > 0x7fffffffL) return false;
+  if (d.cache_len <= 0 || d.cache_tokens <= 0) return false;
   if (!ix_embed_rmsnorm_serves(d.hidden)) return false;
   // ix_moe_combine_add_rmsnorm's widths
   const long ng = d.hidden / 512;
@@ -269,7 +289,7 @@ extern "C" size_t ix_decode_step_workspace_bytes(const IxDecodeDims* dims) {
 extern "C" int ix_decode_step(const IxDecodeDims* dims, const IxDecodeLayer* layers, const void* embed, const void* pre_norm,
                               const void* cos_table, const void* sin_table, const int64_t* tokens, const int64_t* slots,
                               int* ctx, const int64_t* kv_start, float eps, void* workspace, size_t workspace_bytes,
-                              void* out, void* stream) {
+                              void* out, int* error, void* stream) {
   if (!dims || !layers || !embed || !pre_norm || !cos_table || !sin_table || !tokens || !slots || !ctx || !kv_start ||
       !workspace || !out)
     return IX_ERR_ARG;
@@ -287,6 +307,7 @@ extern "C" int ix_decode_step(const IxDecodeDims* dims, const IxDecodeLayer* lay
     if (rc_ != IX_OK) return rc_ > 0 ? IX_ERR_ARG : rc_; \
   }
   {
+    const IxStepLimits lim{ctx, kv_start, d.cache_len < d.max_positions ? d.cache_len : d.max_positions, d.cache_tokens};
     long l = 0;
     int row_base = 0;
     bool first = true;
@@ -296,14 +317,14 @@ extern "C" int ix_decode_step(const IxDecodeDims* dims, const IxDecodeLayer* lay
       for (; l < d.layers && cnt < IX_STEP_GDN_MAX; ++l)
         if (layers[l].kind == 0)
           maps.m[cnt++] = IxStepMap{layers[l].slot2row, layers[l].map_n, layers[l].last_used, layers[l].clock};
-      hipLaunchKernelGGL(k_step_begin, dim3((unsigned)(cnt + 1)), dim3(256), 0, st, maps, cnt, slots, (int)n,
-                         w.rows + (long)row_base * n, first ? ctx : nullptr, w.pos, w.cu);
+      hipLaunchKernelGGL(k_step_begin, dim3((unsigned)(cnt + 1)), dim3(256), 0, st, maps, cnt, slots, (int)n, lim,
+                         w.rows + (long)row_base * n, first ? w.pos : nullptr, w.cu, error);
       row_base += cnt;
       first = false;
     }
     IX_STEP(ix_launch_status());
   }
-  IX_STEP(ix_embed_rmsnorm(embed, d.vocab, tokens, pre_norm, w.h[0], w.x, n, Hd, eps, st));
+  IX_STEP(ix_embed_rmsnorm(embed, d.vocab, tokens, w.pos, ctx, pre_norm, w.h[0], w.x, n, Hd, eps, st));
   auto linear = [&](const bf16_t* a, long K, const void* weight, const void* packed, bf16_t* c, long N) -> int {
     if (packed && n <= 64) {
       const int rc = ix_gemm_bf16_nt_decode(a, K, packed, c, N, n, N, K, stream);
@@ -334,8 +355,8 @@ extern "C" int ix_decode_step(const IxDecodeDims* dims, const IxDecodeLayer* lay
       IX_STEP(linear(w.x, Hd, y.w_in, y.w_in_packed, w.proj, pw));
       const unsigned per = (unsigned)((HQ + 2 * HKV) * (D / 16));
       hipLaunchKernelGGL(k_rope_append, dim3((per + 255) / 256, (unsigned)n), dim3(256), 0, st, w.proj, pw,
-                         (const bf16_t*)cos_table, (const bf16_t*)sin_table, (int)d.max_positions, w.pos, kv_start,
-                         (bf16_t*)y.k_cache, (bf16_t*)y.v_cache, (int)HQ, (int)HKV, (int)D);
+                         (const bf16_t*)cos_table, (const bf16_t*)sin_table, w.pos, kv_start, (bf16_t*)y.k_cache,
+                         (bf16_t*)y.v_cache, (int)HQ, (int)HKV, (int)D);
       IX_STEP(ix_launch_status());
       IX_STEP(ix_attn_varlen(w.proj, pw, y.k_cache, y.v_cache, HKV * D, w.o, w.cu, (const long*)kv_start, w.pos, n, 1, HQ,
                              HKV, D, (float)pow((double)D, -0.5), stream));

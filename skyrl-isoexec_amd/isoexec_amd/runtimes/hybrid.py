@@ -418,7 +418,7 @@ class RolloutEngine:
             self.blocks.pack_expert_weights()
             self.blocks.pack_dense_weights()
         dev = weights.embed.device
-        self.max_len = max_len
+        self.max_len, self.max_num_seqs = max_len, max_num_seqs
         self.gdn, self.kv = {}, {}
         for i in range(cfg.layers):
             lw = weights.layers[i]
@@ -435,6 +435,7 @@ class RolloutEngine:
         self.kv_rows: dict[int, int] = {}
         self.free_kv_rows = list(range(max_num_seqs, 0, -1))
         self.context: dict[int, int] = {}
+        self._step_error: torch.Tensor | None = None  # pinned host int32 that a native step reports into
 
     def _kv_row(self, slot: int) -> int:
         if slot not in self.kv_rows:
@@ -456,6 +457,7 @@ class RolloutEngine:
         """Prompts packed in ``tokens``; returns the final-normed hidden state of each prompt's LAST
         token ``[N, H]`` (the row the first response token is sampled from)."""
         b, c = self.blocks, self.cfg
+        self._raise_step_error()
         check_lengths(c, lens, "prefill")
         if int(max(lens)) > self.max_len:
             raise ValueError(f"[isoexec-amd] prefill: a prompt of {int(max(lens))} tokens exceeds the cache length {self.max_len}")
@@ -491,6 +493,24 @@ class RolloutEngine:
         for s, n in zip(slots, lens):
             self.context[s] = n
         return x.index_select(0, torch.from_numpy(offs[1:].astype(np.int64) - 1).to(dev))
+
+    def _step_error_flag(self) -> torch.Tensor:
+        if self._step_error is None:
+            self._step_error = torch.zeros(1, dtype=torch.int32, pin_memory=True)
+        return self._step_error
+
+    def _raise_step_error(self) -> None:
+        """Raise what an earlier native step has reported. Read without waiting for the device, so a fault of the step in
+        flight is seen by the call after it (``check_steps`` waits)."""
+        if self._step_error is not None and int(self._step_error[0]):
+            self._step_error.zero_()
+            raise RuntimeError("[isoexec-amd] decode: a sequence's position in an earlier step lay outside its part of the "
+                               "key/value cache; nothing was stored for it and its output is NaN")
+
+    def check_steps(self) -> None:
+        """Wait for the steps issued so far and raise if one of them reported a fault."""
+        torch.cuda.current_stream(self.blocks.w.embed.device).synchronize()
+        self._raise_step_error()
 
     def _decode_state(self, slots: list):
         """Device-resident description of a decode batch: slot ids, each sequence's context length
@@ -556,7 +576,7 @@ class RolloutEngine:
                     row += [ptr(pk.weight, bf16, *shape), ptr(pk.packed, bf16, shape[0] * shape[1])]
             if attention:
                 kv = self.kv[i]
-                cache = (kv.k.shape[0], self.max_len, c.kv_heads, c.head_dim)
+                cache = (self.max_num_seqs + 1, self.max_len, c.kv_heads, c.head_dim)
                 row += [0] * 11 + [ptr(kv.k, bf16, *cache), ptr(kv.v, bf16, *cache)]
             else:
                 g = self.gdn[i]
@@ -576,7 +596,8 @@ class RolloutEngine:
         if not ok:
             return None
         dims = array("q", [n, c.layers, H, c.vocab, b.cos.shape[0], c.gdn_k_heads, c.gdn_v_heads, c.gdn_head_dim, c.q_heads,
-                           c.kv_heads, c.head_dim, E, c.topk, F, int(packed_all), int(c.moe_combine_dtype == "fp32")])
+                           c.kv_heads, c.head_dim, E, c.topk, F, int(packed_all), int(c.moe_combine_dtype == "fp32"),
+                           (self.max_num_seqs + 1) * self.max_len, self.max_len])
         return dims, array("q", table)
 
     def _decode_native(self, st: dict, tokens: torch.Tensor):
@@ -597,13 +618,15 @@ class RolloutEngine:
             return None
         dev = w.embed.device
         _lib.require_device(tokens, w.embed)
+        error = self._step_error_flag()
         work = torch.empty(need, dtype=torch.uint8, device=dev)
         out = torch.empty(n, self.cfg.hidden, dtype=torch.bfloat16, device=dev)
         rc = _lib.check(
             L.ix_decode_step(dims.buffer_info()[0], layers.buffer_info()[0], w.embed.data_ptr(),
                              w.layers[0]["pre_norm"].data_ptr(), b.cos.data_ptr(), b.sin.data_ptr(), tokens.data_ptr(),
                              st["slots_t"].data_ptr(), st["ctx"].data_ptr(), st["kv_start"].data_ptr(), float(self.cfg.eps),
-                             work.data_ptr(), need, out.data_ptr(), _lib.current_stream(dev)), "ix_decode_step")
+                             work.data_ptr(), need, out.data_ptr(), error.data_ptr(),
+                             _lib.current_stream(dev)), "ix_decode_step")
         return out if rc == _lib.IX_OK else None
 
     def _decode_device(self, st: dict, tokens: torch.Tensor) -> torch.Tensor:
@@ -633,6 +656,7 @@ class RolloutEngine:
     @torch.no_grad()
     def decode(self, slots: list, tokens: torch.Tensor) -> torch.Tensor:
         """Feed one token per sequence; returns the final-normed hidden states ``[N, H]``."""
+        self._raise_step_error()
         if max(self.context[s] for s in slots) >= self.max_len:
             raise RuntimeError(f"[isoexec-amd] a sequence reached the cache length {self.max_len}")
         x = self._decode_device(self._decode_state(slots), tokens)
@@ -696,6 +720,7 @@ class DecodeGraph:
         self.tokens = torch.zeros(len(slots), dtype=torch.int64, device=dev)
         for layer in engine.gdn.values():
             layer.flush_slot_map()  # the slot map is read, never written, inside the graph
+        engine._step_error_flag()  # allocated outside the capture; the graph keeps its address, and the engine
         self.graph = torch.cuda.CUDAGraph()
         saved = self.state["ctx"].clone()
         with torch.cuda.graph(self.graph):
@@ -707,6 +732,7 @@ class DecodeGraph:
     @torch.no_grad()
     def step(self, tokens: torch.Tensor) -> torch.Tensor:
         eng = self.engine
+        eng._raise_step_error()
         if max(eng.context[s] for s in self.slots) >= eng.max_len:
             raise RuntimeError(f"[isoexec-amd] a sequence reached the cache length {eng.max_len}")
         self.tokens.copy_(tokens)

@@ -492,8 +492,9 @@ size_t ix_decode_step_workspace_bytes(const IxDecodeDims* dims); /* 0: not serve
 
 /* dims and layers in HOST memory, read during the call. tokens, slots int64 [n]; ctx int32 [n]: each sequence's position of
  * this token, advanced by one on the device; kv_start int64 [n]. out bf16 [n, hidden]: the normed hidden states. A sequence
- * whose position lies outside its part of the cache, the cache or the rotary tables stores nothing, gets a row of NaNs and
- * sets error[0] to 1 (error: int32 in host memory that the device can write, or NULL). */
+ * whose position lies outside its part of the cache, the cache or the rotary tables, or whose token lies outside [0, vocab),
+ * stores nothing, gets a row of NaNs and sets error[0] (the position) or error[1] (the token) to 1 (error: int32 [2] in host
+ * memory that the device can write, or NULL). */
 int ix_decode_step(const IxDecodeDims* dims, const IxDecodeLayer* layers, const void* embed, const void* pre_norm,
                    const void* cos_table, const void* sin_table, const int64_t* tokens, const int64_t* slots, int* ctx,
                    const int64_t* kv_start, float eps, void* workspace, size_t workspace_bytes, void* out,

@@ -28,21 +28,25 @@ struct IxStepMaps {
 };
 
 // What a sequence's next token is checked against: nothing behind this kernel knows an extent.
+enum { IX_STEP_FITS = -1, IX_STEP_BAD_POSITION = 0, IX_STEP_BAD_TOKEN = 1 };  // the latter two: index into error[]
 struct IxStepLimits {
+  const int64_t* tokens;    // [n]
+  int64_t vocab;
   const int* ctx;           // [n] the position of this token
   const int64_t* kv_start;  // [n] first cache token of the sequence
   int64_t cache_len;        // positions that the sequence's part of the cache and the rotary tables both hold
   int64_t cache_tokens;     // tokens of the whole cache
-  __device__ __forceinline__ bool fits(int i) const {
-    const int64_t p = ctx[i], start = kv_start[i];
-    return p >= 0 && p < cache_len && start >= 0 && start < cache_tokens && p < cache_tokens - start;
+  __device__ __forceinline__ int check(int i) const {
+    const int64_t p = ctx[i], start = kv_start[i], t = tokens[i];
+    if (!(p >= 0 && p < cache_len && start >= 0 && start < cache_tokens && p < cache_tokens - start)) return IX_STEP_BAD_POSITION;
+    return t >= 0 && t < vocab ? IX_STEP_FITS : IX_STEP_BAD_TOKEN;
   }
 };
 
 // Workgroup l < layers: layer l's rows; the last workgroup (pos not NULL): positions and offsets. A sequence whose position
-// does not fit takes the step as a null lane -- row 0 of every state pool, position -1: no key and no state is stored, none
-// is read, its output is NaN -- and is reported in error[0]. The counters are advanced by a later launch (k_embed_rmsnorm),
-// so every workgroup here checks the same values.
+// does not fit or whose token the embedding does not hold takes the step as a null lane -- row 0 of every state pool,
+// position -1: no key and no state is stored, none is read, its output is NaN -- and is reported in error[0] or error[1]. The
+// counters are advanced by a later launch (k_embed_rmsnorm), so every workgroup here checks the same values.
 __global__ __launch_bounds__(256) void k_step_begin(IxStepMaps maps, int layers, const int64_t* __restrict__ slots, int n,
                                                     IxStepLimits lim, int* __restrict__ rows, int* __restrict__ pos,
                                                     int* __restrict__ cu, int* __restrict__ error) {
@@ -53,7 +57,7 @@ __global__ __launch_bounds__(256) void k_step_begin(IxStepMaps maps, int layers,
     for (int i = threadIdx.x; i < n; i += 256) {
       int64_t s = slots[i];
       s = s < 0 ? 0 : (s > m.map_n - 1 ? m.map_n - 1 : s);
-      const int64_t r = lim.fits(i) ? m.slot2row[s] : 0;
+      const int64_t r = lim.check(i) == IX_STEP_FITS ? m.slot2row[s] : 0;
       rows[(long)l * n + i] = (int)r;
       m.last_used[r] = stamp;
     }
@@ -65,18 +69,18 @@ __global__ __launch_bounds__(256) void k_step_begin(IxStepMaps maps, int layers,
   for (int i = threadIdx.x; i <= n; i += 256) {
     cu[i] = i;
     if (i < n) {
-      const bool fits = lim.fits(i);
-      pos[i] = fits ? lim.ctx[i] : -1;
+      const int bad = lim.check(i);
+      pos[i] = bad == IX_STEP_FITS ? lim.ctx[i] : -1;
       // host memory: seen by the host once the launch has ended, whatever the caller waits for
-      if (!fits && error) __hip_atomic_store(error, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+      if (bad != IX_STEP_FITS && error) __hip_atomic_store(error + bad, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
     }
   }
 }
 
 // h[i] = table[tokens[i]], x[i] = norm(h[i]): k_rmsnorm_reg<64, 0, NG>'s statements (ix_norm.hip) on the gathered row. A
-// token outside the table reads nothing and gives a row of NaNs, a null lane (pos < 0) as well. Advances ctx.
+// null lane (pos < 0: its token may lie outside the table) reads nothing and gives a row of NaNs. Advances ctx.
 template <int NG>
-__global__ __launch_bounds__(64) void k_embed_rmsnorm(const bf16_t* __restrict__ table, long vocab,
+__global__ __launch_bounds__(64) void k_embed_rmsnorm(const bf16_t* __restrict__ table,
                                                       const int64_t* __restrict__ tokens, const int* __restrict__ pos,
                                                       int* __restrict__ ctx, const bf16_t* __restrict__ w,
                                                       bf16_t* __restrict__ h, bf16_t* __restrict__ x, float eps,
@@ -84,10 +88,9 @@ __global__ __launch_bounds__(64) void k_embed_rmsnorm(const bf16_t* __restrict__
   constexpr int LPR = 64, N = LPR * 8 * NG;
   const int sub = threadIdx.x;
   const long row = blockIdx.x;
-  const int64_t t = tokens[row];
-  const bool held = t >= 0 && t < vocab && pos[row] >= 0;
+  const bool held = pos[row] >= 0;
   if (sub == 0) ctx[row] += 1;
-  const bf16_t* src = table + (held ? t : 0) * N + sub * 8;
+  const bf16_t* src = table + (held ? tokens[row] : 0) * N + sub * 8;
   uint4 xp[NG], wp[NG];
 #pragma unroll
   for (int c = 0; c < NG; ++c) xp[c] = *reinterpret_cast<const uint4*>(src + c * LPR * 8);
@@ -125,11 +128,11 @@ __global__ __launch_bounds__(64) void k_embed_rmsnorm(const bf16_t* __restrict__
 
 static bool ix_embed_rmsnorm_serves(long N) { return N == 512 || N == 1024 || N == 2048 || N == 4096; }
 
-static int ix_embed_rmsnorm(const void* table, long vocab, const int64_t* tokens, const int* pos, int* ctx, const void* w,
-                            void* h, void* x, long n, long N, float eps, hipStream_t st) {
+static int ix_embed_rmsnorm(const void* table, const int64_t* tokens, const int* pos, int* ctx, const void* w, void* h,
+                            void* x, long n, long N, float eps, hipStream_t st) {
 #define IX_EMB(NG_)                                                                                                     \
   if (N == 512 * NG_) {                                                                                                 \
-    hipLaunchKernelGGL((k_embed_rmsnorm<NG_>), dim3((unsigned)n), dim3(64), 0, st, (const bf16_t*)table, vocab, tokens, \
+    hipLaunchKernelGGL((k_embed_rmsnorm<NG_>), dim3((unsigned)n), dim3(64), 0, st, (const bf16_t*)table, tokens, \
                        pos, ctx, (const bf16_t*)w, (bf16_t*)h, (bf16_t*)x, eps, 1);                                     \
     return ix_launch_status();                                                                                          \
   }
@@ -307,7 +310,8 @@ extern "C" int ix_decode_step(const IxDecodeDims* dims, const IxDecodeLayer* lay
     if (rc_ != IX_OK) return rc_ > 0 ? IX_ERR_ARG : rc_; \
   }
   {
-    const IxStepLimits lim{ctx, kv_start, d.cache_len < d.max_positions ? d.cache_len : d.max_positions, d.cache_tokens};
+    const IxStepLimits lim{tokens, d.vocab, ctx, kv_start, d.cache_len < d.max_positions ? d.cache_len : d.max_positions,
+                           d.cache_tokens};
     long l = 0;
     int row_base = 0;
     bool first = true;
@@ -324,7 +328,7 @@ extern "C" int ix_decode_step(const IxDecodeDims* dims, const IxDecodeLayer* lay
     }
     IX_STEP(ix_launch_status());
   }
-  IX_STEP(ix_embed_rmsnorm(embed, d.vocab, tokens, w.pos, ctx, pre_norm, w.h[0], w.x, n, Hd, eps, st));
+  IX_STEP(ix_embed_rmsnorm(embed, tokens, w.pos, ctx, pre_norm, w.h[0], w.x, n, Hd, eps, st));
   auto linear = [&](const bf16_t* a, long K, const void* weight, const void* packed, bf16_t* c, long N) -> int {
     if (packed && n <= 64) {
       const int rc = ix_gemm_bf16_nt_decode(a, K, packed, c, N, n, N, K, stream);

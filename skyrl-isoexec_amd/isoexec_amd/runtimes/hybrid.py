@@ -435,7 +435,7 @@ class RolloutEngine:
         self.kv_rows: dict[int, int] = {}
         self.free_kv_rows = list(range(max_num_seqs, 0, -1))
         self.context: dict[int, int] = {}
-        self._step_error: torch.Tensor | None = None  # pinned host int32 that a native step reports into
+        self._step_error: torch.Tensor | None = None  # pinned host int32 [2] that native steps report into
 
     def _kv_row(self, slot: int) -> int:
         if slot not in self.kv_rows:
@@ -496,16 +496,21 @@ class RolloutEngine:
 
     def _step_error_flag(self) -> torch.Tensor:
         if self._step_error is None:
-            self._step_error = torch.zeros(1, dtype=torch.int32, pin_memory=True)
+            self._step_error = torch.zeros(2, dtype=torch.int32, pin_memory=True)
         return self._step_error
 
     def _raise_step_error(self) -> None:
         """Raise what an earlier native step has reported. Read without waiting for the device, so a fault of the step in
         flight is seen by the call after it (``check_steps`` waits)."""
-        if self._step_error is not None and int(self._step_error[0]):
+        if self._step_error is None:
+            return
+        position, token = self._step_error.tolist()
+        if position or token:
             self._step_error.zero_()
-            raise RuntimeError("[isoexec-amd] decode: a sequence's position in an earlier step lay outside its part of the "
-                               "key/value cache; nothing was stored for it and its output is NaN")
+            what = " and ".join((["a sequence's position outside its part of the key/value cache"] if position else [])
+                                + (["a token id outside the vocabulary"] if token else []))
+            raise RuntimeError(f"[isoexec-amd] decode: an earlier step was given {what}; nothing was stored for that "
+                               "sequence and its output is NaN")
 
     def check_steps(self) -> None:
         """Wait for the steps issued so far and raise if one of them reported a fault."""

@@ -149,11 +149,12 @@ def test_a_pool_table_or_copy_of_another_shape_is_not_handed_to_the_native_step(
 
 @pytest.mark.parametrize("captured", [False, True])
 @pytest.mark.parametrize("field,value", [("ctx", 32), ("ctx", -1), ("ctx", 2**31 - 2), ("kv_start", 4 * 32), ("kv_start", -32),
-                                         ("kv_start", 4 * 32 - 2), ("kv_start", 2**62)])
-def test_a_position_outside_the_cache_stores_nothing_and_is_reported(field, value, captured):
+                                         ("kv_start", 4 * 32 - 2), ("kv_start", 2**62), ("token", 1024), ("token", -1),
+                                         ("token", 2**62)])
+def test_a_position_or_token_out_of_range_stores_nothing_and_is_reported(field, value, captured):
     """The step's own counters can run past what the host's bookkeeping says. Sequence 1 of 3 gets a position (or a first cache
-    token) that does not fit the 4 x 32 tokens of the cache: its output is NaN, no pool changes for it, the others' bits are
-    those of the untouched step, and the next call raises."""
+    token) that does not fit the 4 x 32 tokens of the cache, or a token id that the vocabulary of 1024 does not hold: its
+    output is NaN, no pool changes for it, the others' bits are those of the untouched step, and the next call raises."""
     from isoexec_amd.runtimes.hybrid import HybridWeights, RolloutEngine
 
     cfg = config()
@@ -165,14 +166,12 @@ def test_a_position_outside_the_cache_stores_nothing_and_is_reported(field, valu
         engine.decode([0, 1, 2], tok)
     row = e.kv_rows[1]
     before = {name: t.clone() for name, t in pools(e)}
+    st, given = e._decode_state([0, 1, 2]), tok.clone()
     if captured:
         graph = e.capture_decode([0, 1, 2])
-        graph.state[field][1] = value
-        out = graph.step(tok).clone()
-    else:
-        st = e._decode_state([0, 1, 2])
-        st[field][1] = value
-        out = e._decode_native(st, tok)
+        st = graph.state
+    (given if field == "token" else st[field])[1] = value
+    out = graph.step(given).clone() if captured else e._decode_native(st, given)
     want = ref.decode([0, 1, 2], tok)
     assert out[1].isnan().all() and same_bits(out[[0, 2]], want[[0, 2]])
     for (name, got), (_, other) in zip(pools(e), pools(ref)):
@@ -181,6 +180,6 @@ def test_a_position_outside_the_cache_stores_nothing_and_is_reported(field, valu
         r = e.gdn[0].table.row_of[1] if name.startswith("gdn") else row
         keep = [i for i in range(1, 4) if i != r]  # row 0 is the null row
         assert torch.equal(got[r], before[name][r]) and torch.equal(got[keep], other[keep]), name
-    with pytest.raises(RuntimeError, match="outside its part"):
+    with pytest.raises(RuntimeError, match="outside the vocabulary" if field == "token" else "outside its part"):
         graph.step(tok) if captured else e.decode([0, 1, 2], tok)
     e.check_steps()  # reported once

@@ -84,8 +84,9 @@ NOT_HOOKED: Dict[str, str] = {
 
 # Regions whose doors cover only part of the op.
 PARTIAL: Dict[str, str] = {
-    "gdn.state": "read side only (chunk_boundary_states): the pools are advanced in place by the scan, there is no value "
-                 "to digest at the write. The runtimes' per-layer records (`_Blocks.region_log`) see the state's effect.",
+    "gdn.state": "read side only (chunk_boundary_states, which the boundary form calls while the trace is on; one launch "
+                 "stands for it otherwise): the pools are advanced in place by the scan, there is no value to digest at the "
+                 "write. The runtimes' per-layer records (`_Blocks.region_log`) see the state's effect.",
     "gdn.gating": "subsumed by the fused core when gating runs inside the scan's preparation (decode: ix_gdn_decode_prep).",
     "gdn.l2norm": "subsumed likewise in a decode step.",
     "moe.combine": "the runtimes fold combine + residual add + norm into one launch unless a region log is attached; with "

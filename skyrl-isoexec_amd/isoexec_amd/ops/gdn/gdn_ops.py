@@ -12,6 +12,7 @@ from __future__ import annotations
 import torch
 
 from ... import _lib
+from ...debug.trace import get_tracer
 
 L2NORM_EPS = 1e-6  # gdn_ops.py:173
 
@@ -386,9 +387,11 @@ def _recurrent_scratch_state(q, v, cu_seqlens):
 
 
 def _stateless(q, k, v, g, beta, cu_seqlens, gated_norm=None):
-    o = stateless_forward(q, k, v, g, beta, cu_seqlens=cu_seqlens, gated_norm=gated_norm)
-    if o is not None:
-        return o
+    # not while a trace is attached: the scan behind it is a door of the trace, the single launch is none
+    if get_tracer() is None:
+        o = stateless_forward(q, k, v, g, beta, cu_seqlens=cu_seqlens, gated_norm=gated_norm)
+        if o is not None:
+            return o
     ssm_state, idx = _recurrent_scratch_state(q, v, cu_seqlens)
     return gdn_recurrent_kernel(q, k, v, g, beta, ssm_state=ssm_state, state_indices=idx, cu_seqlens=cu_seqlens,
                                 gated_norm=gated_norm)

@@ -206,3 +206,44 @@ def test_installed_doors_record_what_the_runtime_calls_and_change_nothing(tmp_pa
     finally:
         install.uninstall_debug_hooks()
         trace._forget_for_tests()
+
+
+def test_doors_of_the_delta_rule_without_a_pool(tmp_path, monkeypatch):
+    """The boundary form's states and the scan of a stateless forward are regions while the trace is attached: the single
+    launches that stand for them otherwise have no door. Same bits either way."""
+    from isoexec_amd.debug import install, trace
+    from isoexec_amd.debug.compare import load_dir
+    from isoexec_amd.ops.gdn import gdn_cpr, gdn_ops
+
+    g = torch.Generator().manual_seed(3)
+    lens, H, HV, K = [70, 5, 16], 2, 4, 64
+    T = sum(lens)
+    cu = torch.tensor([0, 70, 75, 91], dtype=torch.int32, device="cuda")
+    draw = lambda *s: torch.randn(*s, generator=g).to(torch.bfloat16).cuda()
+    q, k, v, a, b = draw(1, T, H, K), draw(1, T, H, K), draw(1, T, HV, K), draw(T, HV), draw(T, HV)
+    A_log, dt = torch.randn(HV, generator=g).cuda(), torch.randn(HV, generator=g).cuda()
+
+    def calls():
+        qn, kn = gdn_ops.gdn_l2norm(q), gdn_ops.gdn_l2norm(k)
+        return {"cpr": gdn_cpr.gdn_native_cpr_fwd(q, k, v, a, b, A_log, dt, cu_seqlens=cu, chunk_size=16),
+                "cpr normed": gdn_cpr.gdn_native_cpr_normed(qn, kn, v, a, b, A_log, dt, cu_seqlens=cu, chunk_size=16),
+                "core": gdn_ops.gdn_native_core(q, k, v, a, b, A_log, dt, cu_seqlens=cu),
+                "core normed": gdn_ops.gdn_native_core_normed(qn, kn, v, a, b, A_log, dt, cu_seqlens=cu)}
+
+    trace._forget_for_tests()
+    monkeypatch.delenv(trace.ENV_TRACE, raising=False)
+    plain = calls()
+    trace._forget_for_tests()
+    monkeypatch.setenv(trace.ENV_TRACE, str(tmp_path / "doors"))
+    try:
+        assert install.install_debug_hooks() > 0
+        traced = calls()
+        trace.flush()
+        records = load_dir(str(tmp_path / "doors"))
+        count = lambda region: len([r for r in records if r["region"] == region and r["out"] == "0"])
+        assert count("gdn.state") == 2 and count("gdn.core") == 4
+        for name, want in plain.items():
+            assert torch.equal(traced[name].view(torch.int16), want.view(torch.int16)), name
+    finally:
+        install.uninstall_debug_hooks()
+        trace._forget_for_tests()

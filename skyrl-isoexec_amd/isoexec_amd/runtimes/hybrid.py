@@ -406,6 +406,8 @@ class TrainerModel:
 class RolloutEngine:
     """Prefill, then one token per step per sequence, out of per-layer state."""
 
+    _step_error: torch.Tensor | None = None  # pinned host int32 [2] that native steps report into, made by the first
+
     def __init__(self, cfg: HybridConfig, weights: HybridWeights, max_num_seqs: int, max_len: int,
                  pack_expert_weights: bool = True):
         if max_len > cfg.max_positions:
@@ -435,7 +437,6 @@ class RolloutEngine:
         self.kv_rows: dict[int, int] = {}
         self.free_kv_rows = list(range(max_num_seqs, 0, -1))
         self.context: dict[int, int] = {}
-        self._step_error: torch.Tensor | None = None  # pinned host int32 [2] that native steps report into
 
     def _kv_row(self, slot: int) -> int:
         if slot not in self.kv_rows:

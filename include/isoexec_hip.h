@@ -169,11 +169,15 @@ int ix_gemm_bf16_nt_batched(const void* A, long lda, long stride_a, const void* 
  * ix_gemm_pack_decode: Wf (N * K bf16, 16-byte aligned) <- W [N,K] with row pitch ldw. Serves N a multiple of 32 and
  * K in {1024, 2048, 3072, 4096}; ix_gemm_decode_serves_shape(N, K) says so without touching memory (1 = served).
  * ix_gemm_bf16_nt_decode: C [M,N] bf16 (row pitch ldc, a multiple of 4; C 8-byte aligned) = A [M,K] (row pitch lda, a
- * multiple of 8; A 16-byte aligned) . W^T; no bias, no row maxima, M <= 64: declines (IX_DECLINED) anything else. */
+ * multiple of 8; A 16-byte aligned) . W^T; no bias, no row maxima, M <= 64: declines (IX_DECLINED) anything else.
+ * _footprint: the same with what the caller knows of the bytes that are read between two readings of these weights. From
+ * 256 MiB (the launch's own weights count too) they are loaded past the caches. Never changes a bit. */
 int ix_gemm_decode_serves_shape(long N, long K);
 int ix_gemm_pack_decode(const void* W, long ldw, void* Wf, long N, long K, void* stream);
 int ix_gemm_bf16_nt_decode(const void* A, long lda, const void* Wf, void* C, long ldc, long M, long N, long K,
                            void* stream);
+int ix_gemm_bf16_nt_decode_footprint(const void* A, long lda, const void* Wf, void* C, long ldc, long M, long N, long K,
+                                     size_t footprint, void* stream);
 
 /* Router gating GEMM (moe/_register.py:59-66): C fp32 [M,N] = A[M,K] . W[N,K]^T with W fp32 and
  * A fp32 or bf16 (a_dtype), fp32 accumulate in a fixed K order. */
@@ -432,11 +436,15 @@ int ix_moe_experts_tile(const void* x, long ldx, const int* sorted_token, const 
  *   W2f [E][Hd / 256][wave 4][F / 64][b 2][s 4][lane 64]   row = 256 nt + 64 wave + 32 b + r
  * Serves Hd % 256 == 0, F % 128 == 0 with Hd / 64 and F / 64 in {8, 12, 16, 24, 32, 48, 64}; else declined. Pack once per
  * weight version (one pass over each matrix), not per step. ix_moe_experts_packed takes a block map of BM = 32 or 64,
- * ix_moe_experts_decode one of BM = 32. */
+ * ix_moe_experts_decode one of BM = 32. _footprint: as ix_gemm_bf16_nt_decode_footprint. */
 int ix_moe_pack_decode(const void* W1, const void* W2, void* W1f, void* W2f, long E, long Hd, long F, void* stream);
 int ix_moe_experts_packed(const void* x, long ldx, const int* sorted_token, const float* permuted_prob, const void* W1f,
                           const void* W2f, const int* tile_meta, long max_tiles, long BM, void* inter, void* expert_out,
                           long T, long rows, long Hd, long F, void* stream);
+int ix_moe_experts_packed_footprint(const void* x, long ldx, const int* sorted_token, const float* permuted_prob,
+                                    const void* W1f, const void* W2f, const int* tile_meta, long max_tiles, long BM,
+                                    void* inter, void* expert_out, long T, long rows, long Hd, long F, size_t footprint,
+                                    void* stream);
 int ix_moe_experts_decode(const void* x, long ldx, const int* sorted_token, const float* permuted_prob, const void* W1f,
                           const void* W2f, const int* tile_meta, long max_tiles, void* inter, void* expert_out, long T,
                           long rows, long Hd, long F, void* stream);

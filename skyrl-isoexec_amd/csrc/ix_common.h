@@ -212,7 +212,8 @@ __device__ __forceinline__ void ix_load8(const float* __restrict__ p, long valid
 }
 
 // Sixteen bytes that nobody reads again soon: loaded without claiming a place in the caches. Weights that one launch streams
-// once are read at 6.9-7.1 TB/s this way, at 6.0-6.3 TB/s with the default policy.
+// once are read at 6.9-7.1 TB/s this way, at 6.0-6.3 TB/s with the default policy, out of memory; weights that the 256 MiB
+// memory-side cache still holds from their last use are slower by up to a third (ix_streams_once).
 __device__ __forceinline__ uint4 ix_load16_once(const uint4* p) {
   typedef __attribute__((ext_vector_type(4))) uint32_t v4;
   const v4 v = __builtin_nontemporal_load(reinterpret_cast<const v4*>(p));
@@ -222,6 +223,16 @@ __device__ __forceinline__ uint4 ix_load16_once(const uint4* p) {
 __device__ __forceinline__ void ix_store16_once(uint4* p, uint4 u) {
   typedef __attribute__((ext_vector_type(4))) uint32_t v4;
   __builtin_nontemporal_store(v4{u.x, u.y, u.z, u.w}, reinterpret_cast<v4*>(p));
+}
+
+// Whether a launch that reads its weights once reads them past the caches: when more bytes than the memory-side cache holds
+// are read between two readings of the same weight (`footprint`: what the caller knows of them, 0 for nothing; at least the
+// launch's own). A model whose weights stay in that cache would pay for it. Packed streams, us per launch, default / past the
+// caches, cycling through 193 and 1592 MiB of weights: dense 12352 x 1024 at 64 rows 7.7 / 9.2 and 9.1 / 8.7, 12352 x 2048
+// at 1 row 8.8 / 9.5 and 10.4 / 9.2, at 32 9.5 / 12.1 and 11.9 / 10.8, at 64 12.8 / 14.7 and 15.8 / 14.9; fc1 + fc2 of 8
+// experts of 1024 x 512, 64 tokens, 9.1 / 11.0 and 11.0 / 10.4, of 16, 8 tokens, 11.1 / 11.9 and 12.2 / 11.3.
+static inline bool ix_streams_once(size_t launch, size_t footprint) {
+  return (launch > footprint ? launch : footprint) >= ((size_t)256 << 20);
 }
 
 // Eight bf16 held in a 16-byte register group, widened.

@@ -8,8 +8,8 @@
 //     wave's four matrix instructions take as their A operands, in (step, lane) order, so a load instruction is 1 KiB
 //     of contiguous memory and a wave walks one contiguous stream;
 //   * a lane holds the fragments of the next D = 8 k-tiles in registers (32 loads of 16 bytes in flight per lane; with
-//     eight waves on a CU 256 KiB of weight bytes in flight per CU), loaded past the caches (ix_load16_once: LM head
-//     151936 x 4096 at M = 16 216 -> 189 us = 6.6 TB/s, 151936 x 2048 115 -> 101 us);
+//     eight waves on a CU 256 KiB of weight bytes in flight per CU), loaded past the caches where ix_streams_once says so
+//     (LM head 151936 x 4096 at M = 16 216 -> 189 us = 6.6 TB/s, 151936 x 2048 115 -> 101 us);
 //   * the activations -- the same at most 64 rows for every unit -- are staged once per workgroup: each k-tile of A is
 //     fetched straight into LDS in B-operand fragment order (memory -> LDS, 1 KiB pieces shared out over the waves), as
 //     far ahead as the weights, and every wave reads its B fragments from there. One barrier per k-tile, which couples
@@ -47,8 +47,9 @@ __global__ __launch_bounds__(256) void k_gemm_pack_frag(const bf16_t* __restrict
       *reinterpret_cast<const uint4*>(W + (32 * u + r) * ldw + 64 * kt + 32 * g + 8 * st);
 }
 
-// TB: 32-row blocks of A (1: M <= 32, 2: M <= 64). NW: waves per workgroup, one unit of 32 weight rows each.
-template <int KT, int TB, int NW>
+// TB: 32-row blocks of A (1: M <= 32, 2: M <= 64). NW: waves per workgroup, one unit of 32 weight rows each. ONCE: weights
+// past the caches.
+template <int KT, int TB, int NW, bool ONCE>
 __global__ __launch_bounds__(NW * 64) void k_gemm_dec(const bf16_t* __restrict__ A, long lda, int M,
                                                       const bf16_t* __restrict__ Wf, bf16_t* __restrict__ C, long ldc,
                                                       int units) {
@@ -91,7 +92,10 @@ __global__ __launch_bounds__(NW * 64) void k_gemm_dec(const bf16_t* __restrict__
   auto load_w = [&](auto ktc) {
     constexpr int kt = decltype(ktc)::value;
 #pragma unroll
-    for (int c = 0; c < 4; ++c) wreg[kt % D][c] = ix_load16_once(wp + kt * 256 + c * 64);
+    for (int c = 0; c < 4; ++c) {
+      const uint4* p = wp + kt * 256 + c * 64;
+      wreg[kt % D][c] = ONCE ? ix_load16_once(p) : *p;
+    }
   };
 
   ix_f32x16 acc[TB];
@@ -170,11 +174,11 @@ extern "C" int ix_gemm_pack_decode(const void* W, long ldw, void* Wf, long N, lo
   return ix_launch_status();
 }
 
-template <int KT, int TB, int NW>
+template <int KT, int TB, int NW, bool ONCE>
 static int ix_gemm_dec_launch(const bf16_t* A, long lda, int M, const bf16_t* Wf, bf16_t* C, long ldc, int units,
                               hipStream_t st) {
   constexpr int LDS = (IX_GD_D + 1) * TB * 4 * 1024;
-  auto kern = k_gemm_dec<KT, TB, NW>;
+  auto kern = k_gemm_dec<KT, TB, NW, ONCE>;
   static bool attr_set = false;
   if (!attr_set) {
     if (hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, LDS) != hipSuccess)
@@ -190,6 +194,11 @@ static int ix_gemm_dec_launch(const bf16_t* A, long lda, int M, const bf16_t* Wf
 // the activations for fewer units).
 extern "C" int ix_gemm_bf16_nt_decode(const void* A, long lda, const void* Wf, void* C, long ldc, long M, long N, long K,
                                       void* stream) {
+  return ix_gemm_bf16_nt_decode_footprint(A, lda, Wf, C, ldc, M, N, K, 0, stream);
+}
+
+extern "C" int ix_gemm_bf16_nt_decode_footprint(const void* A, long lda, const void* Wf, void* C, long ldc, long M, long N,
+                                                long K, size_t footprint, void* stream) {
   if (!A || !Wf || !C || M < 0 || N <= 0 || K <= 0 || lda < K || ldc < N) return IX_ERR_ARG;
   if (M > 64 || !ix_gemm_decode_serves(N, K) || (lda % 8) || (ldc % 4) || !ix_aligned(A, 16) || !ix_aligned(Wf, 16) ||
       !ix_aligned(C, 8))
@@ -200,17 +209,19 @@ extern "C" int ix_gemm_bf16_nt_decode(const void* A, long lda, const void* Wf, v
   const bf16_t *a = (const bf16_t*)A, *wf = (const bf16_t*)Wf;
   bf16_t* c = (bf16_t*)C;
   const int units = (int)(N / 32), m = (int)M;
-  const bool wide = units >= 2048;
+  const bool wide = units >= 2048, once = ix_streams_once((size_t)N * K * 2, footprint);
+#define IX_GD_NW(KT_, TB_, ONCE_)                                                                       \
+  return wide ? ix_gemm_dec_launch<KT_, TB_, 4, ONCE_>(a, lda, m, wf, c, ldc, units, st)                \
+              : ix_gemm_dec_launch<KT_, TB_, 2, ONCE_>(a, lda, m, wf, c, ldc, units, st)
 #define IX_GD_GO(KT_)                                                                                   \
   if (K / 64 == KT_) {                                                                                  \
-    if (M > 32) {                                                                                       \
-      if (wide) return ix_gemm_dec_launch<KT_, 2, 4>(a, lda, m, wf, c, ldc, units, st);                 \
-      return ix_gemm_dec_launch<KT_, 2, 2>(a, lda, m, wf, c, ldc, units, st);                           \
-    }                                                                                                   \
-    if (wide) return ix_gemm_dec_launch<KT_, 1, 4>(a, lda, m, wf, c, ldc, units, st);                   \
-    return ix_gemm_dec_launch<KT_, 1, 2>(a, lda, m, wf, c, ldc, units, st);                             \
+    if (M > 32 && once) IX_GD_NW(KT_, 2, true);                                                         \
+    if (M > 32) IX_GD_NW(KT_, 2, false);                                                                \
+    if (once) IX_GD_NW(KT_, 1, true);                                                                   \
+    IX_GD_NW(KT_, 1, false);                                                                            \
   }
   IX_GD_KTS(IX_GD_GO)
 #undef IX_GD_GO
+#undef IX_GD_NW
   return IX_DECLINED;
 }

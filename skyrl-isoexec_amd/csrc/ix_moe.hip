@@ -1459,7 +1459,7 @@ extern "C" int ix_moe_experts(const void* x, long ldx, const int* sorted_token, 
 //     eight matrix instructions of that k-tile take as their A operands, in (block, step, lane) order, so that a load
 //     instruction is 1 KiB of contiguous memory and a wave walks one contiguous stream;
 //   * a lane keeps the fragments of the next D k-tiles in registers (D x 8 loads of 16 bytes in flight per lane, eight
-//     waves per CU: up to 256 KiB of weight bytes in flight per CU), loaded past the caches (ix_load16_once);
+//     waves per CU: up to 256 KiB of weight bytes in flight per CU), loaded past the caches where ix_streams_once says so;
 //   * activations (at most 32 token rows per block, typically four live ones) come straight from memory as B operands,
 //     a lane loading the 16 bytes of its own token, as far ahead as the weights; a dead token's lanes load a live row
 //     and multiply zeros instead;
@@ -1494,8 +1494,9 @@ __global__ __launch_bounds__(256) void k_moe_pack_frag(const bf16_t* __restrict_
   *reinterpret_cast<uint4*>(Wf + i * 8) = v;
 }
 
-// D: k-tiles of fragments a lane holds ahead of the matrix instructions. TB: blocks of 32 token rows.
-template <int D, int TB>
+// D: k-tiles of fragments a lane holds ahead of the matrix instructions. TB: blocks of 32 token rows. ONCE: weights past the
+// caches.
+template <int D, int TB, bool ONCE>
 struct IxDecStream {
   const uint4* wp;       // this lane's first chunk of the wave's stream: k-tile kt, chunk c at wp[kt * 512 + c * 64]
   const bf16_t* xp[TB];  // this lane's token row + 32 g (a dead token's lanes point at a live row and discard what they load)
@@ -1508,7 +1509,10 @@ struct IxDecStream {
 #pragma unroll
       for (int st = 0; st < 4; ++st) xreg[d][t][st] = *reinterpret_cast<const uint4*>(xp[t] + 64 * kt + 8 * st);
 #pragma unroll
-    for (int c = 0; c < 8; ++c) wreg[d][c] = ix_load16_once(wp + (long)kt * 512 + c * 64);
+    for (int c = 0; c < 8; ++c) {
+      const uint4* p = wp + (long)kt * 512 + c * 64;
+      wreg[d][c] = ONCE ? ix_load16_once(p) : *p;
+    }
   }
   __device__ __forceinline__ void multiply(int d, ix_f32x16 (&a0)[TB], ix_f32x16 (&a1)[TB]) {
 #pragma unroll
@@ -1566,13 +1570,13 @@ struct IxDecUnit {
   }
 };
 
-template <int D, int TB, int KT>
+template <int D, int TB, bool ONCE, int KT>
 __device__ __forceinline__ void ix_moe_fc1_dec_unit(const IxDecUnit& un, const bf16_t* __restrict__ x, long ldx,
                                                     const int* __restrict__ sorted_token,
                                                     const float* __restrict__ permuted_prob, const bf16_t* __restrict__ W1f,
                                                     bf16_t* __restrict__ inter, int F) {
   const int lane = threadIdx.x, r = lane & 31, g = lane >> 5;
-  IxDecStream<D, TB> st;
+  IxDecStream<D, TB, ONCE> st;
   st.wp = reinterpret_cast<const uint4*>(W1f) + un.stream * (long)KT * 512 + lane;
 #pragma unroll
   for (int t = 0; t < TB; ++t) {
@@ -1598,11 +1602,11 @@ __device__ __forceinline__ void ix_moe_fc1_dec_unit(const IxDecUnit& un, const b
   }
 }
 
-template <int D, int TB, int KT>
+template <int D, int TB, bool ONCE, int KT>
 __device__ __forceinline__ void ix_moe_fc2_dec_unit(const IxDecUnit& un, const bf16_t* __restrict__ inter,
                                                     const bf16_t* __restrict__ W2f, bf16_t* __restrict__ out, int Hd, int F) {
   const int lane = threadIdx.x, r = lane & 31, g = lane >> 5;
-  IxDecStream<D, TB> st;
+  IxDecStream<D, TB, ONCE> st;
   st.wp = reinterpret_cast<const uint4*>(W2f) + un.stream * (long)KT * 512 + lane;
 #pragma unroll
   for (int t = 0; t < TB; ++t) {
@@ -1626,7 +1630,7 @@ __device__ __forceinline__ void ix_moe_fc2_dec_unit(const IxDecUnit& un, const b
 
 // BM = 32 or 64: the block map's rows per tile. Four k-tiles ahead for one block of tokens (three where a long K's addresses
 // would push registers out to memory), two for two: both leave two waves per SIMD; deeper rings with one wave measured slower.
-template <int KT, int BM>
+template <int KT, int BM, bool ONCE>
 __global__ __launch_bounds__(64, 2) void k_moe_fc1_dec(const bf16_t* __restrict__ x, long ldx,
                                                        const int* __restrict__ sorted_token,
                                                        const float* __restrict__ permuted_prob,
@@ -1635,21 +1639,21 @@ __global__ __launch_bounds__(64, 2) void k_moe_fc1_dec(const bf16_t* __restrict_
   IxDecUnit un;
   if (!un.init(meta, max_tiles, nb_n)) return;
   if (BM == 32 || un.nrows <= 32)
-    ix_moe_fc1_dec_unit<(KT <= 32 ? 4 : 3), 1, KT>(un, x, ldx, sorted_token, permuted_prob, W1f, inter, F);
+    ix_moe_fc1_dec_unit<(KT <= 32 ? 4 : 3), 1, ONCE, KT>(un, x, ldx, sorted_token, permuted_prob, W1f, inter, F);
   else
-    ix_moe_fc1_dec_unit<2, 2, KT>(un, x, ldx, sorted_token, permuted_prob, W1f, inter, F);
+    ix_moe_fc1_dec_unit<2, 2, ONCE, KT>(un, x, ldx, sorted_token, permuted_prob, W1f, inter, F);
 }
 
-template <int KT, int BM>
+template <int KT, int BM, bool ONCE>
 __global__ __launch_bounds__(64, 2) void k_moe_fc2_dec(const bf16_t* __restrict__ inter, const bf16_t* __restrict__ W2f,
                                                        const int* __restrict__ meta, int max_tiles,
                                                        bf16_t* __restrict__ out, int Hd, int F, int nb_n) {
   IxDecUnit un;
   if (!un.init(meta, max_tiles, nb_n)) return;
   if (BM == 32 || un.nrows <= 32)
-    ix_moe_fc2_dec_unit<(KT <= 12 ? 4 : 3), 1, KT>(un, inter, W2f, out, Hd, F);
+    ix_moe_fc2_dec_unit<(KT <= 12 ? 4 : 3), 1, ONCE, KT>(un, inter, W2f, out, Hd, F);
   else
-    ix_moe_fc2_dec_unit<2, 2, KT>(un, inter, W2f, out, Hd, F);
+    ix_moe_fc2_dec_unit<2, 2, ONCE, KT>(un, inter, W2f, out, Hd, F);
 }
 
 // The k-tile counts the straight-line kernels are instantiated for (K = 64 KT).
@@ -1685,6 +1689,14 @@ extern "C" int ix_moe_pack_decode(const void* W1, const void* W2, void* W1f, voi
 extern "C" int ix_moe_experts_packed(const void* x, long ldx, const int* sorted_token, const float* permuted_prob,
                                      const void* W1f, const void* W2f, const int* tile_meta, long max_tiles, long BM,
                                      void* inter, void* expert_out, long T, long rows, long Hd, long F, void* stream) {
+  return ix_moe_experts_packed_footprint(x, ldx, sorted_token, permuted_prob, W1f, W2f, tile_meta, max_tiles, BM, inter,
+                                         expert_out, T, rows, Hd, F, 0, stream);
+}
+
+extern "C" int ix_moe_experts_packed_footprint(const void* x, long ldx, const int* sorted_token, const float* permuted_prob,
+                                               const void* W1f, const void* W2f, const int* tile_meta, long max_tiles, long BM,
+                                               void* inter, void* expert_out, long T, long rows, long Hd, long F,
+                                               size_t footprint, void* stream) {
   if (!x || !sorted_token || !permuted_prob || !W1f || !W2f || !tile_meta || !inter || !expert_out) return IX_ERR_ARG;
   if (T < 0 || rows < 0 || Hd <= 0 || F <= 0 || max_tiles < 0 || ldx < Hd || (BM != 32 && BM != 64)) return IX_ERR_ARG;
   if (!ix_moe_decode_serves(Hd, F) || (ldx % 8) || !ix_aligned(x, 16) || !ix_aligned(W1f, 16) || !ix_aligned(W2f, 16) ||
@@ -1696,29 +1708,30 @@ extern "C" int ix_moe_experts_packed(const void* x, long ldx, const int* sorted_
   const long u1 = tiles * nb1 * 4, u2 = tiles * nb2 * 4;
   if (u1 > 0x7ffffff0L || u2 > 0x7ffffff0L) return IX_DECLINED;
   const dim3 g1((unsigned)(8 * ((u1 + 7) / 8))), g2((unsigned)(8 * ((u2 + 7) / 8)));
+  const bool once = ix_streams_once((size_t)tiles * 3 * F * Hd * 2, footprint);
   hipStream_t st = (hipStream_t)stream;
-#define IX_DEC_FC1_BM(KT_, BM_)                                                                                     \
-  hipLaunchKernelGGL((k_moe_fc1_dec<KT_, BM_>), g1, dim3(64), 0, st, (const bf16_t*)x, ldx, sorted_token, permuted_prob, \
-                     (const bf16_t*)W1f, tile_meta, (int)max_tiles, (bf16_t*)inter, (int)F, (int)nb1)
-#define IX_DEC_FC2_BM(KT_, BM_)                                                                                      \
-  hipLaunchKernelGGL((k_moe_fc2_dec<KT_, BM_>), g2, dim3(64), 0, st, (const bf16_t*)inter, (const bf16_t*)W2f, tile_meta, \
-                     (int)max_tiles, (bf16_t*)expert_out, (int)Hd, (int)F, (int)nb2)
-#define IX_DEC_FC1(KT_)                          \
-  if (Hd / 64 == KT_) {                          \
-    if (BM == 32) IX_DEC_FC1_BM(KT_, 32);        \
-    else IX_DEC_FC1_BM(KT_, 64);                 \
-  }
-#define IX_DEC_FC2(KT_)                          \
-  if (F / 64 == KT_) {                           \
-    if (BM == 32) IX_DEC_FC2_BM(KT_, 32);        \
-    else IX_DEC_FC2_BM(KT_, 64);                 \
-  }
+#define IX_DEC_FC1_GO(KT_, BM_, ONCE_)                                                                              \
+  hipLaunchKernelGGL((k_moe_fc1_dec<KT_, BM_, ONCE_>), g1, dim3(64), 0, st, (const bf16_t*)x, ldx, sorted_token,     \
+                     permuted_prob, (const bf16_t*)W1f, tile_meta, (int)max_tiles, (bf16_t*)inter, (int)F, (int)nb1)
+#define IX_DEC_FC2_GO(KT_, BM_, ONCE_)                                                                               \
+  hipLaunchKernelGGL((k_moe_fc2_dec<KT_, BM_, ONCE_>), g2, dim3(64), 0, st, (const bf16_t*)inter, (const bf16_t*)W2f, \
+                     tile_meta, (int)max_tiles, (bf16_t*)expert_out, (int)Hd, (int)F, (int)nb2)
+#define IX_DEC_CASE(GO, KT_)                     \
+  if (BM == 32 && once) GO(KT_, 32, true);       \
+  else if (BM == 32) GO(KT_, 32, false);         \
+  else if (once) GO(KT_, 64, true);              \
+  else GO(KT_, 64, false);
+#define IX_DEC_FC1(KT_) \
+  if (Hd / 64 == KT_) { IX_DEC_CASE(IX_DEC_FC1_GO, KT_) }
+#define IX_DEC_FC2(KT_) \
+  if (F / 64 == KT_) { IX_DEC_CASE(IX_DEC_FC2_GO, KT_) }
   IX_DEC_KTS(IX_DEC_FC1)
   IX_DEC_KTS(IX_DEC_FC2)
 #undef IX_DEC_FC1
 #undef IX_DEC_FC2
-#undef IX_DEC_FC1_BM
-#undef IX_DEC_FC2_BM
+#undef IX_DEC_CASE
+#undef IX_DEC_FC1_GO
+#undef IX_DEC_FC2_GO
   return ix_launch_status();
 }
 

@@ -283,6 +283,20 @@ bool served(const IxDecodeDims& d) {
   return proj_width(d, false) % 8 == 0 && proj_width(d, true) % 8 == 0;
 }
 
+// Bytes a step moves at least, hence between two readings of one weight: every layer's projections, as many experts as the
+// step can touch, the recurrent states read and written.
+size_t step_bytes(const IxDecodeDims& d, const IxDecodeLayer* layers) {
+  const long touched = d.n * d.topk < d.experts ? d.n * d.topk : d.experts;
+  size_t sum = 0;
+  for (long l = 0; l < d.layers; ++l) {
+    const bool attention = layers[l].kind != 0;
+    const long out = attention ? d.q_heads * d.head_dim : d.gdn_v_heads * d.gdn_head_dim;
+    sum += (size_t)(proj_width(d, attention) + out + touched * 3 * d.expert_inter) * d.hidden * 2;
+    if (!attention) sum += (size_t)d.n * d.gdn_v_heads * d.gdn_head_dim * d.gdn_head_dim * 8;
+  }
+  return sum;
+}
+
 }  // namespace
 
 extern "C" size_t ix_decode_step_workspace_bytes(const IxDecodeDims* dims) {
@@ -329,9 +343,10 @@ extern "C" int ix_decode_step(const IxDecodeDims* dims, const IxDecodeLayer* lay
     IX_STEP(ix_launch_status());
   }
   IX_STEP(ix_embed_rmsnorm(embed, tokens, w.pos, ctx, pre_norm, w.h[0], w.x, n, Hd, eps, st));
+  const size_t footprint = step_bytes(d, layers);
   auto linear = [&](const bf16_t* a, long K, const void* weight, const void* packed, bf16_t* c, long N) -> int {
     if (packed && n <= 64) {
-      const int rc = ix_gemm_bf16_nt_decode(a, K, packed, c, N, n, N, K, stream);
+      const int rc = ix_gemm_bf16_nt_decode_footprint(a, K, packed, c, N, n, N, K, footprint, stream);
       if (rc != IX_DECLINED) return rc;
     }
     return ix_gemm_bf16_nt(a, K, weight, K, nullptr, c, IX_DT_BF16, N, n, N, K, 0, nullptr, 0, stream);
@@ -380,8 +395,8 @@ extern "C" int ix_decode_step(const IxDecodeDims* dims, const IxDecodeLayer* lay
     }
     const bool streamed = d.packed_experts && (w.bm == 32 || w.bm == 64);
     if (streamed) {
-      IX_STEP(ix_moe_experts_packed(w.x, Hd, w.sorted, w.pprob, y.w1_packed, y.w2_packed, w.meta, w.max_tiles, w.bm, w.inter,
-                                    w.eo, n, n * d.topk, Hd, d.expert_inter, stream));
+      IX_STEP(ix_moe_experts_packed_footprint(w.x, Hd, w.sorted, w.pprob, y.w1_packed, y.w2_packed, w.meta, w.max_tiles,
+                                              w.bm, w.inter, w.eo, n, n * d.topk, Hd, d.expert_inter, footprint, stream));
     } else {
       IX_STEP(ix_moe_experts_tile(w.x, Hd, w.sorted, w.pprob, y.w1, y.w2, w.meta, w.max_tiles, w.bm, w.bn, w.inter, w.eo, n,
                                   n * d.topk, Hd, d.expert_inter, stream));

@@ -75,6 +75,7 @@ SIGNATURES = {
     "ix_gemm_decode_serves_shape": (c_int, [c_long, c_long]),
     "ix_gemm_pack_decode": (c_int, [P, c_long, P, c_long, c_long, P]),
     "ix_gemm_bf16_nt_decode": (c_int, [P, c_long, P, P, c_long, c_long, c_long, c_long, P]),
+    "ix_gemm_bf16_nt_decode_footprint": (c_int, [P, c_long, P, P, c_long, c_long, c_long, c_long, c_size_t, P]),
     "ix_gemm_f32_nt": (c_int, [P, c_int, c_long, P, c_long, P, c_long, c_long, c_long, c_long, P]),
     "ix_gdn_scan": (
         c_int,
@@ -133,6 +134,10 @@ SIGNATURES = {
     "ix_moe_experts_packed": (
         c_int,
         [P, c_long, P, P, P, P, P, c_long, c_long, P, P, c_long, c_long, c_long, c_long, P],
+    ),
+    "ix_moe_experts_packed_footprint": (
+        c_int,
+        [P, c_long, P, P, P, P, P, c_long, c_long, P, P, c_long, c_long, c_long, c_long, c_size_t, P],
     ),
     "ix_moe_experts_decode": (
         c_int,

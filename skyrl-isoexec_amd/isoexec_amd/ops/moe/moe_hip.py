@@ -185,11 +185,13 @@ def experts_forward(x: torch.Tensor, w1: torch.Tensor, w2: torch.Tensor, p: Perm
         w1f, w2f = packed
         if w1f.shape != w1.shape or w2f.shape != w2.shape or w1f.dtype is not torch.bfloat16 or w2f.dtype is not torch.bfloat16:
             raise RuntimeError("[isoexec-amd] packed must come from pack_decode(w1, w2)")
+        # other tokens touch other experts: between two uses of one, up to all of this layer's are read
         rc = _lib.check(
-            _lib.lib().ix_moe_experts_packed(xc.data_ptr(), xc.stride(0), p.sorted_token.data_ptr(),
-                                             p.permuted_prob.data_ptr(), w1f.data_ptr(), w2f.data_ptr(),
-                                             p.tile_meta.data_ptr(), p.max_tiles, p.BM, inter.data_ptr(), out.data_ptr(), T,
-                                             rows, H, F, _lib.current_stream(dev)), "ix_moe_experts_packed")
+            _lib.lib().ix_moe_experts_packed_footprint(xc.data_ptr(), xc.stride(0), p.sorted_token.data_ptr(),
+                                                       p.permuted_prob.data_ptr(), w1f.data_ptr(), w2f.data_ptr(),
+                                                       p.tile_meta.data_ptr(), p.max_tiles, p.BM, inter.data_ptr(),
+                                                       out.data_ptr(), T, rows, H, F, w1f.nbytes + w2f.nbytes,
+                                                       _lib.current_stream(dev)), "ix_moe_experts_packed")
         if rc == _lib.IX_OK:
             return (out, inter) if return_inter else out
     w1c, w2c = w1.contiguous(), w2.contiguous()  # named: the copies have to outlive the call

@@ -34,3 +34,51 @@ def test_experts(tokens):
     got = M.experts_forward(x, w1, w2, M.permute(idx, prob, e, BM=256))
     want = M.experts_forward(x, w1, w2, M.permute(idx, prob, e, BM=128))
     assert torch.equal(got, want)
+
+
+MEMORY_SIDE_CACHE = 256 << 20  # the line of the packed streams
+
+
+@pytest.mark.parametrize("m", [1, 32, 33, 64])
+@pytest.mark.parametrize("n", [96, 65568])  # two and four waves per workgroup, a last unit without a neighbour
+def test_packed_dense_on_either_side_of_the_line(m, n):
+    from isoexec_amd import _lib
+    from isoexec_amd.ops.mm.mm_hip import linear_nt, pack_nt_decode
+
+    k = 1024
+    g = torch.Generator(device="cuda")
+    g.manual_seed(n + m)
+    x = torch.randn(m, k, generator=g, device="cuda").to(torch.bfloat16)
+    w = (0.02 * torch.randn(n, k, generator=g, device="cuda")).to(torch.bfloat16)
+    wf = pack_nt_decode(w).packed
+    want = linear_nt(x, w)
+    for footprint in (0, MEMORY_SIDE_CACHE - 1, MEMORY_SIDE_CACHE):
+        got = torch.full_like(want, float("nan"))
+        rc = _lib.lib().ix_gemm_bf16_nt_decode_footprint(x.data_ptr(), k, wf.data_ptr(), got.data_ptr(), n, m, n, k, footprint,
+                                                         _lib.current_stream(x.device))
+        assert rc == _lib.IX_OK and torch.equal(got, want)
+
+
+@pytest.mark.parametrize("bm, tokens", [(32, 1), (32, 33), (64, 33), (64, 130)])
+def test_packed_experts_on_either_side_of_the_line(bm, tokens):
+    from isoexec_amd import _lib
+    from isoexec_amd.ops.moe import moe_hip as M
+
+    e, h, f, k = 4, 512, 512, 2
+    g = torch.Generator(device="cuda")
+    g.manual_seed(tokens)
+    x = torch.randn(tokens, h, generator=g, device="cuda").to(torch.bfloat16)
+    w1 = (0.02 * torch.randn(e, 2 * f, h, generator=g, device="cuda")).to(torch.bfloat16)
+    w2 = (0.02 * torch.randn(e, h, f, generator=g, device="cuda")).to(torch.bfloat16)
+    w1f, w2f = M.pack_decode(w1, w2)
+    idx, prob, _, _ = M.router_topk(torch.randn(tokens, e, generator=g, device="cuda"), k, pre_softmax=True)
+    want = M.experts_forward(x, w1, w2, M.permute(idx, prob, e, BM=256))
+    p = M.permute(idx, prob, e, BM=bm)
+    for footprint in (0, MEMORY_SIDE_CACHE - 1, MEMORY_SIDE_CACHE):
+        inter = torch.full((tokens * k, f), float("nan"), dtype=torch.bfloat16, device="cuda")
+        got = torch.full_like(want, float("nan"))
+        rc = _lib.lib().ix_moe_experts_packed_footprint(
+            x.data_ptr(), h, p.sorted_token.data_ptr(), p.permuted_prob.data_ptr(), w1f.data_ptr(), w2f.data_ptr(),
+            p.tile_meta.data_ptr(), p.max_tiles, bm, inter.data_ptr(), got.data_ptr(), tokens, tokens * k, h, f, footprint,
+            _lib.current_stream(x.device))
+        assert rc == _lib.IX_OK and torch.equal(got, want)

@@ -74,3 +74,17 @@ def cpu_gen(seed: int) -> torch.Generator:
     g = torch.Generator(device="cpu")
     g.manual_seed(seed)
     return g
+
+
+def lane_pairs_serve(n_seq: int, H: int, HV: int, device) -> bool:
+    """Whether a scan of ``n_seq`` sequences (K = V = 128, one state row each) takes the lane-pair layout: the form with the
+    gated norm is served exactly there. Asked with empty sequences, which the kernel leaves at once."""
+    from isoexec_amd import _lib
+
+    z = torch.zeros(max(1, 128 * HV), dtype=torch.bfloat16, device=device)
+    f, i = torch.zeros(HV, device=device), torch.zeros(n_seq + 1, dtype=torch.int32, device=device)
+    rc = _lib.lib().ix_gdn_scan_gated_norm(z.data_ptr(), z.data_ptr(), z.data_ptr(), f.data_ptr(), z.data_ptr(), z.data_ptr(),
+                                           H * 128, H * 128, HV * 128, f.data_ptr(), i.data_ptr(), i.data_ptr(), n_seq, H, HV,
+                                           128, 128, 128 ** -0.5, 0, z.data_ptr(), HV * 128, z.data_ptr(), 1e-6, 1,
+                                           _lib.current_stream(torch.device(device)))
+    return rc == _lib.IX_OK

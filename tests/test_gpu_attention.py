@@ -323,7 +323,8 @@ def test_single_reader_form_equals_the_tiled_form(HQ, HKV, extra):
     lens = [1, tile, max(1, tile - 1)]
     context = [0, 63, 1027]                      # keys in front of the first query
     starts = [5, 200, 700]
-    q, k, v = (t.to(DEV) for t in rand_qkv(sum(lens) + tile + extra, HQ, HKV, HQ + extra)[:1] + rand_qkv(2048, HQ, HKV, 9)[1:])
+    longer = tile + 1 + extra * tile             # more than one tile, more than two
+    q, k, v = (t.to(DEV) for t in rand_qkv(sum(lens) + longer, HQ, HKV, HQ + extra)[:1] + rand_qkv(2048, HQ, HKV, 9)[1:])
     i32 = dict(dtype=torch.int32, device=DEV)
 
     def call(lengths, ctx, first):
@@ -332,5 +333,5 @@ def test_single_reader_form_equals_the_tiled_form(HQ, HKV, extra):
                                 kv_start=torch.tensor(first, dtype=torch.int64, device=DEV))
 
     n = sum(lens)
-    both = call(lens + [tile + extra], context + [30], starts + [0])   # extra = 1: more than one tile
+    both = call(lens + [longer], context + [30], starts + [0])
     assert same_bits(call(lens, context, starts), both[:n])

@@ -4,7 +4,7 @@ import numpy as np
 import pytest
 import torch
 
-from _util import DevicePrims, bf16_to_np, cpu_gen, np_bits, np_to_bf16, same_bits
+from _util import DevicePrims, bf16_to_np, cpu_gen, lane_pairs_serve, np_bits, np_to_bf16, same_bits
 from oracle import gdn as o_gdn
 
 pytestmark = pytest.mark.gpu
@@ -409,14 +409,15 @@ def test_scan_with_the_gated_output_norm_folded_in_equals_the_two_launches():
     """``gdn_recurrent_kernel(..., gated_norm=...)``: the lane-pair scan applies the layer's gated output norm to its own
     outputs. Against the scan followed by ``fused_gated_out_norm``: outputs and final states bit for bit, a packed batch
     with short, long and empty sequences, null lanes (state index 0) included, a gate that is a column slice of a wider
-    buffer; where the lane-pair layout does not run the library declines the form before it touches the state and the
-    wrapper makes the two calls."""
+    buffer. The scan to compare with is the walk (code 17), so neither side is made of the other; where the lane-pair layout
+    does not run the library declines the form before it touches the state and the wrapper makes the two calls."""
     from isoexec_amd.ops.gdn.gdn_ops import gdn_l2norm, gdn_recurrent_kernel
     from isoexec_amd.ops.norms.fused_outnorm import fused_gated_out_norm
 
     H, HV, K, V = 16, 32, 128, 128
     g = cpu_gen(91)
-    lens = [70, 1, 0, 33, 16, 5, 129, 17, 2, 64, 48, 31, 7, 96, 3, 40, 12, 100]        # 18 sequences x 32 heads >= 512 pairs
+    lens = [70, 1, 0, 33, 16, 5, 129, 17, 2, 64, 48, 31, 7, 96, 3, 40, 12, 100] + [(5 * i) % 19 for i in range(46)]
+    assert lane_pairs_serve(len(lens), H, HV, DEV)                                     # 64 sequences x 32 heads
     T, N = sum(lens), len(lens)
     bf = lambda t: t.to(torch.bfloat16).to(DEV)
     q = gdn_l2norm(bf(torch.randn(T, H, K, generator=g)))
@@ -433,7 +434,8 @@ def test_scan_with_the_gated_output_norm_folded_in_equals_the_two_launches():
     pool0 = torch.randn(N + 1, HV, V, K, generator=g).to(DEV) * 0.1
     u = lambda t: t.unsqueeze(0)
     pa, pb = pool0.clone(), pool0.clone()
-    o = gdn_recurrent_kernel(u(q), u(k), u(v), u(gate), u(beta), ssm_state=pa, state_indices=rows, cu_seqlens=cu)[0]
+    o = gdn_recurrent_kernel(u(q), u(k), u(v), u(gate), u(beta), ssm_state=pa, state_indices=rows, cu_seqlens=cu,
+                             time_tile=17 << 8)[0]
     want = fused_gated_out_norm(o, z, w, 1e-6).view(T, HV, V)
     got = gdn_recurrent_kernel(u(q), u(k), u(v), u(gate), u(beta), ssm_state=pb, state_indices=rows, cu_seqlens=cu,
                                gated_norm=(z, w, 1e-6, True))
@@ -450,13 +452,14 @@ def test_scan_with_the_gated_output_norm_folded_in_equals_the_two_launches():
     w2[9] = float("inf")
     z2 = wide2[:, :HV * V].unflatten(1, (HV, V))
     pe, pf = pool0.clone(), pool0.clone()
-    o2 = gdn_recurrent_kernel(u(q), u(k), u(v2), u(gate), u(beta), ssm_state=pe, state_indices=rows, cu_seqlens=cu)[0]
+    o2 = gdn_recurrent_kernel(u(q), u(k), u(v2), u(gate), u(beta), ssm_state=pe, state_indices=rows, cu_seqlens=cu,
+                              time_tile=17 << 8)[0]
     want2 = fused_gated_out_norm(o2, z2, w2, 1e-6).view(T, HV, V)
     got_nf = gdn_recurrent_kernel(u(q), u(k), u(v2), u(gate), u(beta), ssm_state=pf, state_indices=rows, cu_seqlens=cu,
                                   gated_norm=(z2, w2, 1e-6, True))
     assert not torch.isfinite(want2.float()).all()
     assert got_nf is not None and same_bits(got_nf[0], want2) and same_bits(pe, pf)
-    # fewer than 512 (sequence, head) pairs: the 16-lane layout runs; the library declines the fused form untouched ...
+    # few (sequence, head) pairs: the 16-lane layout runs; the library declines the fused form untouched ...
     from isoexec_amd import _lib
 
     pc = pool0.clone()

@@ -8,7 +8,7 @@ import numpy as np
 import pytest
 import torch
 
-from _util import cpu_gen, same_bits
+from _util import cpu_gen, lane_pairs_serve, same_bits
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
@@ -202,7 +202,7 @@ def test_decode_step_replays_from_a_graph_across_boundaries():
 
 
 def test_wide_heads_take_the_lane_pair_scan_in_the_boundary_pass():
-    """K = V = 128 and a pool of more than 128 rows: the state-only boundary scan over the buffer pool then runs in
+    """K = V = 128 and a pool of 521 rows x 4 heads: the state-only boundary scan over the buffer pool then runs in
     the lane-pair layout (every row that is not due a null lane). Same check as above: prefill, decode across
     boundaries, against the one-pass forward."""
     from isoexec_amd.ops.gdn.gdn_cpr import gdn_cpr_fwd
@@ -213,7 +213,9 @@ def test_wide_heads_take_the_lane_pair_scan_in_the_boundary_pass():
     d = 2 * h * k_ + hv * v_
     g = cpu_gen(41)
     bf = lambda t: t.to(torch.bfloat16).to(DEV)
-    layer = CprGDN(capacity=140, chunk_size=c_, num_k_heads=h, head_k_dim=k_, num_v_heads=hv, head_v_dim=v_, device=DEV,
+    capacity = 520
+    assert lane_pairs_serve(capacity + 1, h, hv, DEV)
+    layer = CprGDN(capacity=capacity, chunk_size=c_, num_k_heads=h, head_k_dim=k_, num_v_heads=hv, head_v_dim=v_, device=DEV,
                    conv_weight=bf(torch.randn(d, w_, generator=g) * 0.4), conv_bias=bf(torch.randn(d, generator=g) * 0.1),
                    A_log=(torch.randn(hv, generator=g) * 0.3).to(DEV), dt_bias=(torch.randn(hv, generator=g) * 0.3).to(DEV))
     total, lens, slots = 40, [13, 16, 30], [5, 6, 7]

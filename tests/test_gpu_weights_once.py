@@ -18,12 +18,13 @@ def test_dense(n, k, m, tile):
     want, want_top = linear_nt(x, w, tile=6, want_row_max=True)
     assert torch.equal(got, want) and torch.equal(top, want_top)
 
+@pytest.mark.parametrize("f", [704, 768])  # 11 k-tiles of the second product, the fewest its streaming form takes; and both streamed
 @pytest.mark.parametrize("tokens", [223, 224, 225, 449])  # mean rows per expert on either side of 224, a last row tile
-def test_experts(tokens):
+def test_experts(tokens, f):
     from isoexec_amd.ops.moe import moe_hip as M
 
-    # few experts; 704 output columns are 11 k-tiles of the second product, the fewest its streaming form takes
-    e, h, f, k = 64, 1024, 768, 1
+    # few experts; five column tiles of the second product give its streaming form the 512 tiles it starts at
+    e, h, k = 64, 1280, 1
     g = torch.Generator(device="cuda")
     g.manual_seed(tokens)
     rows = tokens * e

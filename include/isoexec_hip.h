@@ -476,7 +476,6 @@ typedef struct IxDecodeDims {
   int64_t experts, topk, expert_inter;            /* softmax, top-k, renormalise */
   int64_t packed_experts;                         /* 1: every layer has w1_packed / w2_packed */
   int64_t combine_fp32;                           /* sum of a token's expert rows in fp32 (else bf16) */
-  int64_t cache_tokens, cache_len;                /* tokens of k_cache / v_cache, and of one sequence's part of them */
 } IxDecodeDims;
 
 /* Device pointers of one layer; every tensor contiguous and 16-byte aligned, bf16 unless noted. Fields of the other kind of
@@ -498,15 +497,26 @@ typedef struct IxDecodeLayer {
 
 size_t ix_decode_step_workspace_bytes(const IxDecodeDims* dims); /* 0: not served */
 
-/* dims and layers in HOST memory, read during the call. tokens, slots int64 [n]; ctx int32 [n]: each sequence's position of
- * this token, advanced by one on the device; kv_start int64 [n]. out bf16 [n, hidden]: the normed hidden states. A sequence
- * whose position lies outside its part of the cache, the cache or the rotary tables, or whose token lies outside [0, vocab),
- * stores nothing, gets a row of NaNs and sets error[0] (the position) or error[1] (the token) to 1 (error: int32 [2] in host
- * memory that the device can write, or NULL). */
+/* What a step's positions are checked against, and where a step that does not fit is reported. */
+typedef struct IxDecodeCache {
+  int64_t tokens, len; /* tokens of k_cache / v_cache, and of one sequence's part of them */
+  int* error;          /* int32 [2] in host memory that the device can write, or NULL */
+} IxDecodeCache;
+
+/* dims, cache and layers in HOST memory, read during the call. tokens, slots int64 [n]; ctx int32 [n]: each sequence's
+ * position of this token, advanced by one on the device; kv_start int64 [n]. out bf16 [n, hidden]: the normed hidden states. A
+ * sequence whose position lies outside its part of the cache, the cache or the rotary tables, or whose token lies outside
+ * [0, vocab), stores nothing, gets a row of NaNs and sets error[0] (the position) or error[1] (the token) to 1. */
+int ix_decode_step_checked(const IxDecodeDims* dims, const IxDecodeCache* cache, const IxDecodeLayer* layers,
+                           const void* embed, const void* pre_norm, const void* cos_table, const void* sin_table,
+                           const int64_t* tokens, const int64_t* slots, int* ctx, const int64_t* kv_start, float eps,
+                           void* workspace, size_t workspace_bytes, void* out, void* stream);
+
+/* The same for a caller that keeps every position inside its part of the cache itself: without the cache's extent only the
+ * rotary tables, negative positions and the vocabulary are checked, and nothing is reported. */
 int ix_decode_step(const IxDecodeDims* dims, const IxDecodeLayer* layers, const void* embed, const void* pre_norm,
                    const void* cos_table, const void* sin_table, const int64_t* tokens, const int64_t* slots, int* ctx,
-                   const int64_t* kv_start, float eps, void* workspace, size_t workspace_bytes, void* out,
-                   int* error, void* stream);
+                   const int64_t* kv_start, float eps, void* workspace, size_t workspace_bytes, void* out, void* stream);
 
 /* ---- order-invariant digests: debug/thash ------------------------------------------------- */
 

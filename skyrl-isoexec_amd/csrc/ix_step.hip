@@ -269,7 +269,6 @@ Work carve(const IxDecodeDims& d, void* base) {
 
 bool served(const IxDecodeDims& d) {
   if (d.n <= 0 || d.n > 65535 || d.layers <= 0 || d.vocab <= 0 || d.max_positions <= 0 || d.max_positions > 0x7fffffffL) return false;
-  if (d.cache_len <= 0 || d.cache_tokens <= 0) return false;
   if (!ix_embed_rmsnorm_serves(d.hidden)) return false;
   // ix_moe_combine_add_rmsnorm's widths
   const long ng = d.hidden / 512;
@@ -303,15 +302,15 @@ extern "C" size_t ix_decode_step_workspace_bytes(const IxDecodeDims* dims) {
   return dims && served(*dims) ? carve(*dims, nullptr).bytes : 0;
 }
 
-extern "C" int ix_decode_step(const IxDecodeDims* dims, const IxDecodeLayer* layers, const void* embed, const void* pre_norm,
-                              const void* cos_table, const void* sin_table, const int64_t* tokens, const int64_t* slots,
-                              int* ctx, const int64_t* kv_start, float eps, void* workspace, size_t workspace_bytes,
-                              void* out, int* error, void* stream) {
-  if (!dims || !layers || !embed || !pre_norm || !cos_table || !sin_table || !tokens || !slots || !ctx || !kv_start ||
-      !workspace || !out)
+extern "C" int ix_decode_step_checked(const IxDecodeDims* dims, const IxDecodeCache* cache, const IxDecodeLayer* layers,
+                                      const void* embed, const void* pre_norm, const void* cos_table, const void* sin_table,
+                                      const int64_t* tokens, const int64_t* slots, int* ctx, const int64_t* kv_start,
+                                      float eps, void* workspace, size_t workspace_bytes, void* out, void* stream) {
+  if (!dims || !cache || !layers || !embed || !pre_norm || !cos_table || !sin_table || !tokens || !slots || !ctx ||
+      !kv_start || !workspace || !out)
     return IX_ERR_ARG;
   const IxDecodeDims& d = *dims;
-  if (!served(d)) return IX_DECLINED;
+  if (!served(d) || cache->tokens <= 0 || cache->len <= 0) return IX_DECLINED;
   const Work w = carve(d, workspace);
   if (workspace_bytes < w.bytes || !ix_aligned(workspace, 256) || !ix_aligned(out, 16)) return IX_ERR_ARG;
   hipStream_t st = (hipStream_t)stream;
@@ -324,8 +323,8 @@ extern "C" int ix_decode_step(const IxDecodeDims* dims, const IxDecodeLayer* lay
     if (rc_ != IX_OK) return rc_ > 0 ? IX_ERR_ARG : rc_; \
   }
   {
-    const IxStepLimits lim{tokens, d.vocab, ctx, kv_start, d.cache_len < d.max_positions ? d.cache_len : d.max_positions,
-                           d.cache_tokens};
+    const IxStepLimits lim{tokens, d.vocab, ctx, kv_start, cache->len < d.max_positions ? cache->len : d.max_positions,
+                           cache->tokens};
     long l = 0;
     int row_base = 0;
     bool first = true;
@@ -336,7 +335,7 @@ extern "C" int ix_decode_step(const IxDecodeDims* dims, const IxDecodeLayer* lay
         if (layers[l].kind == 0)
           maps.m[cnt++] = IxStepMap{layers[l].slot2row, layers[l].map_n, layers[l].last_used, layers[l].clock};
       hipLaunchKernelGGL(k_step_begin, dim3((unsigned)(cnt + 1)), dim3(256), 0, st, maps, cnt, slots, (int)n, lim,
-                         w.rows + (long)row_base * n, first ? w.pos : nullptr, w.cu, error);
+                         w.rows + (long)row_base * n, first ? w.pos : nullptr, w.cu, cache->error);
       row_base += cnt;
       first = false;
     }
@@ -407,4 +406,13 @@ extern "C" int ix_decode_step(const IxDecodeDims* dims, const IxDecodeLayer* lay
   }
 #undef IX_STEP
   return IX_OK;
+}
+
+extern "C" int ix_decode_step(const IxDecodeDims* dims, const IxDecodeLayer* layers, const void* embed, const void* pre_norm,
+                              const void* cos_table, const void* sin_table, const int64_t* tokens, const int64_t* slots,
+                              int* ctx, const int64_t* kv_start, float eps, void* workspace, size_t workspace_bytes,
+                              void* out, void* stream) {
+  const IxDecodeCache unknown{INT64_MAX, INT64_MAX, nullptr};
+  return ix_decode_step_checked(dims, &unknown, layers, embed, pre_norm, cos_table, sin_table, tokens, slots, ctx, kv_start,
+                                eps, workspace, workspace_bytes, out, stream);
 }

@@ -146,7 +146,8 @@ SIGNATURES = {
     "ix_moe_combine": (c_int, [P, P, P, c_long, c_long, c_long, c_int, P]),
     "ix_moe_combine_weighted": (c_int, [P, c_int, P, c_int, P, P, c_int, c_long, c_long, c_long, P]),
     "ix_decode_step_workspace_bytes": (c_size_t, [P]),
-    "ix_decode_step": (c_int, [P, P, P, P, P, P, P, P, P, P, c_float, P, c_size_t, P, P, P]),
+    "ix_decode_step": (c_int, [P, P, P, P, P, P, P, P, P, P, c_float, P, c_size_t, P, P]),
+    "ix_decode_step_checked": (c_int, [P, P, P, P, P, P, P, P, P, P, P, c_float, P, c_size_t, P, P]),
     "ix_digest_sums": (c_int, [P, c_int, c_long, c_uint64, P, c_int, P, c_size_t, P, P]),
     "ix_digest_segment_sums": (c_int, [P, c_int, c_long, c_long, c_long, c_uint64, c_uint64, P, c_size_t, P, P]),
     "ix_digest_workspace_words": (c_size_t, [c_long, c_long, c_int]),

@@ -536,7 +536,7 @@ class RolloutEngine:
         }
 
     def _native_step_tables(self, n: int):
-        """``(dims, layers)`` for ``ix_decode_step``: the layers' device pointers as they are now (tables are built anew for
+        """``(dims, layers)`` for ``ix_decode_step_checked``: the layers' device pointers as they are now (tables are built anew for
         every step, so a replaced weight or a moved pool is seen), or ``None`` when the step has to be taken op by op: a
         log or a trace wants the ops' outputs, the fused row lookup is switched off, or something is not the plain
         contiguous tensor the call expects."""
@@ -602,12 +602,11 @@ class RolloutEngine:
         if not ok:
             return None
         dims = array("q", [n, c.layers, H, c.vocab, b.cos.shape[0], c.gdn_k_heads, c.gdn_v_heads, c.gdn_head_dim, c.q_heads,
-                           c.kv_heads, c.head_dim, E, c.topk, F, int(packed_all), int(c.moe_combine_dtype == "fp32"),
-                           (self.max_num_seqs + 1) * self.max_len, self.max_len])
+                           c.kv_heads, c.head_dim, E, c.topk, F, int(packed_all), int(c.moe_combine_dtype == "fp32")])
         return dims, array("q", table)
 
     def _decode_native(self, st: dict, tokens: torch.Tensor):
-        """The step by ``ix_decode_step``: every launch of every layer from one call. Same bits as the ops one by one.
+        """The step by ``ix_decode_step_checked``: every launch of every layer from one call. Same bits as the ops one by one.
         ``None`` when it has to be taken op by op (nothing launched)."""
         b = self.blocks
         n = tokens.shape[0]
@@ -624,15 +623,15 @@ class RolloutEngine:
             return None
         dev = w.embed.device
         _lib.require_device(tokens, w.embed)
-        error = self._step_error_flag()
+        cache = array("q", [(self.max_num_seqs + 1) * self.max_len, self.max_len, self._step_error_flag().data_ptr()])
         work = torch.empty(need, dtype=torch.uint8, device=dev)
         out = torch.empty(n, self.cfg.hidden, dtype=torch.bfloat16, device=dev)
         rc = _lib.check(
-            L.ix_decode_step(dims.buffer_info()[0], layers.buffer_info()[0], w.embed.data_ptr(),
-                             w.layers[0]["pre_norm"].data_ptr(), b.cos.data_ptr(), b.sin.data_ptr(), tokens.data_ptr(),
-                             st["slots_t"].data_ptr(), st["ctx"].data_ptr(), st["kv_start"].data_ptr(), float(self.cfg.eps),
-                             work.data_ptr(), need, out.data_ptr(), error.data_ptr(),
-                             _lib.current_stream(dev)), "ix_decode_step")
+            L.ix_decode_step_checked(dims.buffer_info()[0], cache.buffer_info()[0], layers.buffer_info()[0],
+                                     w.embed.data_ptr(), w.layers[0]["pre_norm"].data_ptr(), b.cos.data_ptr(),
+                                     b.sin.data_ptr(), tokens.data_ptr(), st["slots_t"].data_ptr(), st["ctx"].data_ptr(),
+                                     st["kv_start"].data_ptr(), float(self.cfg.eps), work.data_ptr(), need,
+                                     out.data_ptr(), _lib.current_stream(dev)), "ix_decode_step_checked")
         return out if rc == _lib.IX_OK else None
 
     def _decode_device(self, st: dict, tokens: torch.Tensor) -> torch.Tensor:

@@ -37,6 +37,15 @@ def test_host_only_entry_points():
     assert h.ix_logprob_workspace_bytes(4, 151937, 8) == 0
 
 
+def test_a_decode_step_is_described_by_sixteen_numbers():
+    """``IxDecodeDims`` as callers of this ABI version lay it out; what lies behind it in memory is not read."""
+    dims = (ctypes.c_int64 * 18)(4, 2, 512, 1024, 256, 2, 4, 128, 4, 2, 128, 16, 4, 256, 0, 1)
+    need = _lib.lib().ix_decode_step_workspace_bytes(ctypes.addressof(dims))
+    assert need > 0
+    dims[16] = dims[17] = -1
+    assert _lib.lib().ix_decode_step_workspace_bytes(ctypes.addressof(dims)) == need
+
+
 def test_gemm_tile_choice_is_a_host_decision_with_sane_answers():
     """ix_gemm_bf16_n_tiles reports the row-max parts of the tile shape that would run: forced shapes give
     ceil(N / width), twice that for the four-wave 256 x 256 tile in any of its forms (one part per wave column); the

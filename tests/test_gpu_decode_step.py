@@ -66,6 +66,32 @@ def test_native_step_equals_the_step_op_by_op(n, kw, packed):
         assert graph.state["ctx"].tolist() == [one.context[s] for s in slots]
 
 
+def test_the_step_without_the_cache_extent_gives_the_same_bits():
+    """``ix_decode_step``, for callers that keep positions in range themselves, against the checked form."""
+    from isoexec_amd import _lib
+    from isoexec_amd.runtimes.hybrid import HybridWeights, RolloutEngine
+
+    cfg = config()
+    w = HybridWeights.make(cfg, seed=7, device=DEV)
+    one, plain = (RolloutEngine(cfg, w, max_num_seqs=2, max_len=32) for _ in range(2))
+    tok = torch.tensor([5, 6], device=DEV)
+    for e in (one, plain):
+        e.prefill([0, 1], torch.tensor([1, 2, 3], device=DEV), [2, 1])
+    want = one.decode([0, 1], tok)
+    dims, layers = plain._native_step_tables(2)
+    st, b = plain._decode_state([0, 1]), plain.blocks
+    need = _lib.lib().ix_decode_step_workspace_bytes(dims.buffer_info()[0])
+    work = torch.empty(need, dtype=torch.uint8, device=DEV)
+    out = torch.empty(2, cfg.hidden, dtype=torch.bfloat16, device=DEV)
+    rc = _lib.lib().ix_decode_step(
+        dims.buffer_info()[0], layers.buffer_info()[0], w.embed.data_ptr(), w.layers[0]["pre_norm"].data_ptr(),
+        b.cos.data_ptr(), b.sin.data_ptr(), tok.data_ptr(), st["slots_t"].data_ptr(), st["ctx"].data_ptr(),
+        st["kv_start"].data_ptr(), float(cfg.eps), work.data_ptr(), need, out.data_ptr(), _lib.current_stream(out.device))
+    assert rc == _lib.IX_OK and same_bits(out, want) and st["ctx"].tolist() == [3, 2]
+    for (name, a), (_, c) in zip(pools(plain), pools(one)):
+        assert torch.equal(a.reshape(-1).view(torch.uint8), c.reshape(-1).view(torch.uint8)), name
+
+
 def test_native_step_is_taken_and_sees_replaced_weights():
     from isoexec_amd.runtimes.hybrid import HybridWeights, RolloutEngine
 

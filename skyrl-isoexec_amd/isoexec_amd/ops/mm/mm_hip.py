@@ -32,12 +32,13 @@ DECODE_ROWS = 64  # the streaming form serves products of at most this many rows
 
 class PackedWeight:
     """A weight ``[N, K]`` and its fragment-packed copy for products of at most ``DECODE_ROWS`` rows. The copy is made
-    by ``pack_nt_decode`` and is as large as the weight; it has to be made again when the weight changes."""
+    by ``pack_nt_decode`` and is as large as the weight; it has to be made again when the weight changes. ``footprint``: the
+    bytes the owner knows to be read between two products with this weight (0: nothing known; a cache choice, not a bit)."""
 
-    __slots__ = ("weight", "packed")
+    __slots__ = ("weight", "packed", "footprint")
 
-    def __init__(self, weight: torch.Tensor, packed: torch.Tensor):
-        self.weight, self.packed = weight, packed
+    def __init__(self, weight: torch.Tensor, packed: torch.Tensor, footprint: int = 0):
+        self.weight, self.packed, self.footprint = weight, packed, footprint
 
     @property
     def shape(self):
@@ -70,9 +71,10 @@ def linear_nt_decode(x: torch.Tensor, packed: PackedWeight):
         return None
     n = packed.weight.shape[0]
     out = torch.empty(m, n, dtype=torch.bfloat16, device=x.device)
-    rc = _lib.check(_lib.lib().ix_gemm_bf16_nt_decode(x.data_ptr(), x.stride(0), packed.packed.data_ptr(), out.data_ptr(),
-                                                      out.stride(0), m, n, k, _lib.current_stream(x.device)),
-                    "ix_gemm_bf16_nt_decode")
+    rc = _lib.check(
+        _lib.lib().ix_gemm_bf16_nt_decode_footprint(x.data_ptr(), x.stride(0), packed.packed.data_ptr(), out.data_ptr(),
+                                                    out.stride(0), m, n, k, packed.footprint,
+                                                    _lib.current_stream(x.device)), "ix_gemm_bf16_nt_decode")
     return out if rc == _lib.IX_OK else None
 
 

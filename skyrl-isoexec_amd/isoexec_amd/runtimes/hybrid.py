@@ -207,7 +207,9 @@ class _Blocks:
             packed = pack_nt_decode(weight)
             if packed is not None:
                 self.packed_dense[key] = packed
-                total += packed.packed.numel() * packed.packed.element_size()
+                total += packed.packed.nbytes
+        for packed in self.packed_dense.values():
+            packed.footprint = total  # a step that goes op by op reads each of them once
         return total
 
     def _dense(self, key, weight):

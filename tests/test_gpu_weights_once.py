@@ -60,6 +60,33 @@ def test_packed_dense_on_either_side_of_the_line(m, n):
         assert rc == _lib.IX_OK and torch.equal(got, want)
 
 
+def test_a_step_op_by_op_says_what_its_dense_products_read(monkeypatch):
+    """The products of a layer are below the line one by one; what decides is the model's packed weights together."""
+    from isoexec_amd.runtimes.hybrid import HybridConfig, HybridWeights, RolloutEngine
+
+    cfg = HybridConfig(hidden=1024, vocab=16384, layers=2, attention_every=2, gdn_k_heads=32, gdn_v_heads=32, q_heads=4,
+                       kv_heads=2, experts=8, topk=2, expert_inter=128, max_positions=64, gdn_kernel="cpr")
+    e = RolloutEngine(cfg, HybridWeights.make(cfg, seed=1, device="cuda:0"), max_num_seqs=1, max_len=32)
+    packed = e.blocks.packed_dense
+    total = sum(p.packed.numel() * 2 for p in packed.values())
+    assert len(packed) == 2 and all(p.footprint == total > p.packed.numel() * 2 for p in packed.values())
+    from isoexec_amd import _lib
+
+    real, told = _lib.lib(), []
+
+    class Told:
+        def __getattr__(self, name):
+            entry = getattr(real, name)
+            if name != "ix_gemm_bf16_nt_decode_footprint":
+                return entry
+            return lambda *args: told.append(args[8]) or entry(*args)
+
+    e.prefill([0], torch.tensor([1, 2], device="cuda:0"), [2])
+    monkeypatch.setattr(_lib, "lib", Told)
+    e.blocks.logits(e.decode([0], torch.tensor([3], device="cuda:0")))
+    assert told == [total, total]
+
+
 @pytest.mark.parametrize("bm, tokens", [(32, 1), (32, 33), (64, 33), (64, 130)])
 def test_packed_experts_on_either_side_of_the_line(bm, tokens):
     from isoexec_amd import _lib

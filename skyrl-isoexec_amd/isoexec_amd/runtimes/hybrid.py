@@ -408,7 +408,7 @@ class TrainerModel:
 class RolloutEngine:
     """Prefill, then one token per step per sequence, out of per-layer state."""
 
-    _step_error: torch.Tensor | None = None  # pinned host int32 [2] that native steps report into, made by the first
+    _step_error: torch.Tensor | None = None  # pinned host int32 [2] that native steps report into
 
     def __init__(self, cfg: HybridConfig, weights: HybridWeights, max_num_seqs: int, max_len: int,
                  pack_expert_weights: bool = True):
@@ -434,6 +434,8 @@ class RolloutEngine:
                           head_k_dim=cfg.gdn_head_dim, num_v_heads=cfg.gdn_v_heads, head_v_dim=cfg.gdn_head_dim,
                           device=dev, driver_managed=True)
                 self.gdn[i] = CprGDN(chunk_size=cfg.gdn_chunk, **kw) if cfg.gdn_kernel == "cpr" else RecurrentGDN(**kw)
+        if dev.type == "cuda":
+            self._step_error_flag()  # a pinned allocation: here, not in a step
         # One row table names a request's place in the key/value caches; the GatedDeltaNet layers keep
         # their own (identical) tables so each can be released or evicted with its pool.
         self.kv_rows: dict[int, int] = {}

@@ -451,26 +451,8 @@ void k_gdn_scan_pairs(const TIO* __restrict__ q, const TIO* __restrict__ k, cons
 // vector issue alone would be 75), five of 33..1203 tokens 883 / 247, 8 x 1000 1330 / 667; boundary form of nine sequences
 // of 120..1500 tokens, boundary pass + segmented scan / walk: 3900 / 975. With first and second halves of the 8-element
 // slices apart in LDS a 16-byte read of sixteen lanes is one contiguous row (8 x 1000: 714 -> 667).
-template <typename TIO>
-struct IxRaw8 {
-  uint4 u;
-  __device__ __forceinline__ void load(const TIO* p) { u = *reinterpret_cast<const uint4*>(p); }
-  __device__ __forceinline__ void get(float (&o)[8]) const { ix_unpack8(u, o); }
-};
-template <>
-struct IxRaw8<float> {
-  float4 a, b;
-  __device__ __forceinline__ void load(const float* p) {
-    a = *reinterpret_cast<const float4*>(p);
-    b = *reinterpret_cast<const float4*>(p + 4);
-  }
-  __device__ __forceinline__ void get(float (&o)[8]) const {
-    o[0] = a.x; o[1] = a.y; o[2] = a.z; o[3] = a.w; o[4] = b.x; o[5] = b.y; o[6] = b.z; o[7] = b.w;
-  }
-};
 __device__ __forceinline__ float ix_wire(float x, const bf16_t*) { return ix_rbf(x); }
 __device__ __forceinline__ float ix_wire(float x, const float*) { return x; }
-
 
 template <int KS, int RPL, typename TIO, bool CPR>
 __global__ __launch_bounds__(256) void k_gdn_walk(const TIO* __restrict__ q, const TIO* __restrict__ k,
@@ -577,7 +559,7 @@ __global__ __launch_bounds__(256) void k_gdn_walk(const TIO* __restrict__ q, con
       if (QK % 256 == 0 || i < QK) {
         const int e = i % (T * KS), isq = i / (T * KS);
         float x[8];
-        rq[c].get(x);
+        rq[c].widen(x);
         const float m = isq ? scale : 1.0f;  // k * 1 is k
         float* d = &kq[b][isq][e / KS][(e % KS) * 4];  // first halves of all slices, then second halves
         *reinterpret_cast<float4*>(d) = make_float4(x[0] * m, x[1] * m, x[2] * m, x[3] * m);

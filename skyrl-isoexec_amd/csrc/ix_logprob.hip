@@ -26,28 +26,6 @@
 #define IX_LP_SPLIT_BELOW 192
 #define IX_LP_SEG 8192  // columns per partial-max / full-row-write workgroup in the split shape
 
-// Eight consecutive elements as they lie in memory (a 16-byte-aligned group of bf16, a 32-byte-aligned group of
-// fp32): loading and widening are separate steps so that several loads can be in flight before the first is used.
-template <typename T>
-struct IxRaw8;
-template <>
-struct IxRaw8<bf16_t> {
-  uint4 v;
-  __device__ __forceinline__ void load(const bf16_t* __restrict__ p) { v = *reinterpret_cast<const uint4*>(p); }
-  __device__ __forceinline__ void widen(float (&o)[8]) const { ix_unpack8(v, o); }
-};
-template <>
-struct IxRaw8<float> {
-  float4 a, b;
-  __device__ __forceinline__ void load(const float* __restrict__ p) {
-    a = *reinterpret_cast<const float4*>(p);
-    b = *reinterpret_cast<const float4*>(p + 4);
-  }
-  __device__ __forceinline__ void widen(float (&o)[8]) const {
-    o[0] = a.x; o[1] = a.y; o[2] = a.z; o[3] = a.w; o[4] = b.x; o[5] = b.y; o[6] = b.z; o[7] = b.w;
-  }
-};
-
 // One wave sums one block. `blk` points at the block's first column, n_valid <= 4096 columns
 // exist. Returns the block sum in every lane.
 // `row_max()` yields the row maximum; it is called after the block's loads are issued, so a maximum that is itself

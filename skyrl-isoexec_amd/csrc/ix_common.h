@@ -280,6 +280,56 @@ __device__ __forceinline__ void ix_store8_bf16(bf16_t* __restrict__ p, long vali
   }
 }
 
+// The norm's chain, in the one place that every kernel rounding with ix_rbf takes it from: bits of the row kernels and of
+// the decode step's embedding launch agree by construction. Eight columns of a row into the slot sums (multiply rounded,
+// then add rounded); the slot sums of a row of N columns to its reciprocal root; the row times it, then the weight.
+__device__ __forceinline__ void ix_sumsq8(const float (&x)[8], float (&acc)[8]) {
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    const float sq = x[i] * x[i];
+    acc[i] = acc[i] + sq;
+  }
+}
+template <int LPR>
+__device__ __forceinline__ float ix_norm_rstd(const float (&acc)[8], int N, float eps) {
+  const float s = ix_lane_tree<LPR>(ix_tree8(acc));
+  const float ms = s / (float)N;
+  return ix_rsqrt_ieee(ms + eps);
+}
+__device__ __forceinline__ void ix_norm8(const float (&x)[8], float rstd, const float (&w)[8], int zero_centered,
+                                         float (&o)[8]) {
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    const float nb = ix_rbf(x[i] * rstd);
+    const float gam = zero_centered ? ix_rbf(1.0f + w[i]) : w[i];
+    o[i] = ix_rbf(nb * gam);
+  }
+}
+
+// Rotary embedding of eight pairs (a4[i], b4[i]) by the two halves of the cosine and sine rows: lo = a cos0 - b sin0,
+// hi = b cos1 + a sin1. The products are rounded by the hardware pack-convert, two at a time (ix_rbf2_hw: ix_rbf on
+// everything but a NaN, whose payload it keeps); a NaN stays a NaN through the add whatever its payload, and the sums are
+// stored with their NaNs made canonical (ix_pack_bf2_canon_hw), so the stored bits are those of the chain in ix_rbf.
+__device__ __forceinline__ void ix_rope_pairs8(const uint4 a4, const uint4 b4, const uint4 c0, const uint4 c1, const uint4 s0,
+                                               const uint4 s1, uint4& lo4, uint4& hi4) {
+  const uint32_t* aw = &a4.x; const uint32_t* bw = &b4.x;
+  const uint32_t* c0w = &c0.x; const uint32_t* c1w = &c1.x; const uint32_t* s0w = &s0.x; const uint32_t* s1w = &s1.x;
+  uint32_t* low = &lo4.x; uint32_t* hiw = &hi4.x;
+  auto lo16 = [](uint32_t u) { return __uint_as_float(u << 16); };
+  auto hi16 = [](uint32_t u) { return __uint_as_float(u & 0xffff0000u); };
+#pragma unroll
+  for (int w = 0; w < 4; ++w) {
+    const float a0 = lo16(aw[w]), a1 = hi16(aw[w]), b0 = lo16(bw[w]), b1 = hi16(bw[w]);
+    float t0, t1, u0, u1;
+    ix_rbf2_hw(a0 * lo16(c0w[w]), a1 * hi16(c0w[w]), t0, t1);
+    ix_rbf2_hw((b0 * -1.0f) * lo16(s0w[w]), (b1 * -1.0f) * hi16(s0w[w]), u0, u1);
+    low[w] = ix_pack_bf2_canon_hw(t0 + u0, t1 + u1);
+    ix_rbf2_hw(b0 * lo16(c1w[w]), b1 * hi16(c1w[w]), t0, t1);
+    ix_rbf2_hw(a0 * lo16(s1w[w]), a1 * hi16(s1w[w]), u0, u1);
+    hiw[w] = ix_pack_bf2_canon_hw(t0 + u0, t1 + u1);
+  }
+}
+
 // Workgroup id -> position in a linear work order, for kernels that stream memory in that order. Hardware deals
 // consecutive workgroup ids to the 8 XCDs round-robin; here the order is cut into 8 equal runs and XCD x walks run x,
 // so every XCD (its own L2, its own path to memory) streams one contiguous region instead of every eighth piece of

@@ -17,8 +17,8 @@
 #include "../../include/isoexec_hip.h"
 
 template <int LPR>
-__device__ __forceinline__ float ix_row_sumsq(const bf16_t* __restrict__ xr, const bf16_t* __restrict__ rr,
-                                              int N, int sub, bool vec) {
+__device__ __forceinline__ float ix_row_rstd(const bf16_t* __restrict__ xr, const bf16_t* __restrict__ rr, int N,
+                                             float eps, int sub, bool vec) {
   float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
   for (int off = sub * 8; off < N; off += LPR * 8) {
     float x[8];
@@ -29,13 +29,9 @@ __device__ __forceinline__ float ix_row_sumsq(const bf16_t* __restrict__ xr, con
 #pragma unroll
       for (int i = 0; i < 8; ++i) x[i] = ix_rbf(x[i] + r[i]);
     }
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const float sq = x[i] * x[i];
-      acc[i] = acc[i] + sq;
-    }
+    ix_sumsq8(x, acc);
   }
-  return ix_lane_tree<LPR>(ix_tree8(acc));
+  return ix_norm_rstd<LPR>(acc, N, eps);
 }
 
 // MODE 0: plain; 1: gated (gate strided by token); 2: residual add (writes h too).
@@ -55,9 +51,7 @@ __global__ __launch_bounds__(256) void k_rmsnorm(const bf16_t* __restrict__ x, c
   const bf16_t* xr = x + rrow * N;
   const bf16_t* rr = nullptr;
   if (MODE == 2) rr = aux + rrow * N;
-  const float s = ix_row_sumsq<LPR>(xr, rr, N, sub, vec != 0);
-  const float ms = s / (float)N;
-  const float rstd = ix_rsqrt_ieee(ms + eps);
+  const float rstd = ix_row_rstd<LPR>(xr, rr, N, eps, sub, vec != 0);
   const bf16_t* gr = nullptr;
   if (MODE == 1) {
     const long t = rrow / HV, hh = rrow % HV;
@@ -76,12 +70,7 @@ __global__ __launch_bounds__(256) void k_rmsnorm(const bf16_t* __restrict__ x, c
       for (int i = 0; i < 8; ++i) xv[i] = ix_rbf(xv[i] + r[i]);
       ix_store8_bf16(h_out + row * N + off, N - off, vec != 0, xv);
     }
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const float nb = ix_rbf(xv[i] * rstd);
-      const float gam = zero_centered ? ix_rbf(1.0f + wv[i]) : wv[i];
-      o[i] = ix_rbf(nb * gam);
-    }
+    ix_norm8(xv, rstd, wv, zero_centered, o);
     if (MODE == 1) {
       float g[8];
       ix_load8(gr + off, N - off, vec != 0 && (aux_stride_t % 8 == 0), 0.0f, g);
@@ -93,7 +82,7 @@ __global__ __launch_bounds__(256) void k_rmsnorm(const bf16_t* __restrict__ x, c
 }
 
 // The same chain for a row that fits the registers of its lanes: N = LPR * 8 * NG columns, 16-byte aligned. Every
-// operand is fetched once, all loads are issued before the first use, and the sums run in the order of ix_row_sumsq
+// operand is fetched once, all loads are issued before the first use, and the sums run in the order of ix_row_rstd
 // (chunks ascending per slot, ix_tree8, lane tree), so the results are those of k_rmsnorm.
 template <int LPR, int MODE, int NG>
 __global__ __launch_bounds__(256) void k_rmsnorm_reg(const bf16_t* __restrict__ x, const bf16_t* __restrict__ w,
@@ -135,15 +124,9 @@ __global__ __launch_bounds__(256) void k_rmsnorm_reg(const bf16_t* __restrict__ 
 #pragma unroll
       for (int i = 0; i < 8; ++i) xv[c][i] = ix_rbf(xv[c][i] + r[i]);
     }
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const float sq = xv[c][i] * xv[c][i];
-      acc[i] = acc[i] + sq;
-    }
+    ix_sumsq8(xv[c], acc);
   }
-  const float s = ix_lane_tree<LPR>(ix_tree8(acc));
-  const float ms = s / (float)N;
-  const float rstd = ix_rsqrt_ieee(ms + eps);
+  const float rstd = ix_norm_rstd<LPR>(acc, N, eps);
   if (!live) return;
   bf16_t* orow = out + row * N + sub * 8;
 #pragma unroll
@@ -151,12 +134,7 @@ __global__ __launch_bounds__(256) void k_rmsnorm_reg(const bf16_t* __restrict__ 
     float wv[8], o[8];
     ix_unpack8(wp[c], wv);
     if (MODE == 2) ix_store8_bf16(h_out + row * N + sub * 8 + c * LPR * 8, 8, true, xv[c]);
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const float nb = ix_rbf(xv[c][i] * rstd);
-      const float gam = zero_centered ? ix_rbf(1.0f + wv[i]) : wv[i];
-      o[i] = ix_rbf(nb * gam);
-    }
+    ix_norm8(xv[c], rstd, wv, zero_centered, o);
     if (MODE == 1) {
       float g[8];
       ix_unpack8(ap[c], g);
@@ -308,15 +286,9 @@ __global__ __launch_bounds__(256) void k_combine_add_rmsnorm_reg(const bf16_t* _
     }
     if (live)
       *reinterpret_cast<uint4*>(h_out + row * N + sub * 8 + c * LPR * 8) = make_uint4(hp[0], hp[1], hp[2], hp[3]);
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const float sq = xv[c][i] * xv[c][i];
-      acc[i] = acc[i] + sq;
-    }
+    ix_sumsq8(xv[c], acc);
   }
-  const float s = ix_lane_tree<LPR>(ix_tree8(acc));
-  const float ms = s / (float)N;
-  const float rstd = ix_rsqrt_ieee(ms + eps);
+  const float rstd = ix_norm_rstd<LPR>(acc, N, eps);
   if (!live) return;
   bf16_t* orow = out + row * N + sub * 8;
 #pragma unroll

@@ -10,7 +10,7 @@
 //                    otherwise), the step's positions copied out of the context counters and checked, the packed offsets
 //                    0..n
 //   k_embed_rmsnorm  the embedding rows gathered into the residual stream and normalised, the context counters advanced
-//   k_rope_append    q and k rotated (k_rope8's statements), k and v written to the caches at the step's positions
+//   k_rope_append    q and k rotated (ix_rope_pairs8), k and v written to the caches at the step's positions
 #include "ix_common.h"
 #include "../../include/isoexec_hip.h"
 #include <math.h>
@@ -77,7 +77,7 @@ __global__ __launch_bounds__(256) void k_step_begin(IxStepMaps maps, int layers,
   }
 }
 
-// h[i] = table[tokens[i]], x[i] = norm(h[i]): k_rmsnorm_reg<64, 0, NG>'s statements (ix_norm.hip) on the gathered row. A
+// h[i] = table[tokens[i]], x[i] = norm(h[i]): the layout and sums of k_rmsnorm_reg<64, 0, NG> on the gathered row. A
 // null lane (pos < 0: its token may lie outside the table) reads nothing and gives a row of NaNs. Advances ctx.
 template <int NG>
 __global__ __launch_bounds__(64) void k_embed_rmsnorm(const bf16_t* __restrict__ table,
@@ -103,25 +103,14 @@ __global__ __launch_bounds__(64) void k_embed_rmsnorm(const bf16_t* __restrict__
     if (!held) xp[c] = make_uint4(0x7fc07fc0u, 0x7fc07fc0u, 0x7fc07fc0u, 0x7fc07fc0u);
     *reinterpret_cast<uint4*>(h + row * N + sub * 8 + c * LPR * 8) = xp[c];
     ix_unpack8(xp[c], xv[c]);
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const float sq = xv[c][i] * xv[c][i];
-      acc[i] = acc[i] + sq;
-    }
+    ix_sumsq8(xv[c], acc);
   }
-  const float s = ix_lane_tree<LPR>(ix_tree8(acc));
-  const float ms = s / (float)N;
-  const float rstd = ix_rsqrt_ieee(ms + eps);
+  const float rstd = ix_norm_rstd<LPR>(acc, N, eps);
 #pragma unroll
   for (int c = 0; c < NG; ++c) {
     float wv[8], o[8];
     ix_unpack8(wp[c], wv);
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const float nb = ix_rbf(xv[c][i] * rstd);
-      const float gam = zero_centered ? ix_rbf(1.0f + wv[i]) : wv[i];
-      o[i] = ix_rbf(nb * gam);
-    }
+    ix_norm8(xv[c], rstd, wv, zero_centered, o);
     ix_store8_bf16(x + row * N + sub * 8 + c * LPR * 8, 8, true, o);
   }
 }
@@ -144,7 +133,7 @@ static int ix_embed_rmsnorm(const void* table, const int64_t* tokens, const int*
 // The projection row of a token holds HQ + HKV heads to rotate and HKV value heads, D each. Rotated q heads go back to the
 // row, rotated k heads and the v heads to cache token kv_start[n] + pos[n] ([*, HKV, D]), which k_step_begin has checked
 // against the cache and the tables; a null lane (pos < 0) stores neither. Eight pairs (or, for v, sixteen values) per
-// thread; the rotation is k_rope8's (ix_attn.hip), statement for statement.
+// thread; the rotation is ix_rope_pairs8, as in k_rope8.
 __global__ __launch_bounds__(256) void k_rope_append(bf16_t* __restrict__ proj, long pitch, const bf16_t* __restrict__ cs,
                                                      const bf16_t* __restrict__ sn, const int* __restrict__ pos,
                                                      const int64_t* __restrict__ kv_start, bf16_t* __restrict__ kc,
@@ -173,22 +162,7 @@ __global__ __launch_bounds__(256) void k_rope_append(bf16_t* __restrict__ proj, 
     const bf16_t* st = sn + (long)p * D + c * 8;
     const uint4 c0 = *reinterpret_cast<const uint4*>(ct), c1 = *reinterpret_cast<const uint4*>(ct + half);
     const uint4 s0 = *reinterpret_cast<const uint4*>(st), s1 = *reinterpret_cast<const uint4*>(st + half);
-    const uint32_t* aw = &a4.x; const uint32_t* bw = &b4.x;
-    const uint32_t* c0w = &c0.x; const uint32_t* c1w = &c1.x; const uint32_t* s0w = &s0.x; const uint32_t* s1w = &s1.x;
-    uint32_t* low = &lo4.x; uint32_t* hiw = &hi4.x;
-    auto lo16 = [](uint32_t u) { return __uint_as_float(u << 16); };
-    auto hi16 = [](uint32_t u) { return __uint_as_float(u & 0xffff0000u); };
-#pragma unroll
-    for (int w = 0; w < 4; ++w) {
-      const float a0 = lo16(aw[w]), a1 = hi16(aw[w]), b0 = lo16(bw[w]), b1 = hi16(bw[w]);
-      float t0, t1, u0, u1;
-      ix_rbf2_hw(a0 * lo16(c0w[w]), a1 * hi16(c0w[w]), t0, t1);
-      ix_rbf2_hw((b0 * -1.0f) * lo16(s0w[w]), (b1 * -1.0f) * hi16(s0w[w]), u0, u1);
-      low[w] = ix_pack_bf2_canon_hw(t0 + u0, t1 + u1);
-      ix_rbf2_hw(b0 * lo16(c1w[w]), b1 * hi16(c1w[w]), t0, t1);
-      ix_rbf2_hw(a0 * lo16(s1w[w]), a1 * hi16(s1w[w]), u0, u1);
-      hiw[w] = ix_pack_bf2_canon_hw(t0 + u0, t1 + u1);
-    }
+    ix_rope_pairs8(a4, b4, c0, c1, s0, s1, lo4, hi4);
   }
   bf16_t* d = hd < HQ ? row : kc + (slot * HKV + (hd - HQ)) * D + c * 8;
   *reinterpret_cast<uint4*>(d) = lo4;

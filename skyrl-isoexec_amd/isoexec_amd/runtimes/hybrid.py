@@ -550,63 +550,60 @@ class RolloutEngine:
         if not fused_rows_enabled():
             return None
         bf16, f32, i64 = torch.bfloat16, torch.float32, torch.int64
-        dev = b.w.embed.device
-        ok = dev.type == "cuda"
+        ok, dev = b.w.embed.is_cuda, b.w.embed.get_device()
 
-        def ptr(t, dtype, *shape):  # the kernels have no extents to check an index against: every shape is pinned here
+        def ptr(t, dtype, shape):  # the kernels have no extents to check an index against: every shape is pinned here
             nonlocal ok
             p = t.data_ptr()
-            if t.dtype is not dtype or t.shape != shape or not t.is_contiguous() or p % 16 or t.device != dev:
+            if t.dtype is not dtype or t.shape != shape or not t.is_contiguous() or p & 15 or t.get_device() != dev:
                 ok = False
             return p
 
-        H, F, E, D = c.hidden, c.expert_inter, c.experts, c.gdn_qkv
-        packed_all = len(b.packed_experts) == c.layers
+        H, F, E, D, HV, Z = c.hidden, c.expert_inter, c.experts, c.gdn_qkv, c.gdn_v_heads, c.gdn_z
+        kh, q_width = c.gdn_head_dim, c.q_heads * c.head_dim
+        hidden, router, w1, w2 = (H,), (E, H), (E, 2 * F, H), (E, H, F)
+        kv_cache = (self.max_num_seqs + 1, self.max_len, c.kv_heads, c.head_dim)
+        attention_dense = (("qkv_proj", (q_width + 2 * c.kv_heads * c.head_dim, H)), ("o_proj", (H, q_width)))
+        gdn_dense = (("in_proj", (D + Z + 2 * HV, H)), ("out_proj", (H, Z)))
+        packed_all, packed_dense = len(b.packed_experts) == c.layers, b.packed_dense
         table = []
         for i, lw in enumerate(b.w.layers):
             attention = c.is_attention(i)
             nxt = b.w.layers[i + 1]["pre_norm"] if i + 1 < c.layers else b.w.final_norm
-            row = [int(attention), ptr(lw["post_norm"], bf16, H), ptr(nxt, bf16, H), ptr(lw["router"], bf16, E, H),
-                   ptr(lw["w1"], bf16, E, 2 * F, H), ptr(lw["w2"], bf16, E, H, F)]
+            table += (int(attention), ptr(lw["post_norm"], bf16, hidden), ptr(nxt, bf16, hidden),
+                      ptr(lw["router"], bf16, router), ptr(lw["w1"], bf16, w1), ptr(lw["w2"], bf16, w2))
             if packed_all:
                 w1f, w2f = b.packed_experts[i]
-                row += [ptr(w1f, bf16, E, 2 * F, H), ptr(w2f, bf16, E, H, F)]
+                table += (ptr(w1f, bf16, w1), ptr(w2f, bf16, w2))
             else:
-                row += [0, 0]
-            if attention:
-                q_width = c.q_heads * c.head_dim
-                shapes = {"qkv_proj": (q_width + 2 * c.kv_heads * c.head_dim, H), "o_proj": (H, q_width)}
-            else:
-                shapes = {"in_proj": (D + c.gdn_z + 2 * c.gdn_v_heads, H), "out_proj": (H, c.gdn_z)}
-            for name, shape in shapes.items():
-                pk = b.packed_dense.get((i, name))
+                table += (0, 0)
+            for name, shape in attention_dense if attention else gdn_dense:
+                pk = packed_dense.get((i, name))
                 if pk is None:
-                    row += [ptr(lw[name], bf16, *shape), 0]
+                    table += (ptr(lw[name], bf16, shape), 0)
                 else:  # as linear_nt: the weight the copy was made of beside the copy
-                    row += [ptr(pk.weight, bf16, *shape), ptr(pk.packed, bf16, shape[0] * shape[1])]
+                    table += (ptr(pk.weight, bf16, shape), ptr(pk.packed, bf16, (shape[0] * shape[1],)))
             if attention:
                 kv = self.kv[i]
-                cache = (self.max_num_seqs + 1, self.max_len, c.kv_heads, c.head_dim)
-                row += [0] * 11 + [ptr(kv.k, bf16, *cache), ptr(kv.v, bf16, *cache)]
-            else:
-                g = self.gdn[i]
-                if type(g) is not RecurrentGDN or g.table is None or g.activation not in ("silu", "swish") or not g.fused_decode_prep:
-                    return None
-                row += [ptr(g.conv_weight, bf16, D, 4), 0 if g.conv_bias is None else ptr(g.conv_bias, bf16, D),
-                        ptr(g.A_log, f32, c.gdn_v_heads), ptr(g.dt_bias, f32, c.gdn_v_heads), ptr(lw["out_norm"], bf16, c.gdn_head_dim),
-                        ptr(g.ssm_state, f32, g.capacity + 1, c.gdn_v_heads, c.gdn_head_dim, c.gdn_head_dim),
-                        ptr(g.conv_state, bf16, g.capacity + 1, D, c.conv_width - 1),
-                        ptr(g.slot2row, i64, g.table.map_size), g.table.map_size, ptr(g.last_used, i64, g.capacity + 1),
-                        ptr(g._clock, i64), 0, 0]
-            table += row
-        ptr(b.w.embed, bf16, c.vocab, H)
-        ptr(b.w.layers[0]["pre_norm"], bf16, H)
-        ptr(b.cos, bf16, b.cos.shape[0], c.head_dim)
-        ptr(b.sin, bf16, b.cos.shape[0], c.head_dim)
+                table += (0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, ptr(kv.k, bf16, kv_cache), ptr(kv.v, bf16, kv_cache))
+                continue
+            g = self.gdn[i]
+            if type(g) is not RecurrentGDN or g.table is None or g.activation not in ("silu", "swish") or not g.fused_decode_prep:
+                return None
+            rows, slots = g.capacity + 1, g.table.map_size
+            table += (ptr(g.conv_weight, bf16, (D, 4)), 0 if g.conv_bias is None else ptr(g.conv_bias, bf16, (D,)),
+                      ptr(g.A_log, f32, (HV,)), ptr(g.dt_bias, f32, (HV,)), ptr(lw["out_norm"], bf16, (kh,)),
+                      ptr(g.ssm_state, f32, (rows, HV, kh, kh)), ptr(g.conv_state, bf16, (rows, D, c.conv_width - 1)),
+                      ptr(g.slot2row, i64, (slots,)), slots, ptr(g.last_used, i64, (rows,)), ptr(g._clock, i64, ()), 0, 0)
+        ptr(b.w.embed, bf16, (c.vocab, H))
+        ptr(b.w.layers[0]["pre_norm"], bf16, hidden)
+        rotary = (b.cos.shape[0], c.head_dim)
+        ptr(b.cos, bf16, rotary)
+        ptr(b.sin, bf16, rotary)
         if not ok:
             return None
-        dims = array("q", [n, c.layers, H, c.vocab, b.cos.shape[0], c.gdn_k_heads, c.gdn_v_heads, c.gdn_head_dim, c.q_heads,
-                           c.kv_heads, c.head_dim, E, c.topk, F, int(packed_all), int(c.moe_combine_dtype == "fp32")])
+        dims = array("q", [n, c.layers, H, c.vocab, rotary[0], c.gdn_k_heads, HV, kh, c.q_heads, c.kv_heads, c.head_dim, E,
+                           c.topk, F, int(packed_all), int(c.moe_combine_dtype == "fp32")])
         return dims, array("q", table)
 
     def _decode_native(self, st: dict, tokens: torch.Tensor):

@@ -174,7 +174,8 @@ def experts_forward(x: torch.Tensor, w1: torch.Tensor, w2: torch.Tensor, p: Perm
     if x.dtype is not torch.bfloat16 or w1.dtype is not torch.bfloat16 or w2.dtype is not torch.bfloat16:
         raise RuntimeError("[isoexec-amd] experts serve bf16 only")
     T, H = x.shape
-    E, F2, _ = w1.shape
+    shape1 = w1.shape
+    E, F2, _ = shape1
     F = F2 // 2
     rows = T * p.k
     dev = x.device
@@ -183,14 +184,14 @@ def experts_forward(x: torch.Tensor, w1: torch.Tensor, w2: torch.Tensor, p: Perm
     xc = x if x.stride(1) == 1 else x.contiguous()
     if packed is not None and p.BM in (32, 64) and p.BN == 256:
         w1f, w2f = packed
-        if w1f.shape != w1.shape or w2f.shape != w2.shape or w1f.dtype is not torch.bfloat16 or w2f.dtype is not torch.bfloat16:
+        if w1f.shape != shape1 or w2f.shape != w2.shape or w1f.dtype is not torch.bfloat16 or w2f.dtype is not torch.bfloat16:
             raise RuntimeError("[isoexec-amd] packed must come from pack_decode(w1, w2)")
-        # other tokens touch other experts: between two uses of one, up to all of this layer's are read
+        # other tokens touch other experts: between two uses of one, up to all of this layer's bytes (3 E F2 H) are read
         rc = _lib.check(
             _lib.lib().ix_moe_experts_packed_footprint(xc.data_ptr(), xc.stride(0), p.sorted_token.data_ptr(),
                                                        p.permuted_prob.data_ptr(), w1f.data_ptr(), w2f.data_ptr(),
                                                        p.tile_meta.data_ptr(), p.max_tiles, p.BM, inter.data_ptr(),
-                                                       out.data_ptr(), T, rows, H, F, w1f.nbytes + w2f.nbytes,
+                                                       out.data_ptr(), T, rows, H, F, 3 * E * F2 * H,
                                                        _lib.current_stream(dev)), "ix_moe_experts_packed")
         if rc == _lib.IX_OK:
             return (out, inter) if return_inter else out

@@ -440,35 +440,55 @@ void k_gdn_scan_pairs(const TIO* __restrict__ q, const TIO* __restrict__ k, cons
 //     written to LDS after them; one barrier per tile;
 //   * no LDS store between a tile's tokens (an LDS load may not pass one): a token's output is the same in all lanes of
 //     its row, so lane tt keeps token tt's and the tile is written out at its end;
-//   * sixteen tokens of straight-line code, so the output's tree runs in the shadow of the next token's decay and dot.
+//   * sixteen tokens of straight-line code, so the output's tree runs in the shadow of the next token's decay and dot;
+//   * LONE, at a workgroup or two per CU: a fifth wave stages the tiles and writes the outputs out, so that the four others
+//     meet nothing but their tokens and the barrier (a fifth of the walk at one wave per SIMD, which waits for its own every
+//     instruction: 1147 -> 988 us for 8192 tokens, 121 ns a token);
+//   * E = 4, where SIMDs would stand idle: a slice's two chains in two lanes, joined by the tree's first level. A token is then
+//     29 vector instructions of a wave instead of 45 (256 tokens at K = 64: 33 -> 24 us).
 // The statements per token are ix_gdn_step's: same bits as k_gdn_scan and k_gdn_scan_pairs.
 // Sequences are taken longest first when there are 2..256 of them (ranked by every workgroup from cu), and a sequence's
 // workgroups are spread over all XCDs with the row blocks of a key head on one of them.
 // CPR: the boundary form (gdn_cpr.py:296-319). Two states walk together: the fp32 chain, and the running state, which
 // restarts from the chain rounded to the io type at every multiple of `chunk` tokens and makes the outputs. The pass that
 // first computes every boundary state, its pool, and the second pass over all tokens are then not there at all.
-// Measured (HV = 32, V = K = 128, bf16), k_gdn_scan / walk: one sequence of 8192 tokens 1990 / 1129 us (138 ns a token;
-// vector issue alone would be 75), five of 33..1203 tokens 883 / 247, 8 x 1000 1330 / 667; boundary form of nine sequences
+// Measured (HV = 32, V = K = 128, bf16), k_gdn_scan / walk: without LONE one sequence of 8192 tokens 1990 / 1129 us (138 ns a
+// token; vector issue alone would be 75), five of 33..1203 tokens 883 / 247, 8 x 1000 1330 / 667; boundary form of nine sequences
 // of 120..1500 tokens, boundary pass + segmented scan / walk: 3900 / 975. With first and second halves of the 8-element
 // slices apart in LDS a 16-byte read of sixteen lanes is one contiguous row (8 x 1000: 714 -> 667).
 __device__ __forceinline__ float ix_wire(float x, const bf16_t*) { return ix_rbf(x); }
 __device__ __forceinline__ float ix_wire(float x, const float*) { return x; }
 
-template <int KS, int RPL, typename TIO, bool CPR>
-__global__ __launch_bounds__(256) void k_gdn_walk(const TIO* __restrict__ q, const TIO* __restrict__ k,
+// dot of a lane's slice in the canonical order: eight elements, two chains joined; four elements, one of the two chains (the
+// join is then the first level of the lane tree).
+template <int E>
+__device__ __forceinline__ float ix_dot_slice(const float (&s)[E], const float (&x)[E]) {
+  if constexpr (E == 8) {
+    return ix_dot8(s, x);
+  } else {
+    float p = s[0] * x[0];
+    p = __builtin_fmaf(s[1], x[1], p);
+    p = __builtin_fmaf(s[2], x[2], p);
+    return __builtin_fmaf(s[3], x[3], p);
+  }
+}
+
+template <int K, int E, int RPL, typename TIO, bool CPR, bool LONE>
+__global__ __launch_bounds__(LONE ? 320 : 256) void k_gdn_walk(const TIO* __restrict__ q, const TIO* __restrict__ k,
                                                   const TIO* __restrict__ v, const float* __restrict__ g,
                                                   const TIO* __restrict__ beta, TIO* __restrict__ o,
                                                   float* __restrict__ state, const int* __restrict__ cu,
                                                   const int* __restrict__ sidx, long q_pitch, long k_pitch,
                                                   long v_pitch, int N, int H, int HV, int V, float scale, int chunk) {
-  constexpr int T = KS == 32 ? 8 : 16;  // tokens per tile (K = 256: half as many, for the LDS)
-  constexpr int K = KS * 8;
-  constexpr int RW = 256 / KS;
+  constexpr int T = K == 256 ? 8 : 16;           // tokens per tile (K = 256: half as many, for the LDS)
+  constexpr int L = K / E;                       // lanes per row
+  constexpr int RW = 256 / L;
   constexpr int R = RW * RPL;
-  constexpr int QK = 2 * T * KS;                 // 8-element groups of k and q in a tile
-  constexpr int QC = (QK + 255) / 256;           // groups per thread
-  constexpr int VC = (T * R + 255) / 256;        // v elements per thread
-  constexpr int NK = (T + KS - 1) / KS;          // tokens a lane keeps the output of
+  constexpr int G8 = K / 8;
+  constexpr int QK = 2 * T * G8;                 // 8-element groups of k and q in a tile
+  constexpr int ST = LONE ? 64 : 256;            // threads that stage
+  constexpr int QC = (QK + ST - 1) / ST;         // groups per staging thread
+  constexpr int VC = (T * R + ST - 1) / ST;      // v elements per staging thread
   __shared__ __align__(16) float kq[2][2][T][K];  // [buffer][k, q * scale][token]
   __shared__ float vf[2][T][R];
   __shared__ float of[2][T][R];
@@ -494,36 +514,18 @@ __global__ __launch_bounds__(256) void k_gdn_walk(const TIO* __restrict__ q, con
   const int vb = w % VB;
   const int hv = w / VB;
   const int h = hv / (HV / H);
-  const int sub = tid % KS, r = tid / KS;
   const int t_begin = cu[n];
   const int len = cu[n + 1] - t_begin;
   if (len <= 0) return;
   const int row0 = sidx ? sidx[n] : 1;
   TIO* ob = o + (long)hv * V + vb * R;
   if (row0 <= 0) {  // null lane: no state, outputs defined as zero
-    for (int i = tid; i < len * R; i += 256) ix_st(ob + (long)(t_begin + i / R) * HV * V + i % R, 0.0f);
+    for (int i = tid; i < len * R; i += (int)blockDim.x) ix_st(ob + (long)(t_begin + i / R) * HV * V + i % R, 0.0f);
     return;
   }
+  const int tiles = (len + T - 1) / T;
 
-  float S[RPL][8], C[CPR ? RPL : 1][8];
-#pragma unroll
-  for (int j = 0; j < RPL; ++j) {
-    if (state) {
-      const float* sp = state + (((long)row0 * HV + hv) * V + vb * R + r + j * RW) * K + sub * 8;
-      const float4 a = *reinterpret_cast<const float4*>(sp);
-      const float4 b = *reinterpret_cast<const float4*>(sp + 4);
-      S[j][0] = a.x; S[j][1] = a.y; S[j][2] = a.z; S[j][3] = a.w;
-      S[j][4] = b.x; S[j][5] = b.y; S[j][6] = b.z; S[j][7] = b.w;
-    } else {
-#pragma unroll
-      for (int i = 0; i < 8; ++i) S[j][i] = 0.0f;
-    }
-    if constexpr (CPR) {
-#pragma unroll
-      for (int i = 0; i < 8; ++i) C[j][i] = S[j][i];
-    }
-  }
-
+  const int lane = LONE ? tid - 256 : tid;       // among the staging threads
   IxRaw8<TIO> rq[QC];
   // raw, as loaded: a conversion here would wait for the loads that the tile's tokens are meant to cover
   TIO rv[VC], rb = 0;
@@ -531,23 +533,23 @@ __global__ __launch_bounds__(256) void k_gdn_walk(const TIO* __restrict__ q, con
   auto fetch = [&](int t0) __attribute__((always_inline)) {  // tokens past the end read the last one's values, unused
 #pragma unroll
     for (int c = 0; c < QC; ++c) {
-      const int i = tid + 256 * c;
-      if (QK % 256 == 0 || i < QK) {
-        const int e = i % (T * KS), isq = i / (T * KS);
-        const long tok = t_begin + min(t0 + e / KS, len - 1);
-        rq[c].load((isq ? q + tok * q_pitch : k + tok * k_pitch) + h * K + (e % KS) * 8);
+      const int i = lane + ST * c;
+      if (QK % ST == 0 || i < QK) {
+        const int e = i % (T * G8), isq = i / (T * G8);
+        const long tok = t_begin + min(t0 + e / G8, len - 1);
+        rq[c].load((isq ? q + tok * q_pitch : k + tok * k_pitch) + h * K + (e % G8) * 8);
       }
     }
 #pragma unroll
     for (int c = 0; c < VC; ++c) {
-      const int i = tid + 256 * c;
-      if ((T * R) % 256 == 0 || i < T * R) {
+      const int i = lane + ST * c;
+      if ((T * R) % ST == 0 || i < T * R) {
         const long tok = t_begin + min(t0 + i / R, len - 1);
         rv[c] = v[tok * v_pitch + (long)hv * V + vb * R + i % R];
       }
     }
-    if (tid < T) {
-      const long tok = t_begin + min(t0 + tid, len - 1);
+    if (lane < T) {
+      const long tok = t_begin + min(t0 + lane, len - 1);
       rg = g[tok * HV + hv];
       rb = beta[tok * HV + hv];
     }
@@ -555,72 +557,99 @@ __global__ __launch_bounds__(256) void k_gdn_walk(const TIO* __restrict__ q, con
   auto commit = [&](int b) __attribute__((always_inline)) {
 #pragma unroll
     for (int c = 0; c < QC; ++c) {
-      const int i = tid + 256 * c;
-      if (QK % 256 == 0 || i < QK) {
-        const int e = i % (T * KS), isq = i / (T * KS);
+      const int i = lane + ST * c;
+      if (QK % ST == 0 || i < QK) {
+        const int e = i % (T * G8), isq = i / (T * G8);
         float x[8];
         rq[c].widen(x);
         const float m = isq ? scale : 1.0f;  // k * 1 is k
-        float* d = &kq[b][isq][e / KS][(e % KS) * 4];  // first halves of all slices, then second halves
-        *reinterpret_cast<float4*>(d) = make_float4(x[0] * m, x[1] * m, x[2] * m, x[3] * m);
-        *reinterpret_cast<float4*>(d + K / 2) = make_float4(x[4] * m, x[5] * m, x[6] * m, x[7] * m);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) x[j] = x[j] * m;
+        if constexpr (E == 8) {  // first halves of all slices, then second halves: sixteen lanes read one contiguous row
+          float* d = &kq[b][isq][e / G8][(e % G8) * 4];
+          *reinterpret_cast<float4*>(d) = make_float4(x[0], x[1], x[2], x[3]);
+          *reinterpret_cast<float4*>(d + K / 2) = make_float4(x[4], x[5], x[6], x[7]);
+        } else {  // a slice's even elements, then its odd ones: one chain each
+          float* d = &kq[b][isq][e / G8][(e % G8) * 8];
+          *reinterpret_cast<float4*>(d) = make_float4(x[0], x[2], x[4], x[6]);
+          *reinterpret_cast<float4*>(d + 4) = make_float4(x[1], x[3], x[5], x[7]);
+        }
       }
     }
 #pragma unroll
     for (int c = 0; c < VC; ++c) {
-      const int i = tid + 256 * c;
-      if ((T * R) % 256 == 0 || i < T * R) vf[b][i / R][i % R] = ix_ld(&rv[c]);
+      const int i = lane + ST * c;
+      if ((T * R) % ST == 0 || i < T * R) vf[b][i / R][i % R] = ix_ld(&rv[c]);
     }
-    if (tid < T) eb[b][tid] = make_float2(ix_exp(rg), ix_ld(&rb));
+    if (lane < T) eb[b][lane] = make_float2(ix_exp(rg), ix_ld(&rb));
   };
   auto emit = [&](int t0, int nt, int b) __attribute__((always_inline)) {
 #pragma unroll
     for (int c = 0; c < VC; ++c) {
-      const int i = tid + 256 * c;
+      const int i = lane + ST * c;
       if (i < nt * R) ix_st(ob + (long)(t_begin + t0 + i / R) * HV * V + i % R, of[b][i / R][i % R]);
     }
   };
-  auto token = [&](int b, int tt, float (&ov)[RPL]) __attribute__((always_inline)) {
-    float kk[8], qs[8];
-    {
-      const float4 a = *reinterpret_cast<const float4*>(&kq[b][0][tt][sub * 4]);
-      const float4 c = *reinterpret_cast<const float4*>(&kq[b][0][tt][K / 2 + sub * 4]);
-      kk[0] = a.x; kk[1] = a.y; kk[2] = a.z; kk[3] = a.w; kk[4] = c.x; kk[5] = c.y; kk[6] = c.z; kk[7] = c.w;
-      const float4 d = *reinterpret_cast<const float4*>(&kq[b][1][tt][sub * 4]);
-      const float4 e = *reinterpret_cast<const float4*>(&kq[b][1][tt][K / 2 + sub * 4]);
-      qs[0] = d.x; qs[1] = d.y; qs[2] = d.z; qs[3] = d.w; qs[4] = e.x; qs[5] = e.y; qs[6] = e.z; qs[7] = e.w;
-    }
-    const float2 gb = eb[b][tt];
-#pragma unroll
-    for (int j = 0; j < RPL; ++j) {
-      const float vv = vf[b][tt][j * RW + r];
-      if constexpr (CPR) {  // ix_gdn_step without its output, on the chain
-#pragma unroll
-        for (int i = 0; i < 8; ++i) C[j][i] = C[j][i] * gb.x;
-        const float kv = ix_lane_tree<KS>(ix_dot8(C[j], kk));
-        const float d = (vv - kv) * gb.y;
-#pragma unroll
-        for (int i = 0; i < 8; ++i) C[j][i] = __builtin_fmaf(d, kk[i], C[j][i]);
+  if constexpr (LONE) {
+    if (tid >= 256) {  // the staging wave: as many barriers as the others
+      fetch(0);
+      commit(0);
+      if (tiles > 1) fetch(T);
+      __syncthreads();
+      for (int i = 0; i < tiles; ++i) {
+        const int b = i & 1;
+        if (i + 1 < tiles) commit(b ^ 1);
+        if (i + 2 < tiles) fetch((i + 2) * T);
+        if (i > 0) emit((i - 1) * T, T, b ^ 1);
+        __syncthreads();
       }
-      ov[j] = ix_gdn_step<KS>(S[j], kk, qs, vv, gb.x, gb.y);
+      emit((tiles - 1) * T, len - (tiles - 1) * T, (tiles - 1) & 1);
+      return;
+    }
+    __builtin_amdgcn_s_setprio(2);  // in front of the staging wave, which has a tile's time for its share
+  }
+
+  const int sub = tid % L, r = tid / L;
+  float S[RPL][E], C[CPR ? RPL : 1][E];
+  const int kbase = E == 8 ? sub * 8 : (sub >> 1) * 8 + (sub & 1);
+  constexpr int KSTEP = E == 8 ? 1 : 2;
+#pragma unroll
+  for (int j = 0; j < RPL; ++j) {
+    const float* sp = state + (((long)row0 * HV + hv) * V + vb * R + r + j * RW) * K + kbase;
+#pragma unroll
+    for (int i = 0; i < E; ++i) S[j][i] = state ? sp[i * KSTEP] : 0.0f;
+    if constexpr (CPR) {
+#pragma unroll
+      for (int i = 0; i < E; ++i) C[j][i] = S[j][i];
+    }
+  }
+  auto load_x = [&](const float* row, float (&x)[E]) __attribute__((always_inline)) {
+    const float4 a = *reinterpret_cast<const float4*>(row + sub * 4);
+    x[0] = a.x; x[1] = a.y; x[2] = a.z; x[3] = a.w;
+    if constexpr (E == 8) {
+      const float4 c = *reinterpret_cast<const float4*>(row + K / 2 + sub * 4);
+      x[4] = c.x; x[5] = c.y; x[6] = c.z; x[7] = c.w;
     }
   };
 
-  fetch(0);
-  commit(0);
+  if constexpr (!LONE) {
+    fetch(0);
+    commit(0);
+  }
   __syncthreads();
-  int b = 0;
-  for (int t0 = 0; t0 < len; t0 += T, b ^= 1) {
+  for (int it = 0; it < tiles; ++it) {
+    const int b = it & 1, t0 = it * T;
     const int nt = min(T, len - t0);
-    const bool more = t0 + T < len;
-    if (more) fetch(t0 + T);
-    if (t0 > 0) emit(t0 - T, T, b ^ 1);
+    if constexpr (!LONE) {
+      if (it + 1 < tiles) fetch(t0 + T);
+      if (it > 0) emit(t0 - T, T, b ^ 1);
+    }
     if constexpr (CPR) {
       if (t0 % chunk == 0) {
 #pragma unroll
         for (int j = 0; j < RPL; ++j)
 #pragma unroll
-          for (int i = 0; i < 8; ++i) S[j][i] = ix_wire(C[j][i], (const TIO*)nullptr);
+          for (int i = 0; i < E; ++i) S[j][i] = ix_wire(C[j][i], (const TIO*)nullptr);
       }
     }
     if (nt == T) {
@@ -628,40 +657,32 @@ __global__ __launch_bounds__(256) void k_gdn_walk(const TIO* __restrict__ q, con
       // before, so that neither waits alone for its lane exchanges), updates the state, and issues the dots of its own q
       // and the next token's k. k is loaded two tokens ahead, q one; the scheduling barrier keeps those loads at the top
       // of the iteration, a whole one in front of their use (left alone, the compiler sinks them to it).
-      float keep[RPL][NK];
-      float kb[3][8], qb[2][8], vb3[3][RPL], kp[RPL], qp[RPL], cp[RPL];
+      float kb[3][E], qb[2][E], vb3[3][RPL], kp[RPL], qp[RPL], cp[RPL], keep[RPL];
+      auto put = [&](int tt, int j, float ov) __attribute__((always_inline)) {
+        if ((tt % L) == 0) keep[j] = ov;
+        else keep[j] = sub == tt % L ? ov : keep[j];
+        if (tt % L == L - 1 || tt == T - 1) { if (T - tt / L * L >= L || sub < T % L) of[b][tt / L * L + sub][j * RW + r] = keep[j]; }
+      };
       float2 gb[3];
       auto load_k = [&](int tt) __attribute__((always_inline)) {
-        const float4 a = *reinterpret_cast<const float4*>(&kq[b][0][tt][sub * 4]);
-        const float4 c = *reinterpret_cast<const float4*>(&kq[b][0][tt][K / 2 + sub * 4]);
-        float(&x)[8] = kb[tt % 3];
-        x[0] = a.x; x[1] = a.y; x[2] = a.z; x[3] = a.w; x[4] = c.x; x[5] = c.y; x[6] = c.z; x[7] = c.w;
+        load_x(&kq[b][0][tt][0], kb[tt % 3]);
         gb[tt % 3] = eb[b][tt];
 #pragma unroll
         for (int j = 0; j < RPL; ++j) vb3[tt % 3][j] = vf[b][tt][j * RW + r];
       };
-      auto load_q = [&](int tt) __attribute__((always_inline)) {
-        const float4 a = *reinterpret_cast<const float4*>(&kq[b][1][tt][sub * 4]);
-        const float4 c = *reinterpret_cast<const float4*>(&kq[b][1][tt][K / 2 + sub * 4]);
-        float(&x)[8] = qb[tt % 2];
-        x[0] = a.x; x[1] = a.y; x[2] = a.z; x[3] = a.w; x[4] = c.x; x[5] = c.y; x[6] = c.z; x[7] = c.w;
-      };
+      auto load_q = [&](int tt) __attribute__((always_inline)) { load_x(&kq[b][1][tt][0], qb[tt % 2]); };
       auto decay_dot = [&](int tt) __attribute__((always_inline)) {
 #pragma unroll
         for (int j = 0; j < RPL; ++j) {
 #pragma unroll
-          for (int i = 0; i < 8; ++i) S[j][i] = S[j][i] * gb[tt % 3].x;
-          kp[j] = ix_dot8(S[j], kb[tt % 3]);
+          for (int i = 0; i < E; ++i) S[j][i] = S[j][i] * gb[tt % 3].x;
+          kp[j] = ix_dot_slice(S[j], kb[tt % 3]);
           if constexpr (CPR) {
 #pragma unroll
-            for (int i = 0; i < 8; ++i) C[j][i] = C[j][i] * gb[tt % 3].x;
-            cp[j] = ix_dot8(C[j], kb[tt % 3]);
+            for (int i = 0; i < E; ++i) C[j][i] = C[j][i] * gb[tt % 3].x;
+            cp[j] = ix_dot_slice(C[j], kb[tt % 3]);
           }
         }
-      };
-      auto keep_out = [&](int tt, int j, float ov) __attribute__((always_inline)) {
-        if ((tt % KS) == 0) keep[j][tt / KS] = ov;
-        else keep[j][tt / KS] = sub == tt % KS ? ov : keep[j][tt / KS];
       };
       load_k(0);
       load_k(1);
@@ -675,54 +696,64 @@ __global__ __launch_bounds__(256) void k_gdn_walk(const TIO* __restrict__ q, con
         float ov[RPL], kv[RPL], cv[RPL];
 #pragma unroll
         for (int j = 0; j < RPL; ++j) {
-          kv[j] = ix_lane_tree<KS>(kp[j]);
-          if constexpr (CPR) cv[j] = ix_lane_tree<KS>(cp[j]);
-          if (tt > 0) ov[j] = ix_lane_tree<KS>(qp[j]);
+          kv[j] = ix_lane_tree<L>(kp[j]);
+          if constexpr (CPR) cv[j] = ix_lane_tree<L>(cp[j]);
+          if (tt > 0) ov[j] = ix_lane_tree<L>(qp[j]);
         }
 #pragma unroll
         for (int j = 0; j < RPL; ++j) {
-          if (tt > 0) keep_out(tt - 1, j, ov[j]);
           const float d = (vb3[tt % 3][j] - kv[j]) * gb[tt % 3].y;
 #pragma unroll
-          for (int i = 0; i < 8; ++i) S[j][i] = __builtin_fmaf(d, kb[tt % 3][i], S[j][i]);
-          qp[j] = ix_dot8(S[j], qb[tt % 2]);
+          for (int i = 0; i < E; ++i) S[j][i] = __builtin_fmaf(d, kb[tt % 3][i], S[j][i]);
+          qp[j] = ix_dot_slice(S[j], qb[tt % 2]);
           if constexpr (CPR) {
             const float dc = (vb3[tt % 3][j] - cv[j]) * gb[tt % 3].y;
 #pragma unroll
-            for (int i = 0; i < 8; ++i) C[j][i] = __builtin_fmaf(dc, kb[tt % 3][i], C[j][i]);
+            for (int i = 0; i < E; ++i) C[j][i] = __builtin_fmaf(dc, kb[tt % 3][i], C[j][i]);
           }
+        }
+        if (tt > 0) {
+#pragma unroll
+          for (int j = 0; j < RPL; ++j) put(tt - 1, j, ov[j]);
         }
         if (tt + 1 < T) decay_dot(tt + 1);
       }
 #pragma unroll
-      for (int j = 0; j < RPL; ++j) keep_out(T - 1, j, ix_lane_tree<KS>(qp[j]));
-      if (KS <= T || sub < T) {
-#pragma unroll
-        for (int j = 0; j < RPL; ++j)
-#pragma unroll
-          for (int i = 0; i < NK; ++i) of[b][sub + KS * i][j * RW + r] = keep[j][i];
-      }
+      for (int j = 0; j < RPL; ++j) put(T - 1, j, ix_lane_tree<L>(qp[j]));
     } else {
       for (int tt = 0; tt < nt; ++tt) {
-        float ov[RPL];
-        token(b, tt, ov);
-        if (sub == 0) {
+        float kk[E], qs[E];
+        load_x(&kq[b][0][tt][0], kk);
+        load_x(&kq[b][1][tt][0], qs);
+        const float2 gb = eb[b][tt];
 #pragma unroll
-          for (int j = 0; j < RPL; ++j) of[b][tt][j * RW + r] = ov[j];
+        for (int j = 0; j < RPL; ++j) {
+          const float vv = vf[b][tt][j * RW + r];
+          auto advance = [&](float (&X)[E]) __attribute__((always_inline)) {
+#pragma unroll
+            for (int i = 0; i < E; ++i) X[i] = X[i] * gb.x;
+            const float d = (vv - ix_lane_tree<L>(ix_dot_slice(X, kk))) * gb.y;
+#pragma unroll
+            for (int i = 0; i < E; ++i) X[i] = __builtin_fmaf(d, kk[i], X[i]);
+          };
+          if constexpr (CPR) advance(C[j]);
+          advance(S[j]);
+          of[b][tt][j * RW + r] = ix_lane_tree<L>(ix_dot_slice(S[j], qs));
         }
       }
     }
-    if (more) commit(b ^ 1);
+    if constexpr (!LONE) {
+      if (it + 1 < tiles) commit(b ^ 1);
+    }
     __syncthreads();
   }
-  const int last = (len - 1) / T;
-  emit(last * T, len - last * T, last & 1);
+  if constexpr (!LONE) emit((tiles - 1) * T, len - (tiles - 1) * T, (tiles - 1) & 1);
   if (state && !CPR) {
 #pragma unroll
     for (int j = 0; j < RPL; ++j) {
-      float* sp = state + (((long)row0 * HV + hv) * V + vb * R + r + j * RW) * K + sub * 8;
-      *reinterpret_cast<float4*>(sp) = make_float4(S[j][0], S[j][1], S[j][2], S[j][3]);
-      *reinterpret_cast<float4*>(sp + 4) = make_float4(S[j][4], S[j][5], S[j][6], S[j][7]);
+      float* sp = state + (((long)row0 * HV + hv) * V + vb * R + r + j * RW) * K + kbase;
+#pragma unroll
+      for (int i = 0; i < E; ++i) sp[i * KSTEP] = S[j][i];
     }
   }
 }
@@ -733,21 +764,26 @@ static bool ix_gdn_vec_qk(const void* q, const void* k, long q_pitch, long k_pit
   return q_pitch % 8 == 0 && k_pitch % 8 == 0 && ix_aligned(q, 8 * sizeof(TIO)) && ix_aligned(k, 8 * sizeof(TIO));
 }
 
-template <int KS, typename TIO, bool CPR>
+template <int K, int E, typename TIO, bool CPR>
 static int ix_gdn_walk_launch(const void* q, const void* k, const void* v, const float* g, const void* beta, void* o,
                               float* state, const int* cu, const int* sidx, long q_pitch, long k_pitch, long v_pitch,
-                              long N, int H, int HV, int V, float scale, int chunk, int rpl, hipStream_t st) {
-  constexpr int RW = 256 / KS;
+                              long N, int H, int HV, int V, float scale, int chunk, int rpl, bool lone, hipStream_t st) {
+  constexpr int RW = 256 / (K / E);  // split slices come in the lone form only
   if (V % RW != 0 || !ix_gdn_vec_qk<TIO>(q, k, q_pitch, k_pitch)) return IX_DECLINED;
   if (rpl == 2 && V % (2 * RW) != 0) rpl = 1;
   const long grid = N * HV * (V / (RW * rpl));
   if (grid > 0x7fffffffL) return IX_DECLINED;
-#define IX_WALK(RPL_)                                                                                                \
-  hipLaunchKernelGGL((k_gdn_walk<KS, RPL_, TIO, CPR>), dim3((unsigned)grid), dim3(256), 0, st, (const TIO*)q,        \
-                     (const TIO*)k, (const TIO*)v, g, (const TIO*)beta, (TIO*)o, state, cu, sidx, q_pitch, k_pitch,  \
-                     v_pitch, (int)N, H, HV, V, scale, chunk)
-  if (rpl == 2) IX_WALK(2);
-  else IX_WALK(1);
+#define IX_WALK(RPL_, LONE_)                                                                                           \
+  hipLaunchKernelGGL((k_gdn_walk<K, E, RPL_, TIO, CPR, LONE_>), dim3((unsigned)grid), dim3(LONE_ ? 320 : 256), 0, st, \
+                     (const TIO*)q, (const TIO*)k, (const TIO*)v, g, (const TIO*)beta, (TIO*)o, state, cu, sidx,        \
+                     q_pitch, k_pitch, v_pitch, (int)N, H, HV, V, scale, chunk)
+  if constexpr (E == 4) {
+    IX_WALK(1, true);
+  } else {
+    if (rpl == 2) IX_WALK(2, false);
+    else if (lone) IX_WALK(1, true);
+    else IX_WALK(1, false);
+  }
 #undef IX_WALK
   return ix_launch_status();
 }
@@ -815,24 +851,37 @@ static int ix_gdn_walk(const void* q, const void* k, const void* v, const float*
   // waves. Measured at HV = 32, V = K = 128, us one / two rows: one sequence of 8192 tokens 1129 / 1823, five of 33..1203
   // 247 / 307, nine of 120..1500 608 / 591, 16 x 1000 1266 / 1180; K = V = 64, HV = 16
   // and 32: 8 x 500 72 / 110, 32 x 500 329 / 323. The line: eight waves per SIMD at one row.
-  if (rpl <= 0) rpl = N * HV * V * (K / 8) >= 8L * 1024 * 64 ? 2 : 1;
-#define IX_WALK_CASE(KSV)                                                                                             \
-  if (K == KSV * 8) {                                                                                                 \
-    if (io_dtype == IX_DT_BF16)                                                                                       \
-      return chunk > 0 ? ix_gdn_walk_launch<KSV, bf16_t, true>(q, k, v, g, beta, o, state, cu, sidx, q_pitch, k_pitch, \
-                                                               v_pitch, N, H, HV, V, scale, chunk, rpl, st)           \
-                       : ix_gdn_walk_launch<KSV, bf16_t, false>(q, k, v, g, beta, o, state, cu, sidx, q_pitch,        \
-                                                                k_pitch, v_pitch, N, H, HV, V, scale, 0, rpl, st);    \
-    return chunk > 0 ? ix_gdn_walk_launch<KSV, float, true>(q, k, v, g, beta, o, state, cu, sidx, q_pitch, k_pitch,   \
-                                                            v_pitch, N, H, HV, V, scale, chunk, rpl, st)              \
-                     : ix_gdn_walk_launch<KSV, float, false>(q, k, v, g, beta, o, state, cu, sidx, q_pitch, k_pitch,  \
-                                                             v_pitch, N, H, HV, V, scale, 0, rpl, st);                \
+  // Fewer workgroups: a wave of their own stages the tiles (LONE) up to two of them per CU; with more, its registers and its
+  // share of the issue are missed. us without / with it: one sequence of 8192 tokens 1147 / 988, 2 x 3000 544 / 501, 3 x 2000
+  // 484 / 522; K = V = 64, HV = 32, 8 x 512 92 / 86, 16 x 512 156 / 210. And a slice split over two lanes (E = 4) while one
+  // such workgroup per CU, two at K <= 64, is all there is (at K = 128 a row is then 32 lanes and its tree has a level across
+  // the halves of 16). us whole / split: 2000 tokens of 16 heads at K = 128 245 / 206, of 32 heads (two per CU) 66 / 75 per
+  // 500; K = 64, 2 x 256 of 4 heads 33 / 24, 8 x 512 of 16 heads 66 / 63, of 32 heads 86 / 107.
+  const long lanes = N * HV * V * (K / 8);  // threads at one row per lane group, whole slices
+  const bool auto_shape = rpl <= 0;
+  if (auto_shape) rpl = lanes >= 8L * 1024 * 64 ? 2 : 1;
+  const bool lone = auto_shape && lanes <= 2L * 256 * 256;
+  const bool split = auto_shape && K <= 128 && 2 * lanes <= (K == 128 ? 256L : 512L) * 256 &&
+                     V % (2048 / K) == 0;  // what whole slices decline stays declined
+#define IX_WALK_ARGS(CHUNK_) \
+  q, k, v, g, beta, o, state, cu, sidx, q_pitch, k_pitch, v_pitch, N, H, HV, V, scale, CHUNK_, rpl, lone, st
+#define IX_WALK_CASE(KV, EV)                                                                            \
+  if (K == KV && split == (EV == 4)) {                                                                  \
+    if (io_dtype == IX_DT_BF16)                                                                         \
+      return chunk > 0 ? ix_gdn_walk_launch<KV, EV, bf16_t, true>(IX_WALK_ARGS(chunk))                  \
+                       : ix_gdn_walk_launch<KV, EV, bf16_t, false>(IX_WALK_ARGS(0));                    \
+    return chunk > 0 ? ix_gdn_walk_launch<KV, EV, float, true>(IX_WALK_ARGS(chunk))                     \
+                     : ix_gdn_walk_launch<KV, EV, float, false>(IX_WALK_ARGS(0));                       \
   }
-  IX_WALK_CASE(4)
-  IX_WALK_CASE(8)
-  IX_WALK_CASE(16)
-  IX_WALK_CASE(32)
+  IX_WALK_CASE(32, 4)
+  IX_WALK_CASE(64, 4)
+  IX_WALK_CASE(128, 4)
+  IX_WALK_CASE(32, 8)
+  IX_WALK_CASE(64, 8)
+  IX_WALK_CASE(128, 8)
+  IX_WALK_CASE(256, 8)
 #undef IX_WALK_CASE
+#undef IX_WALK_ARGS
   return IX_DECLINED;
 }
 

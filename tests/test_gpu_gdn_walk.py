@@ -52,6 +52,28 @@ def test_walk_equals_the_token_staged_scan(K, V, dtype, rows_per_group):
     assert same_bits(stateless_forward(*args, cu_seqlens=cu), run(16 | (1 << 8), zero, rows))
 
 
+@pytest.mark.parametrize("K,H,HV,V,dtype,lens", [
+    (32, 2, 4, 64, torch.bfloat16, EDGES), (64, 2, 2, 32, torch.float32, EDGES), (64, 4, 8, 64, torch.bfloat16, [33]),
+    (128, 2, 4, 64, torch.bfloat16, EDGES), (128, 1, 1, 16, torch.float32, [1, 50]),  # slices split over two lanes
+    (64, 8, 16, 64, torch.bfloat16, EDGES), (64, 8, 32, 64, torch.float32, [16, 8, 1, 40, 17, 3, 5, 2]),  # around its line
+    (128, 16, 32, 128, torch.bfloat16, [47]), (128, 16, 32, 128, torch.float32, [32, 17]),  # a staging wave, whole slices
+    (128, 8, 16, 128, torch.bfloat16, EDGES), (256, 1, 2, 64, torch.bfloat16, EDGES), (256, 1, 2, 64, torch.float32, [9])])
+def test_walk_by_the_rule_equals_the_token_staged_scan(K, H, HV, V, dtype, lens):
+    """The forms that the number of workgroups chooses (a staging wave, split slices, neither): output and final state bit for
+    bit against ``k_gdn_scan``, with and without a state."""
+    from isoexec_amd.ops.gdn.gdn_ops import gdn_recurrent_kernel, stateless_forward
+
+    args = make(lens, H, HV, K, V, dtype, K + V + HV)
+    cu, N = offsets(lens), len(lens)
+    rows = torch.arange(1, N + 1, dtype=torch.int32, device=DEV)
+    pa = torch.randn(N + 1, HV, V, K, generator=cpu_gen(4)).to(DEV)
+    pb, zero = pa.clone(), torch.zeros_like(pa)
+    run = lambda code, pool: gdn_recurrent_kernel(*args, ssm_state=pool, state_indices=rows, cu_seqlens=cu, time_tile=code)
+    want = run(16 | (1 << 8), pa)
+    assert same_bits(run(0, pb), want) and same_bits(pb, pa)
+    assert same_bits(stateless_forward(*args, cu_seqlens=cu), run(16 | (1 << 8), zero))
+
+
 def test_more_sequences_than_a_workgroup_ranks():
     from isoexec_amd.ops.gdn.gdn_ops import gdn_recurrent_kernel, stateless_forward
 

@@ -356,6 +356,8 @@ long ix_moe_max_tiles(long T, long k, long E, long BM);   /* ceil(T*k/BM) + E */
 size_t ix_moe_permute_scratch_ints(long T, long E);
 int ix_moe_pick_bm(long T, long k, long E);               /* 32, 128 or 256 */
 int ix_moe_pick_bm_packed(long T, long k, long E);        /* 32, 64, 128 or 256: for callers that hold packed matrices */
+/* The same for callers that know the layer's sizes (fc1 [E, 2F, Hd], fc2 [E, Hd, F]): also 96, 160, 192 and 224. */
+int ix_moe_pick_bm_shape(long T, long k, long E, long Hd, long F, int packed);
 
 /* fused_permute_index / ref_permute_index (moe_router_o2_kernel.py:313-351,389-397) plus the
  * block map (moe_fused_experts.py:156-205) and the inverse permutation of
@@ -409,7 +411,8 @@ int ix_moe_permute_static(const int* topk_idx, const float* topk_prob, long T, l
  * then up rows); W2 bf16 [E, Hd, F]; inter bf16 [rows, F]; expert_out bf16 [rows, Hd];
  * rows = T*k = the length of sorted_token and permuted_prob (the kernels clamp their reads of both to rows - 1, so it
  * must not exceed what the arrays hold). BM must be the value given to ix_moe_permute. With 256-row tiles and at
- * least 512 tiles of work both GEMMs run as streaming kernels (one workgroup per CU walking many tiles); same bits. */
+ * least 512 tiles of work, and with 96, 160, 192 or 224 rows, both GEMMs run as streaming kernels (one workgroup per CU
+ * walking many tiles); same bits. */
 int ix_moe_experts(const void* x, long ldx, const int* sorted_token, const float* permuted_prob,
                    const void* W1, const void* W2, const int* tile_meta, long max_tiles, long BM, void* inter,
                    void* expert_out, long T, long rows, long Hd, long F, void* stream);

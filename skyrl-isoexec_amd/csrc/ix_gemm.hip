@@ -3,47 +3,9 @@
 // override (ops/moe/moe_batch_invariant.py:422-473, ops/mm/mm_tiles.py:127-158) and of its
 // pinned non-split-K provider (ops/mm/csrc/cublaslt_pinned.cpp:1-36).
 #include "ix_gemm_core.h"
-#include "ix_gemm_stream.h"
-#include "../../include/isoexec_hip.h"
+#include "ix_gemm_dense.h"
 #include <algorithm>
 #include <cmath>
-
-// Workgroup -> tile map. Hardware hands consecutive workgroup ids to the 8 XCDs round-robin, and each XCD has
-// its own L2. The tiles are put in one order -- groups of GM M-tiles x GN weight tiles, about what an XCD's 32
-// CUs hold at a time, so that a group pulls GM activation tiles and GN weight tiles through the L2 for GM * GN
-// tiles; groups run down the M-tiles of GN weight-tile columns before moving to the next columns -- and that
-// order is cut into 8 equal runs, one per XCD: every XCD gets the same number of tiles whatever the shape, and
-// a weight tile is fetched by one L2 (two where a run ends inside its column group).
-#ifndef IX_GEMM_GM
-#define IX_GEMM_GM 8  // M-tiles of a group
-#endif
-#ifndef IX_GEMM_GN
-#define IX_GEMM_GN 4  // weight tiles of a group
-#endif
-// Tile number idx of XCD xcd's run of that order, for groups of GM x GN tiles.
-__device__ __forceinline__ bool ix_tile_of_run(unsigned xcd, unsigned idx, int nb_m, int nb_n, int GM, int GN, int* tm,
-                                               int* tn) {
-  // 32-bit arithmetic throughout (the launch refuses more than 2^31 tiles): a 64-bit division costs a workgroup
-  // about a microsecond before its first fetch.
-  const unsigned tiles = (unsigned)nb_m * (unsigned)nb_n;
-  // this XCD's run of the tile order: [tiles * xcd / 8, tiles * (xcd + 1) / 8)
-  const unsigned q = tiles >> 3, r = tiles & 7u;
-  const unsigned lo = q * xcd + ((r * xcd) >> 3), hi = q * (xcd + 1) + ((r * (xcd + 1)) >> 3);
-  const unsigned l = lo + idx;
-  if (l >= hi) return false;
-  const unsigned per_ngroup = (unsigned)GN * (unsigned)nb_m;
-  const unsigned ng = l / per_ngroup;
-  const unsigned rem = l - ng * per_ngroup;
-  const int gn = min(GN, nb_n - (int)ng * GN);  // width of this (possibly last) column group
-  const unsigned per_mgroup = (unsigned)GM * (unsigned)gn;
-  const unsigned mg = rem / per_mgroup;
-  const unsigned r2 = rem - mg * per_mgroup;
-  const int gm = min(GM, nb_m - (int)mg * GM);
-  const unsigned nl = r2 / (unsigned)gm, ml = r2 - nl * (unsigned)gm;
-  *tm = (int)mg * GM + (int)ml;
-  *tn = (int)ng * GN + (int)nl;
-  return true;
-}
 
 __device__ __forceinline__ void ix_store4(bf16_t* p, int valid, bool vec, const float (&v)[4]) {
   ix_store4_bf16(p, valid, vec, v[0], v[1], v[2], v[3]);
@@ -78,7 +40,7 @@ __global__ __launch_bounds__((WM * WN + PW) * 64) void k_gemm_bf16_nt(const bf16
                                                               TC* __restrict__ C, long ldc, int M, int N, int K,
                                                               int nb_m, int nb_n, int vec_store,
                                                               float* __restrict__ row_max_parts, long parts_ld,
-                                                              long batch_a, long batch_w, long batch_c) {
+                                                              long batch_a, long batch_w, long batch_c, int part_copies) {
   using Cfg = IxGemmCfg<BM, BN, WM, WN, PW, W_ONCE>;
   extern __shared__ __align__(16) char ix_lds[];
   // a batch of independent products (bmm): workgroup row blockIdx.y works on matrices batch strides further on
@@ -202,7 +164,9 @@ __global__ __launch_bounds__((WM * WN + PW) * 64) void k_gemm_bf16_nt(const bf16
       if constexpr (ix_gemm_parts_per_tile<BM, BN, WM, WN, PW>() == WN) {
         // one part per wave column: the layout the streaming form of this tile writes without passing through LDS
 #pragma unroll
-        for (int w = 0; w < WN; ++w) row_max_parts[(m0 + r) * parts_ld + tn * WN + w] = s_max[w * BM + r];
+        for (int w = 0; w < WN; ++w)
+          for (int d = 0; d < part_copies; ++d)
+            row_max_parts[(m0 + r) * parts_ld + (tn * WN + w) * part_copies + d] = s_max[w * BM + r];
       } else {
         float v = s_max[r];
 #pragma unroll
@@ -213,110 +177,22 @@ __global__ __launch_bounds__((WM * WN + PW) * 64) void k_gemm_bf16_nt(const bf16
   }
 }
 
-// ---- the streaming form of the four-wave 256 x 256 tile (pipeline F) -----------------------------------------------
-// bf16 output without bias, K a multiple of 64 with at least IX_STREAM_MIN_KT k-tiles, N a multiple of 8, rows of C
-// 16-byte aligned. A workgroup takes every (gridDim.x / 8)-th tile of its XCD's run of the tile order.
-// Tile sequence of the dense product: position idx of XCD xcd's run of the tile order above.
-struct IxDenseStreamSeq {
-  const bf16_t* A;
-  const bf16_t* W;
-  bf16_t* C;
-  float* parts;
-  long lda, ldw, ldc, parts_ld;
-  int M, N, K, nb_m, nb_n, gm, gn;
-  __device__ __forceinline__ bool locate(unsigned xcd, unsigned idx, IxStreamTile& t) const {
-    int tm, tn;
-    if (!ix_tile_of_run(xcd, idx, nb_m, nb_n, gm, gn, &tm, &tn)) return false;
-    const long m0 = (long)tm * 256, n0 = (long)tn * 256;
-    t.x = A + m0 * lda;
-    t.w = W + n0 * ldw;
-    t.c = C + m0 * ldc + n0;
-    t.part = parts + m0 * parts_ld + tn * 2;
-    t.mv = (int)min(256L, (long)M - m0);
-    t.nv = (int)min(256L, (long)N - n0);
-    return true;
-  }
-};
-
-template <bool PARTS, bool W_ONCE>
-__global__ __launch_bounds__(256) void k_gemm_bf16_nt_stream(const bf16_t* __restrict__ A, long lda,
-                                                             const bf16_t* __restrict__ W, long ldw,
-                                                             bf16_t* __restrict__ C, long ldc, int M, int N, int K,
-                                                             int nb_m, int nb_n, int gm, int gn,
-                                                             float* __restrict__ row_max_parts, long parts_ld) {
-  using Cfg = IxGemmCfg<256, 256, 2, 2, 0, W_ONCE>;
-  extern __shared__ __align__(16) char ix_lds[];
-  IxPlainStreamJob<Cfg, IxDenseStreamSeq, PARTS> job;
-  job.seq.gm = gm;
-  job.seq.gn = gn;
-  job.seq.A = A;
-  job.seq.lda = lda;
-  job.seq.W = W;
-  job.seq.ldw = ldw;
-  job.seq.C = C;
-  job.seq.ldc = ldc;
-  job.seq.M = M;
-  job.seq.N = N;
-  job.seq.K = K;
-  job.seq.nb_m = nb_m;
-  job.seq.nb_n = nb_n;
-  job.seq.parts = row_max_parts;
-  job.seq.parts_ld = parts_ld;
-  ix_gemm_stream4<Cfg>(job, K / IX_BK, ix_lds);
-}
-
+template <bool ONCE>
+using IxStreamSquare = IxGemmCfg<256, 256, 2, 2, 0, ONCE>;
 static bool ix_gemm_stream_fits(const void* C, long ldc, long M, long N, long K, const void* bias, long batch) {
   return !bias && batch == 1 && (K % IX_BK == 0) && K / IX_BK >= IX_STREAM_MIN_KT && (N % 8 == 0) && (ldc % 8 == 0) &&
          ix_aligned(C, 16) && ldc * 512 < 0x40000000L;
 }
 
-// Weights with one reader in the launch (ix_dma16): a single row tile, and more of them than the caches would keep for the
-// next launch anyway.
-static bool ix_gemm_once(long nb_m, long N, long K) { return nb_m == 1 && N * K * 2 >= (64L << 20); }
-
-template <auto KERN, typename... Args>
-static int ix_gemm_stream_start(int lds, hipStream_t st, Args... args) {
-  static bool attr_set = false;  // per kernel
-  if (!attr_set) {
-    if (hipFuncSetAttribute((const void*)KERN, hipFuncAttributeMaxDynamicSharedMemorySize, lds) != hipSuccess)
-      return IX_ERR_LAUNCH;
-    attr_set = true;
-  }
-  hipLaunchKernelGGL(KERN, dim3(IX_STREAM_WORKGROUPS), dim3(256), lds, st, args...);
-  return ix_launch_status();
-}
-
-static int ix_gemm_bf16_stream_launch(const bf16_t* A, long lda, const bf16_t* W, long ldw, bf16_t* C, long ldc, long M,
-                                      long N, long K, float* parts, long parts_ld, hipStream_t st) {
-  using Cfg = IxGemmCfg<256, 256, 2, 2>;
-  const long nb_m = (M + 255) / 256, nb_n = (N + 255) / 256;
-  if (nb_m * nb_n > 0x7fffffffL) return IX_DECLINED;
-  if (parts && parts_ld < nb_n * 2) return IX_ERR_ARG;
-  // Group shape of the tile order: with many row tiles the activations are the operand that streams, and a group
-  // that is wider in weight tiles re-uses each activation tile more often (163840 x 2048 x 12352: 6.40 -> 6.20 ms,
-  // 32768 x 2048 x 151936: 15.7 -> 15.5); with few row tiles the default serves the weights better.
-  const int gm = nb_m >= 64 ? 4 : IX_GEMM_GM, gn = nb_m >= 64 ? 16 : IX_GEMM_GN;
-#define IX_STREAM_GO(PARTS_, ONCE_)                                                                                       \
-  return ix_gemm_stream_start<k_gemm_bf16_nt_stream<PARTS_, ONCE_>>(Cfg::LDS_BYTES, st, A, lda, W, ldw, C, ldc, (int)M, (int)N, \
-                                                                    (int)K, (int)nb_m, (int)nb_n, gm, gn, parts, parts_ld)
-  if (ix_gemm_once(nb_m, N, K)) {
-    if (parts) IX_STREAM_GO(true, true);
-    IX_STREAM_GO(false, true);
-  }
-  if (parts) IX_STREAM_GO(true, false);
-  IX_STREAM_GO(false, false);
-#undef IX_STREAM_GO
-}
-
 template <int BM, int BN, int WM, int WN, typename TC, int PW = 0, bool W_ONCE = false>
 static int ix_gemm_bf16_launch(const bf16_t* A, long lda, const bf16_t* W, long ldw, const bf16_t* bias, TC* C,
                                long ldc, long M, long N, long K, float* parts, long parts_ld, hipStream_t st,
-                               long batch = 1, long batch_a = 0, long batch_w = 0, long batch_c = 0) {
+                               long batch = 1, long batch_a = 0, long batch_w = 0, long batch_c = 0, int part_copies = 1) {
   using Cfg = IxGemmCfg<BM, BN, WM, WN, PW>;
   const long nb_m = (M + BM - 1) / BM, nb_n = (N + BN - 1) / BN;
   const long grid = 8 * ((nb_m * nb_n + 7) / 8);  // 8 XCD runs of the tile order, the longest one sets the count
   if (grid > 0x7fffffffL) return IX_DECLINED;
-  if (parts && parts_ld < nb_n * ix_gemm_parts_per_tile<BM, BN, WM, WN, PW>()) return IX_ERR_ARG;
+  if (parts && parts_ld < nb_n * ix_gemm_parts_per_tile<BM, BN, WM, WN, PW>() * part_copies) return IX_ERR_ARG;
   auto kern = k_gemm_bf16_nt<BM, BN, WM, WN, TC, PW, W_ONCE>;
   static bool attr_set = false;  // per instantiation
   if (!attr_set) {
@@ -329,35 +205,44 @@ static int ix_gemm_bf16_launch(const bf16_t* A, long lda, const bf16_t* W, long 
   if (batch > 65535) return IX_DECLINED;
   hipLaunchKernelGGL(kern, dim3((unsigned)grid, (unsigned)batch), dim3(Cfg::NTT), Cfg::LDS_BYTES, st, A, lda, W, ldw,
                      bias, C, ldc, (int)M, (int)N, (int)K, (int)nb_m, (int)nb_n, vec, parts, parts_ld, batch_a, batch_w,
-                     batch_c);
+                     batch_c, part_copies);
   return ix_launch_status();
 }
 
 // Which tile shape runs (0 = choose). Never changes a bit. The choice minimises a cost model: a CU works through
 // ceil(tiles / 256) tiles -- the two small shapes two at a time -- at `fixed` us plus K/64 k-tiles each, and no shape streams
 // the operands faster than `stream` bytes per us. The figures are a fit to 139 measured shapes (weights 2048 x 4096, 5120 x
-// 2048, 12352 x 2048, 8192 x 8192, 151936 x 2048 and x 4096, 1 to 4000 rows): the shape it picks is within 0.2 % of the
-// fastest of the five in the geometric mean, 6 % at worst. The model before it counted waves of whole workgroups and was
-// 4.9 % off, 80 % at worst. us, before -> after: 8192 x 8192 at 384 rows 135 -> 75, 151936 x 4096 at 384 612 -> 488, 12352 x
-// 2048 at 700 54 -> 42, 5120 x 2048 at 4000 100 -> 81, 2048 x 4096 at 1000 40 -> 31.
-static int ix_gemm_tile_for(long M, long N, long K, int tile) {
+// 2048, 12352 x 2048, 8192 x 8192, 151936 x 2048 and x 4096, 1 to 4000 rows) for the five shapes of whole tiles, and to 190
+// of the same weights (16 to 7300 rows) for the bands (`bands`: the call is one they serve), whose k-tile costs what the L2
+// takes for its operands: 256 CUs pull 10 to 13 TB/s whatever the height. us, without -> with bands: 151936 x 4096 at 192
+// rows 290 -> 262, 257 456 -> 358, 320 469 -> 375, 384 492 -> 434, 513 675 -> 587, 769 927 -> 828; 151936 x 2048 at 513 351 ->
+// 307; 12352 x 2048 at 320 32 -> 26; 5120 x 2048 at 3090 86 -> 58.
+#define IX_TILE_BAND 10  // id IX_TILE_BAND + MI: bands of 32 MI rows
+static int ix_gemm_tile_for(long M, long N, long K, int tile, bool bands) {
   if (tile != 0) return tile;
   // One 128-wide column of tiles (the router's gating product): 128-row tiles once there are enough of them to fill
   // the chip, the small tile below that (2048 x 2048 x 128: 20.7 -> 8.5 us; equal at 16384 rows).
   if (M > 128 && N <= 128) return M >= 16384 ? 2 : 6;
   // us_ktile: a tile with its CU to itself; us_ktile_more: one of several (for id 2 and 6: of a pair that shares the CU)
   struct Shape { int id, bm, bn; double us_ktile, us_ktile_more, fixed, stream; };
-  static const Shape shapes[] = {{4, 256, 256, 0.98, 1.4, 4.4, 4.4e6}, {5, 128, 256, 0.95, 1.1, 7.0, 4.1e6},
+  static const Shape shapes[] = {{4, 256, 256, 0.98, 1.4, 4.4, 4.4e6},
+                                 {IX_TILE_BAND + 7, 224, 256, 1.10, 1.44, 4.4, 5.2e6}, {IX_TILE_BAND + 6, 192, 256, 0.96, 1.27, 4.4, 5.2e6},
+                                 {IX_TILE_BAND + 5, 160, 256, 0.78, 1.06, 4.4, 5.2e6}, {IX_TILE_BAND + 4, 128, 256, 0.62, 0.97, 4.4, 5.2e6},
+                                  {5, 128, 256, 0.95, 1.1, 7.0, 4.1e6},
                                  {2, 128, 128, 0.51, 0.95, 5.3, 4.7e6}, {1, 32, 256, 0.38, 0.42, 3.7, 4.4e6},
                                  {6, 64, 32, 0.20, 0.29, 1.3, 3.7e6}};  // preference on ties: larger tiles first
   const double kt = (double)((K + 63) / 64);
   int best = 4;
   double best_cost = 1e300;
+  // up to 64 rows the 128 x 128 tile with its weights past the caches is the better one (7 rows of 151936 x 4096: 202 us
+  // against a band's 226)
+  const bool banded = bands && M > 64 && K % IX_BK == 0 && K / IX_BK >= IX_BAND_MIN_KT && N % 8 == 0;
   for (const Shape& sh : shapes) {
+    if (sh.id > IX_TILE_BAND && !banded) continue;
     const double tiles = (double)((M + sh.bm - 1) / sh.bm) * (double)((N + sh.bn - 1) / sh.bn);
     const double turns = std::ceil(tiles / 256.0);
     double cost;
-    if (sh.id == 4) {  // one workgroup per CU streams its tiles: 3 us between two of them
+    if (sh.id == 4 || sh.id > IX_TILE_BAND) {  // one workgroup per CU streams its tiles: 3 us between two of them
       cost = sh.fixed + turns * (kt * (turns == 1.0 ? sh.us_ktile : sh.us_ktile_more) + 3.0);
     } else if (sh.id == 2 || sh.id == 6) {
       const double pairs = std::floor(turns / 2.0);
@@ -366,7 +251,7 @@ static int ix_gemm_tile_for(long M, long N, long K, int tile) {
       cost = turns * (sh.fixed + kt * (turns == 1.0 ? sh.us_ktile : sh.us_ktile_more));
     }
     cost = std::max(cost, (double)(N + M) * (double)K * 2.0 / sh.stream);
-    if (cost < best_cost * 0.97) {  // a later (smaller) shape must win by a margin
+    if (cost < best_cost * (sh.id > IX_TILE_BAND ? 0.99 : 0.97)) {  // a later (smaller) shape must win by a margin
       best_cost = cost;
       best = sh.id;
     }
@@ -376,9 +261,10 @@ static int ix_gemm_tile_for(long M, long N, long K, int tile) {
 
 // Row-max parts per row of C: one per column tile of the shape that runs.
 extern "C" long ix_gemm_bf16_n_tiles(long M, long N, long K, int tile) {
-  const int t = ix_gemm_tile_for(M, N, K, tile);
+  const int t = ix_gemm_tile_for(M, N, K, tile, true);
   const long bn = (t == 2) ? 128 : (t == 6) ? 32 : 256;  // ids 1, 3, 4, 5, 7, 8 are 256 wide
-  const long per_tile = (t == 4 || t == 7 || t == 8) ? 2 : 1;      // the four-wave tile writes one part per wave column
+  // the four-wave tiles write one part per wave column
+  const long per_tile = t > IX_TILE_BAND ? 4 : ((t == 4 || t == 7 || t == 8) ? 2 : 1);
   return N <= 0 ? 0 : per_tile * ((N + bn - 1) / bn);
 }
 
@@ -388,7 +274,10 @@ static int ix_gemm_bf16_dispatch(const bf16_t* a, long lda, const bf16_t* w, lon
                                  hipStream_t st, long batch = 1, long sa = 0, long sw = 0, long sc = 0) {
   // `tile` only picks which workgroup owns an element (0 = by M); the bits do not depend on it.
 #define IX_BATCH_ARGS , batch, sa, sw, sc
-  switch (ix_gemm_tile_for(M * (batch > 1 ? batch : 1), N, K, tile)) {
+  const bool bands_fit = sizeof(TC) == 2 && ix_gemm_stream_fits(c, ldc, M, N, K, b, batch) && K / IX_BK >= IX_BAND_MIN_KT;
+  // with row-max parts the choice has to be the one ix_gemm_bf16_n_tiles made from the sizes alone
+  const int id = ix_gemm_tile_for(M * (batch > 1 ? batch : 1), N, K, tile, parts || bands_fit);
+  switch (id) {
     case 1: return ix_gemm_bf16_launch<32, 256, 1, 4, TC, 4>(a, lda, w, ldw, b, c, ldc, M, N, K, parts, parts_ld, st IX_BATCH_ARGS);
     case 2:
       if (batch == 1 && ix_gemm_once((M + 127) / 128, N, K))
@@ -399,7 +288,7 @@ static int ix_gemm_bf16_dispatch(const bf16_t* a, long lda, const bf16_t* w, lon
       if constexpr (sizeof(TC) == 2) {
         // with one tile per workgroup too (12352 x 2048 at 700 rows 53 -> 42 us, 8192 x 8192 at 1100 157 -> 145)
         if (ix_gemm_stream_fits(c, ldc, M, N, K, b, batch))
-          return ix_gemm_bf16_stream_launch(a, lda, w, ldw, (bf16_t*)c, ldc, M, N, K, parts, parts_ld, st);
+          return ix_gemm_bf16_stream_launch<IxStreamSquare>(a, lda, w, ldw, (bf16_t*)c, ldc, M, N, K, parts, parts_ld, st);
       }
       [[fallthrough]];
     case 7:  // the same tile, one tile per workgroup
@@ -409,9 +298,20 @@ static int ix_gemm_bf16_dispatch(const bf16_t* a, long lda, const bf16_t* w, lon
     case 8:  // the streaming form whatever the number of tiles (declines what it does not serve)
       if constexpr (sizeof(TC) == 2) {
         if (ix_gemm_stream_fits(c, ldc, M, N, K, b, batch))
-          return ix_gemm_bf16_stream_launch(a, lda, w, ldw, (bf16_t*)c, ldc, M, N, K, parts, parts_ld, st);
+          return ix_gemm_bf16_stream_launch<IxStreamSquare>(a, lda, w, ldw, (bf16_t*)c, ldc, M, N, K, parts, parts_ld, st);
       }
       return IX_DECLINED;
+    case IX_TILE_BAND + 4:  // bands of 128, 160, 192, 224 rows (decline what the streaming form does not serve)
+    case IX_TILE_BAND + 5:
+    case IX_TILE_BAND + 6:
+    case IX_TILE_BAND + 7:
+      if constexpr (sizeof(TC) == 2) {
+        if (bands_fit) return ix_gemm_bf16_bands_launch(id - IX_TILE_BAND, a, lda, w, ldw, (bf16_t*)c, ldc, M, N, K, parts, parts_ld, st);
+      }
+      if (tile != 0) return IX_DECLINED;
+      // chosen by size for a call with a bias, an fp32 result or unaligned rows: the 256-row tile, and every row-max part
+      // stored twice (the caller was told a band's four parts per tile)
+      return ix_gemm_bf16_launch<256, 256, 2, 2, TC>(a, lda, w, ldw, b, c, ldc, M, N, K, parts, parts_ld, st IX_BATCH_ARGS, 2);
     default: return IX_ERR_ARG;
   }
 #undef IX_BATCH_ARGS

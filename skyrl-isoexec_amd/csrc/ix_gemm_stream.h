@@ -263,7 +263,7 @@ struct IxStreamTile {
   const bf16_t* x;  // first activation row of the tile
   const bf16_t* w;  // first weight row
   bf16_t* c;        // the tile's first output element
-  float* part;      // the tile's first row-max part (two per token: one per wave column)
+  float* part;      // the tile's first row-max part (one per token and wave column)
   int mv, nv;       // rows and columns that exist
 };
 
@@ -277,7 +277,8 @@ struct IxPlainStreamJob {
   ix_rsrc_t p_cr, p_pr;      // pending tile: descriptors of its part of C and of the row-max parts
   uint32_t p_voff, p_pvoff;  // this lane's first output element / part in them
   int p_cols;                // columns left from there
-  uint32_t pend[4][4][8];    // the pending tile's outputs, two bf16 per register, accumulator layout
+  static constexpr int MI = Cfg::MI, NI = Cfg::NI, NL = NI / 2;
+  uint32_t pend[MI][NI][8];  // the pending tile's outputs, two bf16 per register, accumulator layout
   uint32_t ta[4][4], tb[4][4];  // [slot][dword] after exchange stage 1 / 2
   float rmax;
 
@@ -299,7 +300,7 @@ struct IxPlainStreamJob {
     p_cols = 0;
     rmax = IX_NEG_INF;
 #pragma unroll
-    for (int i = 0; i < 128; ++i) pend[i >> 5][(i >> 3) & 3][i & 7] = 0u;
+    for (int i = 0; i < MI * NI * 8; ++i) pend[i / (NI * 8)][(i >> 3) % NI][i & 7] = 0u;
     return has_next;
   }
   __device__ __forceinline__ void open_next() {
@@ -322,7 +323,8 @@ struct IxPlainStreamJob {
   template <int J>
   __device__ __forceinline__ uint32_t x_voff() {
     const uint32_t v = xv;
-    asm volatile("v_add_u32 %0, %1, %0" : "+v"(xv) : "s"(J == 7 ? -7 * x_step : x_step));
+    constexpr int LAST = Cfg::X_CH - 1;
+    asm volatile("v_add_u32 %0, %1, %0" : "+v"(xv) : "s"(J == LAST ? -LAST * x_step : x_step));
     return v;
   }
   template <int J>
@@ -332,14 +334,16 @@ struct IxPlainStreamJob {
     return v;
   }
   __device__ __forceinline__ void turn_offsets() const {}  // tile-local descriptors: the offsets never change
-  static constexpr int DMA_IDLE = 0;  // every scalar operand of the loads comes from scalar arithmetic
+  // 0: every scalar operand of the loads comes from scalar arithmetic. With one row of waves and six activation chunks or
+  // more the compiler keeps some of them in lanes of a vector register.
+  static constexpr int DMA_IDLE = Cfg::WM == 1 && Cfg::MI >= 6 ? 3 : 0;
   static constexpr int NSK = IX_STREAM_NSK;
   // (rows sit at the same offsets in every tile: the descriptors carry the tile)
   __device__ __forceinline__ void advance() { cur = nx; }
   template <typename Acc>
   __device__ __forceinline__ void drain(Acc& acc) {
-    ix_static_for<0, 16>([&](auto bc) {
-      constexpr int mi = decltype(bc)::value >> 2, ni = decltype(bc)::value & 3;
+    ix_static_for<0, MI * NI>([&](auto bc) {
+      constexpr int mi = decltype(bc)::value / NI, ni = decltype(bc)::value % NI;
       float a16[16];
       ix_acc_read16<true>(acc[mi][ni], a16);
 #pragma unroll
@@ -347,28 +351,29 @@ struct IxPlainStreamJob {
       __builtin_amdgcn_sched_barrier(0);  // or every read is scheduled ahead of the first pack: 256 registers in flight
     });
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int wm = wave >> 1, wn = wave & 1;
+    const int wm = wave / Cfg::WN, wn = wave % Cfg::WN;
     // after the quad transposes a lane holds piece (lane % 4) of the four tokens of its quad
-    const int r = wm * 128 + (lane & 28), c = wn * 128 + 32 * (lane >> 5) + 8 * (lane & 3);
+    const int r = wm * Cfg::TM + (lane & 28), c = wn * Cfg::TN + 32 * (lane >> 5) + 8 * (lane & 3);
     // Tile-local descriptor of C: rows past the tile's last fall outside its range and are dropped by the hardware;
     // columns past the matrix are sent out of range by hand (p_cols).
     p_cr = ix_make_rsrc(cur.c, (uint32_t)(((long)(cur.mv - 1) * seq.ldc + cur.nv) * 2));
     p_voff = (uint32_t)(((long)r * seq.ldc + c) * 2);
     p_cols = cur.nv - c;
     if constexpr (PARTS) {
-      p_pr = ix_make_rsrc(cur.part, (uint32_t)(((long)(cur.mv - 1) * seq.parts_ld + 2) * 4));
-      p_pvoff = (lane < 32) ? (uint32_t)(((long)(wm * 128 + lane) * seq.parts_ld + wn) * 4) : IX_OOB;
+      p_pr = ix_make_rsrc(cur.part, cur.part ? (uint32_t)(((long)(cur.mv - 1) * seq.parts_ld + Cfg::WN) * 4) : 0u);
+      p_pvoff = (lane < 32) ? (uint32_t)(((long)(wm * Cfg::TM + lane) * seq.parts_ld + wn) * 4) : IX_OOB;
     }
   }
-  // k-tile s of the next tile carries the blocks (mi = s / 2, ni = 2 L and 2 L + 1, L = s % 2): 64 columns of 32 tokens
-  // per wave. Slots 0..7 the row maximum, 8..23 and 24..39 the two exchange stages of the quad transposes, 40..43 the
+  // Group s of 64 micro-steps (k-tile s of the next tile in the 256-row form) carries the blocks (mi = s / NL, ni = 2 L and
+  // 2 L + 1, L = s % NL): 64 columns of 32 tokens per wave. Slots 0..7 the row maximum, 8..23 and 24..39 the two exchange stages of the quad transposes, 40..43 the
   // four stores (a 128-byte line per token), 44 the maximum's store.
   static constexpr int stores_after_p1(int s) { return 4 + ((PARTS && (s & 1)) ? 1 : 0); }
+  static constexpr bool is_store(int i) { return (i % 64 >= 40 && i % 64 < 44) || (PARTS && (i / 64) % NL == NL - 1 && i % 64 == 44); }
   static __device__ __forceinline__ int w_frag_row(int ni, int rho) { return ix_stream_col(ni, rho); }
   template <int I>
   __device__ __forceinline__ void micro() {
     constexpr int s = I / 64, q = I % 64;
-    constexpr int mi = s >> 1, L = s & 1;
+    constexpr int mi = s / NL, L = s % NL;
     if constexpr (PARTS && q < 8) {
       // rounding is monotonic: the maximum of the rounded values is the rounded maximum
       if constexpr (q == 0 && L == 0) rmax = IX_NEG_INF;
@@ -390,7 +395,7 @@ struct IxPlainStreamJob {
       const uint32_t off =
           (64 * L < p_cols) ? p_voff + (uint32_t)(((long)(mi * 32 + t) * seq.ldc + 64 * L) * 2) : IX_OOB;
       ix_buffer_store16<IX_STREAM_STORE_NT_PLAIN>(make_uint4(tb[t][0], tb[t][1], tb[t][2], tb[t][3]), p_cr, off);
-    } else if constexpr (PARTS && L == 1 && q == 44) {
+    } else if constexpr (PARTS && L == NL - 1 && q == 44) {
       const float v = fmaxf(rmax, __shfl_xor(rmax, 32, IX_WAVE));
       ix_buffer_store4(__float_as_uint(v), p_pr,
                        p_pvoff == IX_OOB ? IX_OOB : p_pvoff + (uint32_t)((long)(mi * 32) * seq.parts_ld * 4));

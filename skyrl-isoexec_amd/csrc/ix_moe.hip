@@ -15,7 +15,7 @@
 // map are integer-only and only decide which workgroup computes a row; the GEMM core's K order
 // is fixed (ix_gemm_core.h).
 #include "ix_gemm_core.h"
-#include "ix_gemm_stream.h"
+#include "ix_moe_bands.h"
 #include "../../include/isoexec_hip.h"
 
 #define IX_MOE_KMAX 16
@@ -706,6 +706,35 @@ extern "C" int ix_moe_pick_bm_packed(long T, long k, long E) {
   return rows >= 40 * e ? ix_moe_pick_bm(T, k, E) : (rows >= 16 * e ? 64 : 32);
 }
 
+// The same with the layer's sizes at hand: bands of 96 .. 224 rows (ix_moe_bands.h) from 24 rows per expert on (with or without
+// packed matrices), as long as the mean fits a band, or two, better than 256 rows. us fc1 + fc2 (E = 128, Hd = 2048, F = 768,
+// top-8; even / skewed routing with four experts far more popular):
+//   rows per expert    before     256          96          160         192         224
+//     32            222 / -   253 / 283   207 / 232   207 / 242   209 / 251   223 / 263
+//     62            253 / -   248 / 289   222 / 256   225 / 261   228 / 268   238 / 278
+//     94               -      259 / 304   288 / 272   239 / 273   243 / 280   249 / 293
+//    125               -      270 / 319   296 / 287   247 / 318   252 / 306   259 / 305
+//    156               -      276 / 337   310 / 322   295 / 308   260 / 336   271 / 327
+//    188               -      285 / 369   362 / 371   363 / 325   335 / 337   323 / 359
+//    256               -      400 / 397   436 / 445   383 / 385   413 / 373   446 / 387
+//    312               -      488 / 429   512 / 505   446 / 474   433 / 425   468 / 417
+//    375               -      506 / 481   588 / 597   535 / 555   524 / 541   480 / 475
+//    438               -      551 / 564   662 / 664   581 / 589   607 / 634   579 / 608
+// (before: ring tiles of 128 x 128, or the packed streams). One tile per expert while mean + 3 sqrt(mean) rows fit it, then two
+// of half the height; in between, and from 400 rows on, 256.
+extern "C" int ix_moe_pick_bm_shape(long T, long k, long E, long Hd, long F, int packed) {
+  const long rows = T * k, e = E > 0 ? E : 1, mean = rows / e;
+  if (mean >= 24 && mean < 400 && ix_moe_bands_fit(rows, Hd, F) && e * (F / 128) >= 2 * IX_STREAM_WORKGROUPS) {
+    if (mean < 72) return 96;
+    if (mean < 130) return 160;
+    if (mean < 164) return 192;
+    if (mean < 240) return 256;
+    if (mean < 280) return 160;
+    return mean < 340 ? 192 : 224;
+  }
+  return packed ? ix_moe_pick_bm_packed(T, k, E) : ix_moe_pick_bm(T, k, E);
+}
+
 extern "C" int ix_moe_permute(const int* topk_idx, const float* topk_prob, long T, long E, long k, long BM,
                               int* counts, int* offsets, int* sorted_token, float* permuted_prob,
                               int* combine_rows, int* tile_meta, long max_tiles, int* scratch, void* stream) {
@@ -810,23 +839,6 @@ extern "C" int ix_moe_permute_static(const int* topk_idx, const float* topk_prob
 // Grouped GEMMs over the block map. A workgroup past the device-side tile count exits at once,
 // so the host never reads the routing back.
 //
-// Workgroup -> tile: hardware hands consecutive workgroup ids to the 8 XCDs round-robin and each XCD has its own
-// L2, so the tile order (row tile major, column tile minor: an expert's tiles are adjacent) is cut into 8 equal
-// runs, one per XCD. The ~32 tiles an XCD works on at a time then belong to one or two experts: an expert's
-// weights and a row tile's activations go through one L2 once, instead of through all eight.
-__device__ __forceinline__ bool ix_moe_tile_of_block(unsigned bid, int n_row_tiles, int nb_n, int* mt, int* nt) {
-  const unsigned xcd = bid & 7u;
-  const unsigned idx = bid >> 3;
-  const unsigned tiles = (unsigned)n_row_tiles * (unsigned)nb_n;  // < 2^31: the launch checks the bound
-  const unsigned q = tiles >> 3, r = tiles & 7u;
-  const unsigned lo = q * xcd + ((r * xcd) >> 3), hi = q * (xcd + 1) + ((r * (xcd + 1)) >> 3);
-  const unsigned l = lo + idx;
-  if (l >= hi) return false;
-  *mt = (int)(l / (unsigned)nb_n);
-  *nt = (int)(l - (unsigned)*mt * (unsigned)nb_n);
-  return true;
-}
-
 template <int BM, int BN, int WM, int WN>
 __global__ __launch_bounds__(WM* WN * 64) void k_moe_fc1_glu(const bf16_t* __restrict__ x, long ldx, int T,
                                                              const int* __restrict__ sorted_token,
@@ -1017,52 +1029,6 @@ __global__ __launch_bounds__(WM* WN * 64) void k_moe_fc2(const bf16_t* __restric
       }
     });
   });
-}
-
-// ---- streaming form of the second expert GEMM (pipeline F): the four-wave 256 x 256 tile, Hd a multiple of 256, F a
-// multiple of 64 with at least IX_STREAM_MIN_KT k-tiles. A workgroup takes every (gridDim.x / 8)-th tile of its XCD's run
-// of the (row tile, column tile) order of ix_moe_tile_of_block.
-struct IxMoeFc2Seq {
-  const bf16_t* inter;
-  const bf16_t* W2;
-  bf16_t* out;
-  const int* meta;
-  int max_tiles, Hd, nb_n, K;  // K = F
-  long lda, ldw, ldc, parts_ld;  // F, F, Hd, unused
-  __device__ __forceinline__ bool locate(unsigned xcd, unsigned idx, IxStreamTile& t) const {
-    int mt, nt;
-    if (!ix_moe_tile_of_block(xcd + 8u * idx, meta[0], nb_n, &mt, &nt)) return false;
-    const long e = meta[1 + mt], row0 = meta[1 + max_tiles + mt];
-    t.x = inter + row0 * K;
-    t.w = W2 + (e * Hd + (long)nt * 256) * K;
-    t.c = out + row0 * Hd + (long)nt * 256;
-    t.part = nullptr;
-    t.mv = meta[1 + 2 * max_tiles + mt];
-    t.nv = 256;
-    return true;
-  }
-};
-
-template <bool W_ONCE>
-__global__ __launch_bounds__(256) void k_moe_fc2_stream(const bf16_t* __restrict__ inter, const bf16_t* __restrict__ W2,
-                                                        const int* __restrict__ meta, int max_tiles,
-                                                        bf16_t* __restrict__ out, int Hd, int F, int nb_n) {
-  using Cfg = IxGemmCfg<256, 256, 2, 2, 0, W_ONCE>;
-  extern __shared__ __align__(16) char ix_lds[];
-  IxPlainStreamJob<Cfg, IxMoeFc2Seq, false> job;
-  job.seq.inter = inter;
-  job.seq.W2 = W2;
-  job.seq.out = out;
-  job.seq.meta = meta;
-  job.seq.max_tiles = max_tiles;
-  job.seq.Hd = Hd;
-  job.seq.nb_n = nb_n;
-  job.seq.K = F;
-  job.seq.lda = F;
-  job.seq.ldw = F;
-  job.seq.ldc = Hd;
-  job.seq.parts_ld = 0;
-  ix_gemm_stream4<Cfg>(job, F / IX_BK, ix_lds);
 }
 
 // ---- streaming form of the first expert GEMM (pipeline F) ------------------------------------------------------------
@@ -1342,6 +1308,7 @@ static int ix_moe_experts_launch(const bf16_t* x, long ldx, int T, long rows, co
                                  const bf16_t* W1, const bf16_t* W2, const int* meta, long max_tiles,
                                  bf16_t* inter, bf16_t* out, int Hd, int F, hipStream_t st) {
   using Cfg = IxGemmCfg<BM, BN, WM, WN>;
+  using CfgOnce = IxGemmCfg<BM, BN, WM, WN, 0, true>;
   auto k1 = k_moe_fc1_glu<BM, BN, WM, WN>;
   auto k2 = k_moe_fc2<BM, BN, WM, WN>;
   static bool attr_set = false;
@@ -1391,14 +1358,14 @@ static int ix_moe_experts_launch(const bf16_t* x, long ldx, int T, long rows, co
         max_tiles * nb2 >= 2 * IX_STREAM_WORKGROUPS) {
       static bool attr2_set = false;
       if (!attr2_set) {
-        if (hipFuncSetAttribute((const void*)k_moe_fc2_stream<false>, hipFuncAttributeMaxDynamicSharedMemorySize,
+        if (hipFuncSetAttribute((const void*)k_moe_fc2_stream<Cfg>, hipFuncAttributeMaxDynamicSharedMemorySize,
                                 Cfg::LDS_BYTES) != hipSuccess ||
-            hipFuncSetAttribute((const void*)k_moe_fc2_stream<true>, hipFuncAttributeMaxDynamicSharedMemorySize,
+            hipFuncSetAttribute((const void*)k_moe_fc2_stream<CfgOnce>, hipFuncAttributeMaxDynamicSharedMemorySize,
                                 Cfg::LDS_BYTES) != hipSuccess)
           return IX_ERR_LAUNCH;
         attr2_set = true;
       }
-      hipLaunchKernelGGL(once ? k_moe_fc2_stream<true> : k_moe_fc2_stream<false>, dim3(IX_STREAM_WORKGROUPS), dim3(256), Cfg::LDS_BYTES, st, inter, W2, meta,
+      hipLaunchKernelGGL(once ? k_moe_fc2_stream<CfgOnce> : k_moe_fc2_stream<Cfg>, dim3(IX_STREAM_WORKGROUPS), dim3(256), Cfg::LDS_BYTES, st, inter, W2, meta,
                          (int)max_tiles, out, Hd, F, (int)nb2);
       return ix_launch_status();
     }
@@ -1428,6 +1395,14 @@ extern "C" int ix_moe_experts_tile(const void* x, long ldx, const int* sorted_to
   if (BN == 128)
     return ix_moe_experts_launch<128, 128, 2, 2>(xx, ldx, (int)T, rows, sorted_token, permuted_prob, w1, w2, tile_meta,
                                                  max_tiles, it, eo, (int)Hd, (int)F, st);
+  if (BM == 96 || BM == 160 || BM == 192 || BM == 224) {
+    if (ix_moe_bands_fit(rows, Hd, F) && ix_aligned(expert_out, 16)) {
+      auto bands = BM < 192 ? ix_moe_experts_bands_low : ix_moe_experts_bands_high;
+      return bands((int)BM, xx, ldx, (int)T, rows, sorted_token, permuted_prob, w1, w2, tile_meta, max_tiles, it, eo, (int)Hd,
+                   (int)F, st);
+    }
+    BM = 256;  // a taller tile holds the map's rows as well
+  }
   switch (BM) {
     case 32:
       return ix_moe_experts_launch<32, 256, 1, 4>(xx, ldx, (int)T, rows, sorted_token, permuted_prob, w1, w2, tile_meta,

@@ -108,6 +108,7 @@ SIGNATURES = {
     "ix_moe_max_tiles": (c_long, [c_long, c_long, c_long, c_long]),
     "ix_moe_permute_scratch_ints": (c_size_t, [c_long, c_long]),
     "ix_moe_pick_bm": (c_int, [c_long, c_long, c_long]),
+    "ix_moe_pick_bm_shape": (c_int, [c_long, c_long, c_long, c_long, c_long, c_int]),
     "ix_moe_permute": (
         c_int,
         [P, P, c_long, c_long, c_long, c_long, P, P, P, P, P, P, c_long, P, P],

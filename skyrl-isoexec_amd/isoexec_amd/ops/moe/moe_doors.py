@@ -92,7 +92,7 @@ def _batched_experts_forward(self, permuted_local_hidden_states, tokens_per_expe
         if total != R or counts.numel() != E:
             raise RuntimeError(f"[isoexec-amd] SequentialMLP.forward: tokens_per_expert has {counts.numel()} entries "
                                f"adding up to {total} for {R} permuted rows and {E} local experts")
-    BM = int(L.ix_moe_pick_bm(R, 1, E))
+    BM = int(L.ix_moe_pick_bm_shape(R, 1, E, H, F, 0))
     max_tiles = int(L.ix_moe_max_tiles(R, 1, E, BM))
     meta = torch.empty(1 + 3 * max_tiles, dtype=torch.int32, device=dev)
     stream = _lib.current_stream(dev)

@@ -252,8 +252,12 @@ def moe_ffn_forward(x: torch.Tensor, router_weight: torch.Tensor, w1: torch.Tens
         raise RuntimeError("[isoexec-amd] router GEMM declined")
     if logit_bias is not None:
         logits = logits + logit_bias  # elementwise, per token
-    if BM is None and packed is not None:
-        BM = int(_lib.lib().ix_moe_pick_bm_packed(logits.shape[0], k, logits.shape[1]))
+    if BM is None:
+        L, (T, E) = _lib.lib(), logits.shape
+        if w2.ndim == 3 and w1.is_contiguous() and w2.is_contiguous():  # the bands read the matrices themselves
+            BM = int(L.ix_moe_pick_bm_shape(T, k, E, w2.shape[1], w2.shape[2], int(packed is not None)))
+        elif packed is not None:
+            BM = int(L.ix_moe_pick_bm_packed(T, k, E))
     idx, prob, p = route_and_permute(logits, k, pre_softmax=pre_softmax, scaling_factor=scaling_factor, BM=BM)
     if routing_out is not None:
         routing_out.append(idx)

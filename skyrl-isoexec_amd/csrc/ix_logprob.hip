@@ -380,7 +380,9 @@ __global__ __launch_bounds__(256) void k_lp_backward(const T* __restrict__ x, lo
   }
 }
 
-// rowmax[row] = max over P parts (exact; any order). One wave per row.
+// rowmax[row] = max over P parts (exact; any order). One wave per row, or (many parts) one workgroup per row with all its
+// loads in flight: a wave walks 2376 parts one dependent load after the other (513 rows of 2376 parts 19.7 -> 5.3 us).
+#define IX_LP_MANY_PARTS 512
 __global__ __launch_bounds__(256) void k_lp_reduce_parts(const float* __restrict__ parts, long parts_ld, int P,
                                                          long rows, float* __restrict__ rowmax) {
   const long row = (long)blockIdx.x * 4 + (threadIdx.x >> 6);
@@ -389,9 +391,34 @@ __global__ __launch_bounds__(256) void k_lp_reduce_parts(const float* __restrict
   if ((threadIdx.x & 63) == 0) rowmax[row] = m;
 }
 
+__global__ __launch_bounds__(256) void k_lp_reduce_many_parts(const float* __restrict__ parts, long parts_ld, int P,
+                                                              float* __restrict__ rowmax) {
+  __shared__ float s_w[4];
+  const long row = blockIdx.x;
+  const float* pr = parts + row * parts_ld;
+  float m = IX_NEG_INF;
+  for (int i0 = threadIdx.x; i0 < P; i0 += 256 * 8) {
+    float v[8];
+#pragma unroll
+    for (int c = 0; c < 8; ++c) v[c] = pr[min(i0 + c * 256, P - 1)];
+#pragma unroll
+    for (int c = 0; c < 8; ++c) m = fmaxf(m, v[c]);
+  }
+  m = ix_lane_max<64>(m);
+  if ((threadIdx.x & 63) == 0) s_w[threadIdx.x >> 6] = m;
+  __syncthreads();
+  if (threadIdx.x == 0) rowmax[row] = fmaxf(fmaxf(s_w[0], s_w[1]), fmaxf(s_w[2], s_w[3]));
+}
+
 extern "C" int ix_rowmax_reduce(const float* parts, long parts_ld, long P, long rows, float* rowmax, void* stream) {
   if (!parts || !rowmax || rows < 0 || P <= 0 || parts_ld < P || P > 0x7fffffffL) return IX_ERR_ARG;
   if (rows == 0) return IX_OK;
+  if (P >= IX_LP_MANY_PARTS) {
+    if (rows > 0x7fffffffL) return IX_DECLINED;
+    hipLaunchKernelGGL(k_lp_reduce_many_parts, dim3((unsigned)rows), dim3(256), 0, (hipStream_t)stream, parts, parts_ld, (int)P,
+                       rowmax);
+    return ix_launch_status();
+  }
   const long grid = (rows + 3) / 4;
   if (grid > 0x7fffffffL) return IX_DECLINED;
   hipLaunchKernelGGL(k_lp_reduce_parts, dim3((unsigned)grid), dim3(256), 0, (hipStream_t)stream, parts, parts_ld,

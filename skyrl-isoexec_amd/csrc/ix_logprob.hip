@@ -413,8 +413,7 @@ __global__ __launch_bounds__(256) void k_lp_reduce_many_parts(const float* __res
 extern "C" int ix_rowmax_reduce(const float* parts, long parts_ld, long P, long rows, float* rowmax, void* stream) {
   if (!parts || !rowmax || rows < 0 || P <= 0 || parts_ld < P || P > 0x7fffffffL) return IX_ERR_ARG;
   if (rows == 0) return IX_OK;
-  if (P >= IX_LP_MANY_PARTS) {
-    if (rows > 0x7fffffffL) return IX_DECLINED;
+  if (P >= IX_LP_MANY_PARTS && P <= 0x40000000L && rows <= 0x7fffffffL) {  // the walk's index runs up to 2047 past P
     hipLaunchKernelGGL(k_lp_reduce_many_parts, dim3((unsigned)rows), dim3(256), 0, (hipStream_t)stream, parts, parts_ld, (int)P,
                        rowmax);
     return ix_launch_status();

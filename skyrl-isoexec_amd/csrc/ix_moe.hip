@@ -1812,8 +1812,53 @@ extern "C" int ix_moe_experts_decode(const void* x, long ldx, const int* sorted_
 }
 
 // ---------------------------------------------------------------------------------------------
-// KC > 0: k known at compile time -- the k row numbers and the k rows are requested before the first add, so a thread has
-// k loads in flight instead of one (the sum is the same left-to-right sum). KC = 0: any k.
+// A wave sums 512 columns of one token's KC rows (whole 16-byte groups only). The token is uniform in a wave, so its row
+// numbers and row addresses are scalar work, and the bf16 form's roundings go through the hardware's pack-convert: it keeps
+// a NaN's payload where ix_rbf makes 0x7fc0, but a NaN stays one through the later adds and the store makes it canonical.
+// The thread-per-group form below is bound by its own vector instructions instead (a 64-bit division and an integer rounding
+// per element and row). us at k = 8 of 2048 columns, 4096
+// tokens: 41 -> 28 (5.4 TB/s).
+template <int KC, bool FP32>
+__global__ __launch_bounds__(256) void k_moe_combine_rows(const bf16_t* __restrict__ expert_out,
+                                                          const int* __restrict__ combine_rows, bf16_t* __restrict__ out,
+                                                          unsigned waves, unsigned chunks, int Hd) {
+  const unsigned wave = (unsigned)__builtin_amdgcn_readfirstlane((int)(blockIdx.x * 4 + (threadIdx.x >> 6)));
+  if (wave >= waves) return;
+  const unsigned t = wave / chunks, chunk = wave - t * chunks;
+  const int c0 = (int)chunk * 512 + (int)(threadIdx.x & 63) * 8;
+  if (c0 >= Hd) return;
+  const int* rows = combine_rows + (size_t)t * KC;
+  uint4 e[KC];
+#pragma unroll
+  for (int r = 0; r < KC; ++r) e[r] = *reinterpret_cast<const uint4*>(expert_out + (long)rows[r] * Hd + c0);
+  float sum[8];
+  ix_unpack8(e[0], sum);
+#pragma unroll
+  for (int r = 1; r < KC; ++r) {
+    float x[8];
+    ix_unpack8(e[r], x);
+#pragma unroll
+    for (int i = 0; i < 8; i += 2) {
+      const float s0 = sum[i] + x[i], s1 = sum[i + 1] + x[i + 1];
+      if constexpr (FP32) {
+        sum[i] = s0;
+        sum[i + 1] = s1;
+      } else {
+        ix_rbf2_hw(s0, s1, sum[i], sum[i + 1]);
+      }
+    }
+  }
+  uint4 o;
+  o.x = ix_pack_bf2_canon_hw(sum[0], sum[1]);
+  o.y = ix_pack_bf2_canon_hw(sum[2], sum[3]);
+  o.z = ix_pack_bf2_canon_hw(sum[4], sum[5]);
+  o.w = ix_pack_bf2_canon_hw(sum[6], sum[7]);
+  *reinterpret_cast<uint4*>(out + (size_t)t * Hd + c0) = o;
+}
+
+// Any width and alignment, a thread per 8 columns. KC > 0: k known at compile time -- the k row numbers and the k rows are
+// requested before the first add, so a thread has k loads in flight instead of one (the sum is the same left-to-right sum).
+// KC = 0: any k.
 template <int KC>
 __global__ __launch_bounds__(256) void k_moe_combine(const bf16_t* __restrict__ expert_out,
                                                      const int* __restrict__ combine_rows,
@@ -1870,6 +1915,18 @@ extern "C" int ix_moe_combine(const void* expert_out, const int* combine_rows, v
   const long grid = (T * groups + 255) / 256;
   if (grid > 0x7fffffffL) return IX_DECLINED;
   const int vec = (Hd % 8 == 0) && ix_aligned(expert_out, 16) && ix_aligned(out, 16);
+  const long chunks = (Hd + 511) / 512;
+  if (vec && T * chunks <= 0x7fffffffL && (k == 2 || k == 4 || k == 8)) {
+#define IX_COMBINE_ROWS(KC_, F_)                                                                                       \
+  hipLaunchKernelGGL((k_moe_combine_rows<KC_, F_>), dim3((unsigned)((T * chunks + 3) / 4)), dim3(256), 0,              \
+                     (hipStream_t)stream, (const bf16_t*)expert_out, combine_rows, (bf16_t*)out, (unsigned)(T * chunks), \
+                     (unsigned)chunks, (int)Hd)
+    if (k == 2) { if (fp32_acc) IX_COMBINE_ROWS(2, true); else IX_COMBINE_ROWS(2, false); }
+    if (k == 4) { if (fp32_acc) IX_COMBINE_ROWS(4, true); else IX_COMBINE_ROWS(4, false); }
+    if (k == 8) { if (fp32_acc) IX_COMBINE_ROWS(8, true); else IX_COMBINE_ROWS(8, false); }
+#undef IX_COMBINE_ROWS
+    return ix_launch_status();
+  }
 #define IX_COMBINE(KC_)                                                                                        \
   hipLaunchKernelGGL(k_moe_combine<KC_>, dim3((unsigned)grid), dim3(256), 0, (hipStream_t)stream,             \
                      (const bf16_t*)expert_out, combine_rows, (bf16_t*)out, T, (int)Hd, (int)k, fp32_acc, vec)

@@ -1816,8 +1816,7 @@ extern "C" int ix_moe_experts_decode(const void* x, long ldx, const int* sorted_
 // numbers and row addresses are scalar work, and the bf16 form's roundings go through the hardware's pack-convert: it keeps
 // a NaN's payload where ix_rbf makes 0x7fc0, but a NaN stays one through the later adds and the store makes it canonical.
 // The thread-per-group form below is bound by its own vector instructions instead (a 64-bit division and an integer rounding
-// per element and row). us at k = 8 of 2048 columns, 4096
-// tokens: 41 -> 28 (5.4 TB/s).
+// per element and row): 4096 tokens of 8 rows of 2048 columns 41 -> 28 us (5.4 TB/s).
 template <int KC, bool FP32>
 __global__ __launch_bounds__(256) void k_moe_combine_rows(const bf16_t* __restrict__ expert_out,
                                                           const int* __restrict__ combine_rows, bf16_t* __restrict__ out,

@@ -182,10 +182,12 @@ def experts_forward(x: torch.Tensor, w1: torch.Tensor, w2: torch.Tensor, p: Perm
     inter = torch.empty(rows, F, dtype=torch.bfloat16, device=dev)
     out = torch.empty(rows, H, dtype=torch.bfloat16, device=dev)
     xc = x if x.stride(1) == 1 else x.contiguous()
-    if packed is not None and p.BM in (32, 64) and p.BN == 256:
+    streams = p.BM in (32, 64) and p.BN == 256
+    if packed is not None and (streams or (p.BM == 96 and rows < 40 * E)):  # 96: bands serve some of the sizes that stream
         w1f, w2f = packed
         if w1f.shape != shape1 or w2f.shape != w2.shape or w1f.dtype is not torch.bfloat16 or w2f.dtype is not torch.bfloat16:
             raise RuntimeError("[isoexec-amd] packed must come from pack_decode(w1, w2)")
+    if packed is not None and streams:
         # other tokens touch other experts: between two uses of one, up to all of this layer's bytes (3 E F2 H) are read
         rc = _lib.check(
             _lib.lib().ix_moe_experts_packed_footprint(xc.data_ptr(), xc.stride(0), p.sorted_token.data_ptr(),

@@ -67,3 +67,16 @@ def test_expert_bands_on_sizes_they_do_not_serve():
     prob = torch.rand(t, 2, device=DEV)
     want = experts_forward(x, w1, w2, permute(idx, prob, e, BM=32))
     assert torch.equal(experts_forward(x, w1, w2, permute(idx, prob, e, BM=160)), want)
+
+
+def test_packed_matrices_of_another_layer_stay_refused_where_a_band_takes_over():
+    from isoexec_amd.ops.moe.moe_hip import experts_forward, pack_decode, permute
+
+    t, e, hd, f = 64, 4, 1024, 768  # 32 rows per expert
+    x, w1, w2 = _randn(t, hd, seed=8), _randn(e, 2 * f, hd, seed=9, std=0.05), _randn(e, hd, f, seed=10, std=0.05)
+    idx = torch.arange(2 * t, device=DEV, dtype=torch.int32).view(t, 2) % e
+    p = permute(idx, torch.rand(t, 2, device=DEV), e, BM=96)
+    w1f, w2f = pack_decode(w1, w2)
+    assert torch.equal(experts_forward(x, w1, w2, p, packed=(w1f, w2f)), experts_forward(x, w1, w2, p))
+    with pytest.raises(RuntimeError, match="pack_decode"):
+        experts_forward(x, w1, w2, p, packed=(w1f[:2], w2f[:2]))

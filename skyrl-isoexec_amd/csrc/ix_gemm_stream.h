@@ -277,6 +277,8 @@ struct IxPlainStreamJob {
   ix_rsrc_t p_cr, p_pr;      // pending tile: descriptors of its part of C and of the row-max parts
   uint32_t p_voff, p_pvoff;  // this lane's first output element / part in them
   int p_cols;                // columns left from there
+  int p_mcols;               // columns left from this lane's first one in the accumulator layout
+  uint32_t p_pad;            // 0, or -inf's bits where the piece of the maximum's step is past the matrix
   static constexpr int MI = Cfg::MI, NI = Cfg::NI, NL = NI / 2;
   uint32_t pend[MI][NI][8];  // the pending tile's outputs, two bf16 per register, accumulator layout
   uint32_t ta[4][4], tb[4][4];  // [slot][dword] after exchange stage 1 / 2
@@ -297,7 +299,8 @@ struct IxPlainStreamJob {
     p_cr = ix_make_rsrc(nullptr, 0u);
     p_pr = p_cr;
     p_voff = p_pvoff = IX_OOB;
-    p_cols = 0;
+    p_cols = p_mcols = 0;
+    p_pad = 0u;
     rmax = IX_NEG_INF;
 #pragma unroll
     for (int i = 0; i < MI * NI * 8; ++i) pend[i / (NI * 8)][(i >> 3) % NI][i & 7] = 0u;
@@ -360,6 +363,7 @@ struct IxPlainStreamJob {
     p_voff = (uint32_t)(((long)r * seq.ldc + c) * 2);
     p_cols = cur.nv - c;
     if constexpr (PARTS) {
+      p_mcols = cur.nv - wn * Cfg::TN - 32 * (lane >> 5);
       p_pr = ix_make_rsrc(cur.part, cur.part ? (uint32_t)(((long)(cur.mv - 1) * seq.parts_ld + Cfg::WN) * 4) : 0u);
       p_pvoff = (lane < 32) ? (uint32_t)(((long)(wm * Cfg::TM + lane) * seq.parts_ld + wn) * 4) : IX_OOB;
     }
@@ -377,11 +381,15 @@ struct IxPlainStreamJob {
     if constexpr (PARTS && q < 8) {
       // rounding is monotonic: the maximum of the rounded values is the rounded maximum
       if constexpr (q == 0 && L == 0) rmax = IX_NEG_INF;
+      // Steps q and q + 1 hold a piece of eight columns, which exists as a whole or not at all. Past the matrix the weight rows
+      // read as zeros: such a value is 0 (or, of an activation that is not finite, NaN) and becomes -inf (or stays NaN, which
+      // a maximum passes over) with the bits of -inf set in it.
+      if constexpr ((q & 1) == 0) p_pad = (64 * L + 4 * q < p_mcols) ? 0u : 0xff800000u;
 #pragma unroll
       for (int h = 0; h < 2; ++h) {
         constexpr int k0 = q * 2;
         const uint32_t u = pend[mi][2 * L + ((k0 + h) >> 3)][(k0 + h) & 7];
-        rmax = fmaxf(rmax, fmaxf(__uint_as_float(u << 16), __uint_as_float(u & 0xffff0000u)));
+        rmax = fmaxf(rmax, fmaxf(__uint_as_float((u << 16) | p_pad), __uint_as_float((u & 0xffff0000u) | p_pad)));
       }
     } else if constexpr (q >= 8 && q < 24) {
       // piece pi, dword d of the lane's 64 bytes: pend[mi][2 L + pi / 2][4 (pi % 2) + d]; stage 1 pairs pieces (0, 1), (2, 3)

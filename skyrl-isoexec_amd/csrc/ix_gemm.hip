@@ -32,7 +32,8 @@ __device__ __forceinline__ bool ix_tile_of_block(unsigned bid, int nb_m, int nb_
 
 // TC = bf16_t: C is the bf16 round of the fp32 accumulator; TC = float: the accumulator itself.
 // row_max_parts (optional): [M, parts_ld] fp32, entry (m, tn) = max over the tile's columns of the
-// values stored to C (exact, order-free), so a consumer can skip its own max pass over C.
+// values stored to C (exact, order-free), so a consumer can skip its own max pass over C. part_slots: entries per row, a
+// multiple of them per part (the last part takes the rest) where the caller counted another shape's.
 template <int BM, int BN, int WM, int WN, typename TC, int PW = 0, bool W_ONCE = false>
 __global__ __launch_bounds__((WM * WN + PW) * 64) void k_gemm_bf16_nt(const bf16_t* __restrict__ A, long lda,
                                                               const bf16_t* __restrict__ W, long ldw,
@@ -40,7 +41,7 @@ __global__ __launch_bounds__((WM * WN + PW) * 64) void k_gemm_bf16_nt(const bf16
                                                               TC* __restrict__ C, long ldc, int M, int N, int K,
                                                               int nb_m, int nb_n, int vec_store,
                                                               float* __restrict__ row_max_parts, long parts_ld,
-                                                              long batch_a, long batch_w, long batch_c, int part_copies) {
+                                                              long batch_a, long batch_w, long batch_c, int part_slots) {
   using Cfg = IxGemmCfg<BM, BN, WM, WN, PW, W_ONCE>;
   extern __shared__ __align__(16) char ix_lds[];
   // a batch of independent products (bmm): workgroup row blockIdx.y works on matrices batch strides further on
@@ -160,18 +161,19 @@ __global__ __launch_bounds__((WM * WN + PW) * 64) void k_gemm_bf16_nt(const bf16
       if (computes && lane < 32) s_max[wn * BM + wm * Cfg::TM + mi * 32 + lane] = v;
     }
     __syncthreads();
+    // one part per wave column where the streaming form of this tile writes those, without passing through LDS; else one
+    constexpr int PPT = ix_gemm_parts_per_tile<BM, BN, WM, WN, PW>();
+    const int n_parts = nb_n * PPT, each = part_slots / n_parts;
     for (int r = threadIdx.x; r < m_valid; r += Cfg::NTT) {
-      if constexpr (ix_gemm_parts_per_tile<BM, BN, WM, WN, PW>() == WN) {
-        // one part per wave column: the layout the streaming form of this tile writes without passing through LDS
 #pragma unroll
-        for (int w = 0; w < WN; ++w)
-          for (int d = 0; d < part_copies; ++d)
-            row_max_parts[(m0 + r) * parts_ld + (tn * WN + w) * part_copies + d] = s_max[w * BM + r];
-      } else {
-        float v = s_max[r];
+      for (int p = 0; p < PPT; ++p) {
+        float v = s_max[p * BM + r];
+        if constexpr (PPT == 1) {
 #pragma unroll
-        for (int w = 1; w < WN; ++w) v = fmaxf(v, s_max[w * BM + r]);
-        row_max_parts[(m0 + r) * parts_ld + tn] = v;
+          for (int w = 1; w < WN; ++w) v = fmaxf(v, s_max[w * BM + r]);
+        }
+        const int part = tn * PPT + p, end = part + 1 == n_parts ? part_slots : (part + 1) * each;
+        for (int d = part * each; d < end; ++d) row_max_parts[(m0 + r) * parts_ld + d] = v;
       }
     }
   }
@@ -187,12 +189,13 @@ static bool ix_gemm_stream_fits(const void* C, long ldc, long M, long N, long K,
 template <int BM, int BN, int WM, int WN, typename TC, int PW = 0, bool W_ONCE = false>
 static int ix_gemm_bf16_launch(const bf16_t* A, long lda, const bf16_t* W, long ldw, const bf16_t* bias, TC* C,
                                long ldc, long M, long N, long K, float* parts, long parts_ld, hipStream_t st,
-                               long batch = 1, long batch_a = 0, long batch_w = 0, long batch_c = 0, int part_copies = 1) {
+                               long batch = 1, long batch_a = 0, long batch_w = 0, long batch_c = 0, long part_slots = 0) {
   using Cfg = IxGemmCfg<BM, BN, WM, WN, PW>;
   const long nb_m = (M + BM - 1) / BM, nb_n = (N + BN - 1) / BN;
   const long grid = 8 * ((nb_m * nb_n + 7) / 8);  // 8 XCD runs of the tile order, the longest one sets the count
   if (grid > 0x7fffffffL) return IX_DECLINED;
-  if (parts && parts_ld < nb_n * ix_gemm_parts_per_tile<BM, BN, WM, WN, PW>() * part_copies) return IX_ERR_ARG;
+  if (part_slots == 0) part_slots = nb_n * ix_gemm_parts_per_tile<BM, BN, WM, WN, PW>();
+  if (parts && parts_ld < part_slots) return IX_ERR_ARG;
   auto kern = k_gemm_bf16_nt<BM, BN, WM, WN, TC, PW, W_ONCE>;
   static bool attr_set = false;  // per instantiation
   if (!attr_set) {
@@ -205,7 +208,7 @@ static int ix_gemm_bf16_launch(const bf16_t* A, long lda, const bf16_t* W, long 
   if (batch > 65535) return IX_DECLINED;
   hipLaunchKernelGGL(kern, dim3((unsigned)grid, (unsigned)batch), dim3(Cfg::NTT), Cfg::LDS_BYTES, st, A, lda, W, ldw,
                      bias, C, ldc, (int)M, (int)N, (int)K, (int)nb_m, (int)nb_n, vec, parts, parts_ld, batch_a, batch_w,
-                     batch_c, part_copies);
+                     batch_c, (int)part_slots);
   return ix_launch_status();
 }
 
@@ -273,15 +276,27 @@ static int ix_gemm_bf16_dispatch(const bf16_t* a, long lda, const bf16_t* w, lon
                                  long ldc, long M, long N, long K, int tile, float* parts, long parts_ld,
                                  hipStream_t st, long batch = 1, long sa = 0, long sw = 0, long sc = 0) {
   // `tile` only picks which workgroup owns an element (0 = by M); the bits do not depend on it.
-#define IX_BATCH_ARGS , batch, sa, sw, sc
+#define IX_BATCH_ARGS , batch, sa, sw, sc, slots
   const bool bands_fit = sizeof(TC) == 2 && ix_gemm_stream_fits(c, ldc, M, N, K, b, batch) && K / IX_BK >= IX_BAND_MIN_KT;
   // with row-max parts the choice has to be the one ix_gemm_bf16_n_tiles made from the sizes alone
-  const int id = ix_gemm_tile_for(M * (batch > 1 ? batch : 1), N, K, tile, parts || bands_fit);
+  const long rows = M * (batch > 1 ? batch : 1);
+  int id = ix_gemm_tile_for(rows, N, K, tile, parts || bands_fit);
+  long slots = 0;
+  if (id > IX_TILE_BAND && !bands_fit) {
+    if (tile != 0) return IX_DECLINED;
+    // Chosen by size for a call with a bias, an fp32 result or unaligned rows: the shape that the model takes without bands
+    // fills a band's four slots per tile. The 64 x 32 tile has more parts than that: the 128 x 128 one in its place.
+    // us in the 256-row tile / here, with a bias: 128 rows of 151936 x 2048 277 / 154, 385 of 12352 x 2048 76 / 39, 300 of
+    // 40000 x 768 69 / 44; with an fp32 result 214 / 172, 54 / 37, 65 / 41.
+    id = ix_gemm_tile_for(rows, N, K, 0, false);
+    if (id == 6) id = 2;
+    slots = 4 * ((N + 255) / 256);
+  }
   switch (id) {
     case 1: return ix_gemm_bf16_launch<32, 256, 1, 4, TC, 4>(a, lda, w, ldw, b, c, ldc, M, N, K, parts, parts_ld, st IX_BATCH_ARGS);
     case 2:
       if (batch == 1 && ix_gemm_once((M + 127) / 128, N, K))
-        return ix_gemm_bf16_launch<128, 128, 2, 2, TC, 0, true>(a, lda, w, ldw, b, c, ldc, M, N, K, parts, parts_ld, st);
+        return ix_gemm_bf16_launch<128, 128, 2, 2, TC, 0, true>(a, lda, w, ldw, b, c, ldc, M, N, K, parts, parts_ld, st IX_BATCH_ARGS);
       return ix_gemm_bf16_launch<128, 128, 2, 2, TC>(a, lda, w, ldw, b, c, ldc, M, N, K, parts, parts_ld, st IX_BATCH_ARGS);
     case 3: return ix_gemm_bf16_launch<256, 256, 2, 4, TC>(a, lda, w, ldw, b, c, ldc, M, N, K, parts, parts_ld, st IX_BATCH_ARGS);
     case 4:
@@ -308,10 +323,7 @@ static int ix_gemm_bf16_dispatch(const bf16_t* a, long lda, const bf16_t* w, lon
       if constexpr (sizeof(TC) == 2) {
         if (bands_fit) return ix_gemm_bf16_bands_launch(id - IX_TILE_BAND, a, lda, w, ldw, (bf16_t*)c, ldc, M, N, K, parts, parts_ld, st);
       }
-      if (tile != 0) return IX_DECLINED;
-      // chosen by size for a call with a bias, an fp32 result or unaligned rows: the 256-row tile, and every row-max part
-      // stored twice (the caller was told a band's four parts per tile)
-      return ix_gemm_bf16_launch<256, 256, 2, 2, TC>(a, lda, w, ldw, b, c, ldc, M, N, K, parts, parts_ld, st IX_BATCH_ARGS, 2);
+      return IX_DECLINED;
     default: return IX_ERR_ARG;
   }
 #undef IX_BATCH_ARGS

@@ -45,3 +45,18 @@ def test_logprobs_of_rows_below_zero(rows):
     assert torch.equal(logits, linear_nt(x, head))
     want, _ = sampled_forward(logits, target, leaves())
     assert torch.isfinite(want).all() and torch.equal(got, want)
+
+
+# Sizes for which a band is chosen and does not serve the call; without bands the model takes the 256 x 256, 128 x 128 (odd
+# number of its column tiles), 128 x 256 and 32 x 256 tile.
+@pytest.mark.parametrize("m,n,k", [(138, 40696, 768), (148, 16920, 832), (4883, 776, 3584), (132, 19624, 1792)])
+def test_shapes_that_take_a_bands_place(m, n, k):
+    from isoexec_amd import _lib
+    from isoexec_amd.ops.mm.mm_hip import linear_nt
+
+    assert _lib.lib().ix_gemm_bf16_n_tiles(m, n, k, 0) == 4 * ((n + 255) // 256)
+    x, w, bias = _positive(m, k, seed=2), -_positive(n, k, seed=3), -_positive(n, seed=4)
+    for kw in ({"bias": bias}, {"out_dtype": torch.float32}):
+        want, want_top = linear_nt(x, w, tile=6, want_row_max=True, **kw)
+        got, top = linear_nt(x, w, want_row_max=True, **kw)
+        assert torch.equal(got, want) and torch.equal(top, want_top), kw

@@ -219,8 +219,14 @@ static int ix_gemm_bf16_launch(const bf16_t* A, long lda, const bf16_t* W, long 
 // of the same weights (16 to 7300 rows) for the bands (`bands`: the call is one they serve), whose k-tile costs what the L2
 // takes for its operands: 256 CUs pull 10 to 13 TB/s whatever the height. us, without -> with bands: 151936 x 4096 at 192
 // rows 290 -> 262, 257 456 -> 358, 320 469 -> 375, 384 492 -> 434, 513 675 -> 587, 769 927 -> 828; 151936 x 2048 at 513 351 ->
-// 307; 12352 x 2048 at 320 32 -> 26; 5120 x 2048 at 3090 86 -> 58.
+// 307; 12352 x 2048 at 320 32 -> 26; 5120 x 2048 at 3090 86 -> 58. One turn of fewer bands than CUs: a CU takes its operands at
+// 35 to 39 GB/s where they come from memory, whatever the height (100 rows of 28672 x 4096, 112 column tiles: 64 us
+// in bands, 55 in twice as many 128 x 128 tiles; of 40960 x 2048, 160 column tiles, 42 against 51). Bands of equal cost are
+// bound by that or by the stream: the lowest (50304 x 2048 at 128 rows 52 -> 49 us). Over 448 points of nineteen weights (65 to
+// 4200 rows, no weight read twice out of the caches) the choice is 1.3 % off the fastest shape in the mean and no more than
+// 3 % slower than the choice without bands.
 #define IX_TILE_BAND 10  // id IX_TILE_BAND + MI: bands of 32 MI rows
+#define IX_BAND_CU_RATE 37e3  // bytes per us that a band takes from memory
 static int ix_gemm_tile_for(long M, long N, long K, int tile, bool bands) {
   if (tile != 0) return tile;
   // One 128-wide column of tiles (the router's gating product): 128-row tiles once there are enough of them to fill
@@ -253,8 +259,11 @@ static int ix_gemm_tile_for(long M, long N, long K, int tile, bool bands) {
     } else {
       cost = turns * (sh.fixed + kt * (turns == 1.0 ? sh.us_ktile : sh.us_ktile_more));
     }
-    cost = std::max(cost, (double)(N + M) * (double)K * 2.0 / sh.stream);
-    if (cost < best_cost * (sh.id > IX_TILE_BAND ? 0.99 : 0.97)) {  // a later (smaller) shape must win by a margin
+    const bool band = sh.id > IX_TILE_BAND;
+    const double bytes = (double)(N + M) * (double)K * 2.0;
+    cost = std::max(cost, band ? sh.fixed + bytes / std::min(sh.stream, IX_BAND_CU_RATE * tiles) : bytes / sh.stream);
+    // a later (smaller) shape must win by a margin, but for a band at the cost of a higher one
+    if (cost < best_cost * (band ? 0.99 : 0.97) || (band && best > IX_TILE_BAND && cost <= best_cost)) {
       best_cost = cost;
       best = sh.id;
     }

@@ -871,14 +871,16 @@ static int ix_gdn_walk(const void* q, const void* k, const void* v, const float*
   // and 32: 8 x 500 72 / 110, 32 x 500 329 / 323. The line: eight waves per SIMD at one row.
   // Fewer workgroups: a wave of their own stages the tiles (LONE) up to two of them per CU; with more, its registers and its
   // share of the issue are missed. us without / with it: one sequence of 8192 tokens 1147 / 988, 2 x 3000 544 / 501, 3 x 2000
-  // 484 / 522; K = V = 64, HV = 32, 8 x 512 92 / 86, 16 x 512 156 / 210. And a slice split over two lanes (E = 4) while one
-  // such workgroup per CU, two at K <= 64, is all there is (at K = 128 a row is then 32 lanes and its tree has a level across
-  // the halves of 16). us whole / split: 2000 tokens of 16 heads at K = 128 245 / 206, of 32 heads (two per CU) 66 / 75 per
-  // 500; K = 64, 2 x 256 of 4 heads 33 / 24, 8 x 512 of 16 heads 66 / 63, of 32 heads 86 / 107.
+  // 484 / 522; K = V = 64, HV = 32, 8 x 512 92 / 86, 16 x 512 156 / 210. Two of them per CU are ten waves, which need 128
+  // registers at most: the fp32 forms of K >= 128 (138 and 146, the raw tile in the staging wave) stop at one (16 heads, K =
+  // 128, 3 x 1000 tokens 185 / 240, 4 x 700 132 / 173; K = 256, 8 heads 242 / 305). And a slice split over two lanes (E = 4)
+  // while one such workgroup per CU, two at K <= 64, is all there is (at K = 128 a row is then 32 lanes and its tree has a
+  // level across the halves of 16). us whole / split: 2000 tokens of 16 heads at K = 128 245 / 206, of 32 heads (two per CU)
+  // 66 / 75 per 500; K = 64, 2 x 256 of 4 heads 33 / 24, 8 x 512 of 16 heads 66 / 63, of 32 heads 86 / 107.
   const long lanes = N * HV * V * (K / 8);  // threads at one row per lane group, whole slices
   const bool auto_shape = rpl <= 0;
   if (auto_shape) rpl = lanes >= 8L * 1024 * 64 ? 2 : 1;
-  const bool lone = auto_shape && lanes <= 2L * 256 * 256;
+  const bool lone = auto_shape && lanes <= (io_dtype == IX_DT_F32 && K >= 128 ? 1L : 2L) * 256 * 256;
   const bool split = auto_shape && K <= 128 && 2 * lanes <= (K == 128 ? 256L : 512L) * 256 &&
                      V % (2048 / K) == 0;  // what whole slices decline stays declined
 #define IX_WALK_ARGS(CHUNK_) \

@@ -57,6 +57,8 @@ def test_walk_equals_the_token_staged_scan(K, V, dtype, rows_per_group):
     (128, 2, 4, 64, torch.bfloat16, EDGES), (128, 1, 1, 16, torch.float32, [1, 50]),  # slices split over two lanes
     (64, 8, 16, 64, torch.bfloat16, EDGES), (64, 8, 32, 64, torch.float32, [16, 8, 1, 40, 17, 3, 5, 2]),  # around its line
     (128, 16, 32, 128, torch.bfloat16, [47]), (128, 16, 32, 128, torch.float32, [32, 17]),  # a staging wave, whole slices
+    (128, 16, 32, 128, torch.float32, [47]), (256, 4, 8, 128, torch.float32, [25, 9]),  # in fp32 up to one workgroup per CU
+    (256, 4, 8, 128, torch.float32, [25, 9, 16]),
     (128, 8, 16, 128, torch.bfloat16, EDGES), (256, 1, 2, 64, torch.bfloat16, EDGES), (256, 1, 2, 64, torch.float32, [9])])
 def test_walk_by_the_rule_equals_the_token_staged_scan(K, H, HV, V, dtype, lens):
     """The forms that the number of workgroups chooses (a staging wave, split slices, neither): output and final state bit for

@@ -1915,7 +1915,13 @@ extern "C" int ix_moe_combine(const void* expert_out, const int* combine_rows, v
   if (grid > 0x7fffffffL) return IX_DECLINED;
   const int vec = (Hd % 8 == 0) && ix_aligned(expert_out, 16) && ix_aligned(out, 16);
   const long chunks = (Hd + 511) / 512;
-  if (vec && T * chunks <= 0x7fffffffL && (k == 2 || k == 4 || k == 8)) {
+  // A wave's 512 columns leave lanes idle in narrow rows, and each row of a token costs the wave its scalar addresses: the fewer
+  // the rows, the wider they have to be. us in threads / in waves at 65536 tokens: k = 2 192 columns 14.7 / 15.5, 256 17.6 /
+  // 17.6; k = 4 128 17.2 / 19.2, 160 21.7 / 20.4; k = 8 64 18.0 / 28.3, 128 29.3 / 28.4. With fp32 sums, which leave the threads
+  // little arithmetic, and more than the caches hold several times over, threads again: 2048 columns, k = 8 469 / 477.
+  const long least = k == 2 ? 256 : (k == 4 ? 160 : 128);
+  const bool waves = Hd >= least && !(fp32_acc && T * Hd >= (1L << 26)) && T * chunks <= 0x7fffffffL;
+  if (vec && waves && (k == 2 || k == 4 || k == 8)) {
 #define IX_COMBINE_ROWS(KC_, F_)                                                                                       \
   hipLaunchKernelGGL((k_moe_combine_rows<KC_, F_>), dim3((unsigned)((T * chunks + 3) / 4)), dim3(256), 0,              \
                      (hipStream_t)stream, (const bf16_t*)expert_out, combine_rows, (bf16_t*)out, (unsigned)(T * chunks), \

@@ -11,7 +11,7 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("tokens", [1, 5, 259])
-@pytest.mark.parametrize("width", [8, 504, 512, 520, 2048, 300])
+@pytest.mark.parametrize("width", [8, 120, 128, 152, 160, 248, 256, 504, 512, 520, 2048, 300])
 @pytest.mark.parametrize("k", [2, 3, 4, 8])
 @pytest.mark.parametrize("offset", [0, 4])
 def test_combine_rows(tokens, width, k, offset):

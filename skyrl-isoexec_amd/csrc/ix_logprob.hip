@@ -381,8 +381,10 @@ __global__ __launch_bounds__(256) void k_lp_backward(const T* __restrict__ x, lo
 }
 
 // rowmax[row] = max over P parts (exact; any order). One wave per row, or (many parts) one workgroup per row with all its
-// loads in flight: a wave walks 2376 parts one dependent load after the other (513 rows of 2376 parts 19.7 -> 5.3 us).
-#define IX_LP_MANY_PARTS 512
+// loads in flight: a wave walks 2376 parts one dependent load after the other (513 rows of 2376 parts 19.7 -> 5.3 us). The line:
+// up to 8192 rows the two are equal at 500 to 1000 parts; us wave / workgroup at 16384 rows 512 parts 6.9 / 9.0, 594 9.2 / 9.4, 640
+// 9.5 / 9.5, 768 10.9 / 9.6, 1187 15.7 / 12.4.
+#define IX_LP_MANY_PARTS 640
 __global__ __launch_bounds__(256) void k_lp_reduce_parts(const float* __restrict__ parts, long parts_ld, int P,
                                                          long rows, float* __restrict__ rowmax) {
   const long row = (long)blockIdx.x * 4 + (threadIdx.x >> 6);

@@ -5,7 +5,7 @@ import torch
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("parts", [1, 511, 512, 513, 2376, 5000])
+@pytest.mark.parametrize("parts", [1, 511, 512, 513, 639, 640, 641, 2376, 5000])
 def test_row_maximum_of_parts(parts):
     from isoexec_amd import _lib
 

@@ -482,11 +482,13 @@ __global__ __launch_bounds__(1024) void k_moe_scatter(const int* __restrict__ to
 }
 
 // Scatter with the prefix over the token tiles and the expert offsets in the same launch, for up to IX_MOE_FEW_TILES token
-// tiles: every workgroup adds up the whole count table for itself (ntiles x E integers out of the L2) instead of waiting for
-// two more launches of one dependent chain each; the first one also writes counts, offsets and the block map. Bound by
-// those launches' latencies: prefix + offsets + scatter 15.8 -> 7.2 us at 512 tokens, 19.1 -> 10.7 at 4096 (128 experts), the
-// gaps between them not counted.
+// tiles and IX_MOE_FEW_COUNTS counts: every workgroup adds up the whole count table for itself (ntiles x E integers out of
+// the L2) instead of waiting for two more launches of one dependent chain each; the first one also writes counts, offsets
+// and the block map. Bound by those launches' latencies: prefix + offsets + scatter 15.8 -> 7.2 us at 512 tokens, 19.1 ->
+// 10.7 at 4096 (128 experts), the gaps between them not counted. The table that every workgroup reads sets the line: of 512
+// experts, top-8, 8192 tokens (16384 integers) 17.0 -> 15.5 us, 12000 (24064) 17.4 -> 17.4, 16384 (32768) 18.1 -> 19.8.
 #define IX_MOE_FEW_TILES 64
+#define IX_MOE_FEW_COUNTS 24576
 __global__ __launch_bounds__(1024) void k_moe_offsets_scatter(const int* __restrict__ topk_idx,
                                                               const float* __restrict__ topk_prob, int T, int E, int k,
                                                               int ntiles, int BM, int max_tiles,
@@ -845,7 +847,7 @@ extern "C" int ix_moe_permute(const int* topk_idx, const float* topk_prob, long 
   if (ntiles > 0)
     hipLaunchKernelGGL(k_moe_tile_counts, dim3((unsigned)ntiles), dim3(256), 0, st, topk_idx, (int)T, (int)E, (int)k,
                        tile_counts);
-  if (ntiles > 0 && ntiles <= IX_MOE_FEW_TILES) {
+  if (ntiles > 0 && ntiles <= IX_MOE_FEW_TILES && ntiles * E <= IX_MOE_FEW_COUNTS) {
     hipLaunchKernelGGL(k_moe_offsets_scatter, dim3((unsigned)ntiles), dim3(1024), 0, st, topk_idx, topk_prob, (int)T, (int)E,
                        (int)k, (int)ntiles, (int)BM, (int)max_tiles, tile_counts, counts, offsets, tile_meta, sorted_token,
                        permuted_prob, combine_rows);

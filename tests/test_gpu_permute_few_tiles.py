@@ -6,7 +6,7 @@ import torch
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("t", [257, 512, 700, 64 * 256, 64 * 256 + 1])
+@pytest.mark.parametrize("t", [257, 512, 700, 48 * 256, 48 * 256 + 1, 64 * 256, 64 * 256 + 1])
 @pytest.mark.parametrize("e,k", [(128, 8), (3, 2), (60, 4), (512, 16)])
 def test_permutation(t, e, k):
     from isoexec_amd.ops.moe.moe_hip import permute

@@ -356,7 +356,10 @@ long ix_moe_max_tiles(long T, long k, long E, long BM);   /* ceil(T*k/BM) + E */
 size_t ix_moe_permute_scratch_ints(long T, long E);
 int ix_moe_pick_bm(long T, long k, long E);               /* 32, 128 or 256 */
 int ix_moe_pick_bm_packed(long T, long k, long E);        /* 32, 64, 128 or 256: for callers that hold packed matrices */
-/* The same for callers that know the layer's sizes (fc1 [E, 2F, Hd], fc2 [E, Hd, F]): also 96, 160, 192 and 224. */
+/* The same for callers that know the layer's sizes (fc1 [E, 2F, Hd], fc2 [E, Hd, F]): also 96, 160 and 192, and
+ * IX_MOE_BM_BY_COUNTS + 160 or 192 where the routing decides between that height and 256 rows: the maps then come from
+ * ix_moe_permute_by_counts or ix_moe_block_map_by_counts. */
+#define IX_MOE_BM_BY_COUNTS 0x10000
 int ix_moe_pick_bm_shape(long T, long k, long E, long Hd, long F, int packed);
 
 /* fused_permute_index / ref_permute_index (moe_router_o2_kernel.py:313-351,389-397) plus the
@@ -370,6 +373,15 @@ int ix_moe_pick_bm_shape(long T, long k, long E, long Hd, long F, int packed);
 int ix_moe_permute(const int* topk_idx, const float* topk_prob, long T, long E, long k, long BM, int* counts,
                    int* offsets, int* sorted_token, float* permuted_prob, int* combine_rows, int* tile_meta,
                    long max_tiles, int* scratch, void* stream);
+
+/* ix_moe_permute with two block maps: meta_low of `low` rows a tile (160 or 192) [1 + 3*max_low] and meta_tall of
+ * 256 [1 + 3*max_tall], max_low >= ix_moe_max_tiles(T, k, E, low), max_tall >= ix_moe_max_tiles(T, k, E, 256).
+ * From the counts and the layer's sizes the device decides which of the two holds the rows; the other has n_tiles
+ * = 0. The caller makes the experts call for both maps (BM = low and 256) with the same buffers: one of them finds
+ * nothing to do. T > 256 (declined at or below it). */
+int ix_moe_permute_by_counts(const int* topk_idx, const float* topk_prob, long T, long E, long k, long low, long Hd, long F,
+                             int* counts, int* offsets, int* sorted_token, float* permuted_prob, int* combine_rows,
+                             int* meta_low, long max_low, int* meta_tall, long max_tall, int* scratch, void* stream);
 
 /* fused_router_dense + fused_permute_index back to back (moe_router_o2_kernel.py:272-351) for a batch of at most one
  * token tile (T <= 256, a decode step) and E <= 128: ix_moe_router_topk and ix_moe_permute in ONE launch, the same
@@ -388,6 +400,10 @@ int ix_moe_route_one_tile(const float* logits, long ld, long T, long E, long k, 
  * tile. Integer work only, one launch, nothing read back by the host. */
 int ix_moe_block_map(const void* counts, int counts_i64, long E, long BM, long rows, int* offsets, int* tile_meta,
                      long max_tiles, void* stream);
+
+/* ix_moe_block_map with two maps, as ix_moe_permute_by_counts writes them. */
+int ix_moe_block_map_by_counts(const void* counts, int counts_i64, long E, long low, long Hd, long F, long rows,
+                               int* offsets, int* meta_low, long max_low, int* meta_tall, long max_tall, void* stream);
 
 /* ix_moe_permute for callers that cannot allocate device memory or bring a workspace: code under HIP graph
  * capture, tight serving loops, harnesses that forbid allocation. No counterpart in the reference (its permutation
@@ -411,8 +427,8 @@ int ix_moe_permute_static(const int* topk_idx, const float* topk_prob, long T, l
  * then up rows); W2 bf16 [E, Hd, F]; inter bf16 [rows, F]; expert_out bf16 [rows, Hd];
  * rows = T*k = the length of sorted_token and permuted_prob (the kernels clamp their reads of both to rows - 1, so it
  * must not exceed what the arrays hold). BM must be the value given to ix_moe_permute. With 256-row tiles and at
- * least 512 tiles of work, and with 96, 160, 192 or 224 rows, both GEMMs run as streaming kernels (one workgroup per CU
- * walking many tiles); same bits. */
+ * least 512 tiles of work, and with 96, 160 or 192 rows where the sizes allow it (Hd a multiple of 256, F of 128, at least
+ * 1024 and 768), both GEMMs run as streaming kernels (one workgroup per CU walking many tiles); same bits. 224 runs as 256. */
 int ix_moe_experts(const void* x, long ldx, const int* sorted_token, const float* permuted_prob,
                    const void* W1, const void* W2, const int* tile_meta, long max_tiles, long BM, void* inter,
                    void* expert_out, long T, long rows, long Hd, long F, void* stream);

@@ -392,56 +392,107 @@ __device__ __forceinline__ void ix_moe_write_tiles(int e, int c, int row0, int n
   }
 }
 
-// One workgroup, after k_moe_tile_prefix has left every expert's row count in `counts`: an
-// exclusive scan over the experts in LDS, then every expert writes its own row tiles.
-__global__ __launch_bounds__(256) void k_moe_offsets(int E, int BM, int max_tiles, const int* __restrict__ counts,
-                                                     int* __restrict__ offsets, int* __restrict__ meta) {
-  __shared__ int s_cnt[IX_MOE_EMAX], s_off[IX_MOE_EMAX + 1], s_toff[IX_MOE_EMAX + 1];
+// A second map of 256-row tiles beside one of 160 or 192, of which the counts decide which is used (the other gets no
+// tiles). The kernels of both heights are launched; those of the empty map find no tile and exit.
+struct IxMoeTall {
+  int* meta;               // null: the map has one height
+  int max_tiles;
+  float us_low;            // what the first map's tiles cost
+  int nb1, kt1, nb2, kt2;  // column tiles and k-tiles of the two products
+};
+
+// What both products cost with `tiles` row tiles at `us` per k-tile: turns of the chip's 256 workgroups, where a last turn that
+// is not full costs two thirds of one and the rest by its share. `us` is a fit to 737 launches (seventeen layers, three
+// routings, 24 to 400 rows per expert) whose times it gives with a deviation of 6 %.
+#define IX_MOE_US_160 1.27f
+#define IX_MOE_US_192 1.41f
+#define IX_MOE_US_256 1.64f
+__device__ __forceinline__ float ix_moe_tiles_cost(const IxMoeTall& h, int tiles, float us) {
+  auto turns = [](float t) {
+    const float full = floorf(t);
+    return t > full ? full + 0.68f + 0.32f * (t - full) : full;
+  };
+  return us * (turns((float)tiles * (float)h.nb1 / 256.0f) * (float)h.kt1 +
+               turns((float)tiles * (float)h.nb2 / 256.0f) * (float)h.kt2);
+}
+
+// Exclusive scans over the experts by one wave (rows and row tiles; s_cnt is zero past the last expert): a lane owns EMAX / 64
+// consecutive ones. Returns the rows of a tile: BM, or 256 where the counts decide for the tall map. `write`: also the total to
+// offsets[E] (if there are offsets) and the number of tiles to the maps.
+__device__ __forceinline__ int ix_moe_scan_experts(const int* s_cnt, int E, int BM, int max_tiles, const IxMoeTall& tall,
+                                                   int* s_off, int* s_toff, bool write, int* offsets, int* meta) {
+  constexpr int PER = IX_MOE_EMAX / 64;
+  const int lane = threadIdx.x;
+  auto count = [&](int rows_per_tile, int& rows, int& tiles) {  // this lane's experts, then all up to them
+    rows = tiles = 0;
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+      const int c = s_cnt[lane * PER + i];
+      rows += c;
+      tiles += (c + rows_per_tile - 1) / rows_per_tile;
+    }
+    const int own_rows = rows, own_tiles = tiles;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+      const int a = __shfl_up(rows, d, 64), b = __shfl_up(tiles, d, 64);
+      if (lane >= d) { rows += a; tiles += b; }
+    }
+    return make_int2(rows - own_rows, tiles - own_tiles);
+  };
+  int rows, tiles;
+  int2 before = count(BM, rows, tiles);
+  int total = __shfl(tiles, 63, 64);
+  bool is_tall = false;
+  if (tall.meta) {
+    int tall_tiles;
+    const int2 b = count(256, rows, tall_tiles);
+    const int tall_total = __shfl(tall_tiles, 63, 64);
+    is_tall = ix_moe_tiles_cost(tall, tall_total, IX_MOE_US_256) <= ix_moe_tiles_cost(tall, total, tall.us_low);
+    if (write && lane == 0) {
+      meta[0] = is_tall ? 0 : min(total, max_tiles);
+      tall.meta[0] = is_tall ? min(tall_total, tall.max_tiles) : 0;
+    }
+    if (is_tall) { before = b; BM = 256; }
+  } else if (write && lane == 0) {
+    meta[0] = min(total, max_tiles);
+  }
+  if (write && offsets && lane == 63) offsets[E] = rows;
+#pragma unroll
+  for (int i = 0; i < PER; ++i) {
+    const int c = s_cnt[lane * PER + i];
+    s_off[lane * PER + i] = before.x;
+    s_toff[lane * PER + i] = before.y;
+    before.x += c;
+    before.y += (c + BM - 1) / BM;
+  }
+  return BM;
+}
+
+// The row tiles of every expert and its offset, from those scans, by the whole workgroup.
+__device__ __forceinline__ void ix_moe_write_map(const int* s_cnt, const int* s_off, const int* s_toff, int E, int rows_per_tile,
+                                                 int BM, int max_tiles, const IxMoeTall& tall, int* offsets, int* meta) {
+  const bool is_tall = rows_per_tile != BM;
+  for (int e = threadIdx.x; e < E; e += (int)blockDim.x) {
+    if (offsets) offsets[e] = s_off[e];
+    ix_moe_write_tiles(e, s_cnt[e], s_off[e], s_toff[e], rows_per_tile, is_tall ? tall.max_tiles : max_tiles,
+                       is_tall ? tall.meta : meta);
+  }
+}
+
+// One workgroup, after k_moe_tile_prefix has left every expert's row count in `counts`.
+__global__ __launch_bounds__(256) void k_moe_offsets(int E, int BM, int max_tiles, IxMoeTall tall,
+                                                     const int* __restrict__ counts, int* __restrict__ offsets,
+                                                     int* __restrict__ meta) {
+  __shared__ int s_cnt[IX_MOE_EMAX], s_off[IX_MOE_EMAX], s_toff[IX_MOE_EMAX], s_rows_per_tile;
   const int tid = threadIdx.x;
-  for (int e = tid; e < E; e += 256) s_cnt[e] = counts[e];
+  for (int e = tid; e < IX_MOE_EMAX; e += 256) s_cnt[e] = e < E ? counts[e] : 0;
   __syncthreads();
-  // exclusive scan over the experts (rows and row tiles): lane owns experts 2 tid and 2 tid + 1 (E <= 512)
-  {
-    __shared__ int s_rows[256], s_tiles[256];
-    int c[2], tl[2];
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      const int e = 2 * tid + h;
-      c[h] = e < E ? s_cnt[e] : 0;
-      tl[h] = (c[h] + BM - 1) / BM;
-    }
-    s_rows[tid] = c[0] + c[1];
-    s_tiles[tid] = tl[0] + tl[1];
-    __syncthreads();
-    for (int d = 1; d < 256; d <<= 1) {
-      const int a = tid >= d ? s_rows[tid - d] : 0;
-      const int b = tid >= d ? s_tiles[tid - d] : 0;
-      __syncthreads();
-      s_rows[tid] += a;
-      s_tiles[tid] += b;
-      __syncthreads();
-    }
-    int row0 = s_rows[tid] - (c[0] + c[1]);
-    int tile0 = s_tiles[tid] - (tl[0] + tl[1]);
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      const int e = 2 * tid + h;
-      if (e < E) { s_off[e] = row0; s_toff[e] = tile0; }
-      row0 += c[h];
-      tile0 += tl[h];
-    }
-    if (tid == 255) {
-      s_off[E] = s_rows[255];
-      s_toff[E] = s_tiles[255];
-      offsets[E] = s_rows[255];
-      meta[0] = min(s_tiles[255], max_tiles);
-    }
+  if (tid < 64) {
+    const int r = ix_moe_scan_experts(s_cnt, E, BM, max_tiles, tall, s_off, s_toff, true, offsets, meta);
+    if (tid == 0) s_rows_per_tile = r;
   }
   __syncthreads();
-  for (int e = tid; e < E; e += 256) {
-    offsets[e] = s_off[e];
-    ix_moe_write_tiles(e, s_cnt[e], s_off[e], s_toff[e], BM, max_tiles, meta);
-  }
+  ix_moe_write_map(s_cnt, s_off, s_toff, E, s_rows_per_tile, BM, max_tiles, tall, offsets, meta);
 }
 
 // 1024 threads, a (token, choice) pair at a time: bound by the latency of a pair's lookups (10 us with a token per thread
@@ -491,7 +542,7 @@ __global__ __launch_bounds__(1024) void k_moe_scatter(const int* __restrict__ to
 #define IX_MOE_FEW_COUNTS 24576
 __global__ __launch_bounds__(1024) void k_moe_offsets_scatter(const int* __restrict__ topk_idx,
                                                               const float* __restrict__ topk_prob, int T, int E, int k,
-                                                              int ntiles, int BM, int max_tiles,
+                                                              int ntiles, int BM, int max_tiles, IxMoeTall tall,
                                                               const int* __restrict__ tile_counts, int* __restrict__ counts,
                                                               int* __restrict__ offsets, int* __restrict__ meta,
                                                               int* __restrict__ sorted_token,
@@ -499,7 +550,7 @@ __global__ __launch_bounds__(1024) void k_moe_offsets_scatter(const int* __restr
                                                               int* __restrict__ combine_rows) {
   __shared__ int s_idx[IX_MOE_TILE_T * IX_MOE_KMAX];
   __shared__ uint32_t s_mask[IX_MOE_EMAX * 8];
-  __shared__ int s_cnt[IX_MOE_EMAX], s_before[IX_MOE_EMAX], s_off[IX_MOE_EMAX], s_toff[IX_MOE_EMAX];
+  __shared__ int s_cnt[IX_MOE_EMAX], s_before[IX_MOE_EMAX], s_off[IX_MOE_EMAX], s_toff[IX_MOE_EMAX], s_rows_per_tile;
   const int tid = threadIdx.x, tile = blockIdx.x;
   const int t0 = tile * IX_MOE_TILE_T;
   const int nt = min(IX_MOE_TILE_T, T - t0);
@@ -518,42 +569,14 @@ __global__ __launch_bounds__(1024) void k_moe_offsets_scatter(const int* __restr
     atomicAdd(&s_before[e], before);
   }
   __syncthreads();
-  if (tid < 64) {  // exclusive scan over the experts (rows and row tiles): lane owns EMAX / 64 consecutive ones
-    constexpr int PER = IX_MOE_EMAX / 64;
-    int rows = 0, tiles = 0;
-#pragma unroll
-    for (int i = 0; i < PER; ++i) {
-      const int c = s_cnt[tid * PER + i];
-      rows += c;
-      tiles += (c + BM - 1) / BM;
-    }
-    int rsum = rows, tsum = tiles;
-#pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-      const int a = __shfl_up(rsum, d, 64), b = __shfl_up(tsum, d, 64);
-      if (tid >= d) { rsum += a; tsum += b; }
-    }
-    int r0 = rsum - rows, q0 = tsum - tiles;
-#pragma unroll
-    for (int i = 0; i < PER; ++i) {
-      const int c = s_cnt[tid * PER + i];
-      s_off[tid * PER + i] = r0;
-      s_toff[tid * PER + i] = q0;
-      r0 += c;
-      q0 += (c + BM - 1) / BM;
-    }
-    if (tid == 63 && tile == 0) {
-      offsets[E] = rsum;
-      meta[0] = min(tsum, max_tiles);
-    }
+  if (tid < 64) {
+    const int r = ix_moe_scan_experts(s_cnt, E, BM, max_tiles, tall, s_off, s_toff, tile == 0, offsets, meta);
+    if (tid == 0) s_rows_per_tile = r;
   }
   __syncthreads();
   if (tile == 0) {
-    for (int x = tid; x < E; x += 1024) {
-      counts[x] = s_cnt[x];
-      offsets[x] = s_off[x];
-      ix_moe_write_tiles(x, s_cnt[x], s_off[x], s_toff[x], BM, max_tiles, meta);
-    }
+    for (int x = tid; x < E; x += 1024) counts[x] = s_cnt[x];
+    ix_moe_write_map(s_cnt, s_off, s_toff, E, s_rows_per_tile, BM, max_tiles, tall, offsets, meta);
   }
   ix_moe_scatter_tile(t0, nt, k, s_mask, s_idx, topk_prob, [&](int x) { return s_off[x] + s_before[x]; }, sorted_token,
                       permuted_prob, combine_rows);
@@ -695,10 +718,12 @@ __global__ __launch_bounds__(1024) void k_moe_route_one_tile(const float* __rest
 // before it (counts that add up to more than `rows` lose their tail instead of reaching past the buffers).
 template <typename TI>
 __global__ __launch_bounds__(256) void k_moe_block_map(const TI* __restrict__ counts_in, int E, int BM, int max_tiles,
-                                                       int rows, int* __restrict__ offsets, int* __restrict__ meta) {
-  __shared__ int s_rows[256], s_tiles[256];
+                                                       IxMoeTall tall, int rows, int* __restrict__ offsets,
+                                                       int* __restrict__ meta) {
+  __shared__ int s_rows[256], s_cnt[IX_MOE_EMAX], s_off[IX_MOE_EMAX], s_toff[IX_MOE_EMAX], s_rows_per_tile;
+  static_assert(IX_MOE_EMAX == 2 * 256, "a thread owns two experts");
   const int tid = threadIdx.x;
-  int c[2], tl[2];  // lane owns experts 2 tid and 2 tid + 1 (E <= 512)
+  int c[2];  // thread owns experts 2 tid and 2 tid + 1
 #pragma unroll
   for (int h = 0; h < 2; ++h) {
     const int e = 2 * tid + h;
@@ -717,54 +742,47 @@ __global__ __launch_bounds__(256) void k_moe_block_map(const TI* __restrict__ co
   const int before = tid > 0 ? s_rows[tid - 1] : 0;
   c[0] = min(c[0], rows - before);
   c[1] = min(c[1], rows - before - c[0]);
-#pragma unroll
-  for (int h = 0; h < 2; ++h) tl[h] = (c[h] + BM - 1) / BM;
-  s_tiles[tid] = tl[0] + tl[1];
+  s_cnt[2 * tid] = c[0];
+  s_cnt[2 * tid + 1] = c[1];
   __syncthreads();
-  for (int d = 1; d < 256; d <<= 1) {
-    const int b = tid >= d ? s_tiles[tid - d] : 0;
-    __syncthreads();
-    s_tiles[tid] += b;
-    __syncthreads();
+  if (tid < 64) {
+    const int r = ix_moe_scan_experts(s_cnt, E, BM, max_tiles, tall, s_off, s_toff, true, offsets, meta);
+    if (tid == 0) s_rows_per_tile = r;
   }
-  int row0 = before;
-  int tile0 = s_tiles[tid] - (tl[0] + tl[1]);
-  int* tile_expert = meta + 1;
-  int* tile_row0 = tile_expert + max_tiles;
-  int* tile_nrows = tile_row0 + max_tiles;
-#pragma unroll
-  for (int h = 0; h < 2; ++h) {
-    const int e = 2 * tid + h;
-    if (e < E) {
-      if (offsets) offsets[e] = row0;
-      int nt = tile0;
-      for (int r0 = 0; r0 < c[h] && nt < max_tiles; r0 += BM, ++nt) {
-        tile_expert[nt] = e;
-        tile_row0[nt] = row0 + r0;
-        tile_nrows[nt] = min(BM, c[h] - r0);
-      }
-    }
-    row0 += c[h];
-    tile0 += tl[h];
-  }
-  if (tid == 255) {
-    if (offsets) offsets[E] = s_rows[255];
-    meta[0] = min(s_tiles[255], max_tiles);
-  }
+  __syncthreads();
+  ix_moe_write_map(s_cnt, s_off, s_toff, E, s_rows_per_tile, BM, max_tiles, tall, offsets, meta);
 }
 
-extern "C" int ix_moe_block_map(const void* counts, int counts_i64, long E, long BM, long rows, int* offsets,
-                                int* tile_meta, long max_tiles, void* stream) {
+static IxMoeTall ix_moe_tall(long low, int* meta, long max_tiles, long Hd, long F) {
+  return {meta, (int)max_tiles, low == 160 ? IX_MOE_US_160 : IX_MOE_US_192, (int)(F / 128), (int)(Hd / IX_BK),
+          (int)(Hd / 256), (int)(F / IX_BK)};
+}
+
+static int ix_moe_block_map_launch(const void* counts, int counts_i64, long E, long BM, long rows, int* offsets, int* tile_meta,
+                                   long max_tiles, const IxMoeTall& tall, void* stream) {
   if (!counts || !tile_meta || E <= 0 || BM <= 0 || max_tiles <= 0 || rows < 0) return IX_ERR_ARG;
   if (E > IX_MOE_EMAX || rows > 0x3fffffffL) return IX_DECLINED;  // two clamped counts are added in an int
   hipStream_t st = (hipStream_t)stream;
   if (counts_i64)
     hipLaunchKernelGGL(k_moe_block_map<long>, dim3(1), dim3(256), 0, st, (const long*)counts, (int)E, (int)BM,
-                       (int)max_tiles, (int)rows, offsets, tile_meta);
+                       (int)max_tiles, tall, (int)rows, offsets, tile_meta);
   else
     hipLaunchKernelGGL(k_moe_block_map<int>, dim3(1), dim3(256), 0, st, (const int*)counts, (int)E, (int)BM,
-                       (int)max_tiles, (int)rows, offsets, tile_meta);
+                       (int)max_tiles, tall, (int)rows, offsets, tile_meta);
   return ix_launch_status();
+}
+
+extern "C" int ix_moe_block_map(const void* counts, int counts_i64, long E, long BM, long rows, int* offsets,
+                                int* tile_meta, long max_tiles, void* stream) {
+  return ix_moe_block_map_launch(counts, counts_i64, E, BM, rows, offsets, tile_meta, max_tiles, IxMoeTall{}, stream);
+}
+
+extern "C" int ix_moe_block_map_by_counts(const void* counts, int counts_i64, long E, long low, long Hd, long F, long rows,
+                                          int* offsets, int* meta_low, long max_low, int* meta_tall, long max_tall,
+                                          void* stream) {
+  if (!meta_tall || max_tall <= 0 || Hd < 256 || F < 128 || (low != 160 && low != 192)) return IX_ERR_ARG;
+  return ix_moe_block_map_launch(counts, counts_i64, E, low, rows, offsets, meta_low, max_low,
+                                 ix_moe_tall(low, meta_tall, max_tall, Hd, F), stream);
 }
 
 extern "C" long ix_moe_max_tiles(long T, long k, long E, long BM) {
@@ -796,38 +814,43 @@ extern "C" int ix_moe_pick_bm_packed(long T, long k, long E) {
   return rows >= 40 * e ? ix_moe_pick_bm(T, k, E) : (rows >= 16 * e ? 64 : 32);
 }
 
-// The same with the layer's sizes at hand: bands of 96 .. 224 rows (ix_moe_bands.h) from 24 rows per expert on (with or without
-// packed matrices), as long as the mean fits a band, or two, better than 256 rows. us fc1 + fc2 (E = 128, Hd = 2048, F = 768,
-// top-8; even / skewed routing with four experts far more popular):
-//   rows per expert    before     256          96          160         192         224
-//     32            222 / -   253 / 283   207 / 232   207 / 242   209 / 251   223 / 263
-//     62            253 / -   248 / 289   222 / 256   225 / 261   228 / 268   238 / 278
-//     94               -      259 / 304   288 / 272   239 / 273   243 / 280   249 / 293
-//    125               -      270 / 319   296 / 287   247 / 318   252 / 306   259 / 305
-//    156               -      276 / 337   310 / 322   295 / 308   260 / 336   271 / 327
-//    188               -      285 / 369   362 / 371   363 / 325   335 / 337   323 / 359
-//    256               -      400 / 397   436 / 445   383 / 385   413 / 373   446 / 387
-//    312               -      488 / 429   512 / 505   446 / 474   433 / 425   468 / 417
-//    375               -      506 / 481   588 / 597   535 / 555   524 / 541   480 / 475
-//    438               -      551 / 564   662 / 664   581 / 589   607 / 634   579 / 608
-// (before: ring tiles of 128 x 128, or the packed streams). One tile per expert while mean + 3 sqrt(mean) rows fit it, then two
-// of half the height; in between, and from 400 rows on, 256.
+// The same with the layer's sizes at hand: bands of 96, 160 and 192 rows (ix_moe_bands.h). From 24 rows per expert on (with or
+// without packed matrices) the lowest in which mean + 3 sqrt(mean) rows fit, so that even routing gives every expert one tile;
+// 256 from 155 on; from 240 to 400, where even routing takes two tiles of 160 or 192, these or 256 as the counts say (IxMoeTall). us
+// fc1 + fc2 (E = 128, Hd = 2048, F = 768, top-8; routing even / four experts 2 to 4 times as popular / in every token's choice):
+//   rows per expert   ring 128 x 128     256 rows            96                 160                192
+//     28              235 / 246 / 246                        205 / 229 / 226    206 / 238 / 241
+//     46              245 / 251 / 260                        214 / 237 / 239    216 / 252 / 246
+//     70              259 / 262 / 276                        227 / 248 / 259    232 / 264 / 268
+//     82              262 / 268 / 282                        257 / 256 / 287    234 / 268 / 271
+//     106                                268 / 308 / 308                        246 / 272 / 288    250 / 284 / 291
+//     124                                275 / 312 / 316                        250 / 279 / 313    254 / 289 / 301
+//     133                                278 / 314 / 321                        292 / 286 / 323    256 / 295 / 307
+//     160                                281 / 326 / 330                        322 / 286 / 316    305 / 303 / 341
+//     241                                350 / 358 / 405                        385 / 419 / 378    419 / 414 / 374
+//     277                                485 / 368 / 419                        399 / 468 / 443    428 / 474 / 389
+//     331                                506 / 497 / 452                        525 / 482 / 530    485 / 523 / 487
+// Over sixteen other layers of 16 to 256 experts a band of the mean is 6 % faster than the other tile in the geometric mean
+// below 155 rows, the worst point 13 % slower. From 240 to 400 one of the mean is as often slower as faster (from 240 to
+// 280 rows 8 % faster, 21 % and 4 % slower for the three routings, the worst point 32 %); chosen by the counts it is 5 %
+// faster, the worst point 5 % slower. Both maps' launches cost 3 to 8 us more than one's.
+// Not for two turns of workgroups or fewer (e F / 128 tiles): one expert that needs a second tile adds a third (32 experts
+// of 2048 x 2048, 80 rows each, even / hot: 197 / 207 us in rings, 187 / 233 in bands). And not in place of the packed
+// streams where these are long: us stream / 96 rows at 32 rows per expert, F = 768 (E = 128, 256) 225 / 204 and 456 / 406,
+// F = 1024 (96) 332 / 294, F = 1536 (48 and 64) 166 / 187 and 411 / 412, F = 2048 (64) 269 / 286.
 extern "C" int ix_moe_pick_bm_shape(long T, long k, long E, long Hd, long F, int packed) {
   const long rows = T * k, e = E > 0 ? E : 1, mean = rows / e;
-  if (mean >= 24 && mean < 400 && ix_moe_bands_fit(rows, Hd, F) && e * (F / 128) >= 2 * IX_STREAM_WORKGROUPS) {
-    if (mean < 72) return 96;
-    if (mean < 130) return 160;
-    if (mean < 164) return 192;
-    if (mean < 240) return 256;
-    if (mean < 280) return 160;
-    return mean < 340 ? 192 : 224;
+  const bool streams = packed && rows < 40 * e && F >= 1536;
+  if (!streams && ix_moe_bands_fit(rows, Hd, F) && e * (F / 128) > 2 * IX_STREAM_WORKGROUPS) {
+    if (mean >= 24 && mean < 155) return mean < 71 ? 96 : (mean < 127 ? 160 : 192);
+    if (mean >= 240 && mean < 400 && T > IX_MOE_TILE_T) return IX_MOE_BM_BY_COUNTS + (mean < 290 ? 160 : 192);
   }
   return packed ? ix_moe_pick_bm_packed(T, k, E) : ix_moe_pick_bm(T, k, E);
 }
 
-extern "C" int ix_moe_permute(const int* topk_idx, const float* topk_prob, long T, long E, long k, long BM,
-                              int* counts, int* offsets, int* sorted_token, float* permuted_prob,
-                              int* combine_rows, int* tile_meta, long max_tiles, int* scratch, void* stream) {
+static int ix_moe_permute_launch(const int* topk_idx, const float* topk_prob, long T, long E, long k, long BM, int* counts,
+                                 int* offsets, int* sorted_token, float* permuted_prob, int* combine_rows, int* tile_meta,
+                                 long max_tiles, const IxMoeTall& tall, int* scratch, void* stream) {
   if (!topk_idx || !topk_prob || !counts || !offsets || !sorted_token || !permuted_prob || !combine_rows ||
       !tile_meta || !scratch)
     return IX_ERR_ARG;
@@ -849,18 +872,36 @@ extern "C" int ix_moe_permute(const int* topk_idx, const float* topk_prob, long 
                        tile_counts);
   if (ntiles > 0 && ntiles <= IX_MOE_FEW_TILES && ntiles * E <= IX_MOE_FEW_COUNTS) {
     hipLaunchKernelGGL(k_moe_offsets_scatter, dim3((unsigned)ntiles), dim3(1024), 0, st, topk_idx, topk_prob, (int)T, (int)E,
-                       (int)k, (int)ntiles, (int)BM, (int)max_tiles, tile_counts, counts, offsets, tile_meta, sorted_token,
-                       permuted_prob, combine_rows);
+                       (int)k, (int)ntiles, (int)BM, (int)max_tiles, tall, tile_counts, counts, offsets, tile_meta,
+                       sorted_token, permuted_prob, combine_rows);
     return ix_launch_status();
   }
   hipLaunchKernelGGL(k_moe_tile_prefix, dim3((unsigned)((E + 3) / 4)), dim3(256), 0, st, tile_counts, (int)ntiles, (int)E,
                      tile_base, counts);
-  hipLaunchKernelGGL(k_moe_offsets, dim3(1), dim3(256), 0, st, (int)E, (int)BM, (int)max_tiles, counts, offsets,
+  hipLaunchKernelGGL(k_moe_offsets, dim3(1), dim3(256), 0, st, (int)E, (int)BM, (int)max_tiles, tall, counts, offsets,
                      tile_meta);
   if (ntiles > 0)
     hipLaunchKernelGGL(k_moe_scatter, dim3((unsigned)ntiles), dim3(1024), 0, st, topk_idx, topk_prob, (int)T, (int)E,
                        (int)k, tile_base, offsets, sorted_token, permuted_prob, combine_rows);
   return ix_launch_status();
+}
+
+extern "C" int ix_moe_permute(const int* topk_idx, const float* topk_prob, long T, long E, long k, long BM,
+                              int* counts, int* offsets, int* sorted_token, float* permuted_prob,
+                              int* combine_rows, int* tile_meta, long max_tiles, int* scratch, void* stream) {
+  return ix_moe_permute_launch(topk_idx, topk_prob, T, E, k, BM, counts, offsets, sorted_token, permuted_prob, combine_rows,
+                               tile_meta, max_tiles, IxMoeTall{}, scratch, stream);
+}
+
+extern "C" int ix_moe_permute_by_counts(const int* topk_idx, const float* topk_prob, long T, long E, long k, long low, long Hd,
+                                        long F, int* counts, int* offsets, int* sorted_token, float* permuted_prob, int* combine_rows,
+                                        int* meta_low, long max_low, int* meta_tall, long max_tall, int* scratch,
+                                        void* stream) {
+  if (!meta_tall || Hd < 256 || F < 128 || (low != 160 && low != 192)) return IX_ERR_ARG;
+  if (max_tall < ix_moe_max_tiles(T, k, E, 256)) return IX_ERR_ARG;
+  if (T <= IX_MOE_TILE_T) return IX_DECLINED;  // one token tile: the launch without a count table
+  return ix_moe_permute_launch(topk_idx, topk_prob, T, E, k, low, counts, offsets, sorted_token, permuted_prob,
+                               combine_rows, meta_low, max_low, ix_moe_tall(low, meta_tall, max_tall, Hd, F), scratch, stream);
 }
 
 // ix_moe_router_topk + ix_moe_permute for a batch of at most one token tile (T <= 256) and E <= 128, in one launch.
@@ -1492,12 +1533,12 @@ extern "C" int ix_moe_experts_tile(const void* x, long ldx, const int* sorted_to
     return ix_moe_experts_launch<128, 128, 2, 2>(xx, ldx, (int)T, rows, sorted_token, permuted_prob, w1, w2, tile_meta,
                                                  max_tiles, it, eo, (int)Hd, (int)F, st);
   if (BM == 96 || BM == 160 || BM == 192 || BM == 224) {
-    if (ix_moe_bands_fit(rows, Hd, F) && ix_aligned(expert_out, 16)) {
+    if (BM != 224 && ix_moe_bands_fit(rows, Hd, F) && ix_aligned(expert_out, 16)) {
       auto bands = BM < 192 ? ix_moe_experts_bands_low : ix_moe_experts_bands_high;
       return bands((int)BM, xx, ldx, (int)T, rows, sorted_token, permuted_prob, w1, w2, tile_meta, max_tiles, it, eo, (int)Hd,
                    (int)F, st);
     }
-    BM = 256;  // a taller tile holds the map's rows as well
+    BM = 256;  // a taller tile holds the map's rows as well (224 rows have no kernel of their own)
   }
   switch (BM) {
     case 32:

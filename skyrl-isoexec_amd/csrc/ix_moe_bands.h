@@ -281,15 +281,14 @@ __global__ __launch_bounds__(256) void k_moe_fc1_glu_bands(const bf16_t* __restr
   ix_gemm_bands<Cfg>(job, Hd / IX_BK, ix_lds);
 }
 
-// Both expert GEMMs over a block map of 32 MI rows a tile, or IX_DECLINED. ONCE / SHARED: which forms of the weight loads are
-// built (ix_dma16): the weights past the caches while nearly every expert has one tile.
-template <int MI, bool ONCE, bool SHARED>
+// Both expert GEMMs over a block map of 32 MI rows a tile, or IX_DECLINED. The weights are loaded past the caches (ix_dma16) while
+// nearly every expert has one tile; SHARED: the height is also used where experts have two, with weight loads that cache.
+template <int MI, bool SHARED>
 static int ix_moe_experts_bands(const bf16_t* x, long ldx, int T, long rows, const int* sorted_token,
                                 const float* permuted_prob, const bf16_t* W1, const bf16_t* W2, const int* meta,
                                 long max_tiles, bf16_t* inter, bf16_t* out, int Hd, int F, hipStream_t st) {
-  static_assert(ONCE || SHARED, "at least one form");
   using C0 = IxBandCfg<MI, !SHARED>;
-  using C1 = IxBandCfg<MI, ONCE>;
+  using C1 = IxBandCfg<MI, true>;
   const long nb1 = F / 128, nb2 = Hd / 256;
   if (max_tiles * nb1 > 0x7fffffffL || max_tiles * nb2 > 0x7fffffffL) return IX_DECLINED;
   static bool attr_set = false;
@@ -316,7 +315,7 @@ static inline bool ix_moe_bands_fit(long rows, long Hd, long F) {
          F / IX_BK >= IX_BAND_MIN_KT && rows < 0x20000000L && (F + 128) * Hd * 2 < 0x40000000L && Hd * 512 < 0x40000000L;
 }
 
-// ix_moe_bands_low.hip: 96 and 160 rows; ix_moe_bands_high.hip: 192 and 224
+// ix_moe_bands_low.hip: 96 and 160 rows; ix_moe_bands_high.hip: 192
 #define IX_MOE_BANDS_ARGS                                                                                              \
   int BM, const bf16_t *x, long ldx, int T, long rows, const int *sorted_token, const float *permuted_prob, const bf16_t *W1, \
       const bf16_t *W2, const int *meta, long max_tiles, bf16_t *inter, bf16_t *out, int Hd, int F, hipStream_t st

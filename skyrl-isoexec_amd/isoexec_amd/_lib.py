@@ -19,6 +19,7 @@ IX_DECLINED = 1
 IX_ERR_SIZE = -3
 DT_F32 = 0
 DT_BF16 = 1
+MOE_BM_BY_COUNTS = 0x10000  # + the lower of the two heights
 
 PRIM = {
     "exp": 0,
@@ -113,9 +114,14 @@ SIGNATURES = {
         c_int,
         [P, P, c_long, c_long, c_long, c_long, P, P, P, P, P, P, c_long, P, P],
     ),
+    "ix_moe_permute_by_counts": (
+        c_int,
+        [P, P, c_long, c_long, c_long, c_long, c_long, c_long, P, P, P, P, P, P, c_long, P, c_long, P, P],
+    ),
     "ix_moe_route_one_tile": (c_int, [P, c_long, c_long, c_long, c_long, c_int, c_float, c_long, P, P, P, P, P, P, P, P,
                                       c_long, P]),
     "ix_moe_block_map": (c_int, [P, c_int, c_long, c_long, c_long, P, P, c_long, P]),
+    "ix_moe_block_map_by_counts": (c_int, [P, c_int, c_long, c_long, c_long, c_long, c_long, P, P, c_long, P, c_long, P]),
     "ix_moe_permute_static_max_ints": (c_size_t, []),
     "ix_moe_permute_static_init": (c_int, []),
     "ix_moe_permute_static": (

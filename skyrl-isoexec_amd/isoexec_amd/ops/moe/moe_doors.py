@@ -93,23 +93,31 @@ def _batched_experts_forward(self, permuted_local_hidden_states, tokens_per_expe
             raise RuntimeError(f"[isoexec-amd] SequentialMLP.forward: tokens_per_expert has {counts.numel()} entries "
                                f"adding up to {total} for {R} permuted rows and {E} local experts")
     BM = int(L.ix_moe_pick_bm_shape(R, 1, E, H, F, 0))
-    max_tiles = int(L.ix_moe_max_tiles(R, 1, E, BM))
-    meta = torch.empty(1 + 3 * max_tiles, dtype=torch.int32, device=dev)
+    low = BM - _lib.MOE_BM_BY_COUNTS
+    maps = []  # (rows per tile, map, its capacity); by counts two, of which the device fills one
+    for bm in (low, 256) if low > 0 else (BM,):
+        max_tiles = int(L.ix_moe_max_tiles(R, 1, E, bm))
+        maps.append((bm, torch.empty(1 + 3 * max_tiles, dtype=torch.int32, device=dev), max_tiles))
     stream = _lib.current_stream(dev)
-    rc = _lib.check(L.ix_moe_block_map(counts.data_ptr(), int(counts.dtype is torch.int64), E, BM, R, None,
-                                       meta.data_ptr(), max_tiles, stream), "ix_moe_block_map")
-    if rc != _lib.IX_OK:
+    buffers = [v for _, meta, max_tiles in maps for v in (meta.data_ptr(), max_tiles)]
+    wide = int(counts.dtype is torch.int64)
+    if low > 0:
+        rc = L.ix_moe_block_map_by_counts(counts.data_ptr(), wide, E, low, H, F, R, None, *buffers, stream)
+    else:
+        rc = L.ix_moe_block_map(counts.data_ptr(), wide, E, BM, R, None, *buffers, stream)
+    if _lib.check(rc, "ix_moe_block_map") != _lib.IX_OK:
         raise RuntimeError(f"[isoexec-amd] ix_moe_block_map declined E={E}")
     rows = torch.arange(R, dtype=torch.int32, device=dev)      # the rows are already in expert order
     probs = permuted_probs.to(torch.float32).contiguous()
     xc = x if x.stride(1) == 1 else x.contiguous()
     inter = torch.empty(R, F, dtype=torch.bfloat16, device=dev)
     out = torch.empty(R, H, dtype=torch.bfloat16, device=dev)
-    rc = _lib.check(L.ix_moe_experts(xc.data_ptr(), xc.stride(0), rows.data_ptr(), probs.data_ptr(), w1.data_ptr(),
-                                     w2.data_ptr(), meta.data_ptr(), max_tiles, BM, inter.data_ptr(), out.data_ptr(), R,
-                                     R, H, F, stream), "ix_moe_experts")
-    if rc != _lib.IX_OK:
-        raise RuntimeError(f"[isoexec-amd] ix_moe_experts declined H={H} F={F}")
+    for bm, meta, max_tiles in maps:
+        rc = _lib.check(L.ix_moe_experts(xc.data_ptr(), xc.stride(0), rows.data_ptr(), probs.data_ptr(), w1.data_ptr(),
+                                         w2.data_ptr(), meta.data_ptr(), max_tiles, bm, inter.data_ptr(), out.data_ptr(), R,
+                                         R, H, F, stream), "ix_moe_experts")
+        if rc != _lib.IX_OK:
+            raise RuntimeError(f"[isoexec-amd] ix_moe_experts declined H={H} F={F}")
     return out, None
 
 

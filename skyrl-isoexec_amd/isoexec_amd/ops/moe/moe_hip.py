@@ -45,15 +45,17 @@ def fused_router_dense(logits: torch.Tensor, k: int, *, scaling_factor: float | 
 
 
 class Permutation:
-    """Device-side routing plan: everything the grouped GEMMs and the combine need."""
+    """Device-side routing plan: everything the grouped GEMMs and the combine need. ``tall``: ``None``, or ``(tile_meta,
+    max_tiles)`` of a second map, of 256-row tiles; the device has left one of the two without tiles."""
 
     __slots__ = ("T", "E", "k", "BM", "BN", "counts", "offsets", "sorted_token", "permuted_prob", "combine_rows",
-                 "tile_meta", "max_tiles")
+                 "tile_meta", "max_tiles", "tall")
 
 
 def permute(topk_idx: torch.Tensor, topk_prob: torch.Tensor, E: int, *, BM: int | None = None,
-            BN: int | None = None, static_scratch: bool = False) -> Permutation:
-    """Expert-major, token-ascending permutation + block map (integer only, no host sync).
+            BN: int | None = None, static_scratch: bool = False, layer: tuple | None = None) -> Permutation:
+    """Expert-major, token-ascending permutation + block map (integer only, no host sync). ``BM=MOE_BM_BY_COUNTS + 160``
+    (or 192): maps of that height and of 256, one of which the device fills, for a ``layer`` of ``(hidden, intermediate)`` size.
 
     ``static_scratch=True`` keeps the kernels' internal tables in the library's file-scope device array instead of a
     torch allocation (``ix_moe_permute_static``; calls that overlap on one GPU race on that array)."""
@@ -63,7 +65,11 @@ def permute(topk_idx: torch.Tensor, topk_prob: torch.Tensor, E: int, *, BM: int 
     L = _lib.lib()
     p = Permutation()
     p.T, p.E, p.k = T, E, k
-    p.BM = int(BM or L.ix_moe_pick_bm(T, k, E))
+    by_counts = BM is not None and BM > _lib.MOE_BM_BY_COUNTS
+    if by_counts and (layer is None or static_scratch or BN not in (None, 256)):
+        raise RuntimeError("[isoexec-amd] a map by counts needs the layer's sizes, scratch of its own and 256 columns")
+    p.BM = BM - _lib.MOE_BM_BY_COUNTS if by_counts else int(BM or L.ix_moe_pick_bm(T, k, E))
+    p.tall = None
     p.BN = int(BN or (128 if p.BM == 128 else 256))  # weight-tile width of the grouped GEMMs: 256, or 128 with BM = 128
     p.max_tiles = int(L.ix_moe_max_tiles(T, k, E, p.BM))
     i32 = dict(dtype=torch.int32, device=dev)
@@ -87,6 +93,17 @@ def permute(topk_idx: torch.Tensor, topk_prob: torch.Tensor, E: int, *, BM: int 
         _lib.check(rc, "ix_moe_permute_static")
         return p
     scratch = torch.empty(max(1, int(L.ix_moe_permute_scratch_ints(T, E))), **i32)
+    if by_counts:
+        max_tall = int(L.ix_moe_max_tiles(T, k, E, 256))
+        p.tall = torch.empty(1 + 3 * max_tall, **i32), max_tall
+        rc = _lib.check(
+            L.ix_moe_permute_by_counts(idx.data_ptr(), prob.data_ptr(), T, E, k, p.BM, *layer,
+                                       p.counts.data_ptr(), p.offsets.data_ptr(), p.sorted_token.data_ptr(),
+                                       p.permuted_prob.data_ptr(), p.combine_rows.data_ptr(), p.tile_meta.data_ptr(), p.max_tiles, p.tall[0].data_ptr(),
+                                       max_tall, scratch.data_ptr(), _lib.current_stream(dev)), "ix_moe_permute_by_counts")
+        if rc != _lib.IX_OK:
+            raise RuntimeError(f"[isoexec-amd] ix_moe_permute_by_counts declined T={T} E={E}")
+        return p
     _lib.check(
         L.ix_moe_permute(idx.data_ptr(), prob.data_ptr(), T, E, k, p.BM,
                          p.counts.data_ptr(), p.offsets.data_ptr(), p.sorted_token.data_ptr(),
@@ -96,7 +113,7 @@ def permute(topk_idx: torch.Tensor, topk_prob: torch.Tensor, E: int, *, BM: int 
 
 
 def route_and_permute(logits: torch.Tensor, k: int, *, pre_softmax: bool = False, scaling_factor: float | None = None,
-                      BM: int | None = None):
+                      BM: int | None = None, layer: tuple | None = None):
     """``router_topk`` then ``permute`` -> ``(topk_idx, topk_prob, Permutation)``. A batch of at most one token tile
     (T <= 256, E <= 128: a decode step) takes ONE launch for both (``ix_moe_route_one_tile``); the integers and the
     weights are the same either way."""
@@ -106,13 +123,14 @@ def route_and_permute(logits: torch.Tensor, k: int, *, pre_softmax: bool = False
     T, E = logits.shape
     if T > 256 or E > 128 or T == 0:
         idx, prob, _, _ = router_topk(logits, k, pre_softmax=pre_softmax, scaling_factor=scaling_factor)
-        return idx, prob, permute(idx, prob, E, BM=BM)
+        return idx, prob, permute(idx, prob, E, BM=BM, layer=layer)
     lg = logits if logits.stride(1) == 1 else logits.contiguous()
     dev = lg.device
     L = _lib.lib()
     p = Permutation()
     p.T, p.E, p.k = T, E, k
     p.BM = int(BM or L.ix_moe_pick_bm(T, k, E))
+    p.tall = None
     p.BN = 128 if p.BM == 128 else 256
     p.max_tiles = int(L.ix_moe_max_tiles(T, k, E, p.BM))
     i32 = dict(dtype=torch.int32, device=dev)
@@ -198,14 +216,16 @@ def experts_forward(x: torch.Tensor, w1: torch.Tensor, w2: torch.Tensor, p: Perm
         if rc == _lib.IX_OK:
             return (out, inter) if return_inter else out
     w1c, w2c = w1.contiguous(), w2.contiguous()  # named: the copies have to outlive the call
-    rc = _lib.check(
-        _lib.lib().ix_moe_experts_tile(xc.data_ptr(), xc.stride(0), p.sorted_token.data_ptr(),
-                                       p.permuted_prob.data_ptr(), w1c.data_ptr(), w2c.data_ptr(), p.tile_meta.data_ptr(), p.max_tiles, p.BM,
-                                       p.BN, inter.data_ptr(), out.data_ptr(), T, rows, H, F,
-                                       _lib.current_stream(dev)),
-        "ix_moe_experts")
-    if rc != _lib.IX_OK:
-        raise RuntimeError(f"[isoexec-amd] ix_moe_experts declined H={H} F={F}")
+    maps = [(p.BM, p.tile_meta, p.max_tiles)] + ([(256, *p.tall)] if p.tall else [])
+    for bm, meta, max_tiles in maps:
+        rc = _lib.check(
+            _lib.lib().ix_moe_experts_tile(xc.data_ptr(), xc.stride(0), p.sorted_token.data_ptr(),
+                                           p.permuted_prob.data_ptr(), w1c.data_ptr(), w2c.data_ptr(), meta.data_ptr(),
+                                           max_tiles, bm, p.BN, inter.data_ptr(), out.data_ptr(), T, rows, H, F,
+                                           _lib.current_stream(dev)),
+            "ix_moe_experts")
+        if rc != _lib.IX_OK:
+            raise RuntimeError(f"[isoexec-amd] ix_moe_experts declined H={H} F={F}")
     return (out, inter) if return_inter else out
 
 
@@ -254,13 +274,16 @@ def moe_ffn_forward(x: torch.Tensor, router_weight: torch.Tensor, w1: torch.Tens
         raise RuntimeError("[isoexec-amd] router GEMM declined")
     if logit_bias is not None:
         logits = logits + logit_bias  # elementwise, per token
+    layer = None
     if BM is None:
         L, (T, E) = _lib.lib(), logits.shape
         if w2.ndim == 3 and w1.is_contiguous() and w2.is_contiguous():  # the bands read the matrices themselves
-            BM = int(L.ix_moe_pick_bm_shape(T, k, E, w2.shape[1], w2.shape[2], int(packed is not None)))
+            layer = w2.shape[1], w2.shape[2]
+            BM = int(L.ix_moe_pick_bm_shape(T, k, E, *layer, int(packed is not None)))
         elif packed is not None:
             BM = int(L.ix_moe_pick_bm_packed(T, k, E))
-    idx, prob, p = route_and_permute(logits, k, pre_softmax=pre_softmax, scaling_factor=scaling_factor, BM=BM)
+    idx, prob, p = route_and_permute(logits, k, pre_softmax=pre_softmax, scaling_factor=scaling_factor, BM=BM,
+                                     layer=layer)
     if routing_out is not None:
         routing_out.append(idx)
     expert_out = experts_forward(x, w1, w2, p, packed=packed)

@@ -1,4 +1,5 @@
-"""Which tile a product's sizes choose, on the host: the lines between the bands and the other shapes."""
+"""Which tile a product's sizes choose, on the host: the lines between the bands and the other shapes, and the
+height of an expert tile."""
 import pytest
 
 from isoexec_amd import _lib
@@ -10,3 +11,25 @@ from isoexec_amd import _lib
     (64, 151936, 4096, 128, 1), (256, 151936, 4096, 256, 2)])  # up to 64 rows; a whole 256-row tile
 def test_dense_tiles(m, n, k, tile_width, parts):
     assert _lib.lib().ix_gemm_bf16_n_tiles(m, n, k, 0) == parts * ((n + tile_width - 1) // tile_width)
+
+
+BY_COUNTS = _lib.MOE_BM_BY_COUNTS
+
+
+@pytest.mark.parametrize("mean,plain,packed", [(15, 32, 32), (23, 128, 64), (24, 96, 96), (70, 96, 96), (71, 160, 160), (126, 160, 160),
+                                               (127, 192, 192), (154, 192, 192), (155, 256, 256), (239, 256, 256),
+                                               (240, BY_COUNTS + 160, BY_COUNTS + 160), (289, BY_COUNTS + 160, BY_COUNTS + 160),
+                                               (290, BY_COUNTS + 192, BY_COUNTS + 192), (399, BY_COUNTS + 192, BY_COUNTS + 192),
+                                               (400, 256, 256)])
+def test_expert_tiles(mean, plain, packed):
+    pick = _lib.lib().ix_moe_pick_bm_shape
+    assert pick(16 * mean, 8, 128, 2048, 768, 0) == plain and pick(16 * mean, 8, 128, 2048, 768, 1) == packed
+
+
+@pytest.mark.parametrize("T,k,E,hd,f,packed,rows", [
+    (1024, 2, 64, 2048, 2048, 0, 96), (1024, 2, 64, 2048, 2048, 1, 64), (1280, 2, 64, 2048, 2048, 1, 96),  # long packed streams
+    (1024, 2, 64, 2048, 1024, 0, 128), (640, 4, 32, 2048, 2048, 0, 128), (2400, 4, 32, 4096, 2048, 0, 256),  # two turns of workgroups
+    (256, 1, 1, 2048, 131072, 0, 256),  # one token tile
+    (1024, 2, 64, 896, 2048, 0, 128), (1024, 2, 64, 2048, 2000, 0, 128)])  # sizes that bands do not serve
+def test_expert_tiles_of_other_layers(T, k, E, hd, f, packed, rows):
+    assert _lib.lib().ix_moe_pick_bm_shape(T, k, E, hd, f, packed) == rows

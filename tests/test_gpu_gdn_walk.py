@@ -76,6 +76,28 @@ def test_walk_by_the_rule_equals_the_token_staged_scan(K, H, HV, V, dtype, lens)
     assert same_bits(stateless_forward(*args, cu_seqlens=cu), run(16 | (1 << 8), zero))
 
 
+@pytest.mark.parametrize("K,H,HV,V,dtype,n", [
+    (64, 2, 4, 64, torch.bfloat16, 3), (128, 2, 4, 64, torch.float32, 3),  # slices split over two lanes
+    (128, 16, 32, 128, torch.bfloat16, 2), (64, 16, 32, 64, torch.float32, 8), (256, 2, 4, 64, torch.bfloat16, 3),  # whole slices
+    (128, 16, 32, 128, torch.float32, 1)])
+def test_null_lane_beside_a_staging_wave(K, H, HV, V, dtype, n):
+    """Sequences without a state row: outputs zero, the pool's other rows as in ``k_gdn_scan``, the null row untouched."""
+    from isoexec_amd.ops.gdn.gdn_ops import gdn_recurrent_kernel
+
+    lens = [33, 16, 5, 18, 1, 40, 31, 2][:n]
+    args = make(lens, H, HV, K, V, dtype, n)
+    cu = offsets(lens)
+    rows = torch.arange(1, n + 1, dtype=torch.int32, device=DEV)
+    rows[n // 2] = 0
+    pa = torch.randn(n + 1, HV, V, K, generator=cpu_gen(6)).to(DEV)
+    pb = pa.clone()
+    run = lambda code, pool: gdn_recurrent_kernel(*args, ssm_state=pool, state_indices=rows, cu_seqlens=cu, time_tile=code)
+    want, got = run(16 | (1 << 8), pa), run(0, pb)
+    assert same_bits(got, want) and same_bits(pb, pa)
+    a, b = sum(lens[:n // 2]), sum(lens[:n // 2 + 1])
+    assert not got[0, a:b].any() and (n == 1 or got.any())
+
+
 def test_more_sequences_than_a_workgroup_ranks():
     from isoexec_amd.ops.gdn.gdn_ops import gdn_recurrent_kernel, stateless_forward
 
@@ -98,6 +120,29 @@ def test_boundary_form_in_one_walk_against_the_oracle(K, H, HV, chunk):
     f = lambda t: bf16_to_np(t[0].cpu())
     want, _, _ = o_gdn.cpr_forward(f(q), f(k), f(v), gate[0].cpu().numpy(), f(beta), lens, chunk, prims=DevicePrims(DEV))
     assert same_bits(gdn_cpr_fwd(q, k, v, gate, beta, cu_seqlens=offsets(lens), chunk_size=chunk)[0].cpu(), np_to_bf16(want))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("K,V,n", [(128, 128, 1), (128, 128, 2), (128, 128, 4), (128, 128, 9), (64, 64, 5), (64, 64, 8), (64, 64, 16),
+                                   (64, 64, 33), (256, 64, 2), (256, 64, 4), (256, 64, 17)])
+def test_boundary_form_by_the_rule_equals_few_heads_alone(K, V, n, dtype):
+    """Whole slices with a staging wave, without one, and two rows a lane group, as 32 heads and n sequences choose them, against
+    the same sequence and four heads of it in a call of their own (split slices up to K = 128, which the oracle test above
+    covers; whole slices with a staging wave at K = 256): at least three chunks, lengths around the tile and the chunk."""
+    from isoexec_amd.ops.gdn.gdn_ops import stateless_forward
+
+    H, HV, chunk = 16, 32, 32
+    lens = [(2 * chunk + 13 * i * i) % 101 + 1 for i in range(n)]
+    q, k, v, gate, beta = args = make(lens, H, HV, K, V, dtype, K + n)
+    got = stateless_forward(*args, cu_seqlens=offsets(lens), chunk_size=chunk)
+    at = 0
+    for i, length in enumerate(lens):
+        t, h = slice(at, at + length), 2 * (i % 8)
+        at += length
+        alone = stateless_forward(q[:, t, h:h + 2].contiguous(), k[:, t, h:h + 2].contiguous(), v[:, t, 2 * h:2 * h + 4].contiguous(),
+                                  gate[:, t, 2 * h:2 * h + 4].contiguous(), beta[:, t, 2 * h:2 * h + 4].contiguous(),
+                                  cu_seqlens=offsets([length]), chunk_size=chunk)
+        assert same_bits(got[:, t, 2 * h:2 * h + 4], alone), (i, length)
 
 
 def test_lane_pairs_of_many_sequences_with_the_norm_folded_in():

@@ -148,9 +148,11 @@ int ix_moe_combine_add_rmsnorm(const void* expert_out, const int* combine_rows, 
  * (32x256, 128x128, 256x256 on eight waves, 256x256 on four waves, 128x256, 64x32); 4 takes the streaming form of its
  * tile (one workgroup per CU walks many tiles) when the product has at least 512 tiles and the form serves it (bf16 C,
  * no bias, K a multiple of 64 and >= 704, N and ldc multiples of 8, C 16-byte aligned), 7 never does, 8 always does
- * and declines what the form does not serve. Every choice gives the same bits.
- * row_max_parts: NULL, or fp32 [M, parts_ld] receiving per part the max of the stored values (one part per column
- * tile; two for tiles 4, 7, 8), parts_ld >= ix_gemm_bf16_n_tiles(M, N, K, tile). */
+ * and declines what the form does not serve. 14..17 are bands of 128, 160, 192 and 224 rows x 256 columns of that form, K >= 768:
+ * asked for by number they decline what it does not serve. Every choice gives the same bits.
+ * row_max_parts: NULL, or fp32 [M, parts_ld] receiving per part the max of the stored values, parts_ld >=
+ * ix_gemm_bf16_n_tiles(M, N, K, tile), which alone says how many parts a row has: one per column tile, two for tiles 4, 7 and 8, four
+ * for the bands, which tile 0 may choose (a part may be stored more than once where the call is one that bands do not serve). */
 int ix_gemm_bf16_nt(const void* A, long lda, const void* W, long ldw, const void* bias, void* C, int c_dtype,
                     long ldc, long M, long N, long K, int tile, float* row_max_parts, long parts_ld,
                     void* stream);

@@ -438,8 +438,8 @@ void k_gdn_scan_pairs(const TIO* __restrict__ q, const TIO* __restrict__ k, cons
 // exactly one wave per SIMD), and everything that is not the chain is kept out of its way:
 //   * tiles of 16 tokens, staged twice in LDS: the next tile's global loads are issued before this tile's tokens and
 //     written to LDS after them; one barrier per tile;
-//   * no LDS store between a tile's tokens (an LDS load may not pass one): a token's output is the same in all lanes of
-//     its row, so lane tt keeps token tt's and the tile is written out at its end;
+//   * hardly an LDS store between a tile's tokens (an LDS load may not pass one): a token's output is the same in all lanes of
+//     its row, so lane tt keeps token tt's and the row's lanes store together, once every L tokens;
 //   * sixteen tokens of straight-line code, so the output's tree runs in the shadow of the next token's decay and dot;
 //   * LONE, at a workgroup or two per CU: a fifth wave stages the tiles and writes the outputs out, so that the four others
 //     meet nothing but their tokens and the barrier (a fifth of the walk at one wave per SIMD, which waits for its own every
@@ -591,7 +591,10 @@ __global__ __launch_bounds__(LONE ? 320 : 256) void k_gdn_walk(const TIO* __rest
     }
   };
   if constexpr (LONE) {
-    if (tid >= 256) {  // the staging wave: as many barriers as the others
+    // The staging wave: as many barriers as the others. The branch is the same for a whole wave (256 is a multiple of 64); with the
+    // wave number in a scalar register the compiler keeps both sides' values at once, and two workgroups no longer fit a CU (K = 256,
+    // 3 x 1000 tokens 208 -> 300 us).
+    if (tid >= 256) {
       fetch(0);
       commit(0);
       if (tiles > 1) fetch(T);

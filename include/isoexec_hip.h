@@ -358,11 +358,11 @@ long ix_moe_max_tiles(long T, long k, long E, long BM);   /* ceil(T*k/BM) + E */
 size_t ix_moe_permute_scratch_ints(long T, long E);
 int ix_moe_pick_bm(long T, long k, long E);               /* 32, 128 or 256 */
 int ix_moe_pick_bm_packed(long T, long k, long E);        /* 32, 64, 128 or 256: for callers that hold packed matrices */
-/* The same for callers that know the layer's sizes (fc1 [E, 2F, Hd], fc2 [E, Hd, F]): also 96, 160 and 192, and
- * IX_MOE_BM_BY_COUNTS + 160 or 192 where the routing decides between that height and 256 rows: the maps then come from
- * ix_moe_permute_by_counts or ix_moe_block_map_by_counts. */
-#define IX_MOE_BM_BY_COUNTS 0x10000
+/* The same for callers that know the layer's sizes (fc1 [E, 2F, Hd], fc2 [E, Hd, F]): also 96, 160 and 192. */
 int ix_moe_pick_bm_shape(long T, long k, long E, long Hd, long F, int packed);
+/* 160 or 192 where the routing decides between that height and 256 rows: the faster maps then come from
+ * ix_moe_permute_by_counts or ix_moe_block_map_by_counts with it as `low`. 0 elsewhere. */
+int ix_moe_pick_low_bm(long T, long k, long E, long Hd, long F);
 
 /* fused_permute_index / ref_permute_index (moe_router_o2_kernel.py:313-351,389-397) plus the
  * block map (moe_fused_experts.py:156-205) and the inverse permutation of

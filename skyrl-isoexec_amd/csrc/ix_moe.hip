@@ -838,14 +838,21 @@ extern "C" int ix_moe_pick_bm_packed(long T, long k, long E) {
 // of 2048 x 2048, 80 rows each, even / hot: 197 / 207 us in rings, 187 / 233 in bands). And not in place of the packed
 // streams where these are long: us stream / 96 rows at 32 rows per expert, F = 768 (E = 128, 256) 225 / 204 and 456 / 406,
 // F = 1024 (96) 332 / 294, F = 1536 (48 and 64) 166 / 187 and 411 / 412, F = 2048 (64) 269 / 286.
+static bool ix_moe_bands_pay(long rows, long E, long Hd, long F) {
+  return ix_moe_bands_fit(rows, Hd, F) && E * (F / 128) > 2 * IX_STREAM_WORKGROUPS;
+}
+
 extern "C" int ix_moe_pick_bm_shape(long T, long k, long E, long Hd, long F, int packed) {
   const long rows = T * k, e = E > 0 ? E : 1, mean = rows / e;
   const bool streams = packed && rows < 40 * e && F >= 1536;
-  if (!streams && ix_moe_bands_fit(rows, Hd, F) && e * (F / 128) > 2 * IX_STREAM_WORKGROUPS) {
-    if (mean >= 24 && mean < 155) return mean < 71 ? 96 : (mean < 127 ? 160 : 192);
-    if (mean >= 240 && mean < 400 && T > IX_MOE_TILE_T) return IX_MOE_BM_BY_COUNTS + (mean < 290 ? 160 : 192);
-  }
+  if (!streams && mean >= 24 && mean < 155 && ix_moe_bands_pay(rows, e, Hd, F)) return mean < 71 ? 96 : (mean < 127 ? 160 : 192);
   return packed ? ix_moe_pick_bm_packed(T, k, E) : ix_moe_pick_bm(T, k, E);
+}
+
+extern "C" int ix_moe_pick_low_bm(long T, long k, long E, long Hd, long F) {
+  const long rows = T * k, e = E > 0 ? E : 1, mean = rows / e;
+  if (mean < 240 || mean >= 400 || T <= IX_MOE_TILE_T || !ix_moe_bands_pay(rows, e, Hd, F)) return 0;
+  return mean < 290 ? 160 : 192;
 }
 
 static int ix_moe_permute_launch(const int* topk_idx, const float* topk_prob, long T, long E, long k, long BM, int* counts,

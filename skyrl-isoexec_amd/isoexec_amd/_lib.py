@@ -19,7 +19,6 @@ IX_DECLINED = 1
 IX_ERR_SIZE = -3
 DT_F32 = 0
 DT_BF16 = 1
-MOE_BM_BY_COUNTS = 0x10000  # + the lower of the two heights
 
 PRIM = {
     "exp": 0,
@@ -110,6 +109,7 @@ SIGNATURES = {
     "ix_moe_permute_scratch_ints": (c_size_t, [c_long, c_long]),
     "ix_moe_pick_bm": (c_int, [c_long, c_long, c_long]),
     "ix_moe_pick_bm_shape": (c_int, [c_long, c_long, c_long, c_long, c_long, c_int]),
+    "ix_moe_pick_low_bm": (c_int, [c_long, c_long, c_long, c_long, c_long]),
     "ix_moe_permute": (
         c_int,
         [P, P, c_long, c_long, c_long, c_long, P, P, P, P, P, P, c_long, P, P],

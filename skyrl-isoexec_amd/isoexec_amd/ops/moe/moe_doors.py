@@ -92,19 +92,19 @@ def _batched_experts_forward(self, permuted_local_hidden_states, tokens_per_expe
         if total != R or counts.numel() != E:
             raise RuntimeError(f"[isoexec-amd] SequentialMLP.forward: tokens_per_expert has {counts.numel()} entries "
                                f"adding up to {total} for {R} permuted rows and {E} local experts")
-    BM = int(L.ix_moe_pick_bm_shape(R, 1, E, H, F, 0))
-    low = BM - _lib.MOE_BM_BY_COUNTS
-    maps = []  # (rows per tile, map, its capacity); by counts two, of which the device fills one
-    for bm in (low, 256) if low > 0 else (BM,):
+    low = int(L.ix_moe_pick_low_bm(R, 1, E, H, F))
+    heights = (low, 256) if low else (int(L.ix_moe_pick_bm_shape(R, 1, E, H, F, 0)),)
+    maps = []  # (rows per tile, map, its capacity); of two the device fills one
+    for bm in heights:
         max_tiles = int(L.ix_moe_max_tiles(R, 1, E, bm))
         maps.append((bm, torch.empty(1 + 3 * max_tiles, dtype=torch.int32, device=dev), max_tiles))
     stream = _lib.current_stream(dev)
     buffers = [v for _, meta, max_tiles in maps for v in (meta.data_ptr(), max_tiles)]
     wide = int(counts.dtype is torch.int64)
-    if low > 0:
+    if low:
         rc = L.ix_moe_block_map_by_counts(counts.data_ptr(), wide, E, low, H, F, R, None, *buffers, stream)
     else:
-        rc = L.ix_moe_block_map(counts.data_ptr(), wide, E, BM, R, None, *buffers, stream)
+        rc = L.ix_moe_block_map(counts.data_ptr(), wide, E, *heights, R, None, *buffers, stream)
     if _lib.check(rc, "ix_moe_block_map") != _lib.IX_OK:
         raise RuntimeError(f"[isoexec-amd] ix_moe_block_map declined E={E}")
     rows = torch.arange(R, dtype=torch.int32, device=dev)      # the rows are already in expert order

@@ -54,8 +54,8 @@ class Permutation:
 
 def permute(topk_idx: torch.Tensor, topk_prob: torch.Tensor, E: int, *, BM: int | None = None,
             BN: int | None = None, static_scratch: bool = False, layer: tuple | None = None) -> Permutation:
-    """Expert-major, token-ascending permutation + block map (integer only, no host sync). ``BM=MOE_BM_BY_COUNTS + 160``
-    (or 192): maps of that height and of 256, one of which the device fills, for a ``layer`` of ``(hidden, intermediate)`` size.
+    """Expert-major, token-ascending permutation + block map (integer only, no host sync). With ``layer``, the experts'
+    ``(hidden, intermediate)`` size, maps of two heights, BM (160 or 192) and 256, one of which the device fills.
 
     ``static_scratch=True`` keeps the kernels' internal tables in the library's file-scope device array instead of a
     torch allocation (``ix_moe_permute_static``; calls that overlap on one GPU race on that array)."""
@@ -65,10 +65,9 @@ def permute(topk_idx: torch.Tensor, topk_prob: torch.Tensor, E: int, *, BM: int 
     L = _lib.lib()
     p = Permutation()
     p.T, p.E, p.k = T, E, k
-    by_counts = BM is not None and BM > _lib.MOE_BM_BY_COUNTS
-    if by_counts and (layer is None or static_scratch or BN not in (None, 256)):
-        raise RuntimeError("[isoexec-amd] a map by counts needs the layer's sizes, scratch of its own and 256 columns")
-    p.BM = BM - _lib.MOE_BM_BY_COUNTS if by_counts else int(BM or L.ix_moe_pick_bm(T, k, E))
+    if layer is not None and (BM not in (160, 192) or static_scratch or BN not in (None, 256)):
+        raise RuntimeError("[isoexec-amd] maps of two heights take BM 160 or 192, scratch of their own and 256 columns")
+    p.BM = int(BM or L.ix_moe_pick_bm(T, k, E))
     p.tall = None
     p.BN = int(BN or (128 if p.BM == 128 else 256))  # weight-tile width of the grouped GEMMs: 256, or 128 with BM = 128
     p.max_tiles = int(L.ix_moe_max_tiles(T, k, E, p.BM))
@@ -93,7 +92,7 @@ def permute(topk_idx: torch.Tensor, topk_prob: torch.Tensor, E: int, *, BM: int 
         _lib.check(rc, "ix_moe_permute_static")
         return p
     scratch = torch.empty(max(1, int(L.ix_moe_permute_scratch_ints(T, E))), **i32)
-    if by_counts:
+    if layer is not None:
         max_tall = int(L.ix_moe_max_tiles(T, k, E, 256))
         p.tall = torch.empty(1 + 3 * max_tall, **i32), max_tall
         rc = _lib.check(
@@ -274,12 +273,16 @@ def moe_ffn_forward(x: torch.Tensor, router_weight: torch.Tensor, w1: torch.Tens
         raise RuntimeError("[isoexec-amd] router GEMM declined")
     if logit_bias is not None:
         logits = logits + logit_bias  # elementwise, per token
-    layer = None
+    layer = None  # the layer's sizes where the counts decide between two heights
     if BM is None:
         L, (T, E) = _lib.lib(), logits.shape
         if w2.ndim == 3 and w1.is_contiguous() and w2.is_contiguous():  # the bands read the matrices themselves
-            layer = w2.shape[1], w2.shape[2]
-            BM = int(L.ix_moe_pick_bm_shape(T, k, E, *layer, int(packed is not None)))
+            sizes = w2.shape[1], w2.shape[2]
+            BM = int(L.ix_moe_pick_low_bm(T, k, E, *sizes))
+            if BM:
+                layer = sizes
+            else:
+                BM = int(L.ix_moe_pick_bm_shape(T, k, E, *sizes, int(packed is not None)))
         elif packed is not None:
             BM = int(L.ix_moe_pick_bm_packed(T, k, E))
     idx, prob, p = route_and_permute(logits, k, pre_softmax=pre_softmax, scaling_factor=scaling_factor, BM=BM,

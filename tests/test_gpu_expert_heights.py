@@ -42,12 +42,11 @@ def _tiles(meta, n):
     (12289, 512, 8, 0), (16640, 130, 2, 1), (17000, 512, 8, 4)])  # the last three: more counts than one launch takes
 @pytest.mark.parametrize("low_rows", [160, 192])
 def test_map_by_counts(t, e, k, hot, low_rows):
-    from isoexec_amd import _lib
     from isoexec_amd.ops.moe.moe_hip import permute
 
     idx, prob = _routing(t, e, k, hot, t + e)
     hd, f = 2048, 768
-    p = permute(idx, prob, e, BM=_lib.MOE_BM_BY_COUNTS + low_rows, layer=(hd, f))
+    p = permute(idx, prob, e, BM=low_rows, layer=(hd, f))
     want_rows = _height(p.counts.tolist(), low_rows, hd, f)
     want = permute(idx, prob, e, BM=want_rows)
     for name in ("counts", "offsets", "sorted_token", "permuted_prob", "combine_rows"):
@@ -128,8 +127,7 @@ def test_layer_by_counts_eager_and_captured():
     from isoexec_amd.ops.mm.mm_hip import router_gemm
 
     t, e, k, hd, f = 4480, 128, 8, 1024, 768
-    BM = _lib.lib().ix_moe_pick_bm_shape(t, k, e, hd, f, 0)
-    assert BM == _lib.MOE_BM_BY_COUNTS + 160
+    assert _lib.lib().ix_moe_pick_low_bm(t, k, e, hd, f) == 160
     w1, w2 = _layer(e, hd, f, 12)
     router = (torch.randn(e, hd, generator=_gen(1), device=DEV) * 0.02).to(torch.bfloat16)
     x = torch.randn(t, hd, generator=_gen(2), device=DEV).to(torch.bfloat16)
@@ -138,7 +136,7 @@ def test_layer_by_counts_eager_and_captured():
     run = lambda bias, **kw: moe_ffn_forward(x, router, w1, w2, k, pre_softmax=True, logit_bias=bias, **kw)
     want = [run(b, BM=32) for b in biases]
     for b, w, tall in zip(biases, want, (False, True)):
-        p = route_and_permute(router_gemm(x, router) + b, k, pre_softmax=True, BM=BM, layer=(hd, f))[2]
+        p = route_and_permute(router_gemm(x, router) + b, k, pre_softmax=True, BM=160, layer=(hd, f))[2]
         assert (int(p.tall[0][0]) > 0, int(p.tile_meta[0]) > 0) == (tall, not tall)
         assert torch.equal(run(b), w)
     static = biases[0].clone()

@@ -13,17 +13,20 @@ def test_dense_tiles(m, n, k, tile_width, parts):
     assert _lib.lib().ix_gemm_bf16_n_tiles(m, n, k, 0) == parts * ((n + tile_width - 1) // tile_width)
 
 
-BY_COUNTS = _lib.MOE_BM_BY_COUNTS
-
-
 @pytest.mark.parametrize("mean,plain,packed", [(15, 32, 32), (23, 128, 64), (24, 96, 96), (70, 96, 96), (71, 160, 160), (126, 160, 160),
                                                (127, 192, 192), (154, 192, 192), (155, 256, 256), (239, 256, 256),
-                                               (240, BY_COUNTS + 160, BY_COUNTS + 160), (289, BY_COUNTS + 160, BY_COUNTS + 160),
-                                               (290, BY_COUNTS + 192, BY_COUNTS + 192), (399, BY_COUNTS + 192, BY_COUNTS + 192),
-                                               (400, 256, 256)])
+                                               (240, 256, 256), (400, 256, 256)])
 def test_expert_tiles(mean, plain, packed):
     pick = _lib.lib().ix_moe_pick_bm_shape
     assert pick(16 * mean, 8, 128, 2048, 768, 0) == plain and pick(16 * mean, 8, 128, 2048, 768, 1) == packed
+
+
+@pytest.mark.parametrize("T,k,E,hd,f,low", [
+    (16 * 239, 8, 128, 2048, 768, 0), (16 * 240, 8, 128, 2048, 768, 160), (16 * 289, 8, 128, 2048, 768, 160),
+    (16 * 290, 8, 128, 2048, 768, 192), (16 * 399, 8, 128, 2048, 768, 192), (16 * 400, 8, 128, 2048, 768, 0),
+    (2400, 4, 32, 4096, 2048, 0), (256, 1, 1, 2048, 131072, 0), (257, 1, 1, 1024, 131072, 160), (4000, 8, 128, 2048, 700, 0)])
+def test_the_lower_of_two_heights(T, k, E, hd, f, low):
+    assert _lib.lib().ix_moe_pick_low_bm(T, k, E, hd, f) == low
 
 
 @pytest.mark.parametrize("T,k,E,hd,f,packed,rows", [

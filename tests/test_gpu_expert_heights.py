@@ -154,3 +154,25 @@ def test_layer_by_counts_eager_and_captured():
         torch.cuda.synchronize()
         assert torch.equal(out, want[i]), i
         assert torch.equal(run(static), want[i])
+
+
+@pytest.mark.parametrize("hot", [0, 2])
+def test_grouped_rows_by_counts(hot):
+    """``SequentialMLP.forward``'s door at a size where the counts decide, against the layer's own experts."""
+    from types import SimpleNamespace
+
+    from isoexec_amd import _lib
+    from isoexec_amd.ops.moe import moe_doors
+    from isoexec_amd.ops.moe.moe_hip import experts_forward, permute
+
+    t, e, k, hd, f = 4480, 128, 8, 1024, 768
+    assert _lib.lib().ix_moe_pick_low_bm(t * k, 1, e, hd, f) == 160
+    w1, w2 = _layer(e, hd, f, 13)
+    idx, prob = _routing(t, e, k, hot, 5)
+    x = torch.randn(t, hd, generator=_gen(6), device=DEV).to(torch.bfloat16)
+    p = permute(idx, prob, e, BM=32)
+    experts = [SimpleNamespace(linear_fc1=SimpleNamespace(weight=w1[i]), linear_fc2=SimpleNamespace(weight=w2[i])) for i in range(e)]
+    mlp = SimpleNamespace(local_experts=experts, num_local_experts=e)
+    for counts in (p.counts, p.counts.long().cpu()):
+        out, bias = moe_doors._batched_experts_forward(mlp, x.index_select(0, p.sorted_token.long()), counts, p.permuted_prob)
+        assert bias is None and torch.equal(out, experts_forward(x, w1, w2, p))

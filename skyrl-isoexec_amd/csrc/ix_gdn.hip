@@ -619,17 +619,15 @@ __global__ __launch_bounds__(LONE ? 320 : 256) void k_gdn_walk(const TIO* __rest
   // 120 us instead of 104
 #pragma unroll
   for (int j = 0; j < RPL; ++j) {
-    if (state) {
-      const float* sp = state + (((long)row0 * HV + hv) * V + vb * R + r + j * RW) * K + kbase;
-      if constexpr (E == 8) {
-        const float4 a = *reinterpret_cast<const float4*>(sp);
-        const float4 b = *reinterpret_cast<const float4*>(sp + 4);
-        S[j][0] = a.x; S[j][1] = a.y; S[j][2] = a.z; S[j][3] = a.w;
-        S[j][4] = b.x; S[j][5] = b.y; S[j][6] = b.z; S[j][7] = b.w;
-      } else {
+    const float* sp = state + (((long)row0 * HV + hv) * V + vb * R + r + j * RW) * K + kbase;
+    if constexpr (E == 4) {
 #pragma unroll
-        for (int i = 0; i < E; ++i) S[j][i] = sp[i * 2];
-      }
+      for (int i = 0; i < E; ++i) S[j][i] = state ? sp[i * 2] : 0.0f;
+    } else if (state) {
+      const float4 a = *reinterpret_cast<const float4*>(sp);
+      const float4 b = *reinterpret_cast<const float4*>(sp + 4);
+      S[j][0] = a.x; S[j][1] = a.y; S[j][2] = a.z; S[j][3] = a.w;
+      S[j][4] = b.x; S[j][5] = b.y; S[j][6] = b.z; S[j][7] = b.w;
     } else {
 #pragma unroll
       for (int i = 0; i < E; ++i) S[j][i] = 0.0f;

@@ -205,14 +205,19 @@ __global__ __launch_bounds__(256) void k_gdn_scan(const TIO* __restrict__ q, con
   }
 }
 
-// ---- the same scan with a state row held by a PAIR of lanes (K = 128) ---------------------------------------
-// Lane l and lane l + 32 of a wave own one state row: the lower one k = 0..63, the upper one k = 64..127, 64
-// state floats each. The row's arithmetic is that of k_gdn_scan statement for statement -- per 8-element slice the
-// same two multiply-add chains and their join (ix_dot8), the adjacent-pairwise tree over the 16 slice sums, here
-// three levels inside the lane (ix_tree8) and the last one across the two halves -- so the two kernels agree bit
-// for bit, and which one runs is a staging choice like the time tile. What changes is the cost: 15 of the 16 tree
-// adds per dot product no longer cross lanes, and a wave instruction serves 32 rows with 64 elements each instead
-// of 4 rows x RPL with 8: about 9.4 instead of 11.3 vector instructions per row and token.
+// ---- the same scan with a state row held by FOUR lanes and updated by the matrix pipe (K = 128) ----------------
+// Lanes r, r + 16, r + 32, r + 48 of a wave own state rows r and r + 16 of the wave's 32, lane group g = lane / 16 the
+// elements k = 32 g .. 32 g + 31 of both: 64 state floats per lane. The row's arithmetic is that of k_gdn_scan statement
+// for statement -- per 8-element slice the same two multiply-add chains and their join (ix_dot8), the adjacent-pairwise
+// tree over the 16 slice sums, here two levels inside the lane, one across neighbouring lane groups and one across the
+// wave's halves -- so the two kernels agree bit for bit, and which one runs is a staging choice like the time tile.
+// The rank-one update S += d k is four v_mfma_f32_16x16x1_4b_f32: state rows are the columns (B = d), the elements of k the
+// rows (A, one value per lane), S the accumulator, whose register layout is the one above. With one product per element
+// that instruction is a fused multiply-add, rounded once, subnormals kept (2 M random, tiny and special operands against fmaf:
+// every bit but a NaN's payload); of the four multiply-adds per element and token one leaves the vector pipe, which bounds
+// this kernel: 250 vector and matrix instructions per token for a wave's 32 rows. Two rows per lane, and not one with 64
+// elements, because every lane reads all its elements of k and q from LDS for each token: 18 reads of a wave instead of 34.
+// 64 x 2560 tokens, 32 heads: 10.1 ms on the vector pipe alone (a row held by two lanes), 8.9 ms this way.
 // Compact state form only (one pool row per sequence, stored after the last token; without a pool the sequences start
 // from zero and nothing is stored).
 #define IX_GDN_SORT_MAX 256  // sequences a workgroup ranks by length
@@ -238,24 +243,28 @@ __device__ __forceinline__ float ix_add_halves(float v) {
   const auto r = __builtin_amdgcn_permlane32_swap(u, u, false, false);
   return __uint_as_float(r[0]) + __uint_as_float(r[1]);  // (own half) + (other half) or the reverse: same bits
 }
+// Two sums over the wave's four groups of sixteen lanes, (0 + 1) + (2 + 3): groups 0 and 2 return a's, 1 and 3 b's.
+__device__ __forceinline__ float ix_add_groups2(float a, float b) {
+  const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+  return ix_add_halves(__uint_as_float(r[0]) + __uint_as_float(r[1]));
+}
+typedef float ix_f32x16 __attribute__((ext_vector_type(16)));
 
 template <typename TIO>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3)))
-void k_gdn_scan_pairs(const TIO* __restrict__ q, const TIO* __restrict__ k, const TIO* __restrict__ v,
+void k_gdn_scan_quads(const TIO* __restrict__ q, const TIO* __restrict__ k, const TIO* __restrict__ v,
                       const float* __restrict__ g, const TIO* __restrict__ beta, TIO* __restrict__ o,
                       float* __restrict__ state, const int* __restrict__ cu, const int* __restrict__ sidx,
                       long q_pitch, long k_pitch, long v_pitch, int N, int H, int HV, int V, float scale, int TT,
                       const bf16_t* __restrict__ gate, long gate_stride_t, const bf16_t* __restrict__ norm_w,
                       float norm_eps, int zero_centered) {
   constexpr int K = 128;
-  constexpr int R = 128;  // state rows per workgroup: 4 waves x 32 rows
+  constexpr int KP = K + 12;  // a token's k or q in LDS: 32 floats per lane group and a gap of 4, so that the groups' reads
+                              // fall on different banks
+  constexpr int R = 128;      // state rows per workgroup: 4 waves x 32 rows
+  constexpr int Q = KP, VAT = 2 * KP, OAT = VAT + R, EAT = OAT + R, REC = EAT + 4;
   extern __shared__ __align__(16) char ix_lds[];
-  float* kf = reinterpret_cast<float*>(ix_lds);  // [TT][K]
-  float* qf = kf + TT * K;                       // [TT][K], pre-scaled
-  float* vf = qf + TT * K;                       // [TT][R]
-  float* of = vf + TT * R;                       // [TT][R]
-  float* egf = of + TT * R;                      // [TT]
-  float* btf = egf + TT;                         // [TT]
+  float* rec = reinterpret_cast<float*>(ix_lds);  // a token: k [KP], q [KP] pre-scaled, v [R], o [R], exp(g), beta
 
   const int VB = V / R;
   long bid = blockIdx.x;
@@ -266,9 +275,8 @@ void k_gdn_scan_pairs(const TIO* __restrict__ q, const TIO* __restrict__ k, cons
   const int h = hv / (HV / H);
   const int tid = threadIdx.x;
   const int lane = tid & 63, wave = tid >> 6;
-  const int hf = lane >> 5;
-  const int r = wave * 32 + (lane & 31);
-  const int vrow = vb * R + r;
+  const int grp = lane >> 4;
+  const int r = wave * 32 + (lane & 31);  // the row whose v, d and output this lane has
 
   const int t_begin = cu[n], t_end = cu[n + 1];
   const int len = t_end - t_begin;
@@ -296,7 +304,7 @@ void k_gdn_scan_pairs(const TIO* __restrict__ q, const TIO* __restrict__ k, cons
         ix_unpack8(*reinterpret_cast<const uint4*>(norm_w + sub * 8), wv);
 #pragma unroll
         for (int j = 0; j < 8; j += 2)  // the scan's output is a bf16 tensor
-          ix_rbf2_hw(of[tt * R + sub * 8 + j], of[tt * R + sub * 8 + j + 1], xv[j], xv[j + 1]);
+          ix_rbf2_hw(rec[tt * REC + OAT + sub * 8 + j], rec[tt * REC + OAT + sub * 8 + j + 1], xv[j], xv[j + 1]);
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
           const float sq = xv[j] * xv[j];
@@ -320,26 +328,61 @@ void k_gdn_scan_pairs(const TIO* __restrict__ q, const TIO* __restrict__ k, cons
     } else {
       for (int i = tid; i < nt * R; i += 256) {
         const int tt = i / R, rr = i % R;
-        ix_st(o + ((long)(t_begin + t0 + tt) * HV + hv) * V + vb * R + rr, of[i]);
+        ix_st(o + ((long)(t_begin + t0 + tt) * HV + hv) * V + vb * R + rr, rec[tt * REC + OAT + rr]);
       }
     }
   };
   if (row0 <= 0) {  // null lane: no state, outputs defined as zero (and what the norm makes of zeros)
     if (!o) return;
-    for (int i = tid; i < TT * R; i += 256) of[i] = 0.0f;
+    for (int i = tid; i < TT * R; i += 256) rec[i / R * REC + OAT + i % R] = 0.0f;
     __syncthreads();
     for (int t0 = 0; t0 < len; t0 += TT) emit(t0, min(TT, len - t0));
     return;
   }
   constexpr long AL = 16 * sizeof(TIO) / 2;
   const bool vec_qk = (q_pitch % 8 == 0) && (k_pitch % 8 == 0) && ((uintptr_t)q % AL == 0) && ((uintptr_t)k % AL == 0);
-  float S[64];
-  float* srow = state + (((long)row0 * HV + hv) * V + vrow) * K + 64 * hf;
+  // S[j][c][i]: row wave * 32 + 16 j + lane % 16, k = 32 grp + 16 c + i
+  ix_f32x16 S[2][2];
+  float* srow = state + (((long)row0 * HV + hv) * V + vb * R + wave * 32 + (lane & 15)) * K + 32 * grp;
 #pragma unroll
-  for (int c = 0; c < 16; ++c) {
-    const float4 a = state ? *reinterpret_cast<const float4*>(srow + 4 * c) : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-    S[4 * c] = a.x; S[4 * c + 1] = a.y; S[4 * c + 2] = a.z; S[4 * c + 3] = a.w;
+  for (int j = 0; j < 2; ++j) {
+#pragma unroll
+    for (int c = 0; c < 8; ++c) {
+      const float4 a =
+          state ? *reinterpret_cast<const float4*>(srow + 16 * j * K + 4 * c) : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+      ix_f32x16& d = S[j][c >> 2];
+      const int i = 4 * (c & 3);
+      d[i] = a.x; d[i + 1] = a.y; d[i + 2] = a.z; d[i + 3] = a.w;
+    }
   }
+  // the element of k that this lane hands to the update's first instruction (the second one's: 16 further)
+  const int ka = 36 * ((lane & 15) >> 2) + 4 * grp + (lane & 3);
+  // the eight slice sums of the lane's two rows with 32 elements of k or q, and the tree over each row's sixteen
+  auto dots = [&](const float (&x)[32]) __attribute__((always_inline)) {
+    float part[2][4];
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+#pragma unroll
+      for (int sl = 0; sl < 4; ++sl) {
+        float ss[8], xs[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+          ss[i] = S[j][sl >> 1][8 * (sl & 1) + i];
+          xs[i] = x[8 * sl + i];
+        }
+        part[j][sl] = ix_dot8(ss, xs);
+      }
+    }
+    return ix_add_groups2((part[0][0] + part[0][1]) + (part[0][2] + part[0][3]),
+                          (part[1][0] + part[1][1]) + (part[1][2] + part[1][3]));
+  };
+  auto load_x = [&](const float* row, float (&x)[32]) __attribute__((always_inline)) {
+#pragma unroll
+    for (int c = 0; c < 8; ++c) {
+      const float4 a = *reinterpret_cast<const float4*>(row + 36 * grp + 4 * c);
+      x[4 * c] = a.x; x[4 * c + 1] = a.y; x[4 * c + 2] = a.z; x[4 * c + 3] = a.w;
+    }
+  };
 
   for (int t0 = 0; t0 < len; t0 += TT) {
     const int nt = min(TT, len - t0);
@@ -351,8 +394,8 @@ void k_gdn_scan_pairs(const TIO* __restrict__ q, const TIO* __restrict__ k, cons
         float a[8], b[8];
         ix_load8(k + tok * k_pitch + h * K + kk, 8, true, 0.0f, a);
         ix_load8(q + tok * q_pitch + h * K + kk, 8, true, 0.0f, b);
-        float* kd = kf + tt * K + kk;
-        float* qd = qf + tt * K + kk;
+        float* kd = rec + tt * REC + kk + (kk >> 5) * 4;
+        float* qd = kd + Q;
         *reinterpret_cast<float4*>(kd) = make_float4(a[0], a[1], a[2], a[3]);
         *reinterpret_cast<float4*>(kd + 4) = make_float4(a[4], a[5], a[6], a[7]);
         *reinterpret_cast<float4*>(qd) = make_float4(b[0] * scale, b[1] * scale, b[2] * scale, b[3] * scale);
@@ -362,69 +405,61 @@ void k_gdn_scan_pairs(const TIO* __restrict__ q, const TIO* __restrict__ k, cons
       for (int i = tid; i < nt * K; i += 256) {
         const int tt = i / K, kk = i % K;
         const long tok = t_begin + t0 + tt;
-        kf[i] = ix_ld(k + tok * k_pitch + h * K + kk);
-        qf[i] = ix_ld(q + tok * q_pitch + h * K + kk) * scale;
+        float* at = rec + tt * REC + kk + (kk >> 5) * 4;
+        at[0] = ix_ld(k + tok * k_pitch + h * K + kk);
+        at[Q] = ix_ld(q + tok * q_pitch + h * K + kk) * scale;
       }
     }
     for (int i = tid; i < nt * R; i += 256) {
       const int tt = i / R, rr = i % R;
-      vf[i] = ix_ld(v + (long)(t_begin + t0 + tt) * v_pitch + (long)hv * V + vb * R + rr);
+      rec[tt * REC + VAT + rr] = ix_ld(v + (long)(t_begin + t0 + tt) * v_pitch + (long)hv * V + vb * R + rr);
     }
     for (int i = tid; i < nt; i += 256) {
       const long src = (long)(t_begin + t0 + i) * HV + hv;
-      egf[i] = ix_exp(g[src]);
-      btf[i] = ix_ld(beta + src);
+      rec[i * REC + EAT] = ix_exp(g[src]);
+      rec[i * REC + EAT + 1] = ix_ld(beta + src);
     }
     __syncthreads();
-#pragma unroll 2
-    for (int tt = 0; tt < nt; ++tt) {
-      const float eg = egf[tt], bt = btf[tt], vv = vf[tt * R + r];
-      float x[64];  // this half's 64 elements of k, later of q
-      const float* kp = kf + tt * K + 64 * hf;
+    auto token = [&](int tt) __attribute__((always_inline)) {
+      float* at = rec + tt * REC;
+      const float eg = at[EAT], bt = at[EAT + 1], vv = at[VAT + r];
+      float x[32];  // this lane group's elements of k, later of q
+      load_x(at, x);
 #pragma unroll
-      for (int c = 0; c < 16; ++c) {
-        const float4 a = *reinterpret_cast<const float4*>(kp + 4 * c);
-        x[4 * c] = a.x; x[4 * c + 1] = a.y; x[4 * c + 2] = a.z; x[4 * c + 3] = a.w;
+      for (int j = 0; j < 2; ++j)
+#pragma unroll
+        for (int c = 0; c < 2; ++c)
+#pragma unroll
+          for (int i = 0; i < 16; ++i) S[j][c][i] = S[j][c][i] * eg;
+      const float d = (vv - dots(x)) * bt;
+      // groups 0 and 2 have the first row's d, 1 and 3 the second's: each to all four
+      const auto dd = __builtin_amdgcn_permlane16_swap(__float_as_uint(d), __float_as_uint(d), false, false);
+#pragma unroll
+      for (int c = 0; c < 2; ++c) {
+        const float ke = at[ka + 16 * c];
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+          S[j][c] = __builtin_amdgcn_mfma_f32_16x16x1f32(ke, __uint_as_float(dd[j]), S[j][c], 0, 0, 0);
       }
-      float part[8];
+      load_x(at + Q, x);
+      const float ov = dots(x);
+      at[OAT + r] = ov;  // both halves of the wave have it
+    };
+    int tt = 0;
+    for (; tt + 4 <= nt; tt += 4) {  // four tokens at fixed distances from one set of addresses
 #pragma unroll
-      for (int sl = 0; sl < 8; ++sl) {
-        float ss[8], xs[8];
-#pragma unroll
-        for (int i = 0; i < 8; ++i) {
-          S[8 * sl + i] = S[8 * sl + i] * eg;
-          ss[i] = S[8 * sl + i];
-          xs[i] = x[8 * sl + i];
-        }
-        part[sl] = ix_dot8(ss, xs);
-      }
-      const float kv = ix_add_halves(ix_tree8(part));
-      const float d = (vv - kv) * bt;
-#pragma unroll
-      for (int i = 0; i < 64; ++i) S[i] = __builtin_fmaf(d, x[i], S[i]);
-      const float* qp = qf + tt * K + 64 * hf;
-#pragma unroll
-      for (int c = 0; c < 16; ++c) {
-        const float4 a = *reinterpret_cast<const float4*>(qp + 4 * c);
-        x[4 * c] = a.x; x[4 * c + 1] = a.y; x[4 * c + 2] = a.z; x[4 * c + 3] = a.w;
-      }
-#pragma unroll
-      for (int sl = 0; sl < 8; ++sl) {
-        float ss[8], xs[8];
-#pragma unroll
-        for (int i = 0; i < 8; ++i) {
-          ss[i] = S[8 * sl + i];
-          xs[i] = x[8 * sl + i];
-        }
-        part[sl] = ix_dot8(ss, xs);
-      }
-      const float ov = ix_add_halves(ix_tree8(part));
-      if (hf == 0) of[tt * R + r] = ov;
+      for (int u = 0; u < 4; ++u) token(tt + u);
     }
+    for (; tt < nt; ++tt) token(tt);
     if (state && t0 + nt == len) {
 #pragma unroll
-      for (int c = 0; c < 16; ++c)
-        *reinterpret_cast<float4*>(srow + 4 * c) = make_float4(S[4 * c], S[4 * c + 1], S[4 * c + 2], S[4 * c + 3]);
+      for (int j = 0; j < 2; ++j)
+#pragma unroll
+        for (int c = 0; c < 8; ++c) {
+          const ix_f32x16& a = S[j][c >> 2];
+          const int i = 4 * (c & 3);
+          *reinterpret_cast<float4*>(srow + 16 * j * K + 4 * c) = make_float4(a[i], a[i + 1], a[i + 2], a[i + 3]);
+        }
     }
     __syncthreads();
     if (o) emit(t0, nt);
@@ -446,7 +481,7 @@ void k_gdn_scan_pairs(const TIO* __restrict__ q, const TIO* __restrict__ k, cons
 //     instruction: 1147 -> 988 us for 8192 tokens, 121 ns a token);
 //   * E = 4, where SIMDs would stand idle: a slice's two chains in two lanes, joined by the tree's first level. A token is then
 //     29 vector instructions of a wave instead of 45 (256 tokens at K = 64: 33 -> 24 us).
-// The statements per token are ix_gdn_step's: same bits as k_gdn_scan and k_gdn_scan_pairs.
+// The statements per token are ix_gdn_step's: same bits as k_gdn_scan and k_gdn_scan_quads.
 // Sequences are taken longest first when there are 2..256 of them (ranked by every workgroup from cu), and a sequence's
 // workgroups are spread over all XCDs with the row blocks of a key head on one of them.
 // CPR: the boundary form (gdn_cpr.py:296-319). Two states walk together: the fp32 chain, and the running state, which
@@ -915,27 +950,27 @@ static int ix_gdn_walk(const void* q, const void* k, const void* v, const float*
   return IX_DECLINED;
 }
 
-// Workgroups (128 rows each) from which a batch of whole sequences takes the lane-pair layout. It issues 36 vector
+// Workgroups (128 rows each) from which a batch of whole sequences takes the four-lane layout. It issues 30 vector
 // instructions per four rows and token where the walk issues 42, but a token takes one of its waves five times as long:
 // it wins once every SIMD has several waves through to the end. Measured at HV = 32, V = 128 (one such workgroup per
-// sequence and head), us pairs / walk: 64 x 1000 tokens 3953 / 4364, 32 x 1000 2314 / 2227, 16 x 1000 1201 / 1180, 20
-// sequences of 60..1485 tokens 1788 / 1134.
-#define IX_GDN_PAIR_MIN 2048
+// sequence and head), us four lanes / walk: 64 x 1000 tokens 3749 / 4375, 48 x 1000 2640 / 3295, 16 x 1000 1051 / 1160, 20
+// sequences of 60..1485 tokens 1398 / 1134.
+#define IX_GDN_QUAD_MIN 2048
 
-static int ix_gdn_pairs(const void* q, const void* k, const void* v, const float* g, const void* beta, void* o, int io_dtype,
+static int ix_gdn_quads(const void* q, const void* k, const void* v, const float* g, const void* beta, void* o, int io_dtype,
                         long q_pitch, long k_pitch, long v_pitch, float* state, const int* cu, const int* sidx, long N,
                         int H, int HV, int V, float scale, int TT, const bf16_t* gate, long gate_stride_t,
                         const bf16_t* norm_w, float norm_eps, int zero_centered, hipStream_t st) {
   const long grid = N * HV * (V / 128);
   if (grid > 0x7fffffffL) return IX_DECLINED;
-  size_t lds = ix_gdn_lds_bytes(128, 128, TT);
+  size_t lds = (size_t)TT * (2 * 140 + 2 * 128 + 4) * sizeof(float);
   if (lds < (IX_GDN_SORT_MAX + 1) * sizeof(int)) lds = (IX_GDN_SORT_MAX + 1) * sizeof(int);
   if (io_dtype == IX_DT_BF16)
-    hipLaunchKernelGGL((k_gdn_scan_pairs<bf16_t>), dim3((unsigned)grid), dim3(256), lds, st, (const bf16_t*)q,
+    hipLaunchKernelGGL((k_gdn_scan_quads<bf16_t>), dim3((unsigned)grid), dim3(256), lds, st, (const bf16_t*)q,
                        (const bf16_t*)k, (const bf16_t*)v, g, (const bf16_t*)beta, (bf16_t*)o, state, cu, sidx, q_pitch,
                        k_pitch, v_pitch, (int)N, H, HV, V, scale, TT, gate, gate_stride_t, norm_w, norm_eps, zero_centered);
   else
-    hipLaunchKernelGGL((k_gdn_scan_pairs<float>), dim3((unsigned)grid), dim3(256), lds, st, (const float*)q,
+    hipLaunchKernelGGL((k_gdn_scan_quads<float>), dim3((unsigned)grid), dim3(256), lds, st, (const float*)q,
                        (const float*)k, (const float*)v, g, (const float*)beta, (float*)o, state, cu, sidx, q_pitch, k_pitch,
                        v_pitch, (int)N, H, HV, V, scale, TT, (const bf16_t*)nullptr, 0L, (const bf16_t*)nullptr, 0.0f, 0);
   return ix_launch_status();
@@ -959,16 +994,16 @@ static int ix_gdn_scan_impl(const void* q, const void* k, const void* v, const f
   if (TT <= 0) TT = (N * HV * (V / 16) >= 4096) ? 16 : 64;
   if (TT > 64) TT = 64;
   hipStream_t st = (hipStream_t)stream;
-  // The lane-pair layout: compact state form, K = 128, whole groups of 128 rows, and IX_GDN_PAIR_MIN workgroups (or forced
+  // The four-lane layout: compact state form, K = 128, whole groups of 128 rows, and IX_GDN_QUAD_MIN workgroups (or forced
   // by code 16 in bits 8.. of time_tile). A time tile of 1 says one token per sequence (a decode step): that is a pure
   // stream of the state, which the 16-lane layout does with more waves in flight.
   if (state_indices_stride == 0 && K == 128 && V % 128 == 0 &&
-      (rpl == 16 || (rpl == 0 && (time_tile & 0xff) != 1 && N * HV * (V / 128) >= IX_GDN_PAIR_MIN)))
-    return ix_gdn_pairs(q, k, v, g, beta, o, io_dtype, q_pitch, k_pitch, v_pitch, state_pool, cu_seqlens, state_indices, N,
+      (rpl == 16 || (rpl == 0 && (time_tile & 0xff) != 1 && N * HV * (V / 128) >= IX_GDN_QUAD_MIN)))
+    return ix_gdn_quads(q, k, v, g, beta, o, io_dtype, q_pitch, k_pitch, v_pitch, state_pool, cu_seqlens, state_indices, N,
                         (int)H, (int)HV, (int)V, scale, time_tile > 0 && (time_tile & 0xff) > 0 ? TT : 16, gate,
                         gate_stride_t, norm_w, norm_eps, zero_centered, st);
-  if (gate) return IX_DECLINED;       // the norm rides on the lane-pair layout only
-  if (rpl == 16) return IX_DECLINED;  // the lane-pair layout was asked for and does not apply
+  if (gate) return IX_DECLINED;       // the norm rides on the four-lane layout only
+  if (rpl == 16) return IX_DECLINED;  // the four-lane layout was asked for and does not apply
   // Sequences of more than one token in the compact form: the walk (codes 17 and 18 force it with one and two rows per
   // lane group). k_gdn_scan below keeps the decode step, the per-token index map, the state-only pass and the operands
   // whose rows are not aligned.
@@ -1006,7 +1041,7 @@ extern "C" int ix_gdn_scan(const void* q, const void* k, const void* v, const fl
 
 // ix_gdn_scan whose output leaves through the layer's gated output norm (ix_gated_out_norm with N = V) in the same
 // launch: o receives bf16(norm(o_scan) * silu(gate)) instead of o_scan -- the bits of the two calls. Served where the
-// lane-pair layout runs (one state row per sequence, K = V = 128, bf16, at least IX_GDN_PAIR_MIN (sequence, head) pairs) with
+// four-lane layout runs (one state row per sequence, K = V = 128, bf16, at least IX_GDN_QUAD_MIN (sequence, head) pairs) with
 // 16-byte aligned gate rows and weight; IX_DECLINED otherwise, before anything is launched or the state is touched.
 extern "C" int ix_gdn_scan_gated_norm(const void* q, const void* k, const void* v, const float* g, const void* beta,
                                       void* o, long q_pitch, long k_pitch, long v_pitch, float* state_pool,
@@ -1015,7 +1050,7 @@ extern "C" int ix_gdn_scan_gated_norm(const void* q, const void* k, const void* 
                                       const void* norm_weight, float norm_eps, int zero_centered, void* stream) {
   if (!o || !gate || !norm_weight || gate_stride_t < HV * V) return IX_ERR_ARG;
   if (K != 128 || V != 128 || (gate_stride_t % 8) || !ix_aligned(gate, 16) || !ix_aligned(norm_weight, 16) ||
-      !ix_aligned(o, 16) || (time_tile & 0xff) == 1 || (time_tile >> 8) != 0 || N * HV < IX_GDN_PAIR_MIN)
+      !ix_aligned(o, 16) || (time_tile & 0xff) == 1 || (time_tile >> 8) != 0 || N * HV < IX_GDN_QUAD_MIN)
     return IX_DECLINED;
   return ix_gdn_scan_impl(q, k, v, g, beta, o, IX_DT_BF16, q_pitch, k_pitch, v_pitch, state_pool, cu_seqlens,
                           state_indices, 0, N, H, HV, K, V, scale, time_tile, (const bf16_t*)gate, gate_stride_t,
@@ -1035,13 +1070,13 @@ extern "C" int ix_gdn_forward(const void* q, const void* k, const void* v, const
   if (io_dtype != IX_DT_F32 && io_dtype != IX_DT_BF16) return IX_DECLINED;
   if (chunk % 16 || chunk > 0x7fffffffL) return IX_DECLINED;  // the restart falls on a tile's first token
   hipStream_t st = (hipStream_t)stream;
-  const bool pairs = chunk == 0 && K == 128 && V % 128 == 0 && N * HV * (V / 128) >= IX_GDN_PAIR_MIN;
+  const bool pairs = chunk == 0 && K == 128 && V % 128 == 0 && N * HV * (V / 128) >= IX_GDN_QUAD_MIN;
   if (gate && (!pairs || V != 128 || io_dtype != IX_DT_BF16 || (gate_stride_t % 8) || !ix_aligned(gate, 16) ||
                !ix_aligned(norm_weight, 16) || !ix_aligned(o, 16)))
-    return IX_DECLINED;  // the norm rides on the lane-pair layout only
+    return IX_DECLINED;  // the norm rides on the four-lane layout only
   if (N == 0) return IX_OK;
   if (pairs)
-    return ix_gdn_pairs(q, k, v, g, beta, o, io_dtype, q_pitch, k_pitch, v_pitch, nullptr, cu_seqlens, nullptr, N, (int)H,
+    return ix_gdn_quads(q, k, v, g, beta, o, io_dtype, q_pitch, k_pitch, v_pitch, nullptr, cu_seqlens, nullptr, N, (int)H,
                         (int)HV, (int)V, scale, 16, (const bf16_t*)gate, gate_stride_t, (const bf16_t*)norm_weight,
                         norm_eps, zero_centered, st);
   return ix_gdn_walk(q, k, v, g, beta, o, io_dtype, nullptr, cu_seqlens, nullptr, q_pitch, k_pitch, v_pitch, N, (int)H,

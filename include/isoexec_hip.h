@@ -222,7 +222,8 @@ int ix_arena_destroy(void* arena);
  * time_tile: bits 0-7 = tokens staged per LDS fill (<= 64, 0 = default; 1 also tells the launcher that every
  * sequence has one token, a decode step); bits 8.. = the layout: state rows held per group of 16 lanes (1, 2 or 4),
  * or 16 for the four-lane layout (K = 128, compact state form, V % 128 == 0; declined otherwise), 17 / 18 for the walk with
- * one / two rows per lane group (compact form with an output, q and k rows aligned to 8 elements; declined otherwise);
+ * one / two rows per lane group, 19 with four lanes per row (K = 128, V % 64 == 0) (compact form with an output, q and k rows
+ * aligned to 8 elements; declined otherwise);
  * 0 = chosen from the grid size. Neither changes results. */
 int ix_gdn_scan(const void* q, const void* k, const void* v, const float* g, const void* beta, void* o,
                 int io_dtype, long q_pitch, long k_pitch, long v_pitch, float* state_pool,
@@ -305,7 +306,7 @@ int ix_gdn_cpr_handoff(const float* entry_state, float* running_state, int* due,
  * runtimes/megatron/gdn_fla_shim.py:390-425 `_eager_apply_gated_norm` after the core, ops/norms/fused_outnorm.py:189-271):
  * o [tokens, HV, V] bf16 receives ix_gated_out_norm(o_scan, gate, norm_weight) instead of o_scan; the bits of the two
  * calls. gate bf16 with token pitch gate_stride_t (elements, a multiple of 8), norm_weight bf16 [V]. Served where the
- * four-lane layout of the scan runs: one state row per sequence (state_indices [N]), K = V = 128, bf16, N * HV >= 2048, no
+ * four-lane layout of the scan runs: one state row per sequence (state_indices [N]), K = V = 128, bf16, N * HV >= 1536, no
  * forced time tile of 1 or row code; IX_DECLINED otherwise, before the state is touched (the caller makes the two calls). */
 int ix_gdn_scan_gated_norm(const void* q, const void* k, const void* v, const float* g, const void* beta, void* o,
                            long q_pitch, long k_pitch, long v_pitch, float* state_pool, const int* cu_seqlens,
@@ -317,7 +318,7 @@ int ix_gdn_scan_gated_norm(const void* q, const void* k, const void* v, const fl
  * as ix_gdn_scan's; every sequence starts from a zero state and no state is stored. chunk = 0: the recurrence. chunk > 0
  * (a multiple of 16): the running state restarts at every multiple of chunk tokens from the unrounded fp32 chain rounded to
  * io_dtype, as if the boundary states had been computed first and every chunk scanned from its snapshot. gate, norm_weight
- * (or NULL): as ix_gdn_scan_gated_norm's, where N * HV >= 2048 and chunk = 0. q and k rows start on multiples of 8 elements.
+ * (or NULL): as ix_gdn_scan_gated_norm's, where N * HV >= 1536 and chunk = 0. q and k rows start on multiples of 8 elements.
  * IX_DECLINED otherwise, before anything is launched. */
 int ix_gdn_forward(const void* q, const void* k, const void* v, const float* g, const void* beta, void* o, int io_dtype,
                    long q_pitch, long k_pitch, long v_pitch, const int* cu_seqlens, long N, long H, long HV, long K, long V,

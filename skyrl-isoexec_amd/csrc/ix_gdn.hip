@@ -249,6 +249,32 @@ __device__ __forceinline__ float ix_add_groups2(float a, float b) {
   return ix_add_halves(__uint_as_float(r[0]) + __uint_as_float(r[1]));
 }
 typedef float ix_f32x16 __attribute__((ext_vector_type(16)));
+// A lane group's 32 elements of a token's k or q in LDS. The groups' elements stand 36 floats apart, so that their reads fall
+// on different banks; a token takes IX_QUAD_KP floats.
+#define IX_QUAD_KP 140
+__device__ __forceinline__ int ix_quad_at(int k) { return k + (k >> 5) * 4; }
+__device__ __forceinline__ void ix_quad_load(const float* row, int grp, float (&x)[32]) {
+#pragma unroll
+  for (int c = 0; c < 8; ++c) {
+    const float4 a = *reinterpret_cast<const float4*>(row + 36 * grp + 4 * c);
+    x[4 * c] = a.x; x[4 * c + 1] = a.y; x[4 * c + 2] = a.z; x[4 * c + 3] = a.w;
+  }
+}
+// The lane's four slice sums of one state row, and the two levels of the row's tree that run inside the lane.
+__device__ __forceinline__ float ix_quad_dot(const ix_f32x16 (&S)[2], const float (&x)[32]) {
+  float part[4];
+#pragma unroll
+  for (int sl = 0; sl < 4; ++sl) {
+    float ss[8], xs[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      ss[i] = S[sl >> 1][8 * (sl & 1) + i];
+      xs[i] = x[8 * sl + i];
+    }
+    part[sl] = ix_dot8(ss, xs);
+  }
+  return (part[0] + part[1]) + (part[2] + part[3]);
+}
 
 template <typename TIO>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3)))
@@ -259,12 +285,10 @@ void k_gdn_scan_quads(const TIO* __restrict__ q, const TIO* __restrict__ k, cons
                       const bf16_t* __restrict__ gate, long gate_stride_t, const bf16_t* __restrict__ norm_w,
                       float norm_eps, int zero_centered) {
   constexpr int K = 128;
-  constexpr int KP = K + 12;  // a token's k or q in LDS: 32 floats per lane group and a gap of 4, so that the groups' reads
-                              // fall on different banks
-  constexpr int R = 128;      // state rows per workgroup: 4 waves x 32 rows
-  constexpr int Q = KP, VAT = 2 * KP, OAT = VAT + R, EAT = OAT + R, REC = EAT + 4;
+  constexpr int R = 128;  // state rows per workgroup: 4 waves x 32 rows
+  constexpr int Q = IX_QUAD_KP, VAT = 2 * IX_QUAD_KP, OAT = VAT + R, EAT = OAT + R, REC = EAT + 4;
   extern __shared__ __align__(16) char ix_lds[];
-  float* rec = reinterpret_cast<float*>(ix_lds);  // a token: k [KP], q [KP] pre-scaled, v [R], o [R], exp(g), beta
+  float* rec = reinterpret_cast<float*>(ix_lds);  // a token: k, q pre-scaled [IX_QUAD_KP each], v [R], o [R], exp(g), beta
 
   const int VB = V / R;
   long bid = blockIdx.x;
@@ -357,31 +381,9 @@ void k_gdn_scan_quads(const TIO* __restrict__ q, const TIO* __restrict__ k, cons
   }
   // the element of k that this lane hands to the update's first instruction (the second one's: 16 further)
   const int ka = 36 * ((lane & 15) >> 2) + 4 * grp + (lane & 3);
-  // the eight slice sums of the lane's two rows with 32 elements of k or q, and the tree over each row's sixteen
+  // both rows' dot products with 32 elements of k or q: groups 0 and 2 have the first row's, 1 and 3 the second's
   auto dots = [&](const float (&x)[32]) __attribute__((always_inline)) {
-    float part[2][4];
-#pragma unroll
-    for (int j = 0; j < 2; ++j) {
-#pragma unroll
-      for (int sl = 0; sl < 4; ++sl) {
-        float ss[8], xs[8];
-#pragma unroll
-        for (int i = 0; i < 8; ++i) {
-          ss[i] = S[j][sl >> 1][8 * (sl & 1) + i];
-          xs[i] = x[8 * sl + i];
-        }
-        part[j][sl] = ix_dot8(ss, xs);
-      }
-    }
-    return ix_add_groups2((part[0][0] + part[0][1]) + (part[0][2] + part[0][3]),
-                          (part[1][0] + part[1][1]) + (part[1][2] + part[1][3]));
-  };
-  auto load_x = [&](const float* row, float (&x)[32]) __attribute__((always_inline)) {
-#pragma unroll
-    for (int c = 0; c < 8; ++c) {
-      const float4 a = *reinterpret_cast<const float4*>(row + 36 * grp + 4 * c);
-      x[4 * c] = a.x; x[4 * c + 1] = a.y; x[4 * c + 2] = a.z; x[4 * c + 3] = a.w;
-    }
+    return ix_add_groups2(ix_quad_dot(S[0], x), ix_quad_dot(S[1], x));
   };
 
   for (int t0 = 0; t0 < len; t0 += TT) {
@@ -394,7 +396,7 @@ void k_gdn_scan_quads(const TIO* __restrict__ q, const TIO* __restrict__ k, cons
         float a[8], b[8];
         ix_load8(k + tok * k_pitch + h * K + kk, 8, true, 0.0f, a);
         ix_load8(q + tok * q_pitch + h * K + kk, 8, true, 0.0f, b);
-        float* kd = rec + tt * REC + kk + (kk >> 5) * 4;
+        float* kd = rec + tt * REC + ix_quad_at(kk);
         float* qd = kd + Q;
         *reinterpret_cast<float4*>(kd) = make_float4(a[0], a[1], a[2], a[3]);
         *reinterpret_cast<float4*>(kd + 4) = make_float4(a[4], a[5], a[6], a[7]);
@@ -405,7 +407,7 @@ void k_gdn_scan_quads(const TIO* __restrict__ q, const TIO* __restrict__ k, cons
       for (int i = tid; i < nt * K; i += 256) {
         const int tt = i / K, kk = i % K;
         const long tok = t_begin + t0 + tt;
-        float* at = rec + tt * REC + kk + (kk >> 5) * 4;
+        float* at = rec + tt * REC + ix_quad_at(kk);
         at[0] = ix_ld(k + tok * k_pitch + h * K + kk);
         at[Q] = ix_ld(q + tok * q_pitch + h * K + kk) * scale;
       }
@@ -424,7 +426,7 @@ void k_gdn_scan_quads(const TIO* __restrict__ q, const TIO* __restrict__ k, cons
       float* at = rec + tt * REC;
       const float eg = at[EAT], bt = at[EAT + 1], vv = at[VAT + r];
       float x[32];  // this lane group's elements of k, later of q
-      load_x(at, x);
+      ix_quad_load(at, grp, x);
 #pragma unroll
       for (int j = 0; j < 2; ++j)
 #pragma unroll
@@ -441,7 +443,7 @@ void k_gdn_scan_quads(const TIO* __restrict__ q, const TIO* __restrict__ k, cons
         for (int j = 0; j < 2; ++j)
           S[j][c] = __builtin_amdgcn_mfma_f32_16x16x1f32(ke, __uint_as_float(dd[j]), S[j][c], 0, 0, 0);
       }
-      load_x(at + Q, x);
+      ix_quad_load(at + Q, grp, x);
       const float ov = dots(x);
       at[OAT + r] = ov;  // both halves of the wave have it
     };
@@ -821,6 +823,194 @@ __global__ __launch_bounds__(LONE ? 320 : 256) void k_gdn_walk(const TIO* __rest
   }
 }
 
+// ---- the walk with four lanes per row (K = 128) ---------------------------------------------------------------
+// k_gdn_walk's staging (two tiles of 16 tokens, one barrier per tile) around k_gdn_scan_quads' token with ONE row per lane: a
+// wave has sixteen rows, a workgroup 64. CPR: the lane's second state is the fp32 chain beside the running state, and its row's
+// reads of k serve both. Outputs stay in registers for four tokens, so that those tokens' reads of LDS may pass one another.
+// Bound by vector issue with several waves per SIMD: 128 instructions per token for sixteen rows, 202 in the boundary form.
+// Tried: the next token's reads and dot products between a token's update and its output (168 registers no longer hold it;
+// with two waves per SIMD 64 x 1000 tokens of the boundary form 5466 -> 6221 us); one element of k and q per lane, broadcast on
+// the operand path of the multiply-adds, instead of the LDS reads (those multiply-adds do not run at the full rate: 6646); a higher wave priority for the longer sequences (nothing).
+template <typename TIO, bool CPR>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3)))
+void k_gdn_walk_quads(const TIO* __restrict__ q, const TIO* __restrict__ k, const TIO* __restrict__ v,
+                      const float* __restrict__ g, const TIO* __restrict__ beta, TIO* __restrict__ o,
+                      float* __restrict__ state, const int* __restrict__ cu, const int* __restrict__ sidx, long q_pitch,
+                      long k_pitch, long v_pitch, int N, int H, int HV, int V, float scale, int chunk) {
+  constexpr int K = 128, T = 16, R = 64, J = CPR ? 2 : 1;
+  constexpr int Q = IX_QUAD_KP, VAT = 2 * IX_QUAD_KP, OAT = VAT + R, EAT = OAT + R, REC = EAT + 4;
+  constexpr int VC = T * R / 256;
+  __shared__ __align__(16) float rec[2][T * REC];  // a token: k, q * scale [IX_QUAD_KP each], v [R], o [R], exp(g), beta
+  static_assert(sizeof(rec) >= (IX_GDN_SORT_MAX + 1) * sizeof(int), "the ranking uses the staging buffer");
+
+  const int VB = V / R;
+  const int per_seq = HV * VB;
+  const int tid = threadIdx.x;
+  int n, w;
+  {
+    const unsigned bid = blockIdx.x;
+    if ((per_seq & 7) == 0) {  // hardware deals consecutive ids to the XCDs round-robin
+      const unsigned per8 = (unsigned)per_seq >> 3;
+      // Every second round of 32 workgroups of an XCD, one per CU, runs the other way: the CU with the longest sequence gets the
+      // shortest of the next round.
+      unsigned p = bid >> 3;
+      const unsigned all = (unsigned)N * per8, first = p & ~31u;
+      if (first & 32u) p = first + min(31u, all - 1 - first) - (p & 31u);
+      n = (int)(p / per8);
+      w = (int)((bid & 7u) * per8 + p % per8);
+    } else {
+      n = (int)(bid / (unsigned)per_seq);
+      w = (int)(bid % (unsigned)per_seq);
+    }
+  }
+  n = ix_gdn_nth_longest(cu, N, n, reinterpret_cast<int*>(&rec[0][0]));
+  const int vb = w % VB;
+  const int hv = w / VB;
+  const int h = hv / (HV / H);
+  const int t_begin = cu[n];
+  const int len = cu[n + 1] - t_begin;
+  if (len <= 0) return;
+  const int row0 = sidx ? sidx[n] : 1;
+  TIO* ob = o + (long)hv * V + vb * R;
+  if (row0 <= 0) {  // null lane: no state, outputs defined as zero
+    for (int i = tid; i < len * R; i += 256) ix_st(ob + (long)(t_begin + i / R) * HV * V + i % R, 0.0f);
+    return;
+  }
+  const int tiles = (len + T - 1) / T;
+
+  // staging: a thread has one group of eight of k and of q, VC values of v
+  const int gt = tid >> 4, gk = (tid & 15) * 8;
+  IxRaw8<TIO> rk, rq;
+  TIO rv[VC], rb = 0;
+  float rg = 0.0f;
+  auto fetch = [&](int t0) __attribute__((always_inline)) {  // tokens past the end read the last one's values, unused
+    const long tok = t_begin + min(t0 + gt, len - 1);
+    rk.load(k + tok * k_pitch + h * K + gk);
+    rq.load(q + tok * q_pitch + h * K + gk);
+#pragma unroll
+    for (int c = 0; c < VC; ++c) {
+      const int i = tid + 256 * c;
+      rv[c] = v[(t_begin + min(t0 + i / R, len - 1)) * v_pitch + (long)hv * V + vb * R + i % R];
+    }
+    if (tid < T) {
+      const long src = (t_begin + (long)min(t0 + tid, len - 1)) * HV + hv;
+      rg = g[src];
+      rb = beta[src];
+    }
+  };
+  auto commit = [&](int b) __attribute__((always_inline)) {
+    float x[8], y[8];
+    rk.widen(x);
+    rq.widen(y);
+    float* d = &rec[b][gt * REC + ix_quad_at(gk)];
+    *reinterpret_cast<float4*>(d) = make_float4(x[0], x[1], x[2], x[3]);
+    *reinterpret_cast<float4*>(d + 4) = make_float4(x[4], x[5], x[6], x[7]);
+    *reinterpret_cast<float4*>(d + Q) = make_float4(y[0] * scale, y[1] * scale, y[2] * scale, y[3] * scale);
+    *reinterpret_cast<float4*>(d + Q + 4) = make_float4(y[4] * scale, y[5] * scale, y[6] * scale, y[7] * scale);
+#pragma unroll
+    for (int c = 0; c < VC; ++c) {
+      const int i = tid + 256 * c;
+      rec[b][i / R * REC + VAT + i % R] = ix_ld(&rv[c]);
+    }
+    if (tid < T) *reinterpret_cast<float2*>(&rec[b][tid * REC + EAT]) = make_float2(ix_exp(rg), ix_ld(&rb));
+  };
+  auto emit = [&](int t0, int nt, int b) __attribute__((always_inline)) {
+#pragma unroll
+    for (int c = 0; c < VC; ++c) {
+      const int i = tid + 256 * c;
+      if (i < nt * R) ix_st(ob + (long)(t_begin + t0 + i / R) * HV * V + i % R, rec[b][i / R * REC + OAT + i % R]);
+    }
+  };
+
+  const int lane = tid & 63, wave = tid >> 6;
+  const int grp = lane >> 4;
+  const int r = wave * 16 + (lane & 15);
+  // S[0]: the state that makes the outputs, S[1]: the chain; S[j][c][i]: k = 32 grp + 16 c + i
+  ix_f32x16 S[J][2];
+  float* srow = state + (((long)row0 * HV + hv) * V + vb * R + r) * K + 32 * grp;
+#pragma unroll
+  for (int j = 0; j < J; ++j) {
+#pragma unroll
+    for (int c = 0; c < 8; ++c) {
+      const float4 a = state ? *reinterpret_cast<const float4*>(srow + 4 * c) : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+      ix_f32x16& d = S[j][c >> 2];
+      const int i = 4 * (c & 3);
+      d[i] = a.x; d[i + 1] = a.y; d[i + 2] = a.z; d[i + 3] = a.w;
+    }
+  }
+  // the element of k that this lane hands to the update's first instruction (the second one's: 16 further)
+  const int ka = 36 * ((lane & 15) >> 2) + 4 * grp + (lane & 3);
+
+  fetch(0);
+  commit(0);
+  __syncthreads();
+  for (int it = 0; it < tiles; ++it) {
+    const int b = it & 1, t0 = it * T;
+    const int nt = min(T, len - t0);
+    if (it + 1 < tiles) fetch(t0 + T);
+    if (it > 0) emit(t0 - T, T, b ^ 1);
+    if constexpr (CPR) {
+      if (t0 % chunk == 0) {
+#pragma unroll
+        for (int c = 0; c < 2; ++c)
+#pragma unroll
+          for (int i = 0; i < 16; ++i) S[0][c][i] = ix_wire(S[1][c][i], (const TIO*)nullptr);
+      }
+    }
+    auto token = [&](int tt) __attribute__((always_inline)) {
+      const float* at = &rec[b][tt * REC];
+      const float eg = at[EAT], bt = at[EAT + 1], vv = at[VAT + r];
+      float x[32];  // this lane group's elements of k, later of q
+      ix_quad_load(at, grp, x);
+#pragma unroll
+      for (int j = 0; j < J; ++j)
+#pragma unroll
+        for (int c = 0; c < 2; ++c)
+#pragma unroll
+          for (int i = 0; i < 16; ++i) S[j][c][i] = S[j][c][i] * eg;
+      // CPR: groups 0 and 2 go on with the running state, 1 and 3 with the chain
+      const float p0 = ix_quad_dot(S[0], x);
+      const float p1 = CPR ? ix_quad_dot(S[J - 1], x) : p0;
+      const float d = (vv - ix_add_groups2(p0, p1)) * bt;
+      float dj[2] = {d, d};
+      if constexpr (CPR) {  // each to all four groups
+        const auto dd = __builtin_amdgcn_permlane16_swap(__float_as_uint(d), __float_as_uint(d), false, false);
+        dj[0] = __uint_as_float(dd[0]);
+        dj[1] = __uint_as_float(dd[1]);
+      }
+#pragma unroll
+      for (int c = 0; c < 2; ++c) {
+        const float ke = at[ka + 16 * c];
+#pragma unroll
+        for (int j = 0; j < J; ++j) S[j][c] = __builtin_amdgcn_mfma_f32_16x16x1f32(ke, dj[j], S[j][c], 0, 0, 0);
+      }
+      ix_quad_load(at + Q, grp, x);
+      const float p = ix_quad_dot(S[0], x);
+      return ix_add_groups2(p, p);
+    };
+    int tt = 0;
+    for (; tt + 4 <= nt; tt += 4) {
+      float ov[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) ov[u] = token(tt + u);
+#pragma unroll
+      for (int u = 0; u < 4; ++u) rec[b][(tt + u) * REC + OAT + r] = ov[u];  // every group of the row has it
+    }
+    for (; tt < nt; ++tt) rec[b][tt * REC + OAT + r] = token(tt);
+    if (it + 1 < tiles) commit(b ^ 1);
+    __syncthreads();
+  }
+  emit((tiles - 1) * T, len - (tiles - 1) * T, (tiles - 1) & 1);
+  if (state && !CPR) {
+#pragma unroll
+    for (int c = 0; c < 8; ++c) {
+      const ix_f32x16& a = S[0][c >> 2];
+      const int i = 4 * (c & 3);
+      *reinterpret_cast<float4*>(srow + 4 * c) = make_float4(a[i], a[i + 1], a[i + 2], a[i + 3]);
+    }
+  }
+}
+
 // q and k rows that can be fetched 8 elements at a time: every row start on a 16-byte (bf16) or 32-byte (fp32) boundary
 template <typename TIO>
 static bool ix_gdn_vec_qk(const void* q, const void* k, long q_pitch, long k_pitch) {
@@ -906,7 +1096,7 @@ static int ix_gdn_scan_launch(const void* q, const void* k, const void* v, const
 #undef IX_RPL_CASE
 }
 
-// chunk > 0: the boundary form. rpl: state rows per lane group, 0 = by the rule.
+// chunk > 0: the boundary form. rpl: state rows per lane group, 3 = four lanes per row, 0 = by the rule.
 static int ix_gdn_walk(const void* q, const void* k, const void* v, const float* g, const void* beta, void* o,
                        int io_dtype, float* state, const int* cu, const int* sidx, long q_pitch, long k_pitch, long v_pitch,
                        long N, int H, int HV, long K, int V, float scale, int chunk, int rpl, hipStream_t st) {
@@ -922,6 +1112,30 @@ static int ix_gdn_walk(const void* q, const void* k, const void* v, const float*
   // while one such workgroup per CU, two at K <= 64, is all there is (at K = 128 a row is then 32 lanes and its tree has a
   // level across the halves of 16). us whole / split: 2000 tokens of 16 heads at K = 128 245 / 206, of 32 heads (two per CU)
   // 66 / 75 per 500; K = 64, 2 x 256 of 4 heads 33 / 24, 8 x 512 of 16 heads 66 / 63, of 32 heads 86 / 107.
+  // Four lanes per row (K = 128) issue 8 vector instructions per row and token where the walk issues 11 (boundary form 13 and
+  // 18), but a token takes a wave three times as long, 0.42 us alone on its SIMD (boundary form 0.58), so they wait for enough
+  // workgroups. us walk / four lanes, 32 heads, V = 128 (64 workgroups per sequence), bf16: 12 sequences of 60..1380 tokens 653 /
+  // 680, 16 of 60..1410 870 / 739, 16 x 1000 1156 / 996, 32 x 1000 2242 / 1913, 32 x 200 467 / 379; boundary form 4 x 1000 595 /
+  // 634, 6 x 1000 858 / 829, 8 x 1000 1122 / 906, nine of 120..1500 1008 / 1000 (fp32 1025 / 1119), 32 of 60..1500 3016 / 2303,
+  // 64 x 1000 7339 / 5466.
+  const long quad_wgs = N * HV * (V / 64);
+  const bool quads = K == 128 && V % 64 == 0 && quad_wgs >= (chunk > 0 && io_dtype == IX_DT_BF16 ? 640 : 1024);
+  const bool vec_qk = io_dtype == IX_DT_BF16 ? ix_gdn_vec_qk<bf16_t>(q, k, q_pitch, k_pitch)
+                                             : ix_gdn_vec_qk<float>(q, k, q_pitch, k_pitch);
+  if (rpl == 3 || (rpl <= 0 && quads)) {
+    if (K != 128 || V % 64 != 0 || quad_wgs > 0x7fffffffL || !vec_qk) return IX_DECLINED;
+#define IX_WALK_QUADS(TIO, CPR_)                                                                                     \
+  hipLaunchKernelGGL((k_gdn_walk_quads<TIO, CPR_>), dim3((unsigned)quad_wgs), dim3(256), 0, st, (const TIO*)q, (const TIO*)k, \
+                     (const TIO*)v, g, (const TIO*)beta, (TIO*)o, state, cu, sidx, q_pitch, k_pitch, v_pitch, (int)N, H, \
+                     HV, V, scale, chunk)
+    if (io_dtype == IX_DT_BF16) {
+      if (chunk > 0) { IX_WALK_QUADS(bf16_t, true); } else { IX_WALK_QUADS(bf16_t, false); }
+    } else {
+      if (chunk > 0) { IX_WALK_QUADS(float, true); } else { IX_WALK_QUADS(float, false); }
+    }
+#undef IX_WALK_QUADS
+    return ix_launch_status();
+  }
   const long lanes = N * HV * V * (K / 8);  // threads at one row per lane group, whole slices
   const bool auto_shape = rpl <= 0;
   if (auto_shape) rpl = lanes >= 8L * 1024 * 64 ? 2 : 1;
@@ -953,9 +1167,10 @@ static int ix_gdn_walk(const void* q, const void* k, const void* v, const float*
 // Workgroups (128 rows each) from which a batch of whole sequences takes the four-lane layout. It issues 30 vector
 // instructions per four rows and token where the walk issues 42, but a token takes one of its waves five times as long:
 // it wins once every SIMD has several waves through to the end. Measured at HV = 32, V = 128 (one such workgroup per
-// sequence and head), us four lanes / walk: 64 x 1000 tokens 3749 / 4375, 48 x 1000 2640 / 3295, 16 x 1000 1051 / 1160, 20
-// sequences of 60..1485 tokens 1398 / 1134.
-#define IX_GDN_QUAD_MIN 2048
+// sequence and head), us two rows per lane / one (k_gdn_walk_quads) / walk: 64 x 1000 tokens 3749 / 3677 / 4375, 48 x 1000 2640 /
+// 2982 / 3295, 48 sequences of 60..1470 2106 / 2285 / 2484, 40 x 1000 2347 / 2344 / 2792, 32 x 1000 2058 / 1913 / 2242, 24 x 1000
+// 1382 / 1399 / 1699, 24 of 60..1440 1378 / 1057 / 1275.
+#define IX_GDN_QUAD_MIN 1536
 
 static int ix_gdn_quads(const void* q, const void* k, const void* v, const float* g, const void* beta, void* o, int io_dtype,
                         long q_pitch, long k_pitch, long v_pitch, float* state, const int* cu, const int* sidx, long N,
@@ -963,7 +1178,7 @@ static int ix_gdn_quads(const void* q, const void* k, const void* v, const float
                         const bf16_t* norm_w, float norm_eps, int zero_centered, hipStream_t st) {
   const long grid = N * HV * (V / 128);
   if (grid > 0x7fffffffL) return IX_DECLINED;
-  size_t lds = (size_t)TT * (2 * 140 + 2 * 128 + 4) * sizeof(float);
+  size_t lds = (size_t)TT * (2 * IX_QUAD_KP + 2 * 128 + 4) * sizeof(float);
   if (lds < (IX_GDN_SORT_MAX + 1) * sizeof(int)) lds = (IX_GDN_SORT_MAX + 1) * sizeof(int);
   if (io_dtype == IX_DT_BF16)
     hipLaunchKernelGGL((k_gdn_scan_quads<bf16_t>), dim3((unsigned)grid), dim3(256), lds, st, (const bf16_t*)q,
@@ -1005,9 +1220,9 @@ static int ix_gdn_scan_impl(const void* q, const void* k, const void* v, const f
   if (gate) return IX_DECLINED;       // the norm rides on the four-lane layout only
   if (rpl == 16) return IX_DECLINED;  // the four-lane layout was asked for and does not apply
   // Sequences of more than one token in the compact form: the walk (codes 17 and 18 force it with one and two rows per
-  // lane group). k_gdn_scan below keeps the decode step, the per-token index map, the state-only pass and the operands
+  // lane group, 19 with four lanes per row). k_gdn_scan below keeps the decode step, the per-token index map, the state-only pass and the operands
   // whose rows are not aligned.
-  if (state_indices_stride == 0 && o && (time_tile <= 0 || rpl == 17 || rpl == 18)) {
+  if (state_indices_stride == 0 && o && (time_tile <= 0 || (rpl >= 17 && rpl <= 19))) {
     const int rc = ix_gdn_walk(q, k, v, g, beta, o, io_dtype, state_pool, cu_seqlens, state_indices, q_pitch, k_pitch,
                                v_pitch, N, (int)H, (int)HV, K, (int)V, scale, 0, rpl >= 17 ? rpl - 16 : 0, st);
     if (rc != IX_DECLINED) return rc;

@@ -14,7 +14,7 @@
 // of rows or on which launch shape ran, so a row's bits are the same at any row count.
 //
 // Two launch shapes evaluate that same function:
-//   * rows >= IX_LP_SPLIT_BELOW : one 512-thread workgroup per row, one launch;
+//   * rows >= IX_LP_SPLIT_BELOW : one 512-thread workgroup per row, one launch (wide rows: a workgroup per CU that keeps them);
 //   * fewer rows                : row split over many workgroups (partial max, block sums,
 //                                 finalize) so a single decode row still fills the chip.
 #include "ix_common.h"
@@ -198,6 +198,146 @@ __global__ __launch_bounds__(512) void k_lp_row(const T* __restrict__ x, long ro
 #pragma unroll
       for (int i = 0; i < 8; ++i)
         if (off + i < V) orow[off + i] = (o[i] - mm) - ls;
+    }
+  }
+}
+
+// Shape 1 with the row kept on the CU between the maximum and the sums. A workgroup per CU walks the rows; a wave keeps HU of its
+// blocks in registers and LU in LDS, reads the others twice, and asks for the next row's block as soon as this row's is summed.
+// The blocks, their sums and the fold are k_lp_row's. Bound by HBM: of [1000, 151936] in bf16 all 40 blocks stay (5 a wave, 160
+// registers), 93 -> 70 us; in fp32 24 (two a wave in registers, one in LDS), 181 -> 129; 2900 rows 259 -> 179 and 506 -> 354.
+// Three fp32 blocks in registers leave none to work with (spilled loads have to be waited for: 155). The line: 1000 rows of
+// 65536, 16 blocks, fp32 77 -> 47, bf16 42 -> 35; of 32000, one block a wave, fp32 36 -> 42, bf16 20 -> 22.
+// The registers as they are: no widened copy of them lives on from an earlier use.
+__device__ __forceinline__ void ix_lp_keep(IxRaw8<bf16_t>& r) {
+  asm volatile("" : "+v"(r.v.x), "+v"(r.v.y), "+v"(r.v.z), "+v"(r.v.w));
+}
+__device__ __forceinline__ void ix_lp_keep(IxRaw8<float>&) {}
+#define IX_LP_HELD_UNITS 512
+#define IX_LP_HELD_V 65536  // columns from which a row is kept
+template <typename T, int HU, int LU>
+__global__ __launch_bounds__(512) void k_lp_row_held(const T* __restrict__ x, long row_stride, long rows, int V, int G,
+                                                     const int64_t* __restrict__ target, float* __restrict__ out_lp,
+                                                     float* __restrict__ out_lse) {
+  constexpr int NW = 8, CH = 4;  // CH: groups of a block that is not kept requested at once
+  extern __shared__ __align__(16) char ix_lp_lds[];
+  __shared__ float s_wmax[2][NW];
+  __shared__ float s_bsum[2][IX_LP_HELD_UNITS];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // scalar, and the blocks' addresses with it
+  const int L = V / G;
+  const int NB = (L + IX_LP_BLOCK - 1) / IX_LP_BLOCK;
+  const int units = G * NB;
+  IxRaw8<T>* kept = reinterpret_cast<IxRaw8<T>*>(ix_lp_lds) + (size_t)wave * LU * 8 * 64 + lane;  // [LU][8] of this lane
+
+  unsigned lane8 = lane * 8;
+  auto width = [&](int u) __attribute__((always_inline)) { return min(IX_LP_BLOCK, L - u % NB * IX_LP_BLOCK); };
+  // group c of block u; one past the block's end reads its first columns instead, which changes no maximum
+  auto load = [&](IxRaw8<T>& r, const T* xr, int u, int c) __attribute__((always_inline)) {
+    const T* blk = xr + (long)(u / NB) * L + u % NB * IX_LP_BLOCK;
+    const unsigned off = c * 512 + lane8;
+    r.load(blk + (off + 8 <= (unsigned)width(u) ? off : 0u));
+  };
+  auto add = [&](float (&acc)[8], const IxRaw8<T>& r, float m, int u, int c) __attribute__((always_inline)) {
+    // The term of a group past the end is exp(v - inf) = +0, or a NaN if v is one or +inf: v is a column of this block then,
+    // whose own term is a NaN as well.
+    const float mm = (unsigned)(c * 512) + lane8 + 8 <= (unsigned)width(u) ? m : -IX_NEG_INF;
+    float v[8];
+    r.widen(v);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) acc[i] = acc[i] + ix_exp_fast(v[i] - mm);
+  };
+
+  IxRaw8<T> held[HU][8];
+  long row = blockIdx.x;
+#pragma unroll
+  for (int j = 0; j < HU; ++j) {
+    if (wave + NW * j < units) {
+#pragma unroll
+      for (int c = 0; c < 8; ++c) load(held[j][c], x + row * row_stride, wave + NW * j, c);
+    }
+  }
+  for (int par = 0; row < rows; row += gridDim.x, par ^= 1) {
+    const T* xr = x + row * row_stride;
+    float m = IX_NEG_INF;
+    asm volatile("" : "+v"(lane8));  // the groups' offsets are computed where they are used, not kept in registers from row to row
+    for (int u = wave + NW * HU; u < units; u += NW) {
+      const int l = (u - wave) / NW - HU;
+#pragma unroll
+      for (int c0 = 0; c0 < 8; c0 += CH) {
+        IxRaw8<T> raw[CH];
+#pragma unroll
+        for (int c = 0; c < CH; ++c) load(raw[c], xr, u, c0 + c);
+#pragma unroll
+        for (int c = 0; c < CH; ++c) {
+          float v[8];
+          raw[c].widen(v);
+          m = fmaxf(m, ix_tree8_max(v));
+          if (LU > 0 && l < LU) kept[(l * 8 + c0 + c) * 64] = raw[c];
+        }
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < HU; ++j) {
+      if (wave + NW * j < units) {
+#pragma unroll
+        for (int c = 0; c < 8; ++c) {
+          float v[8];
+          held[j][c].widen(v);
+          m = fmaxf(m, ix_tree8_max(v));
+        }
+      }
+    }
+    m = ix_lane_max<64>(m);
+    if (lane == 0) s_wmax[par][wave] = m;
+    __syncthreads();
+    m = s_wmax[par][0];
+#pragma unroll
+    for (int w = 1; w < NW; ++w) m = fmaxf(m, s_wmax[par][w]);
+
+#pragma unroll
+    for (int j = 0; j < HU; ++j)
+#pragma unroll
+      for (int c = 0; c < 8; ++c) ix_lp_keep(held[j][c]);
+    const long next = row + gridDim.x;
+    asm volatile("" : "+v"(lane8));
+#pragma unroll
+    for (int j = 0; j < HU; ++j) {
+      const int u = wave + NW * j;
+      if (u < units) {
+        float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int c = 0; c < 8; ++c) add(acc, held[j][c], m, u, c);
+        if (next < rows) {
+#pragma unroll
+          for (int c = 0; c < 8; ++c) load(held[j][c], x + next * row_stride, u, c);
+        }
+        const float bs = ix_lane_tree<64>(ix_tree8(acc));
+        if (lane == 0) s_bsum[par][u] = bs;
+      }
+    }
+    for (int u = wave + NW * HU; u < units; u += NW) {
+      const int l = (u - wave) / NW - HU;
+      float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int c0 = 0; c0 < 8; c0 += CH) {
+        IxRaw8<T> raw[CH];
+#pragma unroll
+        for (int c = 0; c < CH; ++c) {
+          if (LU > 0 && l < LU) raw[c] = kept[(l * 8 + c0 + c) * 64];
+          else load(raw[c], xr, u, c0 + c);
+        }
+#pragma unroll
+        for (int c = 0; c < CH; ++c) add(acc, raw[c], m, u, c0 + c);
+      }
+      const float bs = ix_lane_tree<64>(ix_tree8(acc));
+      if (lane == 0) s_bsum[par][u] = bs;
+    }
+    __syncthreads();
+    if (wave == 0) {  // the others go on with the next row: its maxima and sums have places of their own
+      float leaf = lane < G ? ix_kahan_blocks(s_bsum[par] + lane * NB, NB) : 0.0f;
+      for (int s = 1; s < G; s <<= 1) leaf = leaf + __shfl_xor(leaf, s, IX_WAVE);  // ix_fold_leaves: lane 0 has the root
+      if (lane == 0) ix_lp_emit(xr, V, m, ix_log(leaf), target, row, out_lp, out_lse);
     }
   }
 }
@@ -458,6 +598,13 @@ static int ix_lp_launch(const T* x, long rows, long V, long row_stride, int G, c
   // a caller-supplied row max (exact, e.g. from the producing GEMM's epilogue) removes the max
   // pass: the row is then read from HBM once, by the block sums
   const bool split = row_max_in || force_shape == 2 || (force_shape == 0 && rows < IX_LP_SPLIT_BELOW);
+  if (!split && force_shape == 0 && vec && !out_full && V >= IX_LP_HELD_V &&
+      G * ((L + IX_LP_BLOCK - 1) / IX_LP_BLOCK) <= IX_LP_HELD_UNITS) {
+    constexpr int HU = sizeof(T) == 2 ? 5 : 2, LU = sizeof(T) == 2 ? 0 : 1;
+    hipLaunchKernelGGL((k_lp_row_held<T, HU, LU>), dim3((unsigned)(rows < 256 ? rows : 256)), dim3(512),
+                       (size_t)LU * 8 * IX_LP_BLOCK * sizeof(T), st, x, row_stride, rows, (int)V, G, target, out_lp, out_lse);
+    return ix_launch_status();
+  }
   if (!split) {
     hipLaunchKernelGGL((k_lp_row<T>), dim3((unsigned)rows), dim3(512), 0, st, x, row_stride, (int)V, G, target,
                        out_lp, out_lse, out_full, full_stride, vec);

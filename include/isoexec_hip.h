@@ -287,6 +287,15 @@ int ix_gdn_decode_prep(const void* x, long x_pitch, const void* a, long a_pitch,
 int ix_gdn_resolve_rows(const void* slots, int slots_i64, long n, const int64_t* slot2row, long map_n, long blocks,
                         int64_t* rows64, int* rows32, int64_t* last_used, int64_t* clock, void* stream);
 
+/* A prefill's edits of a layer's tables and pools in one launch (gdn_recurrent_state.py prefill: the slot-map scatter, the use
+ * stamps, zeroed fresh rows). map_edits int64 [2][edits]: slot2row[map_edits[0][i]] = map_edits[1][i] (slots outside
+ * [0, map_n) skipped). stamps int64 [2][stamped], rows distinct: last_used[stamps[0][i]] = clock[0] + stamps[1][i], then
+ * clock[0] += advance. fresh int32 [N]: those rows of pool fp32 [pool_rows, row_floats], and of pool2 if it is not NULL, become
+ * zero, and so do pos[fresh[i]] and pos[0] if pos (int64 [pool_rows]) is not NULL. Rows outside the pool are skipped. */
+int ix_gdn_prefill_begin(const int64_t* map_edits, long edits, const int64_t* stamps, long stamped, long advance,
+                         const int* fresh, long N, int64_t* slot2row, long map_n, int64_t* last_used, int64_t* clock,
+                         float* pool, float* pool2, int64_t* pos, long pool_rows, long row_floats, void* stream);
+
 /* cpr_buffer_scatter (gdn_cpr_scatter.py:24-76; eager form in CprGDN.decode, gdn_cpr_state.py): lane n of a decode
  * step appends its prepared k [H*K] (token pitch k_pitch), v [HV*V] (v_pitch), g fp32 [HV], beta [HV] to the
  * open-chunk buffers k_buf [rows, C, H, K], v_buf [rows, C, HV, V], g_buf fp32 [rows, C, HV], b_buf [rows, C, HV] at

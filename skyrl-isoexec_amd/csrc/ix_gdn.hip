@@ -1528,6 +1528,71 @@ extern "C" int ix_gdn_resolve_rows(const void* slots, int slots_i64, long n, con
 }
 
 // ---------------------------------------------------------------------------------------------
+// What a prefill does to a layer's tables and pools in front of its kernels (gdn_recurrent_state.py prefill: slot-map scatter,
+// use stamps, fresh rows zeroed), in one launch and from one upload: ten launches and copies of 4 to 5 us each before, none
+// of which has work to speak of (8192 tokens through one layer 1088 -> 1047 us, the l2norm folded into the convolution with it).
+// Workgroup 0 edits the tables (it alone reads the clock before it advances it), the others zero IX_GDN_ZERO floats each of a
+// fresh row in the pools. The null row is zeroed once, however many sequences start no row.
+#define IX_GDN_ZERO 8192
+__global__ __launch_bounds__(256) void k_gdn_prefill_begin(const int64_t* __restrict__ map_edits, int edits,
+                                                           const int64_t* __restrict__ stamps, int stamped, long advance,
+                                                           const int* __restrict__ fresh, int N, int64_t* __restrict__ slot2row,
+                                                           long map_n, int64_t* __restrict__ last_used,
+                                                           int64_t* __restrict__ clock, float* __restrict__ pool,
+                                                           float* __restrict__ pool2, int64_t* __restrict__ pos, long pool_rows,
+                                                           long row_floats, int per_row) {
+  const int tid = threadIdx.x;
+  if (blockIdx.x == 0) {
+    for (int i = tid; i < edits; i += 256) {
+      const int64_t slot = map_edits[i], row = map_edits[edits + i];
+      if (slot >= 0 && slot < map_n) slot2row[slot] = row;
+    }
+    const int64_t now = clock ? clock[0] : 0;
+    for (int i = tid; i < stamped; i += 256) {
+      const int64_t row = stamps[i];
+      if (row >= 0 && row < pool_rows) last_used[row] = now + stamps[stamped + i];
+    }
+    if (pos) {
+      for (int i = tid; i < N; i += 256)
+        if (fresh[i] >= 0 && fresh[i] < pool_rows) pos[fresh[i]] = 0;
+      if (tid == 0) pos[0] = 0;  // the null row's
+    }
+    __syncthreads();
+    if (clock && tid == 0) clock[0] = now + advance;
+    return;
+  }
+  const long at = blockIdx.x - 1;
+  const int n = (int)(at / per_row);
+  const int row = fresh[n];
+  if (row < 0 || row >= pool_rows) return;
+  if (row == 0)
+    for (int j = 0; j < n; ++j)
+      if (fresh[j] == 0) return;
+  const long lo = at % per_row * (long)IX_GDN_ZERO, hi = min(row_floats, lo + IX_GDN_ZERO);
+  for (long i = lo + 4 * tid; i < hi; i += 1024) {  // row_floats % 4 == 0
+    *reinterpret_cast<float4*>(pool + row * row_floats + i) = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    if (pool2) *reinterpret_cast<float4*>(pool2 + row * row_floats + i) = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+  }
+}
+
+extern "C" int ix_gdn_prefill_begin(const int64_t* map_edits, long edits, const int64_t* stamps, long stamped, long advance,
+                                    const int* fresh, long N, int64_t* slot2row, long map_n, int64_t* last_used,
+                                    int64_t* clock, float* pool, float* pool2, int64_t* pos, long pool_rows, long row_floats,
+                                    void* stream) {
+  if (edits < 0 || stamped < 0 || N < 0 || advance < 0 || pool_rows <= 0 || row_floats <= 0 || !pool) return IX_ERR_ARG;
+  if ((edits > 0 && (!map_edits || !slot2row || map_n <= 0)) || (stamped > 0 && (!stamps || !last_used || !clock)) ||
+      (N > 0 && !fresh))
+    return IX_ERR_ARG;
+  if (row_floats % 4 || !ix_aligned(pool, 16) || (pool2 && !ix_aligned(pool2, 16))) return IX_DECLINED;
+  const long per_row = (row_floats + IX_GDN_ZERO - 1) / IX_GDN_ZERO;
+  if (edits > 0x7fffffffL || stamped > 0x7fffffffL || N * per_row >= 0x7fffffffL) return IX_DECLINED;
+  hipLaunchKernelGGL(k_gdn_prefill_begin, dim3((unsigned)(1 + N * per_row)), dim3(256), 0, (hipStream_t)stream, map_edits,
+                     (int)edits, stamps, (int)stamped, advance, fresh, (int)N, slot2row, map_n, last_used, clock, pool, pool2,
+                     pos, pool_rows, row_floats, (int)per_row);
+  return ix_launch_status();
+}
+
+// ---------------------------------------------------------------------------------------------
 // Causal depthwise conv of width W <= 8 over packed tokens (gdn_ops.py:74-170):
 //   acc = 0; for i = 0..W-1: acc = acc + w[d,i] * xp[t+i]   (multiply rounded, add rounded)
 //   acc = acc + bias[d]; acc = acc * sigmoid(acc); y = bf16(acc)

@@ -454,6 +454,9 @@ class CprGDN(RecurrentGDN):
     def _on_row_released(self, row: int) -> None:
         self._reset_rows([row])
 
+    def _fresh_state(self):
+        return self.entry_state, self.pos
+
     def _zero_fresh_rows(self, fresh_rows: torch.Tensor) -> None:
         super()._zero_fresh_rows(fresh_rows)
         self.entry_state.index_fill_(0, fresh_rows, 0.0)

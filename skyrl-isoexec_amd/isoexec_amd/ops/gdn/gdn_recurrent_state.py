@@ -26,6 +26,8 @@ from typing import Callable, Iterable, Sequence
 import numpy as np
 import torch
 
+from ... import _lib
+from ...debug.trace import get_tracer
 from .gdn_ops import conv_packed, decode_prep, gate_and_beta_fp32, gdn_l2norm, gdn_recurrent_kernel
 
 _SLOT_MAP_ENV = "SKYRL_ISOEXEC_GDN_SLOT_MAP_SIZE"
@@ -475,11 +477,16 @@ class RecurrentGDN:
         has_initial_state=None,
         prefill_query_start_loc: torch.Tensor | None = None,
         gated_norm: tuple | None = None,
+        fuse_l2norm: bool | None = None,
     ) -> torch.Tensor:
         """Prefill a packed batch of N prompts (or prompt chunks). Returns ``o [T, HV, V]``; with ``gated_norm``
-        (``gdn_recurrent_kernel``'s) the output comes back through the layer's gated output norm."""
+        (``gdn_recurrent_kernel``'s) the output comes back through the layer's gated output norm. ``fuse_l2norm=False`` keeps
+        the convolution and the l2norm apart (each op's output is a region of its own; the default while a trace is attached
+        and there is no ``gated_norm``); the same bits."""
+        if fuse_l2norm is None:
+            fuse_l2norm = gated_norm is not None or get_tracer() is None
         rows, is_cont, rows_out, cu, q, k, v, g, beta = self._prefill_prepare(
-            slots_cpu, x, a, b, qsl, has_initial_state, prefill_query_start_loc, fuse_l2norm=gated_norm is not None)
+            slots_cpu, x, a, b, qsl, has_initial_state, prefill_query_start_loc, fuse_l2norm=fuse_l2norm)
         o = gdn_recurrent_kernel(q.unsqueeze(0), k.unsqueeze(0), v.unsqueeze(0), g.unsqueeze(0), beta.unsqueeze(0),
                                  ssm_state=self.ssm_state, state_indices=rows_out, cu_seqlens=cu, gated_norm=gated_norm)
         return o[0]
@@ -490,6 +497,7 @@ class RecurrentGDN:
         device, cu int32 device, q, k, v, g, beta)`` with q, k ``[T, H, K]``, v ``[T, HV, V]``, g, beta ``[T, HV]``."""
         N = len(slots_cpu)
         dev = x.device
+        begin = self._begin_served(dev)
         if len(qsl) != N + 1 or qsl[-1] != x.shape[0]:
             raise ValueError(f"qsl {list(qsl)} does not describe {N} sequences over {x.shape[0]} packed tokens")
         if self._native:
@@ -506,20 +514,11 @@ class RecurrentGDN:
         else:
             # Membership is read before assignment edits the table; fresh and resumed rows may mix.
             is_cont = self._continuation_mask(slots_cpu, has_initial_state)
-            rows = self._assign_many(slots_cpu)
-        # One upload carries the three row lists: where each sequence stores, where it resumes from
-        # (0 = from nothing) and which rows start fresh (0 = none; zeroing the null row is harmless).
-        meta = np.array(
-            [rows, [r if c else 0 for r, c in zip(rows, is_cont)], [0 if c else r for r, c in zip(rows, is_cont)]],
-            dtype=np.int32,
-        )
-        meta_t = torch.from_numpy(meta).to(dev, non_blocking=True)
-        rows_out, rows_in = meta_t[0], meta_t[1]
-        cu = prefill_query_start_loc
-        if cu is None:
-            cu = torch.from_numpy(np.asarray(qsl, dtype=np.int32)).to(dev, non_blocking=True)
-        # A fresh row must start from zero; a resumed row keeps what the previous chunk left.
-        self._zero_fresh_rows(meta_t[2].long())
+            rows = None if begin else self._assign_many(slots_cpu)
+        if begin:
+            rows, rows_in, rows_out, cu = self._prefill_begin(slots_cpu, rows, is_cont, qsl, prefill_query_start_loc, dev)
+        else:
+            rows_in, rows_out, cu = self._prefill_upload(rows, is_cont, qsl, prefill_query_start_loc, dev)
         if fuse_l2norm:  # q and k leave the convolution's launch normalised where the library serves that form
             y = conv_packed(x, self.conv_weight, self.conv_bias, cu_seqlens=cu, conv_state=self.conv_state,
                             rows_in=rows_in, rows_out=rows_out, activation=self.activation,
@@ -531,6 +530,65 @@ class RecurrentGDN:
             q, k, v = self._split_qkv(y)
         g, beta = self._gate_and_beta(a, b)
         return rows, is_cont, rows_out, cu, q, k, v, g, beta
+
+    def _fresh_state(self):
+        """What becomes zero with a fresh row beside ``ssm_state``: (fp32 pool of its shape or None, int64 positions or None)."""
+        return None, None
+
+    def _begin_served(self, dev) -> bool:
+        pools = [self.ssm_state] + [t for t in self._fresh_state() if t is not None]
+        return dev.type == "cuda" and all(t.device == dev and t.is_contiguous() and t.data_ptr() % 16 == 0 for t in pools) \
+            and self.ssm_state[0].numel() % 4 == 0
+
+    def _prefill_begin(self, slots_cpu, rows, is_cont, qsl, cu, dev):
+        """Rows assigned (``rows`` given: a native layer's), the device's tables brought up to date and fresh rows zeroed: one
+        upload and one launch. Returns ``(rows, rows_in, rows_out, cu)``, the last three int32 on the device."""
+        edits, ticks, table = None, {}, self.table
+        if rows is None:
+            rows = table.assign_many(slots_cpu, lru_snapshot=self.last_used.tolist)
+            edits = table.drain_outbox()
+            ticks = {r: j + 1 for j, r in enumerate(rows)}  # a row named twice keeps its last tick
+        N, ne, nt = len(rows), 0 if edits is None else len(edits[0]), len(ticks)
+        # int64: map edits, stamps; int32: where each sequence stores, where it resumes from (0 = from nothing), which rows start
+        # fresh (0 = none), token offsets
+        host = np.empty(2 * (ne + nt) + (4 * N + 2) // 2, dtype=np.int64)
+        if ne:
+            host[:ne], host[ne:2 * ne] = edits
+        if nt:
+            host[2 * ne:2 * ne + nt], host[2 * ne + nt:2 * (ne + nt)] = list(ticks.keys()), list(ticks.values())
+        small = host[2 * (ne + nt):].view(np.int32)
+        small[:N] = rows
+        small[N:2 * N] = [r if c else 0 for r, c in zip(rows, is_cont)]
+        small[2 * N:3 * N] = [0 if c else r for r, c in zip(rows, is_cont)]
+        small[3 * N:4 * N + 1] = qsl
+        t = torch.from_numpy(host).to(dev, non_blocking=True)
+        st = t[2 * (ne + nt):].view(torch.int32)
+        pool2, pos = self._fresh_state()
+        own = table is not None
+        base = t.data_ptr()
+        rc = _lib.check(_lib.lib().ix_gdn_prefill_begin(
+            base, ne, base + 16 * ne, nt, N if own else 0, st[2 * N:].data_ptr(), N, _lib.ptr(self.slot2row) if own else None,
+            self.slot2row.numel() if own else 0, _lib.ptr(self.last_used) if own else None, _lib.ptr(self._clock) if own else None,
+            self.ssm_state.data_ptr(), _lib.ptr(pool2), _lib.ptr(pos), self.ssm_state.shape[0], self.ssm_state[0].numel(),
+            _lib.current_stream(dev)), "ix_gdn_prefill_begin")
+        if rc != _lib.IX_OK:
+            raise RuntimeError(f"[isoexec-gdn] prefill: {N} sequences are more than one launch takes")
+        return rows, st[N:2 * N], st[:N], st[3 * N:4 * N + 1] if cu is None else cu
+
+    def _prefill_upload(self, rows, is_cont, qsl, cu, dev):
+        """The same with torch's operators, for rows already assigned. Returns ``(rows_in, rows_out, cu)``."""
+        # One upload carries the three row lists: where each sequence stores, where it resumes from
+        # (0 = from nothing) and which rows start fresh (0 = none; zeroing the null row is harmless).
+        meta = np.array(
+            [rows, [r if c else 0 for r, c in zip(rows, is_cont)], [0 if c else r for r, c in zip(rows, is_cont)]],
+            dtype=np.int32,
+        )
+        meta_t = torch.from_numpy(meta).to(dev, non_blocking=True)
+        if cu is None:
+            cu = torch.from_numpy(np.asarray(qsl, dtype=np.int32)).to(dev, non_blocking=True)
+        # A fresh row must start from zero; a resumed row keeps what the previous chunk left.
+        self._zero_fresh_rows(meta_t[2].long())
+        return meta_t[1], meta_t[0], cu
 
     def _zero_fresh_rows(self, fresh_rows: torch.Tensor) -> None:
         """Rows that start a new request (device int64, 0 = none)."""

@@ -489,7 +489,8 @@ class RolloutEngine:
                 o = layer.prefill(slots_t, slots, qkv, a, bb, qsl, prefill_query_start_loc=cu, fuse_l2norm=b.fuse_ops)
                 return b.gdn_out(i, o, z)
             if not b.fuse_ops:
-                return b.gdn_out(i, layer.prefill(slots_t, slots, qkv, a, bb, qsl, prefill_query_start_loc=cu), z)
+                return b.gdn_out(i, layer.prefill(slots_t, slots, qkv, a, bb, qsl, prefill_query_start_loc=cu,
+                                                      fuse_l2norm=False), z)
             o = layer.prefill(slots_t, slots, qkv, a, bb, qsl, prefill_query_start_loc=cu,
                               gated_norm=b.gdn_gated_norm(i, z))
             return b.gdn_out(i, o, z, normed=True)

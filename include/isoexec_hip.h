@@ -145,7 +145,7 @@ int ix_moe_combine_add_rmsnorm(const void* expert_out, const int* combine_rows, 
  * split-K. C is bf16 (one round of the accumulator) or, with c_dtype = IX_DT_F32, the fp32
  * accumulator itself (the router's fp32 gating product when its fp32 weight is bf16-exact).
  * lda/ldw/ldc are row pitches in elements. bias (bf16 [N]) may be NULL. tile: 0 auto; 1..6 name a tile shape
- * (32x256, 128x128, 256x256 on eight waves, 256x256 on four waves, 128x256, 64x32); 4 takes the streaming form of its
+ * (32x256, 128x128, 256x256 on eight waves, 256x256 on four waves, 128x256, 64x32), 9 a tile of 32x32; 4 takes the streaming form of its
  * tile (one workgroup per CU walks many tiles) when the product has at least 512 tiles and the form serves it (bf16 C,
  * no bias, K a multiple of 64 and >= 704, N and ldc multiples of 8, C 16-byte aligned), 7 never does, 8 always does
  * and declines what the form does not serve. 14..17 are bands of 128, 160, 192 and 224 rows x 256 columns of that form, K >= 768:

@@ -231,7 +231,8 @@ static int ix_gemm_tile_for(long M, long N, long K, int tile, bool bands) {
   if (tile != 0) return tile;
   // One 128-wide column of tiles (the router's gating product): 128-row tiles once there are enough of them to fill
   // the chip, the small tile below that (2048 x 2048 x 128: 20.7 -> 8.5 us; equal at 16384 rows).
-  if (M > 128 && N <= 128) return M >= 16384 ? 2 : 6;
+  const bool halves = M <= 32 || ((M + 31) / 32) * ((N + 31) / 32) <= 256;  // of the small tile, see below
+  if (M > 128 && N <= 128) return M >= 16384 ? 2 : (halves ? 9 : 6);
   // us_ktile: a tile with its CU to itself; us_ktile_more: one of several (for id 2 and 6: of a pair that shares the CU)
   struct Shape { int id, bm, bn; double us_ktile, us_ktile_more, fixed, stream; };
   static const Shape shapes[] = {{4, 256, 256, 0.98, 1.4, 4.4, 4.4e6},
@@ -268,13 +269,18 @@ static int ix_gemm_tile_for(long M, long N, long K, int tile, bool bands) {
       best = sh.id;
     }
   }
-  return best;
+  // The 64 x 32 tile in halves of 32 rows: for few rows its other half only takes room in the ring, whose bytes under way are
+// what a CU's share of the weight waits for (ten stages of 8 KiB instead of six of 12), and at one turn of tiles the halves are
+// on two CUs. With more turns every weight tile is read twice instead. us 64 x 32 / 32 x 32, weights from memory: 2048 x 4096 at
+// 1 row 12.6 / 10.3, 32 13.4 / 12.2, 64 15.8 / 12.2; 5120 x 2048 at 1 8.9 / 7.7, 32 9.4 / 8.5, 64 (320 halves) 10.4 / 12.4;
+// 12352 x 2048 at 32 17.2 / 15.2, 33 16.8 / 19.6; 4096 x 4096 at 64 16.9 / 13.0, 100 14.8 / 17.4; 128 x 4096 at 2000 11.6 / 10.7, 4096 13.0 / 15.5.
+  return best == 6 && halves ? 9 : best;
 }
 
 // Row-max parts per row of C: one per column tile of the shape that runs.
 extern "C" long ix_gemm_bf16_n_tiles(long M, long N, long K, int tile) {
   const int t = ix_gemm_tile_for(M, N, K, tile, true);
-  const long bn = (t == 2) ? 128 : (t == 6) ? 32 : 256;  // ids 1, 3, 4, 5, 7, 8 are 256 wide
+  const long bn = (t == 2) ? 128 : (t == 6 || t == 9) ? 32 : 256;  // ids 1, 3, 4, 5, 7, 8 are 256 wide
   // the four-wave tiles write one part per wave column
   const long per_tile = t > IX_TILE_BAND ? 4 : ((t == 4 || t == 7 || t == 8) ? 2 : 1);
   return N <= 0 ? 0 : per_tile * ((N + bn - 1) / bn);
@@ -294,11 +300,11 @@ static int ix_gemm_bf16_dispatch(const bf16_t* a, long lda, const bf16_t* w, lon
   if (id > IX_TILE_BAND && !bands_fit) {
     if (tile != 0) return IX_DECLINED;
     // Chosen by size for a call with a bias, an fp32 result or unaligned rows: the shape that the model takes without bands
-    // fills a band's four slots per tile. The 64 x 32 tile has more parts than that: the 128 x 128 one in its place.
+    // fills a band's four slots per tile. The tiles of 32 columns have more parts than that: the 128 x 128 one in their place.
     // us in the 256-row tile / here, with a bias: 128 rows of 151936 x 2048 277 / 154, 385 of 12352 x 2048 76 / 39, 300 of
     // 40000 x 768 69 / 44; with an fp32 result 214 / 172, 54 / 37, 65 / 41.
     id = ix_gemm_tile_for(rows, N, K, 0, false);
-    if (id == 6) id = 2;
+    if (id == 6 || id == 9) id = 2;
     slots = 4 * ((N + 255) / 256);
   }
   switch (id) {
@@ -319,6 +325,7 @@ static int ix_gemm_bf16_dispatch(const bf16_t* a, long lda, const bf16_t* w, lon
       return ix_gemm_bf16_launch<256, 256, 2, 2, TC>(a, lda, w, ldw, b, c, ldc, M, N, K, parts, parts_ld, st IX_BATCH_ARGS);
     case 5: return ix_gemm_bf16_launch<128, 256, 2, 4, TC>(a, lda, w, ldw, b, c, ldc, M, N, K, parts, parts_ld, st IX_BATCH_ARGS);
     case 6: return ix_gemm_bf16_launch<64, 32, 2, 1, TC, 2>(a, lda, w, ldw, b, c, ldc, M, N, K, parts, parts_ld, st IX_BATCH_ARGS);
+    case 9: return ix_gemm_bf16_launch<32, 32, 1, 1, TC, 2>(a, lda, w, ldw, b, c, ldc, M, N, K, parts, parts_ld, st IX_BATCH_ARGS);
     case 8:  // the streaming form whatever the number of tiles (declines what it does not serve)
       if constexpr (sizeof(TC) == 2) {
         if (ix_gemm_stream_fits(c, ldc, M, N, K, b, batch))

@@ -83,8 +83,9 @@ struct IxGemmCfg {
 #ifndef IX_SPLIT_STAGES_SMALL
 #define IX_SPLIT_STAGES_SMALL 6
 #endif
-  static constexpr int SPLIT_STAGES =
-      (144 * 1024) / STAGE_BYTES > IX_SPLIT_STAGES_SMALL ? IX_SPLIT_STAGES_SMALL : (144 * 1024) / STAGE_BYTES;
+  // The 32 x 32 tile's stages are 8 KiB: ten still let two workgroups share a CU.
+  static constexpr int SPLIT_MAX = BM == 32 && BN == 32 ? 10 : IX_SPLIT_STAGES_SMALL;
+  static constexpr int SPLIT_STAGES = (144 * 1024) / STAGE_BYTES > SPLIT_MAX ? SPLIT_MAX : (144 * 1024) / STAGE_BYTES;
   static constexpr int LDS_BYTES =
       PW > 0 ? SPLIT_STAGES * STAGE_BYTES
              : (UNIT_RING ? UNITS * BM * 128

@@ -101,6 +101,13 @@ __device__ __forceinline__ float ix_fold_leaves(float* leaf, int G) {
   return leaf[0];
 }
 
+// log S of a row from its block sums, by one wave: a lane per leaf, folded as ix_fold_leaves does. Valid in lane 0.
+__device__ __forceinline__ float ix_log_total(const float* __restrict__ bsum, int G, int NB, int lane) {
+  float leaf = lane < G ? ix_kahan_blocks(bsum + lane * NB, NB) : 0.0f;
+  for (int s = 1; s < G; s <<= 1) leaf = leaf + __shfl_xor(leaf, s, IX_WAVE);
+  return ix_log(leaf);
+}
+
 template <typename T>
 __device__ __forceinline__ void ix_lp_emit(const T* __restrict__ xr, int V, float m, float log_s,
                                            const int64_t* __restrict__ target, long row, float* out_lp,
@@ -335,9 +342,8 @@ __global__ __launch_bounds__(512) void k_lp_row_held(const T* __restrict__ x, lo
     }
     __syncthreads();
     if (wave == 0) {  // the others go on with the next row: its maxima and sums have places of their own
-      float leaf = lane < G ? ix_kahan_blocks(s_bsum[par] + lane * NB, NB) : 0.0f;
-      for (int s = 1; s < G; s <<= 1) leaf = leaf + __shfl_xor(leaf, s, IX_WAVE);  // ix_fold_leaves: lane 0 has the root
-      if (lane == 0) ix_lp_emit(xr, V, m, ix_log(leaf), target, row, out_lp, out_lse);
+      const float log_s = ix_log_total(s_bsum[par], G, NB, lane);
+      if (lane == 0) ix_lp_emit(xr, V, m, log_s, target, row, out_lp, out_lse);
     }
   }
 }
@@ -346,7 +352,7 @@ __global__ __launch_bounds__(512) void k_lp_row_held(const T* __restrict__ x, lo
 // Shape 2: the row split over many workgroups. Workspace layout (floats):
 //   pmax [rows, P]  P = ceil(V / IX_LP_SEG)
 //   bsum [rows, U]  U = G * NB
-//   fin  [rows, 2]  (m, log S)
+//   (and two floats per row that nothing uses: the size is part of the interface)
 template <typename T>
 __global__ __launch_bounds__(256) void k_lp_partmax(const T* __restrict__ x, long row_stride, int V, int P,
                                                     float* __restrict__ pmax, int vec) {
@@ -403,7 +409,7 @@ __global__ __launch_bounds__(256) void k_lp_blocksums(const T* __restrict__ x, l
 template <typename T>
 __global__ __launch_bounds__(64) void k_lp_finalize(const T* __restrict__ x, long row_stride, int V, int G, int P,
                                                     const float* __restrict__ pmax,
-                                                    const float* __restrict__ bsum, float* __restrict__ fin,
+                                                    const float* __restrict__ bsum,
                                                     const int64_t* __restrict__ target,
                                                     float* __restrict__ out_lp, float* __restrict__ out_lse) {
   __shared__ float s_leaf[IX_LP_MAX_G];
@@ -417,28 +423,70 @@ __global__ __launch_bounds__(64) void k_lp_finalize(const T* __restrict__ x, lon
   if (lane == 0) {
     const float S = ix_fold_leaves(s_leaf, G);
     const float log_s = ix_log(S);
-    fin[row * 2 + 0] = m;
-    fin[row * 2 + 1] = log_s;
     ix_lp_emit(x + row * row_stride, V, m, log_s, target, row, out_lp, out_lse);
   }
 }
 
+// The whole row, and its lse. Every workgroup joins the row's block sums for itself (a wave, while the columns travel) instead
+// of a launch in front that does it once: 4.6 us less for a decode step. Bound by HBM: four columns per lane and access, so that
+// a store instruction is 1 KiB of the row, all of them requested first: 64 rows of 151936 26.5 -> 10.2 us (eight columns
+// per lane stored one by one before).
+__device__ __forceinline__ void ix_lp_load4(const float* p, float (&v)[4]) {
+  const float4 a = *reinterpret_cast<const float4*>(p);
+  v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w;
+}
+__device__ __forceinline__ void ix_lp_load4(const bf16_t* p, float (&v)[4]) {
+  const uint2 a = *reinterpret_cast<const uint2*>(p);
+  v[0] = __uint_as_float(a.x << 16); v[1] = __uint_as_float(a.x & 0xffff0000u);
+  v[2] = __uint_as_float(a.y << 16); v[3] = __uint_as_float(a.y & 0xffff0000u);
+}
 template <typename T>
-__global__ __launch_bounds__(256) void k_lp_fullwrite(const T* __restrict__ x, long row_stride, int V,
-                                                      const float* __restrict__ fin, float* __restrict__ out_full,
-                                                      long full_stride, int vec, int PW) {
+__global__ __launch_bounds__(256) void k_lp_fullwrite(const T* __restrict__ x, long row_stride, int V, int G, int P,
+                                                      const float* __restrict__ pmax, const float* __restrict__ bsum,
+                                                      float* __restrict__ out_full, long full_stride,
+                                                      float* __restrict__ out_lse, int vec, int PW) {
+  constexpr int GROUPS = IX_LP_SEG / (256 * 4);
+  __shared__ float s_fin[2];
   const long row = blockIdx.x / PW;  // segments fastest
   const T* xr = x + row * row_stride;
   float* orow = out_full + row * full_stride;
-  const float mm = fin[row * 2], ls = fin[row * 2 + 1];
-  const long lo = (long)(blockIdx.x % PW) * IX_LP_SEG;
-  const long hi = min((long)V, lo + IX_LP_SEG);
-  for (long off = lo + (long)threadIdx.x * 8; off < hi; off += 256 * 8) {
-    float o[8];
-    ix_load8(xr + off, hi - off, vec != 0, 0.0f, o);
+  const int lo = (int)(blockIdx.x % PW) * IX_LP_SEG;
+  const int hi = min(V, lo + IX_LP_SEG);
+  float v[GROUPS][4];
+  if (vec) {  // whole groups of four; an absent one reads the segment's first columns
 #pragma unroll
-    for (int i = 0; i < 8; ++i)
-      if (off + i < hi) orow[off + i] = (o[i] - mm) - ls;
+    for (int c = 0; c < GROUPS; ++c) {
+      const int off = lo + (c * 256 + (int)threadIdx.x) * 4;
+      ix_lp_load4(xr + (off < hi ? off : lo), v[c]);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  if (threadIdx.x < 64) {
+    const int NB = (V / G + IX_LP_BLOCK - 1) / IX_LP_BLOCK;
+    const float m = ix_row_max_from_parts(pmax + row * P, P, threadIdx.x);
+    const float log_s = ix_log_total(bsum + row * (long)(G * NB), G, NB, threadIdx.x);
+    if (threadIdx.x == 0) {
+      s_fin[0] = m;
+      s_fin[1] = log_s;
+      if (out_lse && lo == 0) out_lse[row] = m + log_s;
+    }
+  }
+  __syncthreads();
+  const float mm = s_fin[0], ls = s_fin[1];
+  if (vec) {
+#pragma unroll
+    for (int c = 0; c < GROUPS; ++c) {
+      const int off = lo + (c * 256 + (int)threadIdx.x) * 4;
+      if (off < hi)
+        *reinterpret_cast<float4*>(orow + off) =
+            make_float4((v[c][0] - mm) - ls, (v[c][1] - mm) - ls, (v[c][2] - mm) - ls, (v[c][3] - mm) - ls);
+    }
+    return;
+  }
+  for (int j = lo + (int)threadIdx.x; j < hi; j += 256) {
+    float o[8];
+    ix_load8(xr + j, 1, false, 0.0f, o);
+    orow[j] = (o[0] - mm) - ls;
   }
 }
 
@@ -618,7 +666,6 @@ static int ix_lp_launch(const T* x, long rows, long V, long row_stride, int G, c
   const int U = G * NB;
   float* ws_pmax = ws;
   float* bsum = ws_pmax + rows * PW;
-  float* fin = bsum + rows * U;
   const int P = row_max_in ? 1 : PW;
   const float* pmax = row_max_in ? row_max_in : ws_pmax;
   if (!row_max_in)
@@ -628,11 +675,14 @@ static int ix_lp_launch(const T* x, long rows, long V, long row_stride, int G, c
   const unsigned total = (unsigned)(rows * ny);
   hipLaunchKernelGGL((k_lp_blocksums<T>), dim3(ix_xcd_run_grid(total)), dim3(256), 0, st, x, row_stride, (int)V, G,
                      P, pmax, bsum, vec, ny, total);
-  hipLaunchKernelGGL((k_lp_finalize<T>), dim3((unsigned)rows), dim3(64), 0, st, x, row_stride, (int)V, G, P, pmax,
-                     bsum, fin, target, out_lp, out_lse);
-  if (out_full)
-    hipLaunchKernelGGL((k_lp_fullwrite<T>), dim3((unsigned)(rows * PW)), dim3(256), 0, st, x, row_stride, (int)V, fin,
-                       out_full, full_stride, vec, PW);
+  if (!out_full) {
+    hipLaunchKernelGGL((k_lp_finalize<T>), dim3((unsigned)rows), dim3(64), 0, st, x, row_stride, (int)V, G, P, pmax,
+                       bsum, target, out_lp, out_lse);
+    return ix_launch_status();
+  }
+  const int vec4 = vec && full_stride % 4 == 0 && ix_aligned(out_full, 16);
+  hipLaunchKernelGGL((k_lp_fullwrite<T>), dim3((unsigned)(rows * PW)), dim3(256), 0, st, x, row_stride, (int)V, G, P, pmax,
+                     bsum, out_full, full_stride, out_lse, vec4, PW);
   return ix_launch_status();
 }
 

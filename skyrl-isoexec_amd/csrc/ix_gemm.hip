@@ -274,6 +274,10 @@ static int ix_gemm_tile_for(long M, long N, long K, int tile, bool bands) {
 // on two CUs. With more turns every weight tile is read twice instead. us 64 x 32 / 32 x 32, weights from memory: 2048 x 4096 at
 // 1 row 12.6 / 10.3, 32 13.4 / 12.2, 64 15.8 / 12.2; 5120 x 2048 at 1 8.9 / 7.7, 32 9.4 / 8.5, 64 (320 halves) 10.4 / 12.4;
 // 12352 x 2048 at 32 17.2 / 15.2, 33 16.8 / 19.6; 4096 x 4096 at 64 16.9 / 13.0, 100 14.8 / 17.4; 128 x 4096 at 2000 11.6 / 10.7, 4096 13.0 / 15.5.
+  // Weight rows 4 KiB apart and a few rows: 128 of them per tile are read at 4.6 TB/s by this memory system, 32 at up to 5.9. us
+  // 128 x 128 / 32 x 32: 151936 x 2048 at 1 row 134 / 105, 16 129 / 117, 24 130 / 126 (with the row maximum and the norm in front 142 / 144), 32 135 / 134; 65536 x 2048 at 7 62 / 57; 32000
+  // x 2048 32.1 / 31.3; rows 8 KiB apart (151936 x 4096 at 7) 195 / 206, 2 KiB 55 / 61.
+  if (M <= 16 && K * 2 == 4096 && N >= 32000) return 9;
   return best == 6 && halves ? 9 : best;
 }
 

@@ -28,7 +28,8 @@ def test_tile_of_32_rows_and_columns(M, N, K):
 
 
 # the sizes at which the rule changes over (32 rows; 256 tiles), with the row maximum of the shape it takes
-@pytest.mark.parametrize("M,N,K", [(32, 5120, 512), (33, 5120, 512), (64, 4096, 512), (65, 4096, 512), (128, 2048, 512), (129, 64, 512)])
+@pytest.mark.parametrize("M,N,K", [(32, 5120, 512), (33, 5120, 512), (64, 4096, 512), (65, 4096, 512), (128, 2048, 512), (129, 64, 512),
+                                   (16, 32000, 2048), (17, 32000, 2048)])
 def test_rule_of_the_small_tiles(M, N, K):
     from isoexec_amd.ops.mm.mm_hip import linear_nt
 

@@ -215,7 +215,7 @@ __global__ __launch_bounds__(256) void k_gdn_scan(const TIO* __restrict__ q, con
 // rows (A, one value per lane), S the accumulator, whose register layout is the one above. With one product per element
 // that instruction is a fused multiply-add, rounded once, subnormals kept (2 M random, tiny and special operands against fmaf:
 // every bit but a NaN's payload); of the four multiply-adds per element and token one leaves the vector pipe, which bounds
-// this kernel: 250 vector and matrix instructions per token for a wave's 32 rows. Two rows per lane, and not one with 64
+// this kernel: 240 vector and matrix instructions per token for a wave's 32 rows. Two rows per lane, and not one with 64
 // elements, because every lane reads all its elements of k and q from LDS for each token: 18 reads of a wave instead of 34.
 // 64 x 2560 tokens, 32 heads: 10.1 ms on the vector pipe alone (a row held by two lanes), 8.9 ms this way.
 // Compact state form only (one pool row per sequence, stored after the last token; without a pool the sequences start

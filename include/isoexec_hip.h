@@ -315,7 +315,7 @@ int ix_gdn_cpr_handoff(const float* entry_state, float* running_state, int* due,
  * runtimes/megatron/gdn_fla_shim.py:390-425 `_eager_apply_gated_norm` after the core, ops/norms/fused_outnorm.py:189-271):
  * o [tokens, HV, V] bf16 receives ix_gated_out_norm(o_scan, gate, norm_weight) instead of o_scan; the bits of the two
  * calls. gate bf16 with token pitch gate_stride_t (elements, a multiple of 8), norm_weight bf16 [V]. Served where the
- * four-lane layout of the scan runs: one state row per sequence (state_indices [N]), K = V = 128, bf16, N * HV >= 1536, no
+ * four-lane layout of the scan runs: one state row per sequence (state_indices [N]), K = V = 128, bf16, N * HV >= 2048, no
  * forced time tile of 1 or row code; IX_DECLINED otherwise, before the state is touched (the caller makes the two calls). */
 int ix_gdn_scan_gated_norm(const void* q, const void* k, const void* v, const float* g, const void* beta, void* o,
                            long q_pitch, long k_pitch, long v_pitch, float* state_pool, const int* cu_seqlens,
@@ -327,12 +327,27 @@ int ix_gdn_scan_gated_norm(const void* q, const void* k, const void* v, const fl
  * as ix_gdn_scan's; every sequence starts from a zero state and no state is stored. chunk = 0: the recurrence. chunk > 0
  * (a multiple of 16): the running state restarts at every multiple of chunk tokens from the unrounded fp32 chain rounded to
  * io_dtype, as if the boundary states had been computed first and every chunk scanned from its snapshot. gate, norm_weight
- * (or NULL): as ix_gdn_scan_gated_norm's, where N * HV >= 1536 and chunk = 0. q and k rows start on multiples of 8 elements.
+ * (or NULL): as ix_gdn_scan_gated_norm's, where N * HV >= 2048 and chunk = 0. q and k rows start on multiples of 8 elements.
  * IX_DECLINED otherwise, before anything is launched. */
 int ix_gdn_forward(const void* q, const void* k, const void* v, const float* g, const void* beta, void* o, int io_dtype,
                    long q_pitch, long k_pitch, long v_pitch, const int* cu_seqlens, long N, long H, long HV, long K, long V,
                    float scale, long chunk, const void* gate, long gate_stride_t, const void* norm_weight, float norm_eps,
                    int zero_centered, void* stream);
+
+/* ix_gdn_scan (compact form, time_tile 0, o not NULL; with a gate ix_gdn_scan_gated_norm) and ix_gdn_forward for a host that
+ * knows the lengths: `tokens` in all, `longest` the longest sequence's (0: not known). They choose the layout, which changes no
+ * result. The gate is served where ix_gdn_layout says 16 and IX_DECLINED otherwise, before anything is launched. */
+int ix_gdn_scan_lens(const void* q, const void* k, const void* v, const float* g, const void* beta, void* o, int io_dtype,
+                     long q_pitch, long k_pitch, long v_pitch, float* state_pool, const int* cu_seqlens,
+                     const int* state_indices, long N, long H, long HV, long K, long V, float scale, long tokens, long longest,
+                     const void* gate, long gate_stride_t, const void* norm_weight, float norm_eps, int zero_centered,
+                     void* stream);
+int ix_gdn_forward_lens(const void* q, const void* k, const void* v, const float* g, const void* beta, void* o, int io_dtype,
+                        long q_pitch, long k_pitch, long v_pitch, const int* cu_seqlens, long N, long H, long HV, long K, long V,
+                        float scale, long chunk, long tokens, long longest, const void* gate, long gate_stride_t,
+                        const void* norm_weight, float norm_eps, int zero_centered, void* stream);
+/* The layout that they take (chunk > 0: the boundary form): 0 sixteen lanes per state row, 16 and 19 as in time_tile. */
+int ix_gdn_layout(long N, long HV, long K, long V, int io_dtype, long chunk, long tokens, long longest);
 
 /* gdn_causal_conv / gdn_causal_conv_batched (gdn_ops.py:74-170) over packed tokens, and the
  * engine's window-slide update (gdn_recurrent_state.py:686-707,814-825) when every sequence has

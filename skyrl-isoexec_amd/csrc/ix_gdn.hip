@@ -1096,7 +1096,43 @@ static int ix_gdn_scan_launch(const void* q, const void* k, const void* v, const
 #undef IX_RPL_CASE
 }
 
-// chunk > 0: the boundary form. rpl: state rows per lane group, 3 = four lanes per row, 0 = by the rule.
+// Which layout runs whole sequences at K = 128: 0 the sixteen-lane walk, IX_GDN_FOUR_ONE four lanes per row with one row per lane
+// (k_gdn_walk_quads), IX_GDN_FOUR_TWO with two (k_gdn_scan_quads); the values are time_tile's layout codes. Four lanes issue 8
+// (two rows per lane 7.5) vector instructions per row and token where the walk issues 11, in the boundary form 13 where it
+// issues 18. But a token takes a lone wave 0.42 us (two rows 0.9, boundary form 0.58) where the walk's takes 0.12 to 0.22, so
+// the longest sequence decides: four lanes pay where enough of the others run beside it to its end. `even`: the tokens as so many
+// sequences of the longest one's length, in workgroups of 64 rows. us walk / one row / two rows, 32 heads, V = 128 (64
+// workgroups a sequence), bf16, `even` in brackets:
+//   1 x 8000 + 15 x 100 tokens (76) 1793 / 3345 / 6722     1 x 4096 + 31 x 64 (95) 912 / 1743 / 3404
+//   4 x 2000 + 12 x 200 (333) 803 / 873 / 1772             6 x 2000 + 10 x 200 (448) 1035 / 1038 / 1823
+//   16 of 60..1410 (534) 820 / 690 / 1299                  1 x 3000 + 47 x 500 (565) 1865 / 1634 / 2933
+//   8 x 2000 + 40 x 100 (640) 1526 / 1172 / 1858           16 x 1000 (1024) 1259 / 984 / 1063
+//   48 of 60..1470 (1599) 2491 / 2009 / 2133               24 x 1000 + 24 x 100 (1690) 1806 / 1432 / 1384
+//   48 x 1000 (3072) 3307 / 2731 / 2631                    12 of 60..1380 (768 workgroups) 653 / 680
+// Two rows per lane also take the gated norm along, which is worth more than the 6 % that they lose at 1599. Short sequences,
+// where a launch's start counts: 16 x 24 39.2 / 41.7, 16 x 48 63.2 / 63.4, 32 x 24 72.1 / 71.2, 32 x 32 86.7 / 79.2, 48 x 16
+// 76.2 / 77.8 / 82.5, 63 x 20 123 / 114 / 127, 63 x 24 142 / 127 / 130; from 64 sequences on two rows are no worse there.
+// Boundary form, walk / one row: 1 x 4096 + 31 x 64 (95) 1346 / 2387, 2 x 2000 + 14 x 200 (218) 801 / 1178, 4 x 2000 + 12 x 200
+// (333) 1205 / 1199, ten of 120..1500 (345) 943 / 917, 8 x 1000 + 2 x 100 (525) 992 / 768, 200 x 9 411 / 261, 64 x 1000 7289 /
+// 5235, nine of 120..1500 (576 workgroups) 1008 / 1000; fp32: 4 x 2000 + 28 x 200 (435) 1543 / 1486, 16 of 60..1500 (532) 1426 / 1183,
+// nine of 120..1500 1025 / 1119.
+// Where the host does not know the lengths (longest <= 0) only IX_GDN_QUAD_MANY workgroups of 128 rows leave the walk: 64 x 1000
+// tokens 4375 / 3677 / 3749.
+#define IX_GDN_FOUR_TWO 16
+#define IX_GDN_FOUR_ONE 19
+#define IX_GDN_QUAD_MANY 2048
+#define IX_GDN_QUAD_MIN 1536  // the same with known lengths, and for a state-only pass
+static int ix_gdn_layout_for(long N, long HV, long V, long tokens, long longest, bool bf16, bool boundary) {
+  const long wgs = N * HV * (V / 64), pairs = V % 128 == 0 ? wgs / 2 : 0;
+  if (longest <= 0) return !boundary && pairs >= IX_GDN_QUAD_MANY ? IX_GDN_FOUR_TWO : 0;
+  if (V % 64 != 0) return 0;
+  const long even = tokens * HV * (V / 64) / longest;
+  if (boundary) return wgs >= (bf16 ? 640 : 1024) && even >= (bf16 ? 320 : 448) ? IX_GDN_FOUR_ONE : 0;
+  if (even >= 1536 && (pairs >= IX_GDN_QUAD_MANY || (pairs >= IX_GDN_QUAD_MIN && tokens >= 24 * N))) return IX_GDN_FOUR_TWO;
+  return wgs >= 1024 && even >= 448 && tokens >= 20 * N && tokens * HV * (V / 64) >= 49152 ? IX_GDN_FOUR_ONE : 0;
+}
+
+// chunk > 0: the boundary form. rpl: state rows per lane group of sixteen, 3 = four lanes per row, 0 = one or two by the rule below.
 static int ix_gdn_walk(const void* q, const void* k, const void* v, const float* g, const void* beta, void* o,
                        int io_dtype, float* state, const int* cu, const int* sidx, long q_pitch, long k_pitch, long v_pitch,
                        long N, int H, int HV, long K, int V, float scale, int chunk, int rpl, hipStream_t st) {
@@ -1112,17 +1148,10 @@ static int ix_gdn_walk(const void* q, const void* k, const void* v, const float*
   // while one such workgroup per CU, two at K <= 64, is all there is (at K = 128 a row is then 32 lanes and its tree has a
   // level across the halves of 16). us whole / split: 2000 tokens of 16 heads at K = 128 245 / 206, of 32 heads (two per CU)
   // 66 / 75 per 500; K = 64, 2 x 256 of 4 heads 33 / 24, 8 x 512 of 16 heads 66 / 63, of 32 heads 86 / 107.
-  // Four lanes per row (K = 128) issue 8 vector instructions per row and token where the walk issues 11 (boundary form 13 and
-  // 18), but a token takes a wave three times as long, 0.42 us alone on its SIMD (boundary form 0.58), so they wait for enough
-  // workgroups. us walk / four lanes, 32 heads, V = 128 (64 workgroups per sequence), bf16: 12 sequences of 60..1380 tokens 653 /
-  // 680, 16 of 60..1410 870 / 739, 16 x 1000 1156 / 996, 32 x 1000 2242 / 1913, 32 x 200 467 / 379; boundary form 4 x 1000 595 /
-  // 634, 6 x 1000 858 / 829, 8 x 1000 1122 / 906, nine of 120..1500 1008 / 1000 (fp32 1025 / 1119), 32 of 60..1500 3016 / 2303,
-  // 64 x 1000 7339 / 5466.
   const long quad_wgs = N * HV * (V / 64);
-  const bool quads = K == 128 && V % 64 == 0 && quad_wgs >= (chunk > 0 && io_dtype == IX_DT_BF16 ? 640 : 1024);
   const bool vec_qk = io_dtype == IX_DT_BF16 ? ix_gdn_vec_qk<bf16_t>(q, k, q_pitch, k_pitch)
                                              : ix_gdn_vec_qk<float>(q, k, q_pitch, k_pitch);
-  if (rpl == 3 || (rpl <= 0 && quads)) {
+  if (rpl == 3) {
     if (K != 128 || V % 64 != 0 || quad_wgs > 0x7fffffffL || !vec_qk) return IX_DECLINED;
 #define IX_WALK_QUADS(TIO, CPR_)                                                                                     \
   hipLaunchKernelGGL((k_gdn_walk_quads<TIO, CPR_>), dim3((unsigned)quad_wgs), dim3(256), 0, st, (const TIO*)q, (const TIO*)k, \
@@ -1164,14 +1193,6 @@ static int ix_gdn_walk(const void* q, const void* k, const void* v, const float*
   return IX_DECLINED;
 }
 
-// Workgroups (128 rows each) from which a batch of whole sequences takes the four-lane layout. It issues 30 vector
-// instructions per four rows and token where the walk issues 42, but a token takes one of its waves five times as long:
-// it wins once every SIMD has several waves through to the end. Measured at HV = 32, V = 128 (one such workgroup per
-// sequence and head), us two rows per lane / one (k_gdn_walk_quads) / walk: 64 x 1000 tokens 3749 / 3677 / 4375, 48 x 1000 2640 /
-// 2982 / 3295, 48 sequences of 60..1470 2106 / 2285 / 2484, 40 x 1000 2347 / 2344 / 2792, 32 x 1000 2058 / 1913 / 2242, 24 x 1000
-// 1382 / 1399 / 1699, 24 of 60..1440 1378 / 1057 / 1275.
-#define IX_GDN_QUAD_MIN 1536
-
 static int ix_gdn_quads(const void* q, const void* k, const void* v, const float* g, const void* beta, void* o, int io_dtype,
                         long q_pitch, long k_pitch, long v_pitch, float* state, const int* cu, const int* sidx, long N,
                         int H, int HV, int V, float scale, int TT, const bf16_t* gate, long gate_stride_t,
@@ -1195,7 +1216,8 @@ static int ix_gdn_scan_impl(const void* q, const void* k, const void* v, const f
                             int io_dtype, long q_pitch, long k_pitch, long v_pitch, float* state_pool,
                             const int* cu_seqlens, const int* state_indices, long state_indices_stride, long N,
                             long H, long HV, long K, long V, float scale, int time_tile, const bf16_t* gate,
-                            long gate_stride_t, const bf16_t* norm_w, float norm_eps, int zero_centered, void* stream) {
+                            long gate_stride_t, const bf16_t* norm_w, float norm_eps, int zero_centered, long tokens,
+                            long longest, void* stream) {
   if (!q || !k || !v || !g || !beta || !state_pool || !cu_seqlens || !state_indices) return IX_ERR_ARG;
   if (N < 0 || H <= 0 || HV <= 0 || K <= 0 || V <= 0 || HV % H != 0 || state_indices_stride < 0) return IX_ERR_ARG;
   if (q_pitch < H * K || k_pitch < H * K || v_pitch < HV * V) return IX_ERR_ARG;
@@ -1209,22 +1231,30 @@ static int ix_gdn_scan_impl(const void* q, const void* k, const void* v, const f
   if (TT <= 0) TT = (N * HV * (V / 16) >= 4096) ? 16 : 64;
   if (TT > 64) TT = 64;
   hipStream_t st = (hipStream_t)stream;
-  // The four-lane layout: compact state form, K = 128, whole groups of 128 rows, and IX_GDN_QUAD_MIN workgroups (or forced
-  // by code 16 in bits 8.. of time_tile). A time tile of 1 says one token per sequence (a decode step): that is a pure
-  // stream of the state, which the 16-lane layout does with more waves in flight.
-  if (state_indices_stride == 0 && K == 128 && V % 128 == 0 &&
-      (rpl == 16 || (rpl == 0 && (time_tile & 0xff) != 1 && N * HV * (V / 128) >= IX_GDN_QUAD_MIN)))
+  // Four lanes per row: compact state form, K = 128, where ix_gdn_layout_for says so (or forced by code 16 or 19 in bits 8.. of
+  // time_tile). A time tile of 1 says one token per sequence (a decode step): that is a pure stream of the state, which
+  // the 16-lane layout does with more waves in flight. A state-only pass (the boundary pass of a decode step: equal lengths, most
+  // rows null lanes) has k_gdn_scan to compare with: 63 rows of 64 tokens, us k_gdn_scan / four lanes with no row live 8.5 / 10.2,
+  // one 46 / 52, four 154 / 54, all 321 / 235.
+  const bool compact = state_indices_stride == 0 && K == 128;
+  int layout = 0;
+  if (compact && rpl == 0 && (time_tile & 0xff) != 1) {
+    layout = ix_gdn_layout_for(N, HV, V, tokens, longest, io_dtype == IX_DT_BF16, false);
+    if (!o && V % 128 == 0 && N * HV * (V / 128) >= IX_GDN_QUAD_MIN) layout = IX_GDN_FOUR_TWO;
+  }
+  if (compact && V % 128 == 0 && (rpl == 16 || layout == IX_GDN_FOUR_TWO))
     return ix_gdn_quads(q, k, v, g, beta, o, io_dtype, q_pitch, k_pitch, v_pitch, state_pool, cu_seqlens, state_indices, N,
                         (int)H, (int)HV, (int)V, scale, time_tile > 0 && (time_tile & 0xff) > 0 ? TT : 16, gate,
                         gate_stride_t, norm_w, norm_eps, zero_centered, st);
-  if (gate) return IX_DECLINED;       // the norm rides on the four-lane layout only
-  if (rpl == 16) return IX_DECLINED;  // the four-lane layout was asked for and does not apply
+  if (gate) return IX_DECLINED;       // the norm rides on two rows per lane only
+  if (rpl == 16) return IX_DECLINED;  // that layout was asked for and does not apply
   // Sequences of more than one token in the compact form: the walk (codes 17 and 18 force it with one and two rows per
   // lane group, 19 with four lanes per row). k_gdn_scan below keeps the decode step, the per-token index map, the state-only pass and the operands
   // whose rows are not aligned.
   if (state_indices_stride == 0 && o && (time_tile <= 0 || (rpl >= 17 && rpl <= 19))) {
+    const int form = rpl >= 17 ? rpl - 16 : (layout == IX_GDN_FOUR_ONE ? 3 : 0);
     const int rc = ix_gdn_walk(q, k, v, g, beta, o, io_dtype, state_pool, cu_seqlens, state_indices, q_pitch, k_pitch,
-                               v_pitch, N, (int)H, (int)HV, K, (int)V, scale, 0, rpl >= 17 ? rpl - 16 : 0, st);
+                               v_pitch, N, (int)H, (int)HV, K, (int)V, scale, 0, form, st);
     if (rc != IX_DECLINED) return rc;
   }
   if (rpl >= 17) return IX_DECLINED;
@@ -1251,51 +1281,80 @@ extern "C" int ix_gdn_scan(const void* q, const void* k, const void* v, const fl
                            const int* cu_seqlens, const int* state_indices, long state_indices_stride, long N,
                            long H, long HV, long K, long V, float scale, int time_tile, void* stream) {
   return ix_gdn_scan_impl(q, k, v, g, beta, o, io_dtype, q_pitch, k_pitch, v_pitch, state_pool, cu_seqlens, state_indices,
-                          state_indices_stride, N, H, HV, K, V, scale, time_tile, nullptr, 0, nullptr, 0.0f, 0, stream);
+                          state_indices_stride, N, H, HV, K, V, scale, time_tile, nullptr, 0, nullptr, 0.0f, 0, 0, 0, stream);
 }
 
-// ix_gdn_scan whose output leaves through the layer's gated output norm (ix_gated_out_norm with N = V) in the same
-// launch: o receives bf16(norm(o_scan) * silu(gate)) instead of o_scan -- the bits of the two calls. Served where the
-// four-lane layout runs (one state row per sequence, K = V = 128, bf16, at least IX_GDN_QUAD_MIN (sequence, head) pairs) with
-// 16-byte aligned gate rows and weight; IX_DECLINED otherwise, before anything is launched or the state is touched.
+// The gated output norm (ix_gated_out_norm with N = V) in the scan's launch: o receives bf16(norm(o_scan) * silu(gate)) instead of
+// o_scan -- the bits of the two calls. What its operands have to be, whatever the layout rule says.
+static bool ix_gdn_norm_fits(const void* o, int io_dtype, long K, long V, const void* gate, long gate_stride_t, const void* w) {
+  return io_dtype == IX_DT_BF16 && K == 128 && V == 128 && gate_stride_t % 8 == 0 && ix_aligned(gate, 16) && ix_aligned(w, 16) &&
+         ix_aligned(o, 16);
+}
+
+// Declines (IX_DECLINED) before anything is launched or the state is touched where two rows per lane do not run.
 extern "C" int ix_gdn_scan_gated_norm(const void* q, const void* k, const void* v, const float* g, const void* beta,
                                       void* o, long q_pitch, long k_pitch, long v_pitch, float* state_pool,
                                       const int* cu_seqlens, const int* state_indices, long N, long H, long HV, long K,
                                       long V, float scale, int time_tile, const void* gate, long gate_stride_t,
                                       const void* norm_weight, float norm_eps, int zero_centered, void* stream) {
   if (!o || !gate || !norm_weight || gate_stride_t < HV * V) return IX_ERR_ARG;
-  if (K != 128 || V != 128 || (gate_stride_t % 8) || !ix_aligned(gate, 16) || !ix_aligned(norm_weight, 16) ||
-      !ix_aligned(o, 16) || (time_tile & 0xff) == 1 || (time_tile >> 8) != 0 || N * HV < IX_GDN_QUAD_MIN)
+  if (!ix_gdn_norm_fits(o, IX_DT_BF16, K, V, gate, gate_stride_t, norm_weight) || (time_tile & 0xff) == 1 ||
+      (time_tile >> 8) != 0 || N * HV < IX_GDN_QUAD_MANY)
     return IX_DECLINED;
   return ix_gdn_scan_impl(q, k, v, g, beta, o, IX_DT_BF16, q_pitch, k_pitch, v_pitch, state_pool, cu_seqlens,
                           state_indices, 0, N, H, HV, K, V, scale, time_tile, (const bf16_t*)gate, gate_stride_t,
-                          (const bf16_t*)norm_weight, norm_eps, zero_centered, stream);
+                          (const bf16_t*)norm_weight, norm_eps, zero_centered, 0, 0, stream);
+}
+
+extern "C" int ix_gdn_scan_lens(const void* q, const void* k, const void* v, const float* g, const void* beta, void* o,
+                                int io_dtype, long q_pitch, long k_pitch, long v_pitch, float* state_pool,
+                                const int* cu_seqlens, const int* state_indices, long N, long H, long HV, long K, long V,
+                                float scale, long tokens, long longest, const void* gate, long gate_stride_t,
+                                const void* norm_weight, float norm_eps, int zero_centered, void* stream) {
+  if (!o || tokens < 0 || longest < 0 || (gate && (!norm_weight || gate_stride_t < HV * V))) return IX_ERR_ARG;
+  if (gate && !ix_gdn_norm_fits(o, io_dtype, K, V, gate, gate_stride_t, norm_weight)) return IX_DECLINED;
+  return ix_gdn_scan_impl(q, k, v, g, beta, o, io_dtype, q_pitch, k_pitch, v_pitch, state_pool, cu_seqlens, state_indices, 0,
+                          N, H, HV, K, V, scale, 0, (const bf16_t*)gate, gate_stride_t, (const bf16_t*)norm_weight, norm_eps,
+                          zero_centered, tokens, longest, stream);
+}
+
+extern "C" int ix_gdn_layout(long N, long HV, long K, long V, int io_dtype, long chunk, long tokens, long longest) {
+  if (N <= 0 || HV <= 0 || V <= 0 || K != 128) return 0;
+  return ix_gdn_layout_for(N, HV, V, tokens, longest, io_dtype == IX_DT_BF16, chunk > 0);
 }
 
 // The stateless forward: every sequence starts from a zero state, which is not kept. chunk 0: the recurrence; chunk > 0:
 // the boundary form, whose running state restarts every `chunk` tokens from the fp32 chain rounded to io_dtype.
-extern "C" int ix_gdn_forward(const void* q, const void* k, const void* v, const float* g, const void* beta, void* o,
-                              int io_dtype, long q_pitch, long k_pitch, long v_pitch, const int* cu_seqlens, long N, long H,
-                              long HV, long K, long V, float scale, long chunk, const void* gate, long gate_stride_t,
-                              const void* norm_weight, float norm_eps, int zero_centered, void* stream) {
-  if (!q || !k || !v || !g || !beta || !o || !cu_seqlens) return IX_ERR_ARG;
+extern "C" int ix_gdn_forward_lens(const void* q, const void* k, const void* v, const float* g, const void* beta, void* o,
+                                   int io_dtype, long q_pitch, long k_pitch, long v_pitch, const int* cu_seqlens, long N,
+                                   long H, long HV, long K, long V, float scale, long chunk, long tokens, long longest,
+                                   const void* gate, long gate_stride_t, const void* norm_weight, float norm_eps,
+                                   int zero_centered, void* stream) {
+  if (!q || !k || !v || !g || !beta || !o || !cu_seqlens || tokens < 0 || longest < 0) return IX_ERR_ARG;
   if (N < 0 || H <= 0 || HV <= 0 || K <= 0 || V <= 0 || HV % H != 0 || chunk < 0) return IX_ERR_ARG;
   if (q_pitch < H * K || k_pitch < H * K || v_pitch < HV * V) return IX_ERR_ARG;
   if (gate && (!norm_weight || gate_stride_t < HV * V)) return IX_ERR_ARG;
   if (io_dtype != IX_DT_F32 && io_dtype != IX_DT_BF16) return IX_DECLINED;
   if (chunk % 16 || chunk > 0x7fffffffL) return IX_DECLINED;  // the restart falls on a tile's first token
   hipStream_t st = (hipStream_t)stream;
-  const bool pairs = chunk == 0 && K == 128 && V % 128 == 0 && N * HV * (V / 128) >= IX_GDN_QUAD_MIN;
-  if (gate && (!pairs || V != 128 || io_dtype != IX_DT_BF16 || (gate_stride_t % 8) || !ix_aligned(gate, 16) ||
-               !ix_aligned(norm_weight, 16) || !ix_aligned(o, 16)))
-    return IX_DECLINED;  // the norm rides on the four-lane layout only
+  const int layout = ix_gdn_layout(N, HV, K, V, io_dtype, chunk, tokens, longest);
+  if (gate && (layout != IX_GDN_FOUR_TWO || !ix_gdn_norm_fits(o, io_dtype, K, V, gate, gate_stride_t, norm_weight)))
+    return IX_DECLINED;  // the norm rides on two rows per lane only
   if (N == 0) return IX_OK;
-  if (pairs)
+  if (layout == IX_GDN_FOUR_TWO)
     return ix_gdn_quads(q, k, v, g, beta, o, io_dtype, q_pitch, k_pitch, v_pitch, nullptr, cu_seqlens, nullptr, N, (int)H,
                         (int)HV, (int)V, scale, 16, (const bf16_t*)gate, gate_stride_t, (const bf16_t*)norm_weight,
                         norm_eps, zero_centered, st);
   return ix_gdn_walk(q, k, v, g, beta, o, io_dtype, nullptr, cu_seqlens, nullptr, q_pitch, k_pitch, v_pitch, N, (int)H,
-                     (int)HV, K, (int)V, scale, (int)chunk, 0, st);
+                     (int)HV, K, (int)V, scale, (int)chunk, layout == IX_GDN_FOUR_ONE ? 3 : 0, st);
+}
+
+extern "C" int ix_gdn_forward(const void* q, const void* k, const void* v, const float* g, const void* beta, void* o,
+                              int io_dtype, long q_pitch, long k_pitch, long v_pitch, const int* cu_seqlens, long N, long H,
+                              long HV, long K, long V, float scale, long chunk, const void* gate, long gate_stride_t,
+                              const void* norm_weight, float norm_eps, int zero_centered, void* stream) {
+  return ix_gdn_forward_lens(q, k, v, g, beta, o, io_dtype, q_pitch, k_pitch, v_pitch, cu_seqlens, N, H, HV, K, V, scale, chunk,
+                             0, 0, gate, gate_stride_t, norm_weight, norm_eps, zero_centered, stream);
 }
 
 // ---------------------------------------------------------------------------------------------

@@ -100,6 +100,17 @@ SIGNATURES = {
         [P, P, P, P, P, P, c_int, c_long, c_long, c_long, P, c_long, c_long, c_long, c_long, c_long, c_float, c_long, P,
          c_long, P, c_float, c_int, P],
     ),
+    "ix_gdn_scan_lens": (
+        c_int,
+        [P, P, P, P, P, P, c_int, c_long, c_long, c_long, P, P, P, c_long, c_long, c_long, c_long, c_long, c_float, c_long,
+         c_long, P, c_long, P, c_float, c_int, P],
+    ),
+    "ix_gdn_forward_lens": (
+        c_int,
+        [P, P, P, P, P, P, c_int, c_long, c_long, c_long, P, c_long, c_long, c_long, c_long, c_long, c_float, c_long, c_long,
+         c_long, P, c_long, P, c_float, c_int, P],
+    ),
+    "ix_gdn_layout": (c_int, [c_long, c_long, c_long, c_long, c_int, c_long, c_long, c_long]),
     "ix_gdn_conv": (c_int, [P, c_long, P, P, P, P, P, P, P, c_long, c_long, c_long, c_long, c_int, P]),
     "ix_gdn_conv_l2norm": (c_int, [P, c_long, P, P, P, P, P, P, P, c_long, c_long, c_long, c_long, c_int, c_long, c_long,
                                    c_float, P]),

@@ -66,6 +66,7 @@ def gdn_recurrent_kernel(
     time_tile: int = 0,
     want_output: bool = True,
     gated_norm: tuple | None = None,
+    longest: int | None = None,
 ) -> torch.Tensor:
     """The delta-rule scan. Advances ``ssm_state`` IN PLACE. Returns ``o`` shaped like ``v`` (``None`` for a
     state-only pass, ``want_output=False``: nothing but the state pool is written).
@@ -78,7 +79,8 @@ def gdn_recurrent_kernel(
     ``v``: ``[B, T, HV, V]``; ``g`` (fp32), ``beta``: ``[B, T, HV]``; ``ssm_state`` fp32 pool
     ``[S, HV, V, K]``; ``state_indices`` ``[N]`` (one row per sequence, stored after its last token) or ``[N, Tmax]``
     (column 0 loads, a positive entry at column t stores after token t); ``cu_seqlens``
-    ``[N+1]`` int32 for a packed batch (then ``B == 1``), ``None`` for ``[B, T, ...]``.
+    ``[N+1]`` int32 for a packed batch (then ``B == 1``), ``None`` for ``[B, T, ...]``. ``longest``: the longest sequence of a
+    packed batch where the host knows it; the kernel's layout follows from it, no result does.
     """
     _lib.require_device(q, k, v, g, beta, ssm_state, state_indices, cu_seqlens)
     if q.ndim != 4 or v.ndim != 4:
@@ -118,6 +120,18 @@ def gdn_recurrent_kernel(
     o = torch.empty(qf.shape[0], HV, V, dtype=io, device=dev) if want_output else None
     if time_tile == 0 and cu_seqlens is None and T == 1:
         time_tile = 1
+    longest = int(longest or 0) if cu_seqlens is not None else T
+    by_length = longest > 0 and time_tile == 0 and idx_stride == 0 and want_output
+
+    def scan_by_length(gate, weight, eps, zero_centered):
+        return _lib.check(
+            _lib.lib().ix_gdn_scan_lens(
+                qf.data_ptr(), kf.data_ptr(), vf.data_ptr(), gf.data_ptr(), bf.data_ptr(), o.data_ptr(), _lib.dtype_code(io),
+                _token_pitch(qf), _token_pitch(kf), _token_pitch(vf), ssm_state.data_ptr(), cu.data_ptr(), idx.data_ptr(),
+                n_seq, H, HV, K, V, float(K) ** -0.5, qf.shape[0], longest, _lib.ptr(gate),
+                0 if gate is None else gate.stride(0), _lib.ptr(weight), float(eps), int(zero_centered),
+                _lib.current_stream(dev)), "ix_gdn_scan_lens")
+
     if gated_norm is not None:
         gate, weight, eps, zero_centered = gated_norm
         _lib.require_device(gate, weight)
@@ -126,7 +140,9 @@ def gdn_recurrent_kernel(
         fusable = (io is torch.bfloat16 and idx_stride == 0 and gate.dtype is io and weight.dtype is io
                    and gate.stride(2) == 1 and gate.stride(1) == V and weight.is_contiguous() and weight.numel() == V)
         rc = _lib.IX_DECLINED
-        if fusable:
+        if fusable and by_length:
+            rc = scan_by_length(gate, weight, eps, zero_centered)
+        elif fusable:
             rc = _lib.check(
                 _lib.lib().ix_gdn_scan_gated_norm(
                     qf.data_ptr(), kf.data_ptr(), vf.data_ptr(), gf.data_ptr(), bf.data_ptr(), o.data_ptr(),
@@ -135,12 +151,15 @@ def gdn_recurrent_kernel(
                     weight.data_ptr(), float(eps), int(zero_centered), _lib.current_stream(dev)), "ix_gdn_scan_gated_norm")
         if rc == _lib.IX_OK:
             return o.view(B, T, HV, V) if cu_seqlens is None else o.unsqueeze(0)
-    rc = _lib.check(
-        _lib.lib().ix_gdn_scan(
-            qf.data_ptr(), kf.data_ptr(), vf.data_ptr(), gf.data_ptr(), bf.data_ptr(), _lib.ptr(o),
-            _lib.dtype_code(io), _token_pitch(qf), _token_pitch(kf), _token_pitch(vf), ssm_state.data_ptr(),
-            cu.data_ptr(), idx.data_ptr(), idx_stride, n_seq, H, HV, K, V, float(K) ** -0.5, time_tile,
-            _lib.current_stream(dev)), "ix_gdn_scan")
+    if by_length:
+        rc = scan_by_length(None, None, 0.0, 0)
+    else:
+        rc = _lib.check(
+            _lib.lib().ix_gdn_scan(
+                qf.data_ptr(), kf.data_ptr(), vf.data_ptr(), gf.data_ptr(), bf.data_ptr(), _lib.ptr(o),
+                _lib.dtype_code(io), _token_pitch(qf), _token_pitch(kf), _token_pitch(vf), ssm_state.data_ptr(),
+                cu.data_ptr(), idx.data_ptr(), idx_stride, n_seq, H, HV, K, V, float(K) ** -0.5, time_tile,
+                _lib.current_stream(dev)), "ix_gdn_scan")
     if rc != _lib.IX_OK:
         raise RuntimeError(f"[isoexec-amd] ix_gdn_scan declined K={K} V={V} dtype={io}")
     if o is None:
@@ -153,11 +172,12 @@ def gdn_recurrent_kernel(
     return o.view(B, T, HV, V) if cu_seqlens is None else o.unsqueeze(0)
 
 
-def stateless_forward(q, k, v, g, beta, *, cu_seqlens=None, chunk_size: int = 0, gated_norm: tuple | None = None):
+def stateless_forward(q, k, v, g, beta, *, cu_seqlens=None, chunk_size: int = 0, gated_norm: tuple | None = None,
+                      longest: int | None = None):
     """The delta-rule forward from a zero state that is not kept (``ix_gdn_forward``): ``q, k`` L2-normalised, layouts as
     ``gdn_recurrent_kernel``'s. ``chunk_size`` > 0 is the boundary form (``gdn_cpr_fwd``), in the same single pass over the
-    tokens. With ``gated_norm`` the output comes back through the layer's gated output norm. Returns ``o`` shaped like
-    ``v``, or ``None`` when the library does not serve the operands (nothing launched: the caller scans with a pool)."""
+    tokens. With ``gated_norm`` the output comes back through the layer's gated output norm. ``longest`` as
+    ``gdn_recurrent_kernel``'s. Returns ``o`` shaped like ``v``, or ``None`` when the library does not serve the operands (nothing launched: the caller scans with a pool)."""
     _lib.require_device(q, k, v, g, beta, cu_seqlens)
     if q.ndim != 4 or v.ndim != 4:
         raise RuntimeError(f"[isoexec-amd] the delta-rule forward expects [B,T,H,K]/[B,T,HV,V], got {tuple(q.shape)}")
@@ -177,14 +197,16 @@ def stateless_forward(q, k, v, g, beta, *, cu_seqlens=None, chunk_size: int = 0,
     gf = _flatten_tokens(g, 1).to(torch.float32).contiguous()
     bf = _flatten_tokens(beta, 1).to(io).contiguous()
     o = torch.empty(qf.shape[0], HV, V, dtype=io, device=dev)
+    longest = int(longest or 0) if cu_seqlens is not None else T
 
     def launch(gate, weight, eps, zero_centered):
         return _lib.check(
-            _lib.lib().ix_gdn_forward(
+            _lib.lib().ix_gdn_forward_lens(
                 qf.data_ptr(), kf.data_ptr(), vf.data_ptr(), gf.data_ptr(), bf.data_ptr(), o.data_ptr(),
                 _lib.dtype_code(io), _token_pitch(qf), _token_pitch(kf), _token_pitch(vf), cu.data_ptr(), n_seq, H, HV, K,
-                V, float(K) ** -0.5, int(chunk_size), _lib.ptr(gate), 0 if gate is None else gate.stride(0),
-                _lib.ptr(weight), float(eps), int(zero_centered), _lib.current_stream(dev)), "ix_gdn_forward")
+                V, float(K) ** -0.5, int(chunk_size), qf.shape[0], longest, _lib.ptr(gate),
+                0 if gate is None else gate.stride(0), _lib.ptr(weight), float(eps), int(zero_centered),
+                _lib.current_stream(dev)), "ix_gdn_forward_lens")
 
     if gated_norm is None:
         return o.view(B, T, HV, V) if launch(None, None, 0.0, 0) == _lib.IX_OK else None
@@ -386,25 +408,26 @@ def _recurrent_scratch_state(q, v, cu_seqlens):
     return ssm_state, idx
 
 
-def _stateless(q, k, v, g, beta, cu_seqlens, gated_norm=None):
+def _stateless(q, k, v, g, beta, cu_seqlens, gated_norm=None, longest=None):
     # not while a trace is attached: the scan behind it is a door of the trace, the single launch is none
     if get_tracer() is None:
-        o = stateless_forward(q, k, v, g, beta, cu_seqlens=cu_seqlens, gated_norm=gated_norm)
+        o = stateless_forward(q, k, v, g, beta, cu_seqlens=cu_seqlens, gated_norm=gated_norm, longest=longest)
         if o is not None:
             return o
     ssm_state, idx = _recurrent_scratch_state(q, v, cu_seqlens)
     return gdn_recurrent_kernel(q, k, v, g, beta, ssm_state=ssm_state, state_indices=idx, cu_seqlens=cu_seqlens,
-                                gated_norm=gated_norm)
+                                gated_norm=gated_norm, longest=longest)
 
 
-def gdn_recurrent(q, k, v, g, beta, *, initial_state=None, output_final_state=False, cu_seqlens=None):
-    """Stateless (training / prefill-from-zero) entry: ``(o, None)`` (gdn_ops.py:997-1027)."""
+def gdn_recurrent(q, k, v, g, beta, *, initial_state=None, output_final_state=False, cu_seqlens=None, longest=None):
+    """Stateless (training / prefill-from-zero) entry: ``(o, None)`` (gdn_ops.py:997-1027). ``longest`` as
+    ``gdn_recurrent_kernel``'s."""
     if initial_state is not None or output_final_state:
         raise NotImplementedError(
             "isoexec GDN: gdn_recurrent is the stateless (training/prefill-from-zero) entry point. "
             "The engine carries state through gdn_recurrent_kernel + a real state pool.")
     with torch.no_grad():
-        return _stateless(q, k, v, g, beta, cu_seqlens), None
+        return _stateless(q, k, v, g, beta, cu_seqlens, longest=longest), None
 
 
 def gdn_kernel_mode() -> str:
@@ -427,9 +450,9 @@ def fla_chunk_size() -> int:
     return 64
 
 
-def gdn_cpr(q, k, v, g, beta, *, initial_state=None, output_final_state=False, cu_seqlens=None):
+def gdn_cpr(q, k, v, g, beta, *, initial_state=None, output_final_state=False, cu_seqlens=None, longest=None):
     """Stateless boundary-form forward: ``(o, None)`` (gdn_ops.py:1063-1116). A padded ``[B, T, ...]`` batch is
-    flattened to B packed sequences."""
+    flattened to B packed sequences. ``longest`` as ``gdn_recurrent_kernel``'s."""
     if initial_state is not None or output_final_state:
         raise NotImplementedError(
             "isoexec GDN: gdn_cpr is the stateless (training/prefill-from-zero) entry point.")
@@ -440,20 +463,21 @@ def gdn_cpr(q, k, v, g, beta, *, initial_state=None, output_final_state=False, c
         if cu_seqlens is None:
             flat = lambda t: t.reshape(1, B * T, *t.shape[2:])
             cu = torch.arange(0, (B + 1) * T, T, dtype=torch.int32, device=q.device)
-            o = gdn_cpr_fwd(flat(q), flat(k), flat(v), flat(g), flat(beta), cu_seqlens=cu, chunk_size=fla_chunk_size())
+            o = gdn_cpr_fwd(flat(q), flat(k), flat(v), flat(g), flat(beta), cu_seqlens=cu, chunk_size=fla_chunk_size(),
+                            longest=T)
             return o.reshape(B, T, *o.shape[2:]), None
-        return gdn_cpr_fwd(q, k, v, g, beta, cu_seqlens=cu_seqlens, chunk_size=fla_chunk_size()), None
+        return gdn_cpr_fwd(q, k, v, g, beta, cu_seqlens=cu_seqlens, chunk_size=fla_chunk_size(), longest=longest), None
 
 
-def gdn_core(q, k, v, g, beta, *, initial_state=None, output_final_state=False, cu_seqlens=None):
+def gdn_core(q, k, v, g, beta, *, initial_state=None, output_final_state=False, cu_seqlens=None, longest=None):
     """The trainer's door (gdn_ops.py:1118-1194): :func:`gdn_recurrent` or :func:`gdn_cpr` per
     :func:`gdn_kernel_mode` (``SKYRL_ISOEXEC_GDN_TRAINER_KERNEL`` overrides it for this door only). The
     chunk-parallel kernel of the vocabulary is not served here: its bits depend on the chunk length, which the
-    recurrent and boundary forms do not have to pay for."""
+    recurrent and boundary forms do not have to pay for. ``longest`` as ``gdn_recurrent_kernel``'s."""
     from ...core.gdn_kernel_env import gdn_trainer_kernel_override
 
     mode = gdn_trainer_kernel_override() or gdn_kernel_mode()
-    kw = dict(initial_state=initial_state, output_final_state=output_final_state, cu_seqlens=cu_seqlens)
+    kw = dict(initial_state=initial_state, output_final_state=output_final_state, cu_seqlens=cu_seqlens, longest=longest)
     if mode == "cpr":
         return gdn_cpr(q, k, v, g, beta, **kw)
     if mode == "recurrent":
@@ -475,15 +499,17 @@ def gdn_native_core_kernel(q, k, v, a, b, A_log, dt_bias, *, ssm_state, state_in
                                 state_indices=state_indices, cu_seqlens=cu_seqlens)
 
 
-def gdn_native_core_normed(qn, kn, v, a, b, A_log, dt_bias, *, cu_seqlens=None, gated_norm: tuple | None = None):
+def gdn_native_core_normed(qn, kn, v, a, b, A_log, dt_bias, *, cu_seqlens=None, gated_norm: tuple | None = None,
+                           longest: int | None = None):
     """``gdn_native_core`` for q and k that are normalised already (``conv_packed(..., l2norm_qk=...)``): the gating and
     the scan of the same composition, without its two l2norm launches. Same bits as ``gdn_native_core`` on the raw heads.
-    ``gated_norm`` as in ``gdn_recurrent_kernel``: the output then comes back through the layer's gated output norm."""
+    ``gated_norm`` and ``longest`` as in ``gdn_recurrent_kernel``: the output then comes back through the layer's gated output
+    norm."""
     with torch.no_grad():
         HV = v.shape[-2]
         g, beta = gate_and_beta_fp32(a.reshape(-1, HV), b.reshape(-1, HV), A_log, dt_bias)
         lead = v.shape[:2]
-        return _stateless(qn, kn, v, g.view(*lead, HV), beta.view(*lead, HV), cu_seqlens, gated_norm)
+        return _stateless(qn, kn, v, g.view(*lead, HV), beta.view(*lead, HV), cu_seqlens, gated_norm, longest)
 
 
 def gdn_native_core(q, k, v, a, b, A_log, dt_bias, *, cu_seqlens=None):

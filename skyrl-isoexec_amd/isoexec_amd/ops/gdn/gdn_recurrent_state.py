@@ -488,7 +488,8 @@ class RecurrentGDN:
         rows, is_cont, rows_out, cu, q, k, v, g, beta = self._prefill_prepare(
             slots_cpu, x, a, b, qsl, has_initial_state, prefill_query_start_loc, fuse_l2norm=fuse_l2norm)
         o = gdn_recurrent_kernel(q.unsqueeze(0), k.unsqueeze(0), v.unsqueeze(0), g.unsqueeze(0), beta.unsqueeze(0),
-                                 ssm_state=self.ssm_state, state_indices=rows_out, cu_seqlens=cu, gated_norm=gated_norm)
+                                 ssm_state=self.ssm_state, state_indices=rows_out, cu_seqlens=cu, gated_norm=gated_norm,
+                                 longest=max((int(e) - int(s) for s, e in zip(qsl, qsl[1:])), default=0))
         return o[0]
 
     def _prefill_prepare(self, slots_cpu, x, a, b, qsl, has_initial_state, prefill_query_start_loc, fuse_l2norm=True):

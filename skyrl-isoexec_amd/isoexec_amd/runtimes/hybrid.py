@@ -19,6 +19,7 @@ from __future__ import annotations
 
 from array import array
 from dataclasses import dataclass, field
+from functools import partial
 
 import numpy as np
 import torch
@@ -378,12 +379,12 @@ class TrainerModel:
             k = y[:, kd : 2 * kd].unflatten(1, (c.gdn_k_heads, c.gdn_head_dim))
             v = y[:, 2 * kd :].unflatten(1, (c.gdn_v_heads, c.gdn_head_dim))
             if c.gdn_kernel == "cpr":
-                core = gdn_native_cpr_normed if fused else gdn_native_cpr_fwd
+                core = partial(gdn_native_cpr_normed, longest=max_len) if fused else gdn_native_cpr_fwd
                 o = core(q.unsqueeze(0), k.unsqueeze(0), v.unsqueeze(0), a, bb, lw["A_log"], lw["dt_bias"], cu_seqlens=cu,
                          chunk_size=c.gdn_chunk)
             elif fused:
                 o = gdn_native_core_normed(q.unsqueeze(0), k.unsqueeze(0), v.unsqueeze(0), a, bb, lw["A_log"],
-                                           lw["dt_bias"], cu_seqlens=cu, gated_norm=b.gdn_gated_norm(i, z))
+                                           lw["dt_bias"], cu_seqlens=cu, gated_norm=b.gdn_gated_norm(i, z), longest=max_len)
                 return b.gdn_out(i, o[0], z, normed=True)
             else:
                 o = gdn_native_core(q.unsqueeze(0), k.unsqueeze(0), v.unsqueeze(0), a, bb, lw["A_log"], lw["dt_bias"], cu_seqlens=cu)

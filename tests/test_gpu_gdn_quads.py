@@ -58,21 +58,61 @@ def test_walk_with_four_lanes_per_row_equals_the_token_staged_scan(V, dtype):
     assert same_bits(run(19 << 8, pb), run(16 | (1 << 8), pa)) and same_bits(pb, pa)
 
 
-# Enough workgroups for four lanes per row, by the rule: 132 sequences (the last turn through the CUs is not a whole one) of the
-# lengths above, plain and in the boundary form, against the same sequences nine at a time (the sixteen-lane walk).
-@pytest.mark.parametrize("HV,dtype", [(8, torch.bfloat16), (16, torch.float32)])
+# By the rule: 132 sequences (the last turn through the CUs is not a whole one) and 300 (more than are ranked by length), plain and
+# in the boundary form, against the same sequences nine at a time (the sixteen-lane walk). q, k and v are column blocks of one
+# buffer with columns of its own, as a layer's convolution leaves them.
+@pytest.mark.parametrize("n,HV,dtype", [(132, 16, torch.bfloat16), (132, 16, torch.float32), (300, 8, torch.bfloat16)])
 @pytest.mark.parametrize("chunk", [0, 16, 32])
-def test_walk_with_four_lanes_per_row_by_the_rule(HV, dtype, chunk):
+def test_walk_with_four_lanes_per_row_by_the_rule(n, HV, dtype, chunk):
+    from isoexec_amd import _lib
     from isoexec_amd.ops.gdn.gdn_ops import stateless_forward
 
-    lens = [LENS[i % 9] + (i // 9) % 2 for i in range(132)]  # one row block per head: 132 * HV workgroups
-    args, cu = operands(lens, HV // 2, HV, 64, dtype, HV + chunk)
-    got = stateless_forward(*args, cu_seqlens=cu, chunk_size=chunk)
+    H, V = HV // 2, 64
+    lens = [LENS[i % 9] and LENS[i % 9] + 20 + (i // 9) % 2 for i in range(n)]
+    T = sum(lens)
+    assert _lib.lib().ix_gdn_layout(n, HV, 128, V, _lib.dtype_code(dtype), chunk, T, max(lens)) == 19
+    (q, k, v, gate, beta), cu = operands(lens, H, HV, V, dtype, HV + chunk)
+    wide = torch.zeros(1, T, 2 * H * 128 + HV * V + 8, dtype=dtype, device=DEV)
+    parts = wide[..., :H * 128], wide[..., H * 128:2 * H * 128], wide[..., 2 * H * 128:2 * H * 128 + HV * V]
+    args = [p.unflatten(2, t.shape[2:]) for p, t in zip(parts, (q, k, v))]
+    for p, t in zip(args, (q, k, v)):
+        p.copy_(t)
+    got = stateless_forward(*args, gate, beta, cu_seqlens=cu, chunk_size=chunk, longest=max(lens))
     at = 0
-    for i in range(0, len(lens), 9):
+    for i in range(0, n, 9):
         part = lens[i:i + 9]
         t = slice(at, at + sum(part))
         at += sum(part)
         _, few = operands(part, 1, 1, 1, dtype, 0)
-        alone = stateless_forward(*(a[:, t].contiguous() for a in args), cu_seqlens=few, chunk_size=chunk)
+        alone = stateless_forward(*(a[:, t].contiguous() for a in (q, k, v, gate, beta)), cu_seqlens=few, chunk_size=chunk)
         assert same_bits(got[:, t], alone), i
+
+
+# One long sequence and many short ones, an even spread and equal lengths: the three layouts, with a state pool and without, with the
+# gated norm and without. The form whose lengths the host does not know takes another layout for the same sequences.
+@pytest.mark.parametrize("lens,layout", [([300] + [3] * 15, 0), ([80 - 2 * i for i in range(16)], 19), ([24] * 48, 16),
+                                         ([300] + [3] * 63, 0), ([5] * 64, 16)])
+def test_lengths_known_on_the_host_change_no_bits(lens, layout):
+    from isoexec_amd import _lib
+    from isoexec_amd.ops.gdn.gdn_ops import gdn_recurrent_kernel, stateless_forward
+    from isoexec_amd.ops.norms.fused_outnorm import fused_gated_out_norm
+
+    H, HV, V, N, T = 16, 32, 128, len(lens), sum(lens)
+    assert _lib.lib().ix_gdn_layout(N, HV, 128, V, 1, 0, T, max(lens)) == layout
+    args, cu = operands(lens, H, HV, V, torch.bfloat16, N)
+    rows = torch.arange(1, N + 1, dtype=torch.int32, device=DEV)
+    z = torch.randn(T, HV, V, generator=cpu_gen(1)).to(torch.bfloat16).to(DEV)
+    w = (0.1 * torch.randn(V, generator=cpu_gen(2))).to(torch.bfloat16).to(DEV)
+    norm = (z, w, 1e-6, True)
+    start = torch.randn(N + 1, HV, V, 128, generator=cpu_gen(3)).to(DEV)
+    run = lambda pool, **kw: gdn_recurrent_kernel(*args, ssm_state=pool, state_indices=rows, cu_seqlens=cu, **kw)
+    pools = [start.clone() for _ in range(3)]
+    want = run(pools[0], time_tile=16 | (1 << 8))
+    normed = fused_gated_out_norm(want[0], z, w, 1e-6).view(1, T, HV, V)
+    assert same_bits(run(pools[1], longest=max(lens)), want) and same_bits(pools[1], pools[0])
+    assert same_bits(run(pools[2], longest=max(lens), gated_norm=norm), normed) and same_bits(pools[2], pools[0])
+    zero = torch.zeros_like(start)
+    want = run(zero, time_tile=16 | (1 << 8))
+    normed = fused_gated_out_norm(want[0], z, w, 1e-6).view(1, T, HV, V)
+    assert same_bits(stateless_forward(*args, cu_seqlens=cu, longest=max(lens)), want)
+    assert same_bits(stateless_forward(*args, cu_seqlens=cu, longest=max(lens), gated_norm=norm), normed)

@@ -81,12 +81,15 @@ int ix_arch_selfcheck_probe(void* workspace, size_t workspace_bytes, unsigned in
 
 /* Workspace the split launch shape needs (bytes); 0 on invalid arguments. */
 size_t ix_logprob_workspace_bytes(long rows, long V, int G);
+/* Whether aligned rows of this size, read by ix_logprob_rowinv_sampled, stay on the CU (force_shape 3). */
+int ix_logprob_keeps_rows(int dtype, long rows, long V, int G);
 
 /* rowinv_sampled_logprobs (rowinv.py:666-712; kernels leaf_sum_exp :136-154, finalize_rows
  * :156-191) at world size 1. logits [rows, V] (row pitch row_stride elements), target int64
  * [rows] (out of range -> logprob 0), G leaves (power of two, V % G == 0 else declined).
  * out_logprob fp32 [rows]; out_lse fp32 [rows] or NULL. force_shape: 0 auto, 1 one workgroup
- * per row, 2 split rows (needs the workspace). row_max_in: NULL, or fp32 [rows] holding each
+ * per row, 2 split rows (needs the workspace), 3 rows kept on the CU (groups of 8 columns aligned, at most 512 blocks of 4096
+ * columns, no row_max_in; declined otherwise), which 0 takes where ix_logprob_keeps_rows says so. row_max_in: NULL, or fp32 [rows] holding each
  * row's exact maximum (e.g. ix_gemm_bf16_nt's row_max_parts reduced by ix_rowmax_reduce): the
  * max pass is skipped and the logits are read once. The workspace is always required with it. */
 int ix_logprob_rowinv_sampled(const void* logits, int dtype, long rows, long V, long row_stride,

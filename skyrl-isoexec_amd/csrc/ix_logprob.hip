@@ -213,15 +213,13 @@ __global__ __launch_bounds__(512) void k_lp_row(const T* __restrict__ x, long ro
 // blocks in registers and LU in LDS, reads the others twice, and asks for the next row's block as soon as this row's is summed.
 // The blocks, their sums and the fold are k_lp_row's. Bound by HBM: of [1000, 151936] in bf16 all 40 blocks stay (5 a wave, 160
 // registers), 93 -> 70 us; in fp32 24 (two a wave in registers, one in LDS), 181 -> 129; 2900 rows 259 -> 179 and 506 -> 354.
-// Three fp32 blocks in registers leave none to work with (spilled loads have to be waited for: 155). The line: 1000 rows of
-// 65536, 16 blocks, fp32 77 -> 47, bf16 42 -> 35; of 32000, one block a wave, fp32 36 -> 42, bf16 20 -> 22.
+// Three fp32 blocks in registers leave none to work with (spilled loads have to be waited for: 155).
 // The registers as they are: no widened copy of them lives on from an earlier use.
 __device__ __forceinline__ void ix_lp_keep(IxRaw8<bf16_t>& r) {
   asm volatile("" : "+v"(r.v.x), "+v"(r.v.y), "+v"(r.v.z), "+v"(r.v.w));
 }
 __device__ __forceinline__ void ix_lp_keep(IxRaw8<float>&) {}
 #define IX_LP_HELD_UNITS 512
-#define IX_LP_HELD_V 65536  // columns from which a row is kept
 template <typename T, int HU, int LU>
 __global__ __launch_bounds__(512) void k_lp_row_held(const T* __restrict__ x, long row_stride, long rows, int V, int G,
                                                      const int64_t* __restrict__ target, float* __restrict__ out_lp,
@@ -636,6 +634,26 @@ extern "C" size_t ix_logprob_workspace_bytes(long rows, long V, int G) {
   return (size_t)rows * (size_t)(P + G * NB + 2) * sizeof(float);
 }
 
+// Whether whole rows go to k_lp_row_held: us twice read (k_lp_row) / kept.
+//   * 65536 columns: 1000 rows fp32 78 / 50, bf16 42 / 36; of 32000, one block a wave, 36 / 42 and 20 / 22.
+//   * A group past its block's end is a load like the others. fp32: blocks half full pay (1000 rows of 131072 in 64 leaves 157 / 133,
+//     257 of 65536 in 32 34 / 31), quarters do not (257 of 65536 in 64 45 / 49).
+//   * fp32 gains at every row count, also just past a whole turn of the CUs, and at every width (257 x 151936 64 / 53, 1025 x 151936
+//     184 / 141, 257 x 2097152 933 / 894).
+//   * bf16, all blocks in registers (40): 256 x 73728 14.3 / 13.4, 257 18.9 / 18.8, 300 20.8 / 20.0; 257 x 151936 39.5 / 36.0. Below
+//     73728 columns a second turn of a few rows is worse (257 x 65536 15.9 / 16.6, 300 17.5 / 17.7; 256 12.5 / 12.1, 384 19.6 / 19.1).
+//   * bf16, some blocks read twice after all: 192 x 196608 28.9 / 29.1, 257 x 262144 63 / 65, and 513 x 524288 203 / 207, 1025 x 1048576
+//     746 / 773; but 384 x 180224 52.0 / 48.5, 384 x 393216 108 / 107, 1537 x 393216 395 / 347, 600 x 524288 227 / 216. Blocks
+//     three quarters full are then not enough (513 x 196608 in 32 leaves 83 / 86).
+extern "C" int ix_logprob_keeps_rows(int dtype, long rows, long V, int G) {
+  if (G < 1 || V < 65536 || V % G != 0) return 0;
+  const long units = G * ((V / G + IX_LP_BLOCK - 1) / IX_LP_BLOCK), columns = units * IX_LP_BLOCK;
+  if (units > IX_LP_HELD_UNITS || rows < IX_LP_SPLIT_BELOW) return 0;
+  if (dtype != IX_DT_BF16) return 2 * V >= columns;
+  if (units <= 40) return V >= 73728 || rows <= 256 || rows >= 384;
+  return units <= (rows >= 576 ? 128 : 96) && rows >= 384 && 8 * V >= 7 * columns;
+}
+
 template <typename T>
 static int ix_lp_launch(const T* x, long rows, long V, long row_stride, int G, const int64_t* target,
                         float* out_lp, float* out_lse, float* out_full, long full_stride, float* ws,
@@ -646,8 +664,10 @@ static int ix_lp_launch(const T* x, long rows, long V, long row_stride, int G, c
   // a caller-supplied row max (exact, e.g. from the producing GEMM's epilogue) removes the max
   // pass: the row is then read from HBM once, by the block sums
   const bool split = row_max_in || force_shape == 2 || (force_shape == 0 && rows < IX_LP_SPLIT_BELOW);
-  if (!split && force_shape == 0 && vec && !out_full && V >= IX_LP_HELD_V &&
-      G * ((L + IX_LP_BLOCK - 1) / IX_LP_BLOCK) <= IX_LP_HELD_UNITS) {
+  const bool can_keep = vec && !out_full && !row_max_in && G * ((L + IX_LP_BLOCK - 1) / IX_LP_BLOCK) <= IX_LP_HELD_UNITS;
+  if (force_shape == 3 && !can_keep) return IX_DECLINED;
+  if (force_shape == 3 ||
+      (force_shape == 0 && can_keep && ix_logprob_keeps_rows(sizeof(T) == 2 ? IX_DT_BF16 : IX_DT_F32, rows, V, G))) {
     constexpr int HU = sizeof(T) == 2 ? 5 : 2, LU = sizeof(T) == 2 ? 0 : 1;
     hipLaunchKernelGGL((k_lp_row_held<T, HU, LU>), dim3((unsigned)(rows < 256 ? rows : 256)), dim3(512),
                        (size_t)LU * 8 * IX_LP_BLOCK * sizeof(T), st, x, row_stride, rows, (int)V, G, target, out_lp, out_lse);

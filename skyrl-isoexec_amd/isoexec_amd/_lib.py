@@ -42,6 +42,7 @@ SIGNATURES = {
     "ix_arch_selfcheck": (c_int, [P, c_size_t, P, P]),
     "ix_arch_selfcheck_probe": (c_int, [P, c_size_t, c_uint, P, P]),
     "ix_logprob_workspace_bytes": (c_size_t, [c_long, c_long, c_int]),
+    "ix_logprob_keeps_rows": (c_int, [c_int, c_long, c_long, c_int]),
     "ix_logprob_rowinv_sampled": (
         c_int,
         [P, c_int, c_long, c_long, c_long, P, c_int, P, P, P, c_size_t, c_int, P, P],

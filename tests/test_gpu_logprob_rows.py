@@ -28,8 +28,8 @@ def test_kept_rows_equal_the_other_shapes(V, G, dtype, rows):
     x[rows - 1, V - 1] = 50.0
     t = torch.randint(0, V, (rows,), generator=g).to(DEV)
     t[1], t[2] = -100, V
-    got = sampled_forward(x, t, G)
-    for shape in (1, 2):
+    got = sampled_forward(x, t, G, force_shape=3)
+    for shape in (0, 1, 2):
         want = sampled_forward(x, t, G, force_shape=shape)
         assert same_bits(torch.nan_to_num(got[0], 7e7), torch.nan_to_num(want[0], 7e7)), shape
         assert same_bits(torch.nan_to_num(got[1], 7e7), torch.nan_to_num(want[1], 7e7)), shape
@@ -40,7 +40,7 @@ def test_kept_rows_with_a_longer_row_stride():
 
     wide = torch.randn(300, 65536 + 64, generator=cpu_gen(1)).to(DEV)
     x, t = wide[:, 32:32 + 65536], torch.randint(0, 65536, (300,), generator=cpu_gen(2)).to(DEV)
-    got, want = sampled_forward(x, t, 8), sampled_forward(x.contiguous(), t, 8, force_shape=2)
+    got, want = sampled_forward(x, t, 8, force_shape=3), sampled_forward(x.contiguous(), t, 8, force_shape=2)
     assert same_bits(got[0], want[0]) and same_bits(got[1], want[1])
 
 

@@ -350,7 +350,7 @@ __global__ __launch_bounds__(512) void k_lp_row_held(const T* __restrict__ x, lo
 // Shape 2: the row split over many workgroups. Workspace layout (floats):
 //   pmax [rows, P]  P = ceil(V / IX_LP_SEG)
 //   bsum [rows, U]  U = G * NB
-//   (and two floats per row that nothing uses: the size is part of the interface)
+//   fin  [rows, 2]  (m, log S), for full rows of many blocks a leaf
 template <typename T>
 __global__ __launch_bounds__(256) void k_lp_partmax(const T* __restrict__ x, long row_stride, int V, int P,
                                                     float* __restrict__ pmax, int vec) {
@@ -407,7 +407,7 @@ __global__ __launch_bounds__(256) void k_lp_blocksums(const T* __restrict__ x, l
 template <typename T>
 __global__ __launch_bounds__(64) void k_lp_finalize(const T* __restrict__ x, long row_stride, int V, int G, int P,
                                                     const float* __restrict__ pmax,
-                                                    const float* __restrict__ bsum,
+                                                    const float* __restrict__ bsum, float* __restrict__ fin,
                                                     const int64_t* __restrict__ target,
                                                     float* __restrict__ out_lp, float* __restrict__ out_lse) {
   __shared__ float s_leaf[IX_LP_MAX_G];
@@ -421,6 +421,10 @@ __global__ __launch_bounds__(64) void k_lp_finalize(const T* __restrict__ x, lon
   if (lane == 0) {
     const float S = ix_fold_leaves(s_leaf, G);
     const float log_s = ix_log(S);
+    if (fin) {
+      fin[row * 2] = m;
+      fin[row * 2 + 1] = log_s;
+    }
     ix_lp_emit(x + row * row_stride, V, m, log_s, target, row, out_lp, out_lse);
   }
 }
@@ -428,7 +432,10 @@ __global__ __launch_bounds__(64) void k_lp_finalize(const T* __restrict__ x, lon
 // The whole row, and its lse. Every workgroup joins the row's block sums for itself (a wave, while the columns travel) instead
 // of a launch in front that does it once: 4.6 us less for a decode step. Bound by HBM: four columns per lane and access, so that
 // a store instruction is 1 KiB of the row, all of them requested first: 64 rows of 151936 26.5 -> 10.2 us (eight columns
-// per lane stored one by one before).
+// per lane stored one by one before). The join is a chain over a leaf's blocks, so with many of them the launch in front does it
+// (fin). us joined everywhere / in front, bf16: 1 row of 192 blocks 24.4 / 25.0, 16 39.4 / 41.3, 64 117 / 97; of 256 29.5 / 29.1,
+// 50.0 / 52.7, 171 / 136; of 384 40.4 / 39.1, 98 / 76, 332 / 209; 64 rows of 136 84 / 71, 16 of 2048 1417 / 442.
+static bool ix_lp_joins_in_front(long rows, int NB) { return NB > 256 || (NB > 128 && rows >= 64); }
 __device__ __forceinline__ void ix_lp_load4(const float* p, float (&v)[4]) {
   const float4 a = *reinterpret_cast<const float4*>(p);
   v[0] = a.x; v[1] = a.y; v[2] = a.z; v[3] = a.w;
@@ -441,7 +448,7 @@ __device__ __forceinline__ void ix_lp_load4(const bf16_t* p, float (&v)[4]) {
 template <typename T>
 __global__ __launch_bounds__(256) void k_lp_fullwrite(const T* __restrict__ x, long row_stride, int V, int G, int P,
                                                       const float* __restrict__ pmax, const float* __restrict__ bsum,
-                                                      float* __restrict__ out_full, long full_stride,
+                                                      const float* __restrict__ fin, float* __restrict__ out_full, long full_stride,
                                                       float* __restrict__ out_lse, int vec, int PW) {
   constexpr int GROUPS = IX_LP_SEG / (256 * 4);
   __shared__ float s_fin[2];
@@ -459,7 +466,9 @@ __global__ __launch_bounds__(256) void k_lp_fullwrite(const T* __restrict__ x, l
     }
     __builtin_amdgcn_sched_barrier(0);
   }
-  if (threadIdx.x < 64) {
+  if (fin) {
+    if (threadIdx.x < 2) s_fin[threadIdx.x] = fin[row * 2 + threadIdx.x];
+  } else if (threadIdx.x < 64) {
     const int NB = (V / G + IX_LP_BLOCK - 1) / IX_LP_BLOCK;
     const float m = ix_row_max_from_parts(pmax + row * P, P, threadIdx.x);
     const float log_s = ix_log_total(bsum + row * (long)(G * NB), G, NB, threadIdx.x);
@@ -695,14 +704,14 @@ static int ix_lp_launch(const T* x, long rows, long V, long row_stride, int G, c
   const unsigned total = (unsigned)(rows * ny);
   hipLaunchKernelGGL((k_lp_blocksums<T>), dim3(ix_xcd_run_grid(total)), dim3(256), 0, st, x, row_stride, (int)V, G,
                      P, pmax, bsum, vec, ny, total);
-  if (!out_full) {
+  float* fin = out_full && ix_lp_joins_in_front(rows, NB) ? bsum + rows * U : nullptr;
+  if (!out_full || fin)
     hipLaunchKernelGGL((k_lp_finalize<T>), dim3((unsigned)rows), dim3(64), 0, st, x, row_stride, (int)V, G, P, pmax,
-                       bsum, target, out_lp, out_lse);
-    return ix_launch_status();
-  }
+                       bsum, fin, target, out_lp, out_lse);
+  if (!out_full) return ix_launch_status();
   const int vec4 = vec && full_stride % 4 == 0 && ix_aligned(out_full, 16);
   hipLaunchKernelGGL((k_lp_fullwrite<T>), dim3((unsigned)(rows * PW)), dim3(256), 0, st, x, row_stride, (int)V, G, P, pmax,
-                     bsum, out_full, full_stride, out_lse, vec4, PW);
+                     bsum, fin, out_full, full_stride, out_lse, vec4, PW);
   return ix_launch_status();
 }
 

@@ -45,8 +45,9 @@ def test_kept_rows_with_a_longer_row_stride():
 
 
 # Segments of 8192 columns that end with a group of eight, one row and several, a row that no 16-byte store fits, a maximum that is
-# given; the row's log-sum joined by every segment for itself.
-@pytest.mark.parametrize("V,G,pad", [(8, 1, 0), (8192, 8, 0), (8200, 1, 0), (151936, 8, 0), (151936, 8, 1), (1000, 8, 0), (16392, 1, 4)])
+# given; the row's log-sum joined by every segment for itself, and by a launch in front (a leaf of more than 256 blocks).
+@pytest.mark.parametrize("V,G,pad", [(8, 1, 0), (8192, 8, 0), (8200, 1, 0), (151936, 8, 0), (151936, 8, 1), (1000, 8, 0), (16392, 1, 4),
+                                     (256 * 4096, 1, 0), (256 * 4096 + 8, 1, 4), (2 * 257 * 4096, 2, 1)])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 def test_full_rows_of_the_split_shape(V, G, pad, dtype):
     from isoexec_amd import _lib

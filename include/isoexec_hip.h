@@ -155,7 +155,8 @@ int ix_moe_combine_add_rmsnorm(const void* expert_out, const int* combine_rows, 
  * asked for by number they decline what it does not serve. Every choice gives the same bits.
  * row_max_parts: NULL, or fp32 [M, parts_ld] receiving per part the max of the stored values, parts_ld >=
  * ix_gemm_bf16_n_tiles(M, N, K, tile), which alone says how many parts a row has: one per column tile, two for tiles 4, 7 and 8, four
- * for the bands, which tile 0 may choose (a part may be stored more than once where the call is one that bands do not serve). */
+ * for the bands, which tile 0 may choose (a part may be stored more than once where the call is not one that the shape counted for
+ * serves: a bias, an fp32 result, weight rows further apart than K). */
 int ix_gemm_bf16_nt(const void* A, long lda, const void* W, long ldw, const void* bias, void* C, int c_dtype,
                     long ldc, long M, long N, long K, int tile, float* row_max_parts, long parts_ld,
                     void* stream);

@@ -270,20 +270,30 @@ static int ix_gemm_tile_for(long M, long N, long K, int tile, bool bands) {
     }
   }
   // The 64 x 32 tile in halves of 32 rows: for few rows its other half only takes room in the ring, whose bytes under way are
-// what a CU's share of the weight waits for (ten stages of 8 KiB instead of six of 12), and at one turn of tiles the halves are
-// on two CUs. With more turns every weight tile is read twice instead. us 64 x 32 / 32 x 32, weights from memory: 2048 x 4096 at
-// 1 row 12.6 / 10.3, 32 13.4 / 12.2, 64 15.8 / 12.2; 5120 x 2048 at 1 8.9 / 7.7, 32 9.4 / 8.5, 64 (320 halves) 10.4 / 12.4;
-// 12352 x 2048 at 32 17.2 / 15.2, 33 16.8 / 19.6; 4096 x 4096 at 64 16.9 / 13.0, 100 14.8 / 17.4; 128 x 4096 at 2000 11.6 / 10.7, 4096 13.0 / 15.5.
-  // Weight rows 4 KiB apart and a few rows: 128 of them per tile are read at 4.6 TB/s by this memory system, 32 at up to 5.9. us
-  // 128 x 128 / 32 x 32: 151936 x 2048 at 1 row 134 / 105, 16 129 / 117, 24 130 / 126 (with the row maximum and the norm in front 142 / 144), 32 135 / 134; 65536 x 2048 at 7 62 / 57; 32000
-  // x 2048 32.1 / 31.3; rows 8 KiB apart (151936 x 4096 at 7) 195 / 206, 2 KiB 55 / 61.
-  if (M <= 16 && K * 2 == 4096 && N >= 32000) return 9;
+  // what a CU's share of the weight waits for (ten stages of 8 KiB instead of six of 12), and at one turn of tiles the halves
+  // are on two CUs. With more turns every weight tile is read twice instead. us 64 x 32 / 32 x 32, weights from memory: 2048 x
+  // 4096 at 1 row 12.6 / 10.3, 32 13.4 / 12.2, 64 15.8 / 12.2; 5120 x 2048 at 1 8.9 / 7.7, 32 9.4 / 8.5, 64 (320 halves) 10.4 /
+  // 12.4; 12352 x 2048 at 32 17.2 / 15.2, 33 16.8 / 19.6; 4096 x 4096 at 64 16.9 / 13.0, 100 14.8 / 17.4; 128 x 4096 at 2000
+  // 11.6 / 10.7, 4096 13.0 / 15.5.
   return best == 6 && halves ? 9 : best;
+}
+
+// A few rows of x and weight rows 4 KiB apart: where the 128 x 128 tile is the choice, the 32 x 32 one reads the weight faster. TB/s
+// 128 x 128 / 32 x 32 at one row of 151936 x 2048: rows 4096 bytes apart 4.5 / 5.9, 4224 5.7 / 6.0, 8192 6.1 / 6.1; K = 1984 in rows of
+// 4096 bytes 4.5 / 5.9, without a gap 5.7 / 6.1. Why that distance costs the larger tile is not known, and weights of other sizes
+// do not show it, so the rule keeps to what was measured to gain. us at 1 / 8 / 16 rows, 128 x 128 then 32 x 32, K = 2048: 80000 77 77 74
+// - 60 62 66; 100000 94 93 95 - 75 77 82; 128256 112 113 113 - 91 94 100; 151936 128 127 125 - 104 108 116; 200000 143 144 147 -
+// 131 138 150; not 65536 (53 51 52 - 53 54 55) nor 250000 (153 156 162 - 161 168 185). Less of such rows: K = 1536 of 151936 97 95
+// 93 - 80 85 93, 1024 73 73 73 - 64 68 75. With the row maximum, the norm and the logprobs around it 140 140 138 - 119 125 134. With
+// a bias it does not gain (136 137 138 - 134 138 142; 100000 85 85 86 - 92 94 97).
+static bool ix_gemm_rows_4k_apart(long M, long N, long K, long ldw) {
+  return ldw * 2 == 4096 && K >= 1536 && N >= 80000 && N <= 200000 && M <= (N <= 160000 ? 16 : 8);
 }
 
 // Row-max parts per row of C: one per column tile of the shape that runs.
 extern "C" long ix_gemm_bf16_n_tiles(long M, long N, long K, int tile) {
-  const int t = ix_gemm_tile_for(M, N, K, tile, true);
+  int t = ix_gemm_tile_for(M, N, K, tile, true);
+  if (tile == 0 && t == 2 && ix_gemm_rows_4k_apart(M, N, K, K)) t = 9;  // weight rows without a gap
   const long bn = (t == 2) ? 128 : (t == 6 || t == 9) ? 32 : 256;  // ids 1, 3, 4, 5, 7, 8 are 256 wide
   // the four-wave tiles write one part per wave column
   const long per_tile = t > IX_TILE_BAND ? 4 : ((t == 4 || t == 7 || t == 8) ? 2 : 1);
@@ -310,6 +320,10 @@ static int ix_gemm_bf16_dispatch(const bf16_t* a, long lda, const bf16_t* w, lon
     id = ix_gemm_tile_for(rows, N, K, 0, false);
     if (id == 6 || id == 9) id = 2;
     slots = 4 * ((N + 255) / 256);
+  }
+  if (tile == 0 && id == 2 && batch == 1) {
+    if (!b && ix_gemm_rows_4k_apart(M, N, K, ldw) && (!parts || K == ldw)) id = 9;
+    else if (parts && ix_gemm_rows_4k_apart(M, N, K, K)) slots = (N + 31) / 32;  // counted for a product without these
   }
   switch (id) {
     case 1: return ix_gemm_bf16_launch<32, 256, 1, 4, TC, 4>(a, lda, w, ldw, b, c, ldc, M, N, K, parts, parts_ld, st IX_BATCH_ARGS);

@@ -39,3 +39,23 @@ def test_rule_of_the_small_tiles(M, N, K):
     want, want_top = linear_nt(x, w, tile=6, want_row_max=True)
     got, top = linear_nt(x, w, want_row_max=True)
     assert same_bits(got, want) and same_bits(top, want_top)
+
+
+# Weight rows 4 KiB apart, with and without a gap, and rows that only the row maximum's count takes for such (a gap, a bias): the
+# columns of a last tile of 32 and of 128, the row maximum of every part that is counted.
+@pytest.mark.parametrize("M,K,pitch", [(1, 2048, 2048), (16, 2048, 2048), (17, 2048, 2048), (7, 1984, 2048), (7, 2048, 2112)])
+def test_few_rows_against_weight_rows_4_kib_apart(M, K, pitch):
+    from isoexec_amd.ops.mm.mm_hip import linear_nt
+
+    N = 80040
+    g = torch.Generator(device=DEV)
+    g.manual_seed(M + K + pitch)
+    w = torch.randn(N, pitch, generator=g, device=DEV, dtype=torch.bfloat16)[:, :K]
+    x = torch.randn(M, K, generator=g, device=DEV, dtype=torch.bfloat16)
+    bias = torch.randn(N, generator=g, device=DEV, dtype=torch.bfloat16)
+    for b in (None, bias):
+        for dtype in (torch.bfloat16, torch.float32):
+            want, want_top = linear_nt(x, w, b, tile=6, out_dtype=dtype, want_row_max=True)
+            got, top = linear_nt(x, w, b, out_dtype=dtype, want_row_max=True)
+            assert same_bits(got, want) and same_bits(top, want_top)
+            assert same_bits(linear_nt(x, w, b, out_dtype=dtype), want)

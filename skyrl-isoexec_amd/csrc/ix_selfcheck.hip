@@ -4,12 +4,15 @@
 // provider whose premise fails on the device it meets is switched off for good. Here the same question is put to the
 // library's own kernels, on the device, through its own entry points:
 //   bit 0  seeded product, operands with a wide exponent spread: every tile shape and launch form of ix_gemm_bf16_nt
-//          (ids 1..8) stores the same bits as id 1;
+//          (ids 1..9 and the bands 14..17) stores the same bits as id 1;
 //   bit 1  small-integer operands (every partial sum exact in fp32, so the result does not depend on any order): every
 //          id stores bf16(the integer product), computed independently by a plain integer kernel;
-//   bit 2  the row-invariant log-softmax + gather gives the same bits in both of its launch shapes (seeded logits);
-//   bit 3  an id declined a shape it documents as served (nothing compared for it).
-// The caller owns the scratch memory; nothing is allocated. The call ends with a stream synchronisation and a 16-byte
+//   bit 2  the row-invariant log-softmax + gather gives the same bits in all three of its launch shapes (seeded logits, more
+//          rows than CUs, and rows of more blocks than a workgroup keeps, in both types);
+//   bit 3  an id declined a shape it documents as served (nothing compared for it);
+//   bit 4  the matrix instruction that updates the delta-rule's state rounds one product per element like fmaf (subnormals and
+//          infinities among the operands; a NaN's payload is not compared).
+// The caller owns the scratch memory; nothing is allocated. The call ends with a stream synchronisation and a 20-byte
 // copy to the host: it is a set-up call, not a hot-path one.
 #include "ix_common.h"
 #include "../../include/isoexec_hip.h"
@@ -77,8 +80,41 @@ __global__ void k_sc_flip(uint32_t* __restrict__ words, long at) {
   if (threadIdx.x == 0 && blockIdx.x == 0) words[at] ^= 1u;
 }
 
+#define IX_SC_FLAGS 5
 __global__ void k_sc_clear(int* __restrict__ flags) {
-  if (threadIdx.x < 4) flags[threadIdx.x] = 0;
+  if (threadIdx.x < IX_SC_FLAGS) flags[threadIdx.x] = 0;
+}
+
+// One product per element through v_mfma_f32_16x16x1_4b_f32 against fmaf, a wave per 1024 elements. The exponents of the
+// operands are spread over the whole range, the addend's lies around the product's. Register i of a lane is block i / 4, row
+// 4 (lane / 16) + i % 4, column lane % 16; an operand lane is block lane / 16, row or column lane % 16.
+typedef float ix_sc_f32x16 __attribute__((ext_vector_type(16)));
+__device__ __forceinline__ float ix_sc_float(uint64_t h, int e) {
+  const uint32_t bits = (uint32_t)(h & 1u) << 31 | (uint32_t)(h >> 32 & 0x7fffffu);
+  if (e >= 255) return __uint_as_float((bits & 0x80000000u) | 0x7f800000u);
+  return __uint_as_float(bits | (uint32_t)max(e, 0) << 23);
+}
+__global__ __launch_bounds__(64) void k_sc_one_product(int* __restrict__ flags, int which, int inject) {
+  const int lane = threadIdx.x;
+  const uint64_t at = ((uint64_t)blockIdx.x * 64 + lane) * 18;
+  const auto exponent = [](uint64_t h) { return (int)(h >> 8 & 0xffffu) % 256; };
+  const uint64_t ha = ix_sc_mix(0xabcdull + at), hb = ix_sc_mix(0xabcdull + at + 1);
+  const int ea = exponent(ha), eb = exponent(hb);
+  const float a = ix_sc_float(ha, ea), b = ix_sc_float(hb, eb);
+  ix_sc_f32x16 c, want;
+#pragma unroll
+  for (int i = 0; i < 16; ++i) {
+    const int la = (i >> 2) * 16 + (lane >> 4) * 4 + (i & 3), lb = (i >> 2) * 16 + (lane & 15);
+    const float x = __shfl(a, la, 64), y = __shfl(b, lb, 64);
+    const uint64_t hc = ix_sc_mix(0xabcdull + at + 2 + i);
+    c[i] = ix_sc_float(hc, __shfl(ea, la, 64) + __shfl(eb, lb, 64) - 127 + (int)(hc >> 24 & 0xffu) % 53 - 26);
+    want[i] = __builtin_fmaf(x, y, c[i]);
+  }
+  if (inject && blockIdx.x == 0 && lane == 5) want[3] = __uint_as_float(__float_as_uint(want[3]) ^ 1u);
+  const ix_sc_f32x16 got = __builtin_amdgcn_mfma_f32_16x16x1f32(a, b, c, 0, 0, 0);
+#pragma unroll
+  for (int i = 0; i < 16; ++i)
+    if (__float_as_uint(got[i]) != __float_as_uint(want[i]) && !(got[i] != got[i] && want[i] != want[i])) flags[which] = 1;
 }
 
 static inline size_t ix_sc_up(size_t x) { return (x + 255) & ~(size_t)255; }
@@ -100,7 +136,7 @@ static IxScLayout ix_sc_layout() {
   L.lp2 = take((size_t)IX_SC_M * 4);
   L.lp_ws_bytes = ix_logprob_workspace_bytes(IX_SC_M, IX_SC_N, IX_SC_G);
   L.lp_ws = take(L.lp_ws_bytes);
-  L.flags = take(16);
+  L.flags = take(IX_SC_FLAGS * sizeof(int));
   L.total = at;
   return L;
 }
@@ -112,7 +148,7 @@ extern "C" int ix_arch_selfcheck(void* workspace, size_t workspace_bytes, unsign
 }
 
 // The self-check with one bit of a comparison's reference side flipped first, for every check named in `inject` (bits
-// 0..2 as in failed_checks): the call must then report exactly those checks. It is how a test (or a suspicious
+// 0..2 and 4 as in failed_checks): the call must then report exactly those checks. It is how a test (or a suspicious
 // operator) shows that the comparisons have teeth; inject = 0 is the self-check itself.
 extern "C" int ix_arch_selfcheck_probe(void* workspace, size_t workspace_bytes, unsigned inject, unsigned* failed_checks,
                                        void* stream) {
@@ -147,7 +183,7 @@ extern "C" int ix_arch_selfcheck_probe(void* workspace, size_t workspace_bytes, 
       hipLaunchKernelGGL(k_sc_int_product, grid(nC), dim3(256), 0, st, A, W, Cref, M, N, K);
     }
     if (inject >> mode & 1u) hipLaunchKernelGGL(k_sc_flip, dim3(1), dim3(64), 0, st, (uint32_t*)Cref, nC / 4 + 17);
-    for (int tile = mode == 0 ? 2 : 1; tile <= 8; ++tile) {
+    for (int tile = mode == 0 ? 2 : 1; tile <= 17; tile = tile == 9 ? 14 : tile + 1) {  // 14..17: the bands
       const int rc = ix_gemm_bf16_nt(A, K, W, K, nullptr, Cgot, IX_DT_BF16, N, M, N, K, tile, nullptr, 0, stream);
       if (rc < 0) return rc;
       if (rc != IX_OK) {
@@ -158,27 +194,39 @@ extern "C" int ix_arch_selfcheck_probe(void* workspace, size_t workspace_bytes, 
                          nC / 2, flags, mode);
     }
     if (mode == 0) {
-      // seeded logits (the product buffer is free again) through both launch shapes of the log-softmax
+      // seeded logits (the product buffer is free again) through the launch shapes of the log-softmax: as rows of N, as two
+      // bf16 rows and as one fp32 row (the pairs' upper halves are logit-sized)
       hipLaunchKernelGGL(k_sc_fill, grid(nC), dim3(256), 0, st, Cgot, nC, 0x4242ull, 2);
-      hipLaunchKernelGGL(k_sc_targets, grid(M), dim3(256), 0, st, targets, (long)M, (long)N, 0x5555ull);
-      float* outs[2] = {lp1, lp2};
-      for (int shape = 1; shape <= 2; ++shape) {
-        const int rc = ix_logprob_rowinv_sampled(Cgot, IX_DT_BF16, M, N, N, targets, IX_SC_G, outs[shape - 1], nullptr,
-                                                 base + L.lp_ws, L.lp_ws_bytes, shape, nullptr, stream);
-        if (rc < 0) return rc;
-        if (rc != IX_OK) declined |= 1u << (8 + shape);
+      const struct { int dtype; long rows; } views[3] = {{IX_DT_BF16, M}, {IX_DT_BF16, 2}, {IX_DT_F32, 1}};
+      for (const auto& view : views) {
+        const long V = nC / (view.dtype == IX_DT_F32 ? 2 : 1) / view.rows;
+        hipLaunchKernelGGL(k_sc_targets, grid(view.rows), dim3(256), 0, st, targets, view.rows, V, 0x5555ull);
+        for (int shape = 1; shape <= 3; ++shape) {
+          const int rc = ix_logprob_rowinv_sampled(Cgot, view.dtype, view.rows, V, V, targets, IX_SC_G, shape == 1 ? lp1 : lp2,
+                                                   nullptr, base + L.lp_ws, L.lp_ws_bytes, shape, nullptr, stream);
+          if (rc < 0) return rc;
+          if (rc != IX_OK) {
+            declined |= 1u << (20 + shape);
+            continue;
+          }
+          if (shape == 1) {
+            if (inject >> 2 & 1u)
+              hipLaunchKernelGGL(k_sc_flip, dim3(1), dim3(64), 0, st, (uint32_t*)lp1, view.rows / 2);
+            continue;
+          }
+          hipLaunchKernelGGL(k_sc_compare, grid(view.rows), dim3(256), 0, st, (const uint32_t*)lp1, (const uint32_t*)lp2,
+                             view.rows, flags, 2);
+        }
       }
-      if (inject >> 2 & 1u) hipLaunchKernelGGL(k_sc_flip, dim3(1), dim3(64), 0, st, (uint32_t*)lp1, (long)(M / 2));
-      hipLaunchKernelGGL(k_sc_compare, grid(M), dim3(256), 0, st, (const uint32_t*)lp1, (const uint32_t*)lp2, (long)M,
-                         flags, 2);
     }
   }
+  hipLaunchKernelGGL(k_sc_one_product, dim3(1024), dim3(64), 0, st, flags, 4, (int)(inject >> 4 & 1u));
   if (ix_launch_status() != IX_OK) return IX_ERR_LAUNCH;
-  int host_flags[4] = {0, 0, 0, 0};
+  int host_flags[IX_SC_FLAGS] = {};
   if (hipMemcpyAsync(host_flags, flags, sizeof(host_flags), hipMemcpyDeviceToHost, st) != hipSuccess) return IX_ERR_LAUNCH;
   if (hipStreamSynchronize(st) != hipSuccess) return IX_ERR_LAUNCH;
   unsigned failed = 0;
-  for (int i = 0; i < 3; ++i)
+  for (int i = 0; i < IX_SC_FLAGS; ++i)
     if (host_flags[i]) failed |= 1u << i;
   if (declined) failed |= 1u << 3;
   if (failed_checks) *failed_checks = failed;

@@ -84,7 +84,8 @@ class HardwareTarget:
 # ---- device self-check -------------------------------------------------------------------------------------------
 SELFCHECK_OBLIGATION = "domain_check:arch.selfcheck"
 SELFCHECK_BITS = ("seeded product differs between tile shapes", "integer product differs from the integer truth",
-                  "log-softmax launch shapes differ", "a tile id declined the check's shape")
+                  "log-softmax launch shapes differ", "a tile id declined the check's shape",
+                  "a matrix instruction of one product does not round like fmaf")
 _SELFCHECK = None   # None = not run in this process, else (ok, evidence)
 
 
@@ -113,7 +114,8 @@ def arch_selfcheck(verbose: bool = True, device=None) -> bool:
         mask = ctypes.c_uint(0)
         rc = L.ix_arch_selfcheck(ws.data_ptr(), need, ctypes.byref(mask), _lib.current_stream(dev))
     if rc == _lib.IX_OK:
-        ok, evidence = True, f"{ARCH}: tile ids 1-8 and both log-softmax shapes agree bit for bit"
+        ok, evidence = True, (f"{ARCH}: tile ids 1-9 and 14-17, the three log-softmax shapes and the one-product matrix "
+                              "instruction agree bit for bit")
     elif rc == _lib.IX_DECLINED:
         failed = [text for bit, text in enumerate(SELFCHECK_BITS) if mask.value >> bit & 1]
         ok, evidence = False, f"{ARCH}: " + "; ".join(failed)

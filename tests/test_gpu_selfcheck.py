@@ -30,7 +30,7 @@ def _run(inject):
 def test_selfcheck_passes_and_every_comparison_has_teeth():
     assert _run(None) == (0, 0)
     assert _run(0) == (0, 0)
-    for inject in (1, 2, 4, 5, 7):
+    for inject in (1, 2, 4, 5, 7, 16, 23):
         assert _run(inject) == (1, inject), inject      # IX_DECLINED, exactly the checks whose reference was touched
     assert _run(None) == (0, 0)                          # nothing is left behind in the library
 

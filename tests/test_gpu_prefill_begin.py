@@ -30,14 +30,16 @@ def layers(kind, capacity=4):
 
 @pytest.mark.parametrize("kind", ["own", "native", "cpr"])
 def test_one_launch_leaves_what_the_operators_leave(kind, monkeypatch):
+    monkeypatch.setenv("SKYRL_ISOEXEC_GDN_CHUNKED_PREFILL", "1")
     (one, d, hv), (ops, _, _) = layers(kind), layers(kind)
     assert one._begin_served(torch.device(DEV))
     monkeypatch.setattr(ops, "_begin_served", lambda dev: False)
     for layer in (one, ops):
         layer.ssm_state.fill_(3.0)
     g = cpu_gen(2)
-    # new slots, a resumed one beside a new one, no fresh row, more slots than free rows (evictions), an empty sequence
-    steps = [([1, 3], [5, 1], None), ([3, 2], [4, 17], [True, False]), ([1, 2], [2, 3], [True, True]), ([4], [0], None)]
+    # new slots, a resumed one beside a new one, no fresh row, an empty sequence beside another, more slots than free rows (evictions)
+    steps = [([1, 3], [5, 1], [False, False]), ([3, 2], [4, 17], [True, False]), ([1, 2], [2, 3], [True, True]),
+             ([4, 1], [0, 3], [False, True])]
     if kind == "own":
         steps += [([900, 901, 902], [3, 1, 2], None), ([900, 5], [6, 2], [True, False])]
     for slots, lens, cont in steps:
@@ -46,14 +48,56 @@ def test_one_launch_leaves_what_the_operators_leave(kind, monkeypatch):
         x = torch.randn(t, d, generator=g).to(torch.bfloat16).to(DEV)
         a, b = (torch.randn(t, hv, generator=g).to(torch.bfloat16).to(DEV) for _ in range(2))
         dev_slots = torch.tensor(slots, device=DEV)
-        if t:
-            out = [ly.prefill(dev_slots, slots, x, a, b, qsl, has_initial_state=cont) for ly in (one, ops)]
-            assert same_bits(*out)
+        before = one.pos.clone() if kind == "cpr" else None
+        out = [ly.prefill(dev_slots, slots, x, a, b, qsl, has_initial_state=cont) for ly in (one, ops)]
+        assert same_bits(*out)
         names = ["ssm_state", "conv_state"] + ([] if kind == "native" else ["slot2row", "last_used", "_clock"])
         for name in names + (["entry_state", "pos"] if kind == "cpr" else []):
             assert torch.equal(getattr(one, name), getattr(ops, name)), (slots, name)
+        for slot, n, resumed in zip(slots, lens, cont or []):
+            if kind == "cpr":
+                row = one.require_row(slot)
+                assert one.pos[row] == n + (before[row] if resumed else 0)
     if kind == "native":
         assert (one.ssm_state[0] == 0).all()  # the null row
+
+
+@pytest.mark.parametrize("kind", ["own", "cpr"])
+def test_what_the_launch_resets_and_what_it_leaves(kind):
+    """Resumed rows and rows of other slots keep their state and position, fresh ones and the null row lose them; a slot named twice
+    has one row and its last stamp; evicted slots lead nowhere."""
+    (one, _, _), (ops, _, _) = layers(kind), layers(kind)
+    dev = torch.device(DEV)
+
+    def both(slots, cont, qsl):
+        got = one._prefill_begin(slots, None, cont, qsl, None, dev)
+        rows = ops._assign_many(slots)
+        want = (rows, *ops._prefill_upload(rows, cont, qsl, None, dev))
+        assert got[0] == want[0] and all(torch.equal(g, w) for g, w in zip(got[1:], want[1:]))
+        for name in ["ssm_state", "slot2row", "last_used", "_clock"] + (["entry_state", "pos"] if kind == "cpr" else []):
+            assert torch.equal(getattr(one, name), getattr(ops, name)), name
+        return got[0]
+
+    def marked():
+        for ly in (one, ops):
+            ly.ssm_state.fill_(3.0)
+            if kind == "cpr":
+                ly.entry_state.fill_(5.0)
+                ly.pos.fill_(7)
+
+    kept = lambda r: bool((one.ssm_state[r] == 3.0).all()) and (kind != "cpr" or bool((one.entry_state[r] == 5.0).all()) and one.pos[r] == 7)
+    zero = lambda r: bool((one.ssm_state[r] == 0.0).all()) and (kind != "cpr" or bool((one.entry_state[r] == 0.0).all()) and one.pos[r] == 0)
+    a, b = both([1, 3], [False, False], [0, 2, 5])
+    marked()
+    (a2, c) = both([1, 2], [True, False], [0, 1, 4])
+    assert a2 == a and kept(a) and kept(b) and zero(c) and zero(0)
+    marked()
+    d, d2, a3 = both([9, 9, 1], [False, False, False], [0, 2, 2, 3])  # one row left, named twice; a slot starts anew
+    assert d == d2 and a3 == a and zero(d) and zero(a) and kept(b) and kept(c)
+    assert one.last_used[d] == one._clock - 1 and one.last_used[a] == one._clock
+    marked()
+    e, f = both([50, 51], [False, False], [0, 1, 2])  # the pool is full: the two least recently used rows go
+    assert {e, f} == {b, c} and one.slot2row[3] == 0 and one.slot2row[2] == 0 and zero(e) and zero(f) and kept(a) and kept(d)
 
 
 def test_prefill_with_and_without_the_l2norm_in_the_convolution():

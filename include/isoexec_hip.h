@@ -229,7 +229,7 @@ int ix_arena_destroy(void* arena);
  * or 16 for the four-lane layout (K = 128, compact state form, V % 128 == 0; declined otherwise), 17 / 18 for the walk with
  * one / two rows per lane group, 19 with four lanes per row (K = 128, V % 64 == 0) (compact form with an output, q and k rows
  * aligned to 8 elements; declined otherwise);
- * 0 = chosen from the grid size. Neither changes results. */
+ * 0 = chosen from the grid size. Neither changes results, but for the payload of a NaN. */
 int ix_gdn_scan(const void* q, const void* k, const void* v, const float* g, const void* beta, void* o,
                 int io_dtype, long q_pitch, long k_pitch, long v_pitch, float* state_pool,
                 const int* cu_seqlens, const int* state_indices, long state_indices_stride, long N, long H,
@@ -341,7 +341,7 @@ int ix_gdn_forward(const void* q, const void* k, const void* v, const float* g, 
 
 /* ix_gdn_scan (compact form, time_tile 0, o not NULL; with a gate ix_gdn_scan_gated_norm) and ix_gdn_forward for a host that
  * knows the lengths: `tokens` in all, `longest` the longest sequence's (0: not known). They choose the layout, which changes no
- * result. The gate is served where ix_gdn_layout says 16 and IX_DECLINED otherwise, before anything is launched. */
+ * result (a NaN's payload aside). The gate is served where ix_gdn_layout says 16 and IX_DECLINED otherwise, before anything is launched. */
 int ix_gdn_scan_lens(const void* q, const void* k, const void* v, const float* g, const void* beta, void* o, int io_dtype,
                      long q_pitch, long k_pitch, long v_pitch, float* state_pool, const int* cu_seqlens,
                      const int* state_indices, long N, long H, long HV, long K, long V, float scale, long tokens, long longest,

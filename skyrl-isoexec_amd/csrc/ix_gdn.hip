@@ -210,7 +210,8 @@ __global__ __launch_bounds__(256) void k_gdn_scan(const TIO* __restrict__ q, con
 // elements k = 32 g .. 32 g + 31 of both: 64 state floats per lane. The row's arithmetic is that of k_gdn_scan statement
 // for statement -- per 8-element slice the same two multiply-add chains and their join (ix_dot8), the adjacent-pairwise
 // tree over the 16 slice sums, here two levels inside the lane, one across neighbouring lane groups and one across the
-// wave's halves -- so the two kernels agree bit for bit, and which one runs is a staging choice like the time tile.
+// wave's halves -- so the two kernels agree bit for bit (a NaN's payload aside), and which one runs is a staging choice like the time
+// tile.
 // The rank-one update S += d k is four v_mfma_f32_16x16x1_4b_f32: state rows are the columns (B = d), the elements of k the
 // rows (A, one value per lane), S the accumulator, whose register layout is the one above. With one product per element
 // that instruction is a fused multiply-add, rounded once, subnormals kept (2 M random, tiny and special operands against fmaf:

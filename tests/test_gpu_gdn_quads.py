@@ -44,6 +44,60 @@ def test_update_on_the_matrix_pipe_rounds_as_the_multiply_adds(V, dtype, size):
     assert not same_bits(pa, start)
 
 
+def nan_alike(a, b):
+    """Equal bits, but for a NaN's: which of two NaN operands an instruction passes on is not part of the contract."""
+    n = lambda t: torch.where(t.isnan(), torch.full_like(t, 7e7), t)
+    return same_bits(n(a), n(b))
+
+
+# Signed zeros, infinities and NaNs in the state and in the values, keys and queries of zero, on both four-lane layouts against the
+# sixteen-lane scan. The first sequence has one token: its infinity is still one in the state.
+@pytest.mark.parametrize("code", [16, 19])
+@pytest.mark.parametrize("V,dtype", [(128, torch.bfloat16), (128, torch.float32)])
+def test_special_values_on_four_lanes_per_row(V, dtype, code):
+    from isoexec_amd.ops.gdn.gdn_ops import gdn_recurrent_kernel
+
+    H, HV, N = 2, 4, len(LENS)
+    (q, k, v, gate, beta), cu = operands(LENS, H, HV, V, dtype, code)
+    start = torch.randn(N + 1, HV, V, 128, generator=cpu_gen(3)).to(DEV)
+    start[1] = 0.0
+    start[2] = -0.0
+    start[3, :, ::3] = -0.0
+    start[5, 0, 5, 7], start[5, 1, 6, 100] = float("inf"), -float("inf")
+    start[6, 2, 9, 64] = float("nan")
+    start[7, :, :, 1::2] = 0.0
+    v, k, q = v.clone(), k.clone(), q.clone()
+    v[0, ::4] = -0.0
+    v[0, 0, 0, 9], v[0, 40, 1, 3], v[0, 41, 2, 4], v[0, 60, 3, 5] = float("inf"), float("inf"), -float("inf"), float("nan")
+    k[0, 5], q[0, 6] = 0.0, -0.0
+    rows = torch.tensor([1, 2, 3, 0, 5, 6, 7, 8, 9], dtype=torch.int32, device=DEV)
+    pa, pb = start.clone(), start.clone()
+    run = lambda c, pool: gdn_recurrent_kernel(q, k, v, gate, beta, ssm_state=pool, state_indices=rows, cu_seqlens=cu, time_tile=c)
+    want, got = run(16 | (1 << 8), pa), run(code << 8, pb)
+    assert nan_alike(got.float(), want.float()) and nan_alike(pb, pa)
+    assert int(want.isnan().sum()) > 0 and int(pa[1].isinf().sum()) > 0 and int(pa[9].isnan().sum()) == 0
+
+
+# The state returns exactly the value that arrives: the update is a product with zero, of either sign.
+@pytest.mark.parametrize("code", [16, 19])
+def test_a_state_that_returns_the_value_exactly(code):
+    from isoexec_amd.ops.gdn.gdn_ops import gdn_recurrent_kernel
+
+    HV, V, T = 4, 128, 6
+    k = torch.zeros(1, T, HV, 128, device=DEV)
+    k[..., 5] = 1.0
+    pool = torch.randn(2, HV, V, 128, generator=cpu_gen(1)).to(DEV)
+    v = pool[1, :, :, 5].expand(1, T, HV, V).contiguous()
+    gate, beta = torch.zeros(1, T, HV, device=DEV), torch.full((1, T, HV), 0.5, device=DEV)
+    q = torch.randn(1, T, HV, 128, generator=cpu_gen(2)).to(DEV)
+    cu, rows = torch.tensor([0, T], dtype=torch.int32, device=DEV), torch.tensor([1], dtype=torch.int32, device=DEV)
+    start = pool.clone()
+    got = gdn_recurrent_kernel(q, k, v, gate, beta, ssm_state=pool, state_indices=rows, cu_seqlens=cu, time_tile=code << 8)
+    other = start.clone()
+    want = gdn_recurrent_kernel(q, k, v, gate, beta, ssm_state=other, state_indices=rows, cu_seqlens=cu, time_tile=16 | (1 << 8))
+    assert same_bits(pool, start) and same_bits(got, want)
+
+
 @pytest.mark.parametrize("V,dtype", [(128, torch.bfloat16), (64, torch.float32)])
 def test_walk_with_four_lanes_per_row_equals_the_token_staged_scan(V, dtype):
     """Code 19: outputs, final states and a null lane, one row block and two."""

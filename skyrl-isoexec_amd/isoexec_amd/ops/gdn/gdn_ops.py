@@ -15,6 +15,7 @@ from ... import _lib
 from ...debug.trace import get_tracer
 
 L2NORM_EPS = 1e-6  # gdn_ops.py:173
+_NORM_LAYOUT = 16  # ix_gdn_layout's code of the layout that takes the gated output norm along
 
 
 def _token_pitch(t: torch.Tensor) -> int:
@@ -35,7 +36,7 @@ def _flatten_tokens(t: torch.Tensor, tail: int) -> torch.Tensor:
     if b == 1:
         return t[0]
     if t.stride(0) == n * t.stride(1):
-        return t.as_strided((b * n, *t.shape[2:]), (t.stride(1), *t.stride()[2:]), t.storage_offset())
+        return t.flatten(0, 1)  # a view
     return t.reshape(b * n, *t.shape[2:])
 
 
@@ -140,8 +141,9 @@ def gdn_recurrent_kernel(
         fusable = (io is torch.bfloat16 and idx_stride == 0 and gate.dtype is io and weight.dtype is io
                    and gate.stride(2) == 1 and gate.stride(1) == V and weight.is_contiguous() and weight.numel() == V)
         rc = _lib.IX_DECLINED
-        if fusable and by_length:
-            rc = scan_by_length(gate, weight, eps, zero_centered)
+        if by_length:
+            if fusable and _lib.lib().ix_gdn_layout(n_seq, HV, K, V, _lib.DT_BF16, 0, qf.shape[0], longest) == _NORM_LAYOUT:
+                rc = scan_by_length(gate, weight, eps, zero_centered)
         elif fusable:
             rc = _lib.check(
                 _lib.lib().ix_gdn_scan_gated_norm(
@@ -177,7 +179,8 @@ def stateless_forward(q, k, v, g, beta, *, cu_seqlens=None, chunk_size: int = 0,
     """The delta-rule forward from a zero state that is not kept (``ix_gdn_forward``): ``q, k`` L2-normalised, layouts as
     ``gdn_recurrent_kernel``'s. ``chunk_size`` > 0 is the boundary form (``gdn_cpr_fwd``), in the same single pass over the
     tokens. With ``gated_norm`` the output comes back through the layer's gated output norm. ``longest`` as
-    ``gdn_recurrent_kernel``'s. Returns ``o`` shaped like ``v``, or ``None`` when the library does not serve the operands (nothing launched: the caller scans with a pool)."""
+    ``gdn_recurrent_kernel``'s. Returns ``o`` shaped like ``v``, or ``None`` when the library does not serve the operands
+    (nothing launched: the caller scans with a pool)."""
     _lib.require_device(q, k, v, g, beta, cu_seqlens)
     if q.ndim != 4 or v.ndim != 4:
         raise RuntimeError(f"[isoexec-amd] the delta-rule forward expects [B,T,H,K]/[B,T,HV,V], got {tuple(q.shape)}")

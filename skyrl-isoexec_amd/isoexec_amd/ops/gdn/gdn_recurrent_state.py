@@ -21,6 +21,7 @@ from __future__ import annotations
 
 import os
 from collections import OrderedDict
+from operator import sub
 from typing import Callable, Iterable, Sequence
 
 import numpy as np
@@ -489,7 +490,7 @@ class RecurrentGDN:
             slots_cpu, x, a, b, qsl, has_initial_state, prefill_query_start_loc, fuse_l2norm=fuse_l2norm)
         o = gdn_recurrent_kernel(q.unsqueeze(0), k.unsqueeze(0), v.unsqueeze(0), g.unsqueeze(0), beta.unsqueeze(0),
                                  ssm_state=self.ssm_state, state_indices=rows_out, cu_seqlens=cu, gated_norm=gated_norm,
-                                 longest=max((int(e) - int(s) for s, e in zip(qsl, qsl[1:])), default=0))
+                                 longest=max(map(sub, qsl[1:], qsl), default=0))
         return o[0]
 
     def _prefill_prepare(self, slots_cpu, x, a, b, qsl, has_initial_state, prefill_query_start_loc, fuse_l2norm=True):

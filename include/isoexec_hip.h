@@ -69,8 +69,8 @@ int ix_prim_unary(int op, const float* x, float* y, long n, void* stream);
  * against fmaf (a million, bits of NaNs aside). workspace: caller-owned device memory, 256-byte aligned, at
  * least ix_arch_selfcheck_workspace_bytes() (about 6 MiB); nothing is allocated. failed_checks (host memory, may be
  * NULL) receives a mask: bit 0 seeded product, bit 1 integer product, bit 2 log-softmax shapes, bit 3 an id declined
- * the shape, bit 4 the matrix instruction. Returns IX_OK (every check passed), IX_DECLINED (a check failed: do not serve from this device), < 0
- * (the checks could not run). Ends with a stream synchronisation: a set-up call, not a hot-path one. */
+ * the shape, bit 4 the matrix instruction. Returns IX_OK (every check passed), IX_DECLINED (a check failed: do not serve
+ * from this device), < 0 (the checks could not run). Ends with a stream synchronisation: a set-up call, not a hot-path one. */
 size_t ix_arch_selfcheck_workspace_bytes(void);
 int ix_arch_selfcheck(void* workspace, size_t workspace_bytes, unsigned* failed_checks, void* stream);
 /* The same call with one bit of the reference side of every check named in `inject` (bits 0..2 and 4) flipped first: it must
@@ -90,8 +90,8 @@ int ix_logprob_keeps_rows(int dtype, long rows, long V, int G);
  * [rows] (out of range -> logprob 0), G leaves (power of two, V % G == 0 else declined).
  * out_logprob fp32 [rows]; out_lse fp32 [rows] or NULL. force_shape: 0 auto, 1 one workgroup
  * per row, 2 split rows (needs the workspace), 3 rows kept on the CU (groups of 8 columns aligned, at most 512 blocks of 4096
- * columns, no row_max_in; declined otherwise), which 0 takes where ix_logprob_keeps_rows says so. row_max_in: NULL, or fp32 [rows] holding each
- * row's exact maximum (e.g. ix_gemm_bf16_nt's row_max_parts reduced by ix_rowmax_reduce): the
+ * columns, no row_max_in; declined otherwise), which 0 takes where ix_logprob_keeps_rows says so. row_max_in: NULL, or fp32
+ * [rows] holding each row's exact maximum (e.g. ix_gemm_bf16_nt's row_max_parts reduced by ix_rowmax_reduce): the
  * max pass is skipped and the logits are read once. The workspace is always required with it. */
 int ix_logprob_rowinv_sampled(const void* logits, int dtype, long rows, long V, long row_stride,
                               const int64_t* target, int G, float* out_logprob, float* out_lse,

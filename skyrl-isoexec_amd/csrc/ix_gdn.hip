@@ -214,8 +214,8 @@ __global__ __launch_bounds__(256) void k_gdn_scan(const TIO* __restrict__ q, con
 // tile.
 // The rank-one update S += d k is four v_mfma_f32_16x16x1_4b_f32: state rows are the columns (B = d), the elements of k the
 // rows (A, one value per lane), S the accumulator, whose register layout is the one above. With one product per element
-// that instruction is a fused multiply-add, rounded once, subnormals kept (2 M random, tiny and special operands against fmaf:
-// every bit but a NaN's payload); of the four multiply-adds per element and token one leaves the vector pipe, which bounds
+// that instruction is a fused multiply-add, rounded once, subnormals kept (a million operands over the whole range against fmaf in
+// ix_selfcheck.hip: every bit but a NaN's payload); of the four multiply-adds per element and token one leaves the vector pipe, which bounds
 // this kernel: 240 vector and matrix instructions per token for a wave's 32 rows. Two rows per lane, and not one with 64
 // elements, because every lane reads all its elements of k and q from LDS for each token: 18 reads of a wave instead of 34.
 // 64 x 2560 tokens, 32 heads: 10.1 ms on the vector pipe alone (a row held by two lanes), 8.9 ms this way.
@@ -831,7 +831,8 @@ __global__ __launch_bounds__(LONE ? 320 : 256) void k_gdn_walk(const TIO* __rest
 // Bound by vector issue with several waves per SIMD: 128 instructions per token for sixteen rows, 202 in the boundary form.
 // Tried: the next token's reads and dot products between a token's update and its output (168 registers no longer hold it;
 // with two waves per SIMD 64 x 1000 tokens of the boundary form 5466 -> 6221 us); one element of k and q per lane, broadcast on
-// the operand path of the multiply-adds, instead of the LDS reads (those multiply-adds do not run at the full rate: 6646); a higher wave priority for the longer sequences (nothing).
+// the operand path of the multiply-adds, instead of the LDS reads (those multiply-adds do not run at the full rate: 6646); a
+// higher wave priority for the longer sequences (nothing).
 template <typename TIO, bool CPR>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3, 3)))
 void k_gdn_walk_quads(const TIO* __restrict__ q, const TIO* __restrict__ k, const TIO* __restrict__ v,
@@ -1104,21 +1105,21 @@ static int ix_gdn_scan_launch(const void* q, const void* k, const void* v, const
 // the longest sequence decides: four lanes pay where enough of the others run beside it to its end. `even`: the tokens as so many
 // sequences of the longest one's length, in workgroups of 64 rows. us walk / one row / two rows, 32 heads, V = 128 (64
 // workgroups a sequence), bf16, `even` in brackets:
-//   1 x 8000 + 15 x 100 tokens (76) 1793 / 3345 / 6722     1 x 4096 + 31 x 64 (95) 912 / 1743 / 3404
-//   4 x 2000 + 12 x 200 (333) 803 / 873 / 1772             6 x 2000 + 10 x 200 (448) 1035 / 1038 / 1823
-//   16 of 60..1410 (534) 820 / 690 / 1299                  1 x 3000 + 47 x 500 (565) 1865 / 1634 / 2933
-//   8 x 2000 + 40 x 100 (640) 1526 / 1172 / 1858           16 x 1000 (1024) 1259 / 984 / 1063
-//   48 of 60..1470 (1599) 2491 / 2009 / 2133               24 x 1000 + 24 x 100 (1690) 1806 / 1432 / 1384
-//   48 x 1000 (3072) 3307 / 2731 / 2631                    12 of 60..1380 (768 workgroups) 653 / 680
-// Two rows per lane also take the gated norm along, which is worth more than the 6 % that they lose at 1599. Short sequences,
-// where a launch's start counts: 16 x 24 39.2 / 41.7, 16 x 48 63.2 / 63.4, 32 x 24 72.1 / 71.2, 32 x 32 86.7 / 79.2, 48 x 16
-// 76.2 / 77.8 / 82.5, 63 x 20 123 / 114 / 127, 63 x 24 142 / 127 / 130; from 64 sequences on two rows are no worse there.
-// Boundary form, walk / one row: 1 x 4096 + 31 x 64 (95) 1346 / 2387, 2 x 2000 + 14 x 200 (218) 801 / 1178, 4 x 2000 + 12 x 200
-// (333) 1205 / 1199, ten of 120..1500 (345) 943 / 917, 8 x 1000 + 2 x 100 (525) 992 / 768, 200 x 9 411 / 261, 64 x 1000 7289 /
-// 5235, nine of 120..1500 (576 workgroups) 1008 / 1000; fp32: 4 x 2000 + 28 x 200 (435) 1543 / 1486, 16 of 60..1500 (532) 1426 / 1183,
-// nine of 120..1500 1025 / 1119.
+//   1 x 8000 + 15 x 100 tokens (76) 1782 / 3335 / 6758     1 x 4096 + 31 x 64 (95) 912 / 1714 / 3401
+//   4 x 2000 + 12 x 200 (332) 779 / 870 / 1755             6 x 2000 + 10 x 200 (448) 1023 / 1033 / 1814
+//   16 of 60..1410 (533) 874 / 706 / 1295                  1 x 3000 + 47 x 500 (565) 1920 / 1565 / 2931
+//   8 x 2000 + 40 x 100 (640) 1453 / 1169 / 1849           16 x 1000 (1024) 1148 / 1000 / 1061
+//   48 of 60..1470 (1598) 2491 / 2085 / 2169               24 x 1000 + 24 x 100 (1689) 1791 / 1479 / 1401
+//   48 x 1000 (3072) 3327 / 2810 / 2720                    12 of 60..1380 (768 workgroups) 595 / 628 / 1165
+// Two rows per lane also take the gated norm along, which is worth more than the 4 % that they lose at 1598. Short sequences,
+// where a launch's start counts: 16 x 24 41 / 42, 16 x 48 64 / 64, 32 x 24 72 / 71, 32 x 32 88 / 80, 48 x 16 77 / 78 / 83, 63 x 20
+// 123 / 113 / 127, 63 x 24 141 / 127 / 130.
+// Boundary form, walk / one row: 1 x 4096 + 31 x 64 (95) 1350 / 2361, 2 x 2000 + 14 x 200 (217) 803 / 1175, 4 x 2000 + 12 x 200
+// (332) 1202 / 1190, ten of 120..1500 (345) 942 / 915, 8 x 1000 + 2 x 100 (524) 994 / 767, 200 x 9 411 / 262, 64 x 1000 7274 /
+// 5414; nine of 120..1500 (576 workgroups) were 1008 / 1000; fp32: 4 x 2000 + 28 x 200 (435) 1650 / 1488, 16 of 60..1500 (532)
+// 1423 / 1200, nine of 120..1500 1025 / 1119.
 // Where the host does not know the lengths (longest <= 0) only IX_GDN_QUAD_MANY workgroups of 128 rows leave the walk: 64 x 1000
-// tokens 4375 / 3677 / 3749.
+// tokens 4413 / 3845 / 3495.
 #define IX_GDN_FOUR_TWO 16
 #define IX_GDN_FOUR_ONE 19
 #define IX_GDN_QUAD_MANY 2048
@@ -1250,8 +1251,8 @@ static int ix_gdn_scan_impl(const void* q, const void* k, const void* v, const f
   if (gate) return IX_DECLINED;       // the norm rides on two rows per lane only
   if (rpl == 16) return IX_DECLINED;  // that layout was asked for and does not apply
   // Sequences of more than one token in the compact form: the walk (codes 17 and 18 force it with one and two rows per
-  // lane group, 19 with four lanes per row). k_gdn_scan below keeps the decode step, the per-token index map, the state-only pass and the operands
-  // whose rows are not aligned.
+  // lane group, 19 with four lanes per row). k_gdn_scan below keeps the decode step, the per-token index map, the state-only
+  // pass and the operands whose rows are not aligned.
   if (state_indices_stride == 0 && o && (time_tile <= 0 || (rpl >= 17 && rpl <= 19))) {
     const int form = rpl >= 17 ? rpl - 16 : (layout == IX_GDN_FOUR_ONE ? 3 : 0);
     const int rc = ix_gdn_walk(q, k, v, g, beta, o, io_dtype, state_pool, cu_seqlens, state_indices, q_pitch, k_pitch,

@@ -279,13 +279,13 @@ static int ix_gemm_tile_for(long M, long N, long K, int tile, bool bands) {
 }
 
 // A few rows of x and weight rows 4 KiB apart: where the 128 x 128 tile is the choice, the 32 x 32 one reads the weight faster. TB/s
-// 128 x 128 / 32 x 32 at one row of 151936 x 2048: rows 4096 bytes apart 4.5 / 5.9, 4224 5.7 / 6.0, 8192 6.1 / 6.1; K = 1984 in rows of
-// 4096 bytes 4.5 / 5.9, without a gap 5.7 / 6.1. Why that distance costs the larger tile is not known, and weights of other sizes
-// do not show it, so the rule keeps to what was measured to gain. us at 1 / 8 / 16 rows, 128 x 128 then 32 x 32, K = 2048: 80000 77 77 74
-// - 60 62 66; 100000 94 93 95 - 75 77 82; 128256 112 113 113 - 91 94 100; 151936 128 127 125 - 104 108 116; 200000 143 144 147 -
-// 131 138 150; not 65536 (53 51 52 - 53 54 55) nor 250000 (153 156 162 - 161 168 185). Less of such rows: K = 1536 of 151936 97 95
-// 93 - 80 85 93, 1024 73 73 73 - 64 68 75. With the row maximum, the norm and the logprobs around it 140 140 138 - 119 125 134. With
-// a bias it does not gain (136 137 138 - 134 138 142; 100000 85 85 86 - 92 94 97).
+// 128 x 128 / 32 x 32 at one row of 151936 x 2048: rows 4096 bytes apart 4.9 / 6.0, 4224 5.7 / 6.0, 8192 6.2 / 6.1; K = 1984 in rows of
+// 4096 bytes 4.9 / 6.0, without a gap 5.7 / 6.1. Why that distance costs the larger tile is not known, and weights of other sizes
+// do not show it, so the rule keeps to what was measured to gain. us at 1 / 8 / 16 rows, 128 x 128 then 32 x 32, K = 2048: 80000 72 72
+// 71 - 59 61 65; 100000 76 76 77 - 70 73 78 (on another card 94 93 95 - 75 77 82); 128256 113 108 113 - 92 94 100; 151936 128 128 125 -
+// 104 108 117; 200000 143 145 148 - 132 137 150; not 65536 (from card to card 51 to 61 - 53 to 59) nor 250000 (154 157 163 - 161 168
+// 184). Less of such rows: K = 1536 of 151936 96 96 94 - 80 86 94, 1024 67 67 68 - 60 66 72. With the row maximum, the norm and the
+// logprobs around it 140 140 138 - 119 125 134. With a bias it does not gain (138 139 139 - 136 139 144; 100000 80 80 81 - 89 92 95).
 static bool ix_gemm_rows_4k_apart(long M, long N, long K, long ldw) {
   return ldw * 2 == 4096 && K >= 1536 && N >= 80000 && N <= 200000 && M <= (N <= 160000 ? 16 : 8);
 }

@@ -647,13 +647,13 @@ extern "C" size_t ix_logprob_workspace_bytes(long rows, long V, int G) {
 //   * 65536 columns: 1000 rows fp32 78 / 50, bf16 42 / 36; of 32000, one block a wave, 36 / 42 and 20 / 22.
 //   * A group past its block's end is a load like the others. fp32: blocks half full pay (1000 rows of 131072 in 64 leaves 157 / 133,
 //     257 of 65536 in 32 34 / 31), quarters do not (257 of 65536 in 64 45 / 49).
-//   * fp32 gains at every row count, also just past a whole turn of the CUs, and at every width (257 x 151936 64 / 53, 1025 x 151936
-//     184 / 141, 257 x 2097152 933 / 894).
-//   * bf16, all blocks in registers (40): 256 x 73728 14.3 / 13.4, 257 18.9 / 18.8, 300 20.8 / 20.0; 257 x 151936 39.5 / 36.0. Below
-//     73728 columns a second turn of a few rows is worse (257 x 65536 15.9 / 16.6, 300 17.5 / 17.7; 256 12.5 / 12.1, 384 19.6 / 19.1).
-//   * bf16, some blocks read twice after all: 192 x 196608 28.9 / 29.1, 257 x 262144 63 / 65, and 513 x 524288 203 / 207, 1025 x 1048576
-//     746 / 773; but 384 x 180224 52.0 / 48.5, 384 x 393216 108 / 107, 1537 x 393216 395 / 347, 600 x 524288 227 / 216. Blocks
-//     three quarters full are then not enough (513 x 196608 in 32 leaves 83 / 86).
+//   * fp32 gains at every row count, also just past a whole turn of the CUs, and at every width (257 x 151936 65 / 53, 1025 x 151936
+//     184 / 141, 257 x 2097152 924 / 892).
+//   * bf16, all blocks in registers (40): 256 x 73728 14.2 / 13.4, 257 18.5 / 18.8, 300 20.7 / 20.1; 257 x 151936 39.9 / 36.2. Below
+//     73728 columns a second turn of a few rows is worse (257 x 65536 16.0 / 16.8, 300 17.6 / 17.7; 256 11.9 / 11.9, 384 19.8 / 18.9).
+//   * bf16, some blocks read twice after all: 192 x 196608 29.1 / 29.1, 257 x 262144 63.8 / 64.5, 513 x 524288 204 / 207, 1025 x
+//     1048576 747 / 770; but 384 x 180224 51.9 / 48.3, 384 x 393216 108 / 106, 1537 x 393216 394 / 348, 600 x 524288 227 / 215. Blocks
+//     three quarters full are then not enough (513 x 196608 in 32 leaves 84 / 87).
 extern "C" int ix_logprob_keeps_rows(int dtype, long rows, long V, int G) {
   if (G < 1 || V < 65536 || V % G != 0) return 0;
   const long units = G * ((V / G + IX_LP_BLOCK - 1) / IX_LP_BLOCK), columns = units * IX_LP_BLOCK;

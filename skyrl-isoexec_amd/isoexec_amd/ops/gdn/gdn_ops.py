@@ -40,6 +40,11 @@ def _flatten_tokens(t: torch.Tensor, tail: int) -> torch.Tensor:
     return t.reshape(b * n, *t.shape[2:])
 
 
+def _packed(t: torch.Tensor, dtype: torch.dtype) -> torch.Tensor:
+    """``t.to(dtype).contiguous()``, without the two calls where it is that already."""
+    return t if t.dtype is dtype and t.is_contiguous() else t.to(dtype).contiguous()
+
+
 _CU_CACHE: dict = {}
 
 
@@ -102,17 +107,17 @@ def gdn_recurrent_kernel(
     else:
         if B != 1:
             raise RuntimeError("[isoexec-amd] a packed batch (cu_seqlens) needs B == 1")
-        cu = cu_seqlens.to(torch.int32).contiguous()
+        cu = _packed(cu_seqlens, torch.int32)
         n_seq = cu.numel() - 1
     qf, kf, vf = _flatten_tokens(q, 2), _flatten_tokens(k, 2), _flatten_tokens(v, 2)
-    gf = _flatten_tokens(g, 1).to(torch.float32).contiguous()
-    bf = _flatten_tokens(beta, 1).to(io).contiguous()
-    idx = state_indices.to(torch.int32)
-    if idx.ndim == 1:
+    gf = _packed(_flatten_tokens(g, 1), torch.float32)
+    bf = _packed(_flatten_tokens(beta, 1), io)
+    if state_indices.ndim == 1:
         # One row per sequence: loaded before its first token, stored once after its last.
-        idx = idx.contiguous()
+        idx = _packed(state_indices, torch.int32)
         idx_stride = 0
     else:
+        idx = state_indices.to(torch.int32)
         if idx.stride(1) != 1:
             idx = idx.contiguous()
         idx_stride = idx.stride(0)
@@ -194,11 +199,11 @@ def stateless_forward(q, k, v, g, beta, *, cu_seqlens=None, chunk_size: int = 0,
     else:
         if B != 1:
             raise RuntimeError("[isoexec-amd] a packed batch (cu_seqlens) needs B == 1")
-        cu = cu_seqlens.to(torch.int32).contiguous()
+        cu = _packed(cu_seqlens, torch.int32)
         n_seq = cu.numel() - 1
     qf, kf, vf = _flatten_tokens(q, 2), _flatten_tokens(k, 2), _flatten_tokens(v, 2)
-    gf = _flatten_tokens(g, 1).to(torch.float32).contiguous()
-    bf = _flatten_tokens(beta, 1).to(io).contiguous()
+    gf = _packed(_flatten_tokens(g, 1), torch.float32)
+    bf = _packed(_flatten_tokens(beta, 1), io)
     o = torch.empty(qf.shape[0], HV, V, dtype=io, device=dev)
     longest = int(longest or 0) if cu_seqlens is not None else T
 

@@ -540,7 +540,7 @@ class RecurrentGDN:
     def _begin_served(self, dev) -> bool:
         pools = [self.ssm_state] + [t for t in self._fresh_state() if t is not None]
         return dev.type == "cuda" and all(t.device == dev and t.is_contiguous() and t.data_ptr() % 16 == 0 for t in pools) \
-            and self.ssm_state[0].numel() % 4 == 0
+            and self.ssm_state.numel() // self.ssm_state.shape[0] % 4 == 0
 
     def _prefill_begin(self, slots_cpu, rows, is_cont, qsl, cu, dev):
         """Rows assigned (``rows`` given: a native layer's), the device's tables brought up to date and fresh rows zeroed: one
@@ -567,11 +567,11 @@ class RecurrentGDN:
         st = t[2 * (ne + nt):].view(torch.int32)
         pool2, pos = self._fresh_state()
         own = table is not None
-        base = t.data_ptr()
+        base, pool_rows = t.data_ptr(), self.ssm_state.shape[0]
         rc = _lib.check(_lib.lib().ix_gdn_prefill_begin(
             base, ne, base + 16 * ne, nt, N if own else 0, st[2 * N:].data_ptr(), N, _lib.ptr(self.slot2row) if own else None,
             self.slot2row.numel() if own else 0, _lib.ptr(self.last_used) if own else None, _lib.ptr(self._clock) if own else None,
-            self.ssm_state.data_ptr(), _lib.ptr(pool2), _lib.ptr(pos), self.ssm_state.shape[0], self.ssm_state[0].numel(),
+            self.ssm_state.data_ptr(), _lib.ptr(pool2), _lib.ptr(pos), pool_rows, self.ssm_state.numel() // pool_rows,
             _lib.current_stream(dev)), "ix_gdn_prefill_begin")
         if rc != _lib.IX_OK:
             raise RuntimeError(f"[isoexec-gdn] prefill: {N} sequences are more than one launch takes")
